@@ -2,8 +2,8 @@
 library on top of it.
 
 ``python -m autogptq.tvm_amd.build`` compiles ``csrc/*.hip`` and ``csrc/*.cpp`` into
-``csrc/libgptq_hip.so`` (no torch in it), then ``csrc/binding.cpp`` against the installed torch headers into
-``csrc/libgptq_hip_torch.so`` (``torch.ops.gptq_hip.*``).  hipcc cross-compiles without a GPU.
+``csrc/libgptq_hip.so`` (no torch in it), then ``csrc/binding.cpp`` and ``csrc/python_call.cpp`` against the installed torch
+headers into ``csrc/libgptq_hip_torch.so`` (``torch.ops.gptq_hip.*`` and the module call).  hipcc cross-compiles without a GPU.
 """
 from __future__ import annotations
 
@@ -75,18 +75,20 @@ def _compile_one(src: str, obj: str, build_id: str):
 
 
 def build_binding(build_id: str) -> str:
-    """binding.cpp -> libgptq_hip_torch.so: host C++ only (no device code), against torch's headers and
-    libraries, linked to libgptq_hip.so beside it."""
+    """binding.cpp and python_call.cpp -> libgptq_hip_torch.so: host C++ only (no device code), against torch's and
+    Python's headers and libraries, linked to libgptq_hip.so beside it."""
+    import sysconfig
+
     import torch
     from torch.utils import cpp_extension as ce
 
-    inc = [f"-I{d}" for d in ce.include_paths()] + ["-I/opt/rocm/include", f"-I{os.path.join(CSRC, '..', '..', '..', 'include')}"]
+    inc = [f"-I{d}" for d in ce.include_paths()] + [f"-I{sysconfig.get_paths()['include']}", "-I/opt/rocm/include", f"-I{os.path.join(CSRC, '..', '..', '..', 'include')}"]
     tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
     cmd = [hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DGPTQ_HIP_BUILD_ID="{build_id}"',
            "-Wno-deprecated-declarations"] + inc + [
-        os.path.join(CSRC, "binding.cpp"), "-o", BINDING_LIB, f"-L{CSRC}", "-lgptq_hip", f"-L{tlib}", "-lc10", "-lc10_hip",
-        "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-Wl,-rpath,$ORIGIN"]
+        os.path.join(CSRC, "binding.cpp"), os.path.join(CSRC, "python_call.cpp"), "-o", BINDING_LIB, f"-L{CSRC}", "-lgptq_hip",
+        f"-L{tlib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-ltorch", "-Wl,-rpath,$ORIGIN"]
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if r.returncode != 0:
         raise RuntimeError("building the torch operator library failed:\n" + r.stdout)

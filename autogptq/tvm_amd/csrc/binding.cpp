@@ -21,27 +21,13 @@
 #include <optional>
 #include <tuple>
 
-#include "gptq_hip.h"
+#include "binding.h"
 
 #ifndef GPTQ_HIP_BUILD_ID
 #define GPTQ_HIP_BUILD_ID "unknown"
 #endif
 
-namespace {
-
-using at::Tensor;
-using OptTensor = std::optional<Tensor>;
-
-void need(const Tensor &t, const char *name, at::ScalarType dtype, const Tensor &like)
-{
-    TORCH_CHECK(t.is_cuda(), name, " is on ", t.device(), ": the GPTQ kernels run on a ROCm GPU only and there is no CPU fallback");
-    TORCH_CHECK(t.device() == like.device(), name, " is on ", t.device(), ", x on ", like.device());
-    TORCH_CHECK(t.scalar_type() == dtype, name, " must be ", dtype, ", got ", t.scalar_type());
-    TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
-}
-
-const void *ptr(const OptTensor &t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
-bool has(const OptTensor &t) { return t.has_value() && t->defined(); }
+namespace gptq_torch {
 
 void raise(int rc, const char *what, int64_t M, int64_t K, int64_t N, int64_t bits, int64_t gs)
 {
@@ -54,8 +40,8 @@ void raise(int rc, const char *what, int64_t M, int64_t K, int64_t N, int64_t bi
 // kind 1: the decode plans of the tiled family with halved tiles, whose kernel keeps their bytes zero between launches
 // (the slots of the halves): nothing else may write there, so they do not share the workspace the other plans pack x
 // or partial sums into.
-std::mutex g_ws_mutex;
-std::map<std::tuple<int, void *, int>, Tensor> g_ws;
+static std::mutex g_ws_mutex;
+static std::map<std::tuple<int, void *, int>, Tensor> g_ws;
 
 int workspace_kind(const gptq_hip_plan &plan)
 {
@@ -63,7 +49,7 @@ int workspace_kind(const gptq_hip_plan &plan)
     return (plan.flags & GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE) ? 1 : 0;
 }
 
-Tensor workspace(const Tensor &like, size_t nbytes, void *stream, int kind = 0)
+Tensor workspace(const Tensor &like, size_t nbytes, void *stream, int kind)
 {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     Tensor &ws = g_ws[{(int)like.get_device(), stream, kind}];
@@ -72,6 +58,47 @@ Tensor workspace(const Tensor &like, size_t nbytes, void *stream, int kind = 0)
         ws = at::zeros({n}, like.options().dtype(at::kByte));
     }
     return ws;
+}
+
+int Bound::choose()
+{
+    const int rc = kind == 2 ? gptq_hip_select_tiled(M, K, N, bits, group_size, &plan)
+                             : gptq_hip_select(M, K, N, bits, group_size, kind == 0 && has(d), &plan);
+    if (rc != GPTQ_HIP_OK) return rc;
+    ws_need = plan.workspace_bytes;
+    // (what the sorted entry needs beyond its plan, x in the sorted order, it says itself)
+    if (kind == 1) ws_need = std::max(ws_need, gptq_hip_sorted_workspace_bytes(M, K, N, bits, group_size));
+    return rc;
+}
+
+int Bound::launch(const Tensor &x, void *y, void *stream) const
+{
+    Tensor ws;
+    if (ws_need) ws = workspace(x, ws_need, stream, workspace_kind(plan));
+    void *wsp = ws.defined() ? ws.data_ptr() : nullptr;
+    const size_t wsb = ws.defined() ? (size_t)ws.numel() : 0;
+    if (kind == 0)
+        return gptq_hip_gemm_plan(x.data_ptr(), (const int32_t *)a.data_ptr(), (const int32_t *)b.data_ptr(), c.data_ptr(),
+                                  (const int32_t *)ptr(d), ptr(bias), y, wsp, wsb, M, K, N, bits, group_size, &plan, stream);
+    if (kind == 1)
+        return gptq_hip_gemm_sorted(x.data_ptr(), (const int32_t *)a.data_ptr(), (const int32_t *)b.data_ptr(), c.data_ptr(),
+                                    (const int32_t *)ptr(d), ptr(bias), y, wsp, wsb, M, K, N, bits, group_size, &plan, stream);
+    return gptq_hip_gemm_tiled(x.data_ptr(), a.data_ptr(), (const uint32_t *)b.data_ptr(), (const int32_t *)ptr(d),
+                               (const uint16_t *)ptr(e), ptr(bias), y, wsp, wsb, M, K, N, bits, group_size, &plan, stream);
+}
+
+}  // namespace gptq_torch
+
+namespace {
+
+using namespace gptq_torch;
+
+void need(const Tensor &t, const char *name, at::ScalarType dtype, const Tensor &like)
+{
+    TORCH_CHECK(t.is_cuda(), name, " is on ", t.device(), ": the GPTQ kernels run on a ROCm GPU only and there is no CPU fallback");
+    TORCH_CHECK(t.device() == like.device(), name, " is on ", t.device(), ", x on ", like.device());
+    TORCH_CHECK(t.scalar_type() == dtype, name, " must be ", dtype, ", got ", t.scalar_type());
+    TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
 }
 
 struct Shape {
@@ -166,23 +193,22 @@ Tensor gemm_sorted(const Tensor &x, const Tensor &qweight_sorted, const Tensor &
     return y;
 }
 
-Tensor gemm_tiled(const Tensor &x, const Tensor &qtile, const Tensor &sz, const OptTensor &xsrc, const OptTensor &kinv,
-                  const OptTensor &bias, int64_t bits, int64_t group_size)
+// the checks of a layer in the tiled format
+void check_tiled(int64_t K, const Tensor &qtile, const Tensor &sz, const OptTensor &xsrc, const OptTensor &kinv,
+                 const OptTensor &bias, int64_t bits, int64_t group_size, const Tensor &like)
 {
-    TORCH_CHECK(x.is_cuda(), "x is on ", x.device(), ": the GPTQ kernels run on a ROCm GPU only and there is no CPU fallback");
-    need(x, "x", at::kHalf, x);
-    need(qtile, "qtile", at::kInt, x);
-    need(sz, "sz", at::kInt, x);
+    need(qtile, "qtile", at::kInt, like);
+    need(sz, "sz", at::kInt, like);
     TORCH_CHECK(has(xsrc) == has(kinv), "xsrc and kinv go together: pass both (activation order) or neither");
     if (has(xsrc)) {
-        need(*xsrc, "xsrc", at::kInt, x);
-        need(*kinv, "kinv", at::kShort, x);
+        need(*xsrc, "xsrc", at::kInt, like);
+        need(*kinv, "kinv", at::kShort, like);
     }
-    if (has(bias)) need(*bias, "bias", at::kHalf, x);
+    if (has(bias)) need(*bias, "bias", at::kHalf, like);
     TORCH_CHECK(bits == 2 || bits == 3 || bits == 4 || bits == 8, "Only 2, 3, 4, 8 bits are supported.");
-    TORCH_CHECK(x.dim() == 2 && sz.dim() == 2, "x must be [M, K] and sz [G, N]");
-    const int64_t M = x.size(0), K = x.size(1), N = sz.size(1);
-    TORCH_CHECK(M < (1LL << 31) && K <= 65536 && N < (1LL << 31), "layer too large");
+    TORCH_CHECK(sz.dim() == 2, "sz must be [G, N]");
+    const int64_t N = sz.size(1);
+    TORCH_CHECK(K <= 65536 && N < (1LL << 31), "layer too large");
     const int64_t Kp = (K + 63) / 64 * 64;
     TORCH_CHECK(qtile.numel() * 4 == Kp * N * bits / 8, "qtile holds ", qtile.numel() * 4, " bytes, a ", K, " x ", N,
                 " layer of ", bits, " bits needs ", Kp * N * bits / 8);
@@ -190,21 +216,33 @@ Tensor gemm_tiled(const Tensor &x, const Tensor &qtile, const Tensor &sz, const 
         TORCH_CHECK(xsrc->dim() == 1 && xsrc->numel() == Kp && kinv->dim() == 1 && kinv->numel() == K, "xsrc must be [", Kp,
                     "] and kinv [", K, "]");
     if (has(bias)) TORCH_CHECK(bias->dim() == 1 && bias->size(0) == N, "bias must be [", N, "]");
-    Tensor y = at::empty({M, N}, x.options());
-    if (M == 0) return y;
+}
+
+void check_groups(int64_t K, const Tensor &sz, int64_t group_size)
+{
+    TORCH_CHECK(group_size == -1 || group_size > 0, "group_size must be -1 or positive, got ", group_size);
+    TORCH_CHECK(sz.size(0) == (group_size == -1 ? 1 : K / group_size), "sz must have one row per group");
+}
+
+Tensor gemm_tiled(const Tensor &x, const Tensor &qtile, const Tensor &sz, const OptTensor &xsrc, const OptTensor &kinv,
+                  const OptTensor &bias, int64_t bits, int64_t group_size)
+{
+    TORCH_CHECK(x.is_cuda(), "x is on ", x.device(), ": the GPTQ kernels run on a ROCm GPU only and there is no CPU fallback");
+    need(x, "x", at::kHalf, x);
+    TORCH_CHECK(x.dim() == 2, "x must be [M, K]");
+    TORCH_CHECK(x.size(0) < (1LL << 31), "too many rows");
+    check_tiled(x.size(1), qtile, sz, xsrc, kinv, bias, bits, group_size, x);
+    Bound q;
+    q.kind = 2, q.bits = (int)bits, q.group_size = (int)group_size;
+    q.M = (int)x.size(0), q.K = (int)x.size(1), q.N = (int)sz.size(1);
+    q.a = qtile, q.b = sz, q.d = xsrc, q.e = kinv, q.bias = bias;
+    Tensor y = at::empty({q.M, q.N}, x.options());
+    if (q.M == 0) return y;
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     void *stream = (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device()).stream();
-    gptq_hip_plan plan;
-    int rc = gptq_hip_select_tiled((int)M, (int)K, (int)N, (int)bits, (int)group_size, &plan);
-    raise(rc, "gptq_hip_gemm_tiled", M, K, N, bits, group_size);
-    TORCH_CHECK(sz.size(0) == (group_size == -1 ? 1 : K / group_size), "sz must have one row per group");
-    Tensor ws;
-    if (plan.workspace_bytes) ws = workspace(x, plan.workspace_bytes, stream, workspace_kind(plan));
-    rc = gptq_hip_gemm_tiled(x.data_ptr(), qtile.data_ptr(), (const uint32_t *)sz.data_ptr(), (const int32_t *)ptr(xsrc),
-                             (const uint16_t *)ptr(kinv), ptr(bias), y.data_ptr(), ws.defined() ? ws.data_ptr() : nullptr,
-                             ws.defined() ? (size_t)ws.numel() : 0, (int)M, (int)K, (int)N, (int)bits, (int)group_size,
-                             &plan, stream);
-    raise(rc, "gptq_hip_gemm_tiled", M, K, N, bits, group_size);
+    raise(q.choose(), "gptq_hip_gemm_tiled", q.M, q.K, q.N, bits, group_size);
+    check_groups(q.K, sz, group_size);
+    raise(q.launch(x, y.data_ptr(), stream), "gptq_hip_gemm_tiled", q.M, q.K, q.N, bits, group_size);
     return y;
 }
 
@@ -229,90 +267,83 @@ Tensor dequant(const Tensor &qweight, const Tensor &qzeros, const Tensor &scales
     return w;
 }
 
-// One layer's constant tensors, bound once: forward(x) then crosses from Python with a single argument (the
-// argument handling of an eight-argument operator costs more host time than the launch itself).
-// kind: 0 = checkpoint tensors (qweight, qzeros, scales, g_idx?), 1 = sorted copy (qweight_sorted, qzeros,
-// scales, kmap), 2 = tiled copy (qtile, sz, -, xsrc?, kinv?).
-struct Layer : torch::CustomClassHolder {
-    int64_t kind, bits, group_size;
-    Tensor a, b, c;
-    OptTensor d, e, bias;
+}  // namespace
 
-    Layer(int64_t kind_, Tensor a_, Tensor b_, OptTensor c_, OptTensor d_, OptTensor e_, OptTensor bias_, int64_t bits_,
-          int64_t group_size_)
-        : kind(kind_), bits(bits_), group_size(group_size_), a(std::move(a_)), b(std::move(b_)),
-          c(has(c_) ? *c_ : Tensor()), d(std::move(d_)), e(std::move(e_)), bias(std::move(bias_))
+void gptq_torch::check_bound(const Bound &q)
+{
+    TORCH_CHECK(q.M > 0, "M must be positive, got ", q.M);
+    TORCH_CHECK(q.a.is_cuda(), "the layer is on ", q.a.device(), ": the GPTQ kernels run on a ROCm GPU only and there is no CPU fallback");
+    if (q.kind == 2) {
+        TORCH_CHECK(q.b.dim() == 2 && q.b.size(1) == q.N, "sz must be [G, ", q.N, "]");
+        check_tiled(q.K, q.a, q.b, q.d, q.e, q.bias, q.bits, q.group_size, q.a);
+        check_groups(q.K, q.b, q.group_size);
+        return;
+    }
+    need(q.a, "qweight", at::kInt, q.a);
+    need(q.b, "qzeros", at::kInt, q.a);
+    need(q.c, "scales", at::kHalf, q.a);
+    if (has(q.d)) need(*q.d, q.kind == 1 ? "kmap" : "g_idx", at::kInt, q.a);
+    if (has(q.bias)) need(*q.bias, "bias", at::kHalf, q.a);
+    const Shape s = check_layer(Tensor(), q.a, q.b, q.c, q.kind == 0 && has(q.d) ? q.d->numel() : -1, q.bias, q.bits, q.group_size, true);
+    TORCH_CHECK(s.K == q.K && s.N == q.N, "the layer is ", s.K, " x ", s.N, ", not ", q.K, " x ", q.N);
+    if (q.kind == 1) TORCH_CHECK(q.d->dim() == 1 && q.d->numel() == 2 * s.K, "kmap must be [", 2 * s.K, "]");
+}
+
+namespace {
+
+// One layer's constant tensors, bound once: forward(x) then crosses from Python with a single argument (the
+// argument handling of an eight-argument operator costs more host time than the launch itself).  kind as in Bound.
+struct Layer : torch::CustomClassHolder {
+    Bound bound;
+
+    Layer(int64_t kind, Tensor a, Tensor b, OptTensor c, OptTensor d, OptTensor e, OptTensor bias, int64_t bits,
+          int64_t group_size)
     {
         TORCH_CHECK(kind >= 0 && kind <= 2, "kind must be 0 (checkpoint tensors), 1 (sorted copy) or 2 (tiled copy)");
-        TORCH_CHECK(kind == 2 || c.defined(), "scales are missing");
-        TORCH_CHECK(kind != 1 || has(d), "the sorted copy needs its kmap");
+        bound.kind = (int)kind, bound.bits = (int)bits, bound.group_size = (int)group_size;
+        bound.a = std::move(a), bound.b = std::move(b), bound.c = has(c) ? *c : Tensor();
+        bound.d = std::move(d), bound.e = std::move(e), bound.bias = std::move(bias);
+        TORCH_CHECK(kind == 2 || bound.c.defined(), "scales are missing");
+        TORCH_CHECK(kind != 1 || has(bound.d), "the sorted copy needs its kmap");
     }
 
     // What the first fully checked call fixed for its row count: later calls with the same M check x only.
     // Written once, under the mutex, before fast_M is published; calls with another M take the checked path.
     std::atomic<int64_t> fast_M{-1};
-    int64_t K = 0, N = 0;
-    gptq_hip_plan plan{};
-    size_t ws_need = 0;
     std::mutex fix_mutex;
 
     Tensor forward(const Tensor &x)
     {
         const int64_t fast_rows = fast_M.load(std::memory_order_acquire);
+        const Bound &q = bound;
         if (x.dim() == 2 && x.size(0) == fast_rows) {
-            TORCH_CHECK(x.is_cuda() && x.device() == a.device(), "x is on ", x.device(), ", the layer on ", a.device(),
+            TORCH_CHECK(x.is_cuda() && x.device() == q.a.device(), "x is on ", x.device(), ", the layer on ", q.a.device(),
                         ": the GPTQ kernels run on a ROCm GPU only and there is no CPU fallback");
-            TORCH_CHECK(x.scalar_type() == at::kHalf && x.is_contiguous() && x.size(1) == K,
-                        "x must be a contiguous fp16 [M, ", K, "] matrix");
-            Tensor y = at::empty({fast_rows, N}, x.options());
+            TORCH_CHECK(x.scalar_type() == at::kHalf && x.is_contiguous() && x.size(1) == q.K,
+                        "x must be a contiguous fp16 [M, ", q.K, "] matrix");
+            Tensor y = at::empty({fast_rows, q.N}, x.options());
             const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
             void *stream = (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device()).stream();
-            Tensor ws;
-            if (ws_need) ws = workspace(x, ws_need, stream, workspace_kind(plan));
-            void *wsp = ws.defined() ? ws.data_ptr() : nullptr;
-            const size_t wsb = ws.defined() ? (size_t)ws.numel() : 0;
-            const int M = (int)fast_rows, bi = (int)bits, gs = (int)group_size;
-            int rc;
-            if (kind == 0)
-                rc = gptq_hip_gemm_plan(x.data_ptr(), (const int32_t *)a.data_ptr(), (const int32_t *)b.data_ptr(), c.data_ptr(),
-                                        (const int32_t *)ptr(d), ptr(bias), y.data_ptr(), wsp, wsb, M, (int)K, (int)N, bi, gs,
-                                        &plan, stream);
-            else if (kind == 1)
-                rc = gptq_hip_gemm_sorted(x.data_ptr(), (const int32_t *)a.data_ptr(), (const int32_t *)b.data_ptr(),
-                                          c.data_ptr(), (const int32_t *)ptr(d), ptr(bias), y.data_ptr(), wsp, wsb, M, (int)K,
-                                          (int)N, bi, gs, &plan, stream);
-            else
-                rc = gptq_hip_gemm_tiled(x.data_ptr(), a.data_ptr(), (const uint32_t *)b.data_ptr(), (const int32_t *)ptr(d),
-                                         (const uint16_t *)ptr(e), ptr(bias), y.data_ptr(), wsp, wsb, M, (int)K, (int)N, bi, gs,
-                                         &plan, stream);
-            raise(rc, "gptq_hip.Layer.forward", fast_rows, K, N, bits, group_size);
+            raise(q.launch(x, y.data_ptr(), stream), "gptq_hip.Layer.forward", fast_rows, q.K, q.N, q.bits, q.group_size);
             return y;
         }
         // the checked path; what it selects is what the operators select
         Tensor y;
-        switch (kind) {
+        switch (q.kind) {
         case 0:
-            y = gemm(x, a, b, c, d, bias, bits, group_size);
+            y = gemm(x, q.a, q.b, q.c, q.d, q.bias, q.bits, q.group_size);
             break;
         case 1:
-            y = gemm_sorted(x, a, b, c, *d, bias, bits, group_size);
+            y = gemm_sorted(x, q.a, q.b, q.c, *q.d, q.bias, q.bits, q.group_size);
             break;
         default:
-            y = gemm_tiled(x, a, b, d, e, bias, bits, group_size);
+            y = gemm_tiled(x, q.a, q.b, q.d, q.e, q.bias, q.bits, q.group_size);
         }
         if (x.size(0) > 0 && fast_rows < 0) {
-            const int M = (int)x.size(0), Ki = (int)x.size(1), Ni = (int)y.size(1), bi = (int)bits, gs = (int)group_size;
-            gptq_hip_plan p;
-            const int rc = kind == 2 ? gptq_hip_select_tiled(M, Ki, Ni, bi, gs, &p)
-                                     : gptq_hip_select(M, Ki, Ni, bi, gs, kind == 0 && has(d), &p);
             const std::lock_guard<std::mutex> lock(fix_mutex);
-            if (rc == GPTQ_HIP_OK && fast_M.load(std::memory_order_relaxed) < 0) {
-                plan = p;
-                ws_need = p.workspace_bytes;
-                if (kind == 1) ws_need = std::max(ws_need, gptq_hip_sorted_workspace_bytes(M, Ki, Ni, bi, gs));
-                K = Ki;
-                N = Ni;
-                fast_M.store(M, std::memory_order_release);
+            if (fast_M.load(std::memory_order_relaxed) < 0) {
+                bound.M = (int)x.size(0), bound.K = (int)x.size(1), bound.N = (int)y.size(1);
+                if (bound.choose() == GPTQ_HIP_OK) fast_M.store(bound.M, std::memory_order_release);
             }
         }
         return y;

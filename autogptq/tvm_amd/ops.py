@@ -376,12 +376,28 @@ def _meta_dequant(qweight, qzeros, scales, g_idx, bits, group_size):
     return scales.new_empty((qweight.shape[0] * 32 // bits, qweight.shape[1]), dtype=torch.float16)
 
 
+# The module call in C (csrc/python_call.cpp, an extension module in the operator library): BoundCall and install();
+# None without the built library.
+CALL = None
+
+
+def _load_call_module():
+    import importlib.machinery
+    import importlib.util
+
+    loader = importlib.machinery.ExtensionFileLoader("gptq_hip_call", BINDING_PATH)
+    spec = importlib.util.spec_from_file_location("gptq_hip_call", BINDING_PATH, loader=loader)
+    module = importlib.util.module_from_spec(spec)
+    loader.exec_module(module)
+    return module
+
+
 BINDING_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc", "libgptq_hip_torch.so")
 NATIVE_OPS = False   # True when torch.ops.gptq_hip.* are the C++ operators
 
 
 def _register_torch_ops():
-    global NATIVE_OPS
+    global NATIVE_OPS, CALL
     keep = []
     native = False
     if os.path.exists(BINDING_PATH) and os.path.exists(_lib.LIB_PATH):
@@ -397,6 +413,7 @@ def _register_torch_ops():
             raise RuntimeError(f"{BINDING_PATH} was built from other sources ({built}) than the kernel library "
                                f"({_lib.build_id()}): run python -m autogptq.tvm_amd.build")
         NATIVE_OPS = True
+        CALL = _load_call_module()
     else:
         lib = torch.library.Library("gptq_hip", "DEF")
         lib.define("gemm(Tensor x, Tensor qweight, Tensor qzeros, Tensor scales, Tensor? g_idx, Tensor? bias, "

@@ -305,9 +305,9 @@ class QuantLinear(nn.Module):
         bits, gs, bias = self.bits, self.groupsize, self.bias
 
         def bind(kind, a, b, c, d, e):
-            if ops.NATIVE_OPS:
-                # the C++ operator library binds a layer's constant tensors once: one argument per call
-                return torch.classes.gptq_hip.Layer(kind, a, b, c, d, e, bias, bits, gs).forward
+            if ops.CALL is not None:
+                # the operator library binds the layer's constant tensors and the plan for M once: one argument per call
+                return ops.CALL.BoundCall(kind, a, b, c, d, e, bias, bits, gs, M, self.infeatures, self.outfeatures)
             if kind == 0:
                 return lambda x2: t.gemm.default(x2, a, b, c, d, bias, bits, gs)
             if kind == 1:
@@ -382,13 +382,8 @@ class QuantLinear(nn.Module):
         return r
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        # the common case first: a contiguous fp16 matrix, no gradient wanted, a row count seen before and
-        # buffers neither replaced nor written since
-        if x.dim() == 2 and x.dtype is torch.float16 and x.is_contiguous() and not (
-                x.requires_grad and torch.is_grad_enabled()):
-            r = self._routes.get(x.size(0))
-            if r is not None and self._fresh(r):
-                return r[3](x)
+        # (the common case, a contiguous fp16 x whose row count was seen before, does not come here: __call__ is a C
+        # function that runs the bound product itself)
         out_shape = x.shape[:-1] + (self.outfeatures,)
         x2 = x.reshape(-1, x.shape[-1])
         if x2.dtype != torch.float16:
@@ -427,6 +422,12 @@ class QuantLinear(nn.Module):
     def extra_repr(self) -> str:
         return (f"bits={self.bits}, groupsize={self.groupsize}, infeatures={self.infeatures}, "
                 f"outfeatures={self.outfeatures}, bias={self.bias is not None}")
+
+
+if ops.CALL is not None:
+    # the module call of the common case as one C function (csrc/python_call.cpp); it comes back to nn.Module.__call__
+    # and forward for everything else
+    ops.CALL.install(QuantLinear)
 
 
 __all__ = ["QuantLinear"]

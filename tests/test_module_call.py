@@ -1,0 +1,81 @@
+"""QuantLinear's C call (csrc/python_call.cpp): what it takes by itself and what it hands to nn.Module.__call__ give the
+same numbers, and the module's ways of being changed or watched still reach it."""
+import pytest
+import torch
+
+from autogptq.tvm_amd import ops
+from autogptq.tvm_amd.qlinear import QuantLinear
+from tests.parity_util import assert_tight, expected_output, layer
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch.device("cuda:0")
+
+
+@pytest.mark.parametrize("bits,desc_act,M", [(4, False, 1), (3, True, 4), (8, True, 9), (4, True, 40)])
+def test_the_call_in_c_equals_forward(dev, bits, desc_act, M):
+    L = layer(4100 + M, 512, 96, bits, 128, desc_act, M=M, bias=True)
+    q = QuantLinear(bits, 128, 512, 96, True)
+    q.load_state_dict({k: L[k] for k in ("qweight", "qzeros", "scales", "g_idx", "bias")})
+    q = q.to(dev)
+    x = L["x"].to(dev)
+    first = q(x)                                   # no route yet: through nn.Module.__call__
+    assert isinstance(q._routes[M][3], ops.CALL.BoundCall)
+    assert_tight(first, expected_output(L), "first call")
+    shapes = [(M, 512), (1, M, 512), (M, 1, 512), (1, 1, M, 512)] + ([(512,)] if M == 1 else [])
+    for shape in shapes:
+        y = q(x.view(shape))
+        assert y.shape == shape[:-1] + (96,) and y.dtype == torch.float16 and not y.requires_grad
+        assert torch.equal(y.view(M, 96), first)
+    # what it does not take: another dtype, a strided x, a keyword, a gradient
+    assert torch.equal(q(x.float()), first)
+    wide = torch.empty((M, 1024), dtype=torch.float16, device=dev)
+    wide[:, ::2] = x
+    assert torch.equal(q(wide[:, ::2]), first) and torch.equal(q(x=x), first)
+    assert q(x.clone().requires_grad_(True)).requires_grad
+    with torch.no_grad():
+        assert torch.equal(q(x.clone().requires_grad_(True)), first)
+    with pytest.raises(Exception):
+        q(x[:, :256].contiguous())
+    with pytest.raises(RuntimeError, match="no CPU fallback"):
+        q(x.cpu())
+
+
+def test_hooks_replaced_buffers_and_instance_forward_are_seen(dev):
+    L = layer(4150, 512, 96, 4, 128, True, M=2, bias=False)
+    q = QuantLinear(4, 128, 512, 96, False)
+    q.load_state_dict({k: L[k] for k in ("qweight", "qzeros", "scales", "g_idx")})
+    q = q.to(dev)
+    x = L["x"].to(dev)
+    first = q(x)
+    assert torch.equal(q(x), first)
+    seen = []
+    for register in (q.register_forward_hook, torch.nn.modules.module.register_module_forward_hook):
+        h = register(lambda m, i, o: seen.append(m))
+        q(x)
+        h.remove()
+        q(x)
+    h = q.register_forward_pre_hook(lambda m, i: seen.append(m))
+    q(x)
+    h.remove()
+    assert seen == [q, q, q]
+    q.forward = lambda t: "replaced"
+    assert q(x) == "replaced"
+    del q.forward
+
+    class Sub(QuantLinear):
+        def forward(self, t):
+            return "subclass"
+
+    s = Sub(4, 128, 512, 96, False).to(dev)
+    s._routes = dict(q._routes)
+    assert s(x) == "subclass"
+    q.scales.mul_(2)                               # written in place: the copies are made again
+    assert torch.allclose(q(x).float(), 2 * first.float(), rtol=1e-3, atol=1e-3)
+    q._buffers["scales"] = q.scales * 0            # swapped behind the module's back
+    assert float(q(x).abs().max()) == 0.0
