@@ -21,6 +21,7 @@ KERNEL_GROUPED = 2
 KERNEL_STREAM = 3
 KERNEL_TILED = 4
 KERNEL_TILED_DECODE = 5
+KERNEL_PANEL = 6
 
 ABI_SYMBOLS = (
     "gptq_hip_select",
@@ -39,6 +40,7 @@ ABI_SYMBOLS = (
     "gptq_hip_tile_prepare",
     "gptq_hip_select_tiled",
     "gptq_hip_select_tiled_decode",
+    "gptq_hip_select_panel",
     "gptq_hip_select_route",
     "gptq_hip_tiled_transposed_bytes",
     "gptq_hip_tiled_transposed_table_bytes",
@@ -80,6 +82,7 @@ class Plan(ctypes.Structure):
 
 
 PLAN_PRIVATE_ZERO_WORKSPACE = 1
+PANEL_TRANSPOSED, PANEL_ACT_ORDER = 1, 2
 
 COPY_CHECKPOINT, COPY_SORTED, COPY_TILED = 1, 2, 4
 ROUTE_CHECKPOINT, ROUTE_SORTED, ROUTE_TILED, ROUTE_LIBRARY = 0, 1, 2, 3
@@ -166,6 +169,8 @@ def lib() -> ctypes.CDLL:
     l.gptq_hip_select_tiled.argtypes = [i, i, i, i, i, ctypes.POINTER(Plan)]
     l.gptq_hip_select_tiled_decode.restype = i
     l.gptq_hip_select_tiled_decode.argtypes = [i, i, i, i, i, ctypes.POINTER(Plan)]
+    l.gptq_hip_select_panel.restype = i
+    l.gptq_hip_select_panel.argtypes = [i, i, i, i, i, ctypes.c_uint, i, i, ctypes.POINTER(Plan)]
     l.gptq_hip_select_route.restype = i
     l.gptq_hip_select_route.argtypes = [i, i, i, i, i, i, ctypes.c_uint, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(Route)]
     l.gptq_hip_gemm_tiled.restype = i
@@ -218,6 +223,20 @@ def select_tiled(M: int, K: int, N: int, bits: int, group_size: int, decode: boo
     rc = fn(M, K, N, bits, group_size, ctypes.byref(plan))
     if rc != OK:
         raise GptqHipError(rc, f"gptq_hip_select_tiled(M={M}, K={K}, N={N}, bits={bits}, group_size={group_size})")
+    return plan
+
+
+def select_panel(M: int, K: int, N: int, bits: int, group_size: int, act_order: bool, transposed: bool = False,
+                 row_tiles: int = 0, split_k: int = 0):
+    """The plan of the PANEL kernel (gptq_hip_select_panel), or None where the format does not cover the layer or
+    (row_tiles = split_k = 0) another kernel is faster."""
+    plan = Plan()
+    flags = (PANEL_TRANSPOSED if transposed else 0) | (PANEL_ACT_ORDER if act_order else 0)
+    rc = lib().gptq_hip_select_panel(M, K, N, bits, group_size, flags, row_tiles, split_k, ctypes.byref(plan))
+    if rc == ERR_UNSUPPORTED:
+        return None
+    if rc != OK:
+        raise GptqHipError(rc, f"gptq_hip_select_panel(M={M}, K={K}, N={N}, bits={bits}, group_size={group_size})")
     return plan
 
 

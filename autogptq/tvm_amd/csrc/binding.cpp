@@ -62,8 +62,14 @@ Tensor workspace(const Tensor &like, size_t nbytes, void *stream, int kind)
 
 int Bound::choose()
 {
-    const int rc = kind == 2 ? gptq_hip_select_tiled(M, K, N, bits, group_size, &plan)
-                             : gptq_hip_select(M, K, N, bits, group_size, kind == 0 && has(d), &plan);
+    int rc = GPTQ_HIP_ERR_UNSUPPORTED;
+    if (kind == 2) {
+        // long prompts: the panel kernel where the library says it is the faster one, else the family's own plan
+        rc = gptq_hip_select_panel(M, K, N, bits, group_size, has(d) ? GPTQ_HIP_PANEL_ACT_ORDER : 0, 0, 0, &plan);
+        if (rc == GPTQ_HIP_ERR_UNSUPPORTED) rc = gptq_hip_select_tiled(M, K, N, bits, group_size, &plan);
+    } else {
+        rc = gptq_hip_select(M, K, N, bits, group_size, kind == 0 && has(d), &plan);
+    }
     if (rc != GPTQ_HIP_OK) return rc;
     ws_need = plan.workspace_bytes;
     // (what the sorted entry needs beyond its plan, x in the sorted order, it says itself)

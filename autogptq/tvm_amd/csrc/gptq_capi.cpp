@@ -307,6 +307,29 @@ extern "C" int gptq_hip_tile_prepare(const int32_t *qweight, const int32_t *qzer
                                      sz, xsrc, kinv, K, N, K / gs, bits, gs, stream);
 }
 
+// The PANEL kernel: the plan must be one it runs, sized for this problem.
+static int run_panel(const void *x, const void *qtile, const uint32_t *sz, const int32_t *xsrc, const void *bias, void *y,
+                     void *workspace, size_t workspace_bytes, int M, int K, int N, int bits, int gs, bool trans,
+                     const gptq_hip_plan &plan, void *stream)
+{
+    const int S_total = ((trans ? N : K) + 63) / 64, cols = trans ? K : N, rt = plan.row_tiles;
+    if (rt < 1 || rt > gptq::kPanelMaxTiles) return GPTQ_HIP_ERR_UNSUPPORTED;
+    if (plan.waves_n != 4 || plan.waves_k != gptq::panel_waves_k(rt) || plan.block != 256 * plan.waves_k || plan.split_k < 1 || plan.k_chunk < 1 || plan.m_blocks < 1 ||
+        plan.grid_x != (cols + gptq::kPanelCols - 1) / gptq::kPanelCols || plan.grid_y != plan.split_k ||
+        plan.grid_z != plan.m_blocks || plan.m_blocks != (M + 32 * rt - 1) / (32 * rt) ||
+        plan.split_k != (S_total + plan.k_chunk - 1) / plan.k_chunk || plan.lds_bytes != gptq::panel_lds_bytes(bits, rt))
+        return GPTQ_HIP_ERR_BAD_ARG;
+    if ((long long)plan.grid_x * plan.m_blocks >= (1LL << 31)) return GPTQ_HIP_ERR_UNSUPPORTED;
+    if (plan.split_k > 1 && (long long)M * cols >= (1LL << 32)) return GPTQ_HIP_ERR_UNSUPPORTED;
+    const size_t part = plan.split_k > 1 ? ((size_t)plan.split_k * M * cols * sizeof(float) + 255) / 256 * 256 : 0;
+    // x in the order of the copy, or the transposed product's result before its channels are put in order
+    const size_t xb = xsrc && (!trans || (plan.split_k == 1 && gptq::panel_scatters(M, K))) ? (size_t)M * K * 2 : 0;
+    if (part + xb > 0 && (!workspace || !aligned(workspace, 16) || workspace_bytes < gptq::kCounterBytes + part + xb))
+        return GPTQ_HIP_ERR_WORKSPACE;
+    char *ws = (char *)workspace + gptq::kCounterBytes;
+    return gptq::launch_panel(x, qtile, sz, xsrc, bias, y, ws + part, (float *)ws, M, K, N, bits, gs, trans, plan, stream);
+}
+
 extern "C" int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint32_t *sz, const int32_t *xsrc,
                                    const uint16_t *kinv, const void *bias, void *y, void *workspace,
                                    size_t workspace_bytes, int M, int K, int N, int bits, int group_size,
@@ -381,6 +404,8 @@ extern "C" int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint3
         }
         return gptq::launch_tiled_decode(x, qtile, sz, kinv, bias, y, part, slots, M, K, N, G_all, bits, gs, *plan, stream);
     }
+    if (plan->kernel == GPTQ_HIP_KERNEL_PANEL)
+        return run_panel(x, qtile, sz, xsrc, bias, y, workspace, workspace_bytes, M, K, N, bits, gs, false, *plan, stream);
     // the plan must be one this family runs, sized for this problem
     const int rts = plan->row_tiles;  // 32-row tiles per workgroup
     const int S_total = (K + 63) / 64;
@@ -451,6 +476,8 @@ extern "C" int gptq_hip_gemm_tiled_transposed(const void *gy, const void *qtile_
         if (rc != GPTQ_HIP_OK) return rc;
         plan = &chosen;
     }
+    if (plan->kernel == GPTQ_HIP_KERNEL_PANEL)
+        return run_panel(gy, qtile_t, szt, xsrc, nullptr, gx, workspace, workspace_bytes, M, K, N, bits, gs, true, *plan, stream);
     // the plan must be one this product runs, sized for this problem
     const int rts = plan->row_tiles, kwv = 4;
     const int S_total = (N + 63) / 64;

@@ -680,6 +680,96 @@ extern "C" int gptq_hip_select_tiled_transposed(int M, int K, int N, int bits, i
 
 namespace {
 
+// Microseconds of the PANEL kernel (its reduce pass included): turns of the chip, each as long as a workgroup's walk.  Fitted to
+// 4000 measurements (3 to 8 sizes of M each on sixteen layers of 1024 to 32768 columns, both products, all widths, one to eight
+// row tiles, one to eight K ranges): 8 % rms, and the plan it names best is 1 % slower than the fastest one on average.  What
+// a step costs besides its matrix instructions (the constant of the first line) is the dequantisation, which every workgroup
+// does for its columns; a turn that is not full runs at a higher clock.
+double panel_us(int rt, int split, int chunk, long long wgs, int bits, double out_elems)
+{
+    const double step = (rt <= 4 ? 0.295 + 0.100 * rt : 0.281 + 0.131 * rt) + (bits == 8 ? 0.01 : (bits == 3 ? 0.07 : 0.0));
+    auto turn = [&](double n) { return chunk * step * (0.79 + 0.21 * n / 256) + 2.7 + 0.71 * rt; };
+    const long long full = wgs / 256, last = wgs % 256;
+    return 4.8 + full * turn(256) + (last ? turn((double)last) : 0.0) + (split > 1 ? 2.2 + 0.86e-6 * split * out_elems : 0.0);
+}
+
+// The same for the matmul kernel's plan (the tables above), 9 % rms over the same layers.
+double tiled_us(const gptq_hip_plan &p, int bits, bool transposed, double out_elems, double in_elems, bool act_order)
+{
+    double step = p.waves_n == 2 ? 2.26 : (p.row_tiles == 1 ? 0.57 : (p.row_tiles == 2 ? 0.79 : 1.32));
+    if (transposed) step *= 1.38;
+    if (bits == 8) step *= 1.5;
+    auto turn = [&](double n) { return p.k_chunk * step * (0.345 + 0.655 * n / 256) + 2.0; };
+    const long long wgs = (long long)p.grid_x * p.grid_y * p.m_blocks, full = wgs / 256, last = wgs % 256;
+    return 4.4 + full * turn(256) + (last ? turn((double)last) : 0.0) + (p.split_k > 1 ? 4.2 + 0.66e-6 * p.split_k * out_elems : 0.0) +
+           (2.9 + 0.4 * act_order) * 1e-6 * in_elems;
+}
+
+}  // namespace
+
+extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_size, unsigned flags, int row_tiles, int split_k,
+                                     gptq_hip_plan *plan)
+{
+    const int ok = tiled_args_ok(M, K, N, bits, group_size, plan);
+    if (ok != GPTQ_HIP_OK) return ok;
+    if ((flags & ~(GPTQ_HIP_PANEL_TRANSPOSED | GPTQ_HIP_PANEL_ACT_ORDER)) || row_tiles < 0 || split_k < 0) return GPTQ_HIP_ERR_BAD_ARG;
+    if ((long long)((K + 63) / 64 * 64) * ((N + 63) / 64 * 64) * bits / 8 >= (1LL << 32)) return GPTQ_HIP_ERR_UNSUPPORTED;
+    const bool transposed = flags & GPTQ_HIP_PANEL_TRANSPOSED, act = flags & GPTQ_HIP_PANEL_ACT_ORDER;
+    const int red = transposed ? N : K, cols = transposed ? K : N;
+    const int S_total = ceil_div(red, 64), col_wgs = ceil_div(cols, gptq::kPanelCols);
+    const double out_elems = (double)M * cols;
+    int rt = row_tiles, split = split_k;
+    if (rt == 0 || split == 0) {
+        if (M <= gptq::kDecodeMaxRows && rt == 0 && split == 0) return GPTQ_HIP_ERR_UNSUPPORTED;   // (the decode kernels' rows)
+        double best = 1e30;
+        for (int r = 1; r <= gptq::kPanelMaxTiles; r++) {
+            if (row_tiles ? r != row_tiles : r > 1 && 32 * (r - 1) >= M) continue;
+            const long long tiles = (long long)col_wgs * ceil_div(M, 32 * r);
+            for (int s = 1; s <= 8; s++) {
+                if (split_k ? s != split_k : s > 1 && (S_total / s < 6 || tiles * s > 768 || s * out_elems > 48e6)) continue;
+                const int chunk = ceil_div(S_total, s);
+                if (ceil_div(S_total, chunk) != s) continue;
+                const double us = panel_us(r, s, chunk, tiles * s, bits, out_elems);
+                if (us < best) best = us, rt = r, split = s;
+            }
+        }
+        if (rt == 0 || split == 0) return GPTQ_HIP_ERR_UNSUPPORTED;
+        if (row_tiles == 0 && split_k == 0) {
+            // an activation order: a pass that puts x (or the result) in the layer's order
+            if (act) best += transposed ? 2.5 + 0.9e-6 * M * K : 3.5 + 0.7e-6 * M * K;
+            gptq_hip_plan other;
+            const int rc = transposed ? gptq_hip_select_tiled_transposed(M, K, N, bits, group_size, &other)
+                                      : gptq_hip_select_tiled(M, K, N, bits, group_size, &other);
+            if (rc == GPTQ_HIP_OK && other.kernel != GPTQ_HIP_KERNEL_TILED) return GPTQ_HIP_ERR_UNSUPPORTED;
+            // (short prompts have other copies to run on, too: there the matmul kernel has to be clearly the slower one)
+            if (rc == GPTQ_HIP_OK &&
+                best > (M <= 128 ? 0.95 : 1.0) * tiled_us(other, bits, transposed, out_elems, (double)M * red, act))
+                return GPTQ_HIP_ERR_UNSUPPORTED;
+        }
+    }
+    if (rt > gptq::kPanelMaxTiles) return GPTQ_HIP_ERR_UNSUPPORTED;
+    const int m_blocks = ceil_div(M, 32 * rt);
+    plan->kernel = GPTQ_HIP_KERNEL_PANEL;
+    plan->row_tiles = rt;
+    plan->m_blocks = m_blocks;
+    plan->waves_n = 4;
+    plan->waves_k = gptq::panel_waves_k(rt);
+    plan->k_chunk = ceil_div(S_total, split);
+    plan->split_k = ceil_div(S_total, plan->k_chunk);
+    plan->grid_x = col_wgs;
+    plan->grid_y = plan->split_k;
+    plan->grid_z = m_blocks;
+    plan->block = 256 * gptq::panel_waves_k(rt);
+    plan->lds_bytes = gptq::panel_lds_bytes(bits, rt);
+    size_t ws = gptq::kCounterBytes;
+    if (plan->split_k > 1) ws += ((size_t)plan->split_k * M * cols * sizeof(float) + 255) / 256 * 256;
+    if (act) ws += ((size_t)M * K * 2 + 255) / 256 * 256;   // x, or the transposed product's result, in the copy's order
+    plan->workspace_bytes = plan->split_k > 1 || act ? ws : 0;
+    return GPTQ_HIP_OK;
+}
+
+namespace {
+
 // Where the tiled kernels were measured faster than the ones that read the checkpoint layout or its channel-sorted
 // copy, on MI355X with the weights cold (us per call, graph replay, group size 128 unless said):
 //   * up to 4 rows, layers of up to 4096 columns (decode kernel with a workgroup per 16 columns, or every tile in two

@@ -269,6 +269,31 @@ int launch_tile_prepare_t(const uint32_t *qweight, const uint32_t *qzeros, const
 int launch_tiled_t(const void *gy, const void *qtile_t, const uint32_t *szt, const int32_t *xsrc, void *gx, char *xpack,
                    float *partial, int M, int K, int N, int bits, int group_size, const gptq_hip_plan &plan,
                    void *stream);
+
+// ---- PANEL kernel (the same layer, long prompts and training batches) -------------------------------
+// A workgroup takes 32 rt rows x 256 columns.  Up to four row tiles: two groups of four waves, each with every other block
+// of K (eight waves of 256 registers); more of them leave a SIMD room for one wave.
+constexpr int kPanelCols = 256, kPanelMaxTiles = 8;
+constexpr int panel_waves_k(int rt) { return rt <= 4 ? 2 : 1; }
+// LDS of a block of 64 positions: x, and the words and (scale, zero) entries of eight column tiles; three blocks per wave
+// group (two where three do not fit) are on their way or in use
+constexpr int panel_tile_bytes(int bits) { return bits == 3 ? 1024 : 256 * bits; }   // (three words per lane take the place of four)
+constexpr int panel_block_bytes(int bits, int rt) { return rt * 4096 + 8 * (panel_tile_bytes(bits) + 256); }
+constexpr int panel_stages(int bits, int rt) { return 3 * panel_waves_k(rt) * panel_block_bytes(bits, rt) <= 160 * 1024 ? 3 : 2; }
+constexpr int panel_lds_bytes(int bits, int rt)
+{
+    // (or what the result is added up and turned around in)
+    const int stages = panel_stages(bits, rt) * panel_waves_k(rt) * panel_block_bytes(bits, rt);
+    const int turn = (panel_waves_k(rt) - 1) * 65536 + 4 * panel_waves_k(rt) * 32 * 272;
+    return stages > turn ? stages : turn;
+}
+// rows x channels from which the transposed product puts its result's channels in order in a pass (2.5 us and 0.9 us per
+// million, against 3.7 us per million for scattered stores)
+inline bool panel_scatters(int M, int K) { return (long long)M * K >= (1LL << 20); }
+int launch_panel(const void *x, const void *qtile, const uint32_t *sz, const int32_t *xsrc, const void *bias, void *y,
+                 void *xs, float *partial, int M, int K, int N, int bits, int group_size, bool trans, const gptq_hip_plan &plan,
+                 void *stream);
+
 int launch_tiled(const void *x, const void *qtile, const uint32_t *sz, const int32_t *xsrc, const void *bias, void *y,
                  char *xpack, float *partial, int M, int K, int N, int G, int bits, int group_size,
                  const gptq_hip_plan &plan, void *stream);

@@ -160,6 +160,34 @@ __device__ __forceinline__ void tile_magic(uint32_t (&mg)[TileCodec<BITS>::KINDS
     for (int k = 0; k < TileCodec<BITS>::KINDS; k++) mg[k] = opaque_vgpr(TileCodec<BITS>::MAGIC[k]);
 }
 
+// One B operand: positions 8 j .. 8 j + 7 of the lane, as fp16(scale * (q - zero)) exactly as the
+// reference rounds it: (base + q) - (base + zero) is exact, the product rounds once.
+template <int BITS>
+__device__ __forceinline__ h8 tiled_bop(const uint32_t (&w)[BITS], int j, h2 s2, const h2 (&zb)[TileCodec<BITS>::KINDS],
+                                        const uint32_t (&mg)[TileCodec<BITS>::KINDS])
+{
+    u4 q;
+    TileCodec<BITS>::operand(w, j, q, mg);
+    u4 o;
+#pragma unroll
+    for (int r = 0; r < 4; r++) o[r] = as_u32((as_h2(q[r]) - zb[r % TileCodec<BITS>::KINDS]) * s2);
+    return __builtin_bit_cast(h8, o);
+}
+
+// The same for the transposed product, where the eight values of an operand are eight COLUMNS of the layer at one
+// position: scale and (base + zero) differ per value and come as ready-made register pairs.
+template <int BITS>
+__device__ __forceinline__ h8 tiled_bop_t(const uint32_t (&w)[BITS], int j, const u4 &s2, const u4 &zb,
+                                          const uint32_t (&mg)[TileCodec<BITS>::KINDS])
+{
+    u4 q;
+    TileCodec<BITS>::operand(w, j, q, mg);
+    u4 o;
+#pragma unroll
+    for (int r = 0; r < 4; r++) o[r] = as_u32((as_h2(q[r]) - as_h2(zb[r])) * as_h2(s2[r]));
+    return __builtin_bit_cast(h8, o);
+}
+
 // ---- shared by the two decode kernels ----
 typedef float f2 __attribute__((ext_vector_type(2)));
 

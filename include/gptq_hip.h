@@ -50,7 +50,7 @@ enum {
                                    workgroup of waves_k = 4 waves along K, m_blocks row blocks along grid_z
                                    (k_chunk = blocks of 64 channels per wave); x is pre-packed into the
                                    workspace; split_k > 1 adds a reduce launch */
-    GPTQ_HIP_KERNEL_TILED_DECODE = 5 /* the same layer for M <= 8 rows, x staged in LDS in the layer's sorted order,
+    GPTQ_HIP_KERNEL_TILED_DECODE = 5, /* the same layer for M <= 8 rows, x staged in LDS in the layer's sorted order,
                                    scales applied per 32 or 64 channels; row_tiles = the rows the kernel is built
                                    for (1, 2, 4 or 8; 8 with waves_n = 1 and at most 8 waves only).  waves_n = 1: a workgroup per 32 columns, waves_k (4, 8 or 16)
                                    waves along K with k_chunk blocks of 64 channels each; split_k > 1 (an x that
@@ -58,6 +58,9 @@ enum {
                                    out evenly over grid_x workgroups of 16 waves, all of K staged per workgroup
                                    (k_chunk = blocks of 128 channels per unit and wave); chosen for layers of up to
                                    4096 columns and fewer than 4096 channels */
+    GPTQ_HIP_KERNEL_PANEL = 6 /* the same layer for long prompts and training batches: a workgroup of four waves takes
+                                   32 * row_tiles rows (shared in LDS) x 256 columns (64 per wave), k_chunk blocks of 64
+                                   channels; grid_x column and m_blocks row positions; split_k > 1 adds a reduce launch */
 };
 
 /* What the dispatcher decided for one problem; filled by gptq_hip_select. */
@@ -217,6 +220,16 @@ int gptq_hip_tile_prepare(const int32_t *qweight, const int32_t *qzeros, const v
 /* The plan of the TILED family for a problem (workspace_bytes included); takes the place of the reference's
  * tile table per M bucket (pycuda_warpper.py:77-127,150-189). */
 int gptq_hip_select_tiled(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan);
+
+/* The plan of the PANEL kernel on the same copy, or (flags: transposed) on the transposed copy below, for
+ * gptq_hip_gemm_tiled / gptq_hip_gemm_tiled_transposed.  row_tiles and split_k: 0 = the planner's choice; with both 0 it answers
+ * GPTQ_HIP_ERR_UNSUPPORTED where the family's other kernels are faster.  No counterpart in the reference. */
+enum {
+    GPTQ_HIP_PANEL_TRANSPOSED = 1,
+    GPTQ_HIP_PANEL_ACT_ORDER = 2   /* the layer has an activation order: the workspace holds x (or gx) in the copy's order */
+};
+int gptq_hip_select_panel(int M, int K, int N, int bits, int group_size, unsigned flags, int row_tiles, int split_k,
+                          gptq_hip_plan *plan);
 
 /* The plan of the family's decode kernel (GPTQ_HIP_KERNEL_TILED_DECODE), M <= 8 rows (GPTQ_HIP_ERR_UNSUPPORTED
  * above); gptq_hip_select_tiled chooses it by itself up to 4 rows, and up to 8 for K <= 11008, the matmul kernel above.  No counterpart in the reference, whose

@@ -1,0 +1,140 @@
+"""GPU parity of the PANEL kernel (long prompts and training batches on the tiled copy, and the transposed product) against
+the CPU oracle's dequantised weight, at the edges of its tiles, and the plans of gptq_hip_select_panel."""
+import ctypes
+
+import pytest
+import torch
+
+from autogptq.tvm_amd import _lib, ops
+from autogptq.tvm_amd.qlinear import QuantLinear
+from tests.parity_util import assert_close, assert_tight, expected_output, expected_weight, layer, to_dev
+
+
+@pytest.fixture(scope="module")
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch.device("cuda:0")
+
+
+def forward(D, plan, out=None):
+    g = D["g_idx"] if D["desc_act"] else None
+    qtile, sz, xsrc, kinv = ops.tile_prepare(D["qweight"], D["qzeros"], D["scales"], g, D["bits"], D["group_size"])
+    if g is None:
+        xsrc = kinv = None
+    return ops.gemm_tiled(D["x"], qtile, sz, xsrc, kinv, D.get("bias"), D["bits"], D["group_size"], plan=plan, out=out)
+
+
+def transposed(D, gy, plan):
+    g = D["g_idx"] if D["desc_act"] else None
+    xsrc = None if g is None else ops.tile_prepare(D["qweight"], D["qzeros"], D["scales"], g, D["bits"], D["group_size"])[2]
+    qtile_t, szt = ops.tile_prepare_transposed(D["qweight"], D["qzeros"], D["scales"], xsrc, D["bits"], D["group_size"])
+    return ops.gemm_tiled_transposed(gy, qtile_t, szt, xsrc, D["K"], D["bits"], D["group_size"], plan=plan)
+
+
+# K: an odd count of blocks, half a block at the end, fewer blocks than stages; N: less than a wave's columns, one column tile
+# past a workgroup; groups of one and of three lane blocks, and one for the layer; rows one short of and one past a row tile
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("K,N,gs,M", [(32, 32, 32, 9), (96, 96, 96, 33), (192, 288, 32, 65), (352, 320, 32, 127), (288, 544, 96, 130),
+                                      (1024, 416, -1, 257)])
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_panel_edges_both_products(dev, bits, K, N, gs, M, desc_act):
+    L = layer(9400 + K + N, K, N, bits, gs, desc_act, M=M, bias=True)
+    D = to_dev(L, dev)
+    gy = torch.randn(M, N, generator=torch.Generator().manual_seed(M)).half()
+    want, want_t = expected_output(L), gy.float() @ expected_weight(L).float().t()
+    for rt, split in ((1, 1), (2, 1), (3, 2), (5, 1), (8, 3)):
+        what = f"panel int{bits} {K}x{N} gs={gs} act={desc_act} M={M} row tiles {rt} ranges {split}"
+        y = forward(D, _lib.select_panel(M, K, N, bits, gs, desc_act, False, rt, split))
+        assert_close(y, want, what)
+        assert_tight(y, want, what)
+        gx = transposed(D, gy.to(dev), _lib.select_panel(M, K, N, bits, gs, desc_act, True, rt, split))
+        assert_close(gx, want_t, "transposed " + what)
+        assert_tight(gx, want_t, "transposed " + what)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits,rt,split", [(4, r, 1) for r in range(1, 9)] + [(8, 4, 2), (8, 8, 1), (3, 4, 3), (2, 7, 2)])
+def test_panel_every_height_on_a_longer_walk(dev, bits, rt, split):
+    # enough blocks for every stage to be used again, several row and column positions, rows past the end in the last one,
+    # the result's channels put in order by the product itself (few rows) and in a pass (many)
+    K, N, gs = 1600, 800, 64
+    for M in (32 * rt + 5, 64 * rt + 600):
+        L = layer(9500 + rt, K, N, bits, gs, True, M=M, bias=True)
+        D = to_dev(L, dev)
+        plan = _lib.select_panel(M, K, N, bits, gs, True, False, rt, split)
+        want = expected_output(L)
+        y = forward(D, plan)
+        assert_close(y, want, f"panel rt={rt} M={M}")
+        assert_tight(y, want, f"panel rt={rt} M={M}")
+        assert torch.equal(y, forward(D, plan)), "two identical calls differ"
+        gy = torch.randn(M, N, generator=torch.Generator().manual_seed(M)).half()
+        gx = transposed(D, gy.to(dev), _lib.select_panel(M, K, N, bits, gs, True, True, rt, split))
+        assert_tight(gx, gy.float() @ expected_weight(L).float().t(), f"panel transposed rt={rt} M={M}")
+
+
+@pytest.mark.gpu
+def test_panel_keeps_to_its_output_and_rejects_other_plans(dev):
+    M, K, N = 70, 512, 96
+    L = layer(9600, K, N, 4, 128, True, M=M)
+    D = to_dev(L, dev)
+    plan = _lib.select_panel(M, K, N, 4, 128, True, False, 2, 1)
+    buf = torch.full((4096 + M * N + 4096,), 1234.0, dtype=torch.float16, device=dev)
+    out = buf[4096: 4096 + M * N].view(M, N)
+    forward(D, plan, out=out)
+    assert_close(out, expected_output(L), "guarded out")
+    assert bool((buf[:4096] == 1234.0).all()) and bool((buf[4096 + M * N:] == 1234.0).all())
+    lib, fake, null = _lib.lib(), ctypes.c_void_p(0x1000), ctypes.c_void_p(None)
+
+    def call(p, m=M, ws=fake):
+        return lib.gptq_hip_gemm_tiled(fake, fake, fake, fake, fake, null, fake, ws, 1 << 24, m, K, N, 4, 128, ctypes.byref(p), null)
+
+    assert call(plan, ws=null) == _lib.ERR_WORKSPACE
+    assert call(plan, m=M + 64) == _lib.ERR_BAD_ARG                      # sized for other rows
+    for field, value in (("block", 256), ("lds_bytes", 1024), ("grid_x", 2), ("k_chunk", 3), ("waves_k", 1)):
+        p = _lib.select_panel(M, K, N, 4, 128, True, False, 2, 1)
+        setattr(p, field, value)
+        assert call(p) == _lib.ERR_BAD_ARG, field
+    p = _lib.select_panel(M, K, N, 4, 128, True, False, 2, 1)
+    p.row_tiles = 9
+    assert call(p) == _lib.ERR_UNSUPPORTED
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_module_runs_long_batches_and_their_gradient_on_the_panel_kernel(dev, desc_act):
+    K, N, gs, M = 2048, 4128, 128, 1300
+    L = layer(9700, K, N, 4, gs, desc_act, M=M, bias=True)
+    q = QuantLinear(4, gs, K, N, True)
+    q.load_state_dict({k: L[k] for k in ("qweight", "qzeros", "scales", "g_idx", "bias")})
+    q = q.to(dev)
+    assert q.route(M) == "library" and q._tiled[1] is not None        # past the switch, on the tiled copy all the same
+    x = L["x"].to(dev).requires_grad_(True)
+    y = q(x)
+    assert_close(y.detach(), expected_output(L), "module")
+    assert_tight(y.detach(), expected_output(L), "module")
+    gy = torch.randn(M, N, generator=torch.Generator().manual_seed(3)).half()
+    y.backward(gy.to(dev))
+    assert_tight(x.grad, gy.float() @ expected_weight(L).float().t(), "module gradient")
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+def test_panel_plans_cover_the_problem(bits):
+    for M, K, N in ((129, 4096, 4096), (333, 5120, 3424), (2000, 9216, 9216), (4096, 8192, 28672), (700, 32, 32), (500, 36864, 96)):
+        for tr in (False, True):
+            red, cols = (N, K) if tr else (K, N)
+            for rt in range(1, 9):
+                p = _lib.select_panel(M, K, N, bits, -1 if K < 128 else 128, True, tr, rt, 2)
+                assert p.kernel == _lib.KERNEL_PANEL and p.row_tiles == rt and p.m_blocks * 32 * rt >= M
+                assert p.grid_x * 256 >= cols and p.split_k * p.k_chunk * 64 >= red > (p.split_k - 1) * p.k_chunk * 64
+                assert p.block == 256 * p.waves_k and p.lds_bytes <= 160 * 1024
+                assert p.workspace_bytes >= 16384 + 2 * M * K + (4 * p.split_k * M * cols if p.split_k > 1 else 0)
+    # short calls and small layers stay with the other kernels; long ones do not
+    assert _lib.select_panel(8, 4096, 11008, bits, 128, False) is None
+    assert _lib.select_panel(300, 1024, 416, bits, 128, False) is None
+    assert _lib.select_panel(512, 4096, 11008, bits, 128, True) is not None
+    assert _lib.select_panel(512, 4096, 11008, bits, 128, True, transposed=True) is not None
+    assert _lib.select_panel(512, 4096, 11008, bits, 16, True) is None
+    with pytest.raises(_lib.GptqHipError):
+        _lib.select_panel(512, 4096, 11008, 5, 128, True)
