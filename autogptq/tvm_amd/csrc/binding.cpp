@@ -35,13 +35,13 @@ void raise(int rc, const char *what, int64_t M, int64_t K, int64_t N, int64_t bi
                 ") failed: ", gptq_hip_strerror(rc), " [status ", rc, "]");
 }
 
-// One workspace per (device, stream) and kind; a replaced one stays alive until the process ends only if a caller
-// still holds it (the allocator keeps it valid for work already queued on its stream).
+// One workspace per (device, stream) and kind (a replaced one stays valid for the work already queued on its stream: the
+// allocator gives its memory to that stream only).
 // kind 1: the decode plans of the tiled family with halved tiles, whose kernel keeps their bytes zero between launches
 // (the slots of the halves): nothing else may write there, so they do not share the workspace the other plans pack x
 // or partial sums into.
-static std::mutex g_ws_mutex;
-static std::map<std::tuple<int, void *, int>, Tensor> g_ws;
+static std::mutex g_ws_mutex;   // of the map; its entries stay where they are
+static std::map<std::tuple<int, void *, int>, Workspace> g_ws;
 
 int workspace_kind(const gptq_hip_plan &plan)
 {
@@ -49,15 +49,18 @@ int workspace_kind(const gptq_hip_plan &plan)
     return (plan.flags & GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE) ? 1 : 0;
 }
 
-Tensor workspace(const Tensor &like, size_t nbytes, void *stream, int kind)
+WorkspaceLease::WorkspaceLease(const Tensor &like, size_t nbytes, void *stream, int kind)
 {
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
-    Tensor &ws = g_ws[{(int)like.get_device(), stream, kind}];
-    if (!ws.defined() || (size_t)ws.numel() < nbytes) {
-        const int64_t n = (int64_t)std::max(nbytes, (size_t)1 << 20);
-        ws = at::zeros({n}, like.options().dtype(at::kByte));
+    if (nbytes == 0) return;
+    {
+        const std::lock_guard<std::mutex> lock(g_ws_mutex);
+        ws = &g_ws[{(int)like.get_device(), stream, kind}];
     }
-    return ws;
+    held = std::unique_lock<std::mutex>(ws->busy);
+    if (!ws->bytes.defined() || (size_t)ws->bytes.numel() < nbytes) {
+        const int64_t n = (int64_t)std::max(nbytes, (size_t)1 << 20);
+        ws->bytes = at::zeros({n}, like.options().dtype(at::kByte));
+    }
 }
 
 int Bound::choose()
@@ -79,10 +82,9 @@ int Bound::choose()
 
 int Bound::launch(const Tensor &x, void *y, void *stream) const
 {
-    Tensor ws;
-    if (ws_need) ws = workspace(x, ws_need, stream, workspace_kind(plan));
-    void *wsp = ws.defined() ? ws.data_ptr() : nullptr;
-    const size_t wsb = ws.defined() ? (size_t)ws.numel() : 0;
+    const WorkspaceLease ws(x, ws_need, stream, workspace_kind(plan));
+    void *wsp = ws.data();
+    const size_t wsb = ws.size();
     if (kind == 0)
         return gptq_hip_gemm_plan(x.data_ptr(), (const int32_t *)a.data_ptr(), (const int32_t *)b.data_ptr(), c.data_ptr(),
                                   (const int32_t *)ptr(d), ptr(bias), y, wsp, wsb, M, K, N, bits, group_size, &plan, stream);
@@ -157,11 +159,10 @@ Tensor gemm(const Tensor &x, const Tensor &qweight, const Tensor &qzeros, const 
     gptq_hip_plan plan;
     int rc = gptq_hip_select((int)s.M, (int)s.K, (int)s.N, (int)bits, (int)group_size, has(g_idx), &plan);
     raise(rc, "gptq_hip_gemm", s.M, s.K, s.N, bits, group_size);
-    Tensor ws;
-    if (plan.workspace_bytes) ws = workspace(x, plan.workspace_bytes, stream);
+    const WorkspaceLease ws(x, plan.workspace_bytes, stream);
     rc = gptq_hip_gemm_plan(x.data_ptr(), (const int32_t *)qweight.data_ptr(), (const int32_t *)qzeros.data_ptr(),
                             scales.data_ptr(), (const int32_t *)ptr(g_idx), ptr(bias), y.data_ptr(),
-                            ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? (size_t)ws.numel() : 0, (int)s.M,
+                            ws.data(), ws.size(), (int)s.M,
                             (int)s.K, (int)s.N, (int)bits, (int)group_size, &plan, stream);
     raise(rc, "gptq_hip_gemm", s.M, s.K, s.N, bits, group_size);
     return y;
@@ -189,11 +190,10 @@ Tensor gemm_sorted(const Tensor &x, const Tensor &qweight_sorted, const Tensor &
     raise(rc, "gptq_hip_gemm_sorted", s.M, s.K, s.N, bits, group_size);
     const size_t need_ws = std::max((size_t)plan.workspace_bytes,
                                     gptq_hip_sorted_workspace_bytes((int)s.M, (int)s.K, (int)s.N, (int)bits, (int)group_size));
-    Tensor ws;
-    if (need_ws) ws = workspace(x, need_ws, stream);
+    const WorkspaceLease ws(x, need_ws, stream);
     rc = gptq_hip_gemm_sorted(x.data_ptr(), (const int32_t *)qweight_sorted.data_ptr(), (const int32_t *)qzeros.data_ptr(),
                               scales.data_ptr(), (const int32_t *)kmap.data_ptr(), ptr(bias), y.data_ptr(),
-                              ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? (size_t)ws.numel() : 0, (int)s.M,
+                              ws.data(), ws.size(), (int)s.M,
                               (int)s.K, (int)s.N, (int)bits, (int)group_size, &plan, stream);
     raise(rc, "gptq_hip_gemm_sorted", s.M, s.K, s.N, bits, group_size);
     return y;

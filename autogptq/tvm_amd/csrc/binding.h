@@ -4,6 +4,7 @@
 #pragma once
 #include <ATen/ATen.h>
 
+#include <mutex>
 #include <optional>
 
 #include "gptq_hip.h"
@@ -19,7 +20,24 @@ inline bool has(const OptTensor &t) { return t.has_value() && t->defined(); }
 void raise(int rc, const char *what, int64_t M, int64_t K, int64_t N, int64_t bits, int64_t gs);
 
 int workspace_kind(const gptq_hip_plan &plan);
-Tensor workspace(const Tensor &like, size_t nbytes, void *stream, int kind = 0);
+
+// The workspace of a stream for the launches of one call (none for nbytes = 0).  Held over all of them: a call is up to three
+// launches that hand x or partial sums on through the workspace, and those of another thread on the same stream must not
+// come between.
+struct Workspace {
+    std::mutex busy;
+    Tensor bytes;
+};
+class WorkspaceLease {
+public:
+    WorkspaceLease(const Tensor &like, size_t nbytes, void *stream, int kind = 0);
+    void *data() const { return ws ? ws->bytes.data_ptr() : nullptr; }
+    size_t size() const { return ws ? (size_t)ws->bytes.numel() : 0; }
+
+private:
+    Workspace *ws = nullptr;
+    std::unique_lock<std::mutex> held;
+};
 
 // One layer's constant tensors, a row count and the plan for it: what a call needs beside x.
 // kind: 0 = checkpoint tensors (qweight, qzeros, scales, g_idx?), 1 = sorted copy (qweight_sorted, qzeros, scales,

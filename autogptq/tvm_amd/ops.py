@@ -1,8 +1,10 @@
 """Torch-tensor front end of the C ABI: pointer plumbing and argument checks only."""
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
+import threading
 from typing import Optional
 
 import torch
@@ -59,20 +61,31 @@ def check_shapes(qweight, qzeros, scales, g_idx, bias, bits: int, group_size: in
     return K, N, G
 
 
+class _Workspace:
+    def __init__(self):
+        self.busy = threading.Lock()
+        self.bytes = None
+
+
 _workspaces = {}
 
 
-def _workspace(device: torch.device, nbytes: int, kind: int = 0) -> torch.Tensor:
-    """A zero-initialised workspace per (device, stream) and kind, grown on demand.  The kernels leave
-    its counters at zero, so it is cleared only when it is (re)allocated.  kind 1: the decode plans of the
-    tiled family with halved tiles, whose kernel keeps ALL their bytes zero between launches (the slots through
-    which the two halves of a tile meet); they do not share the workspace other plans pack x or partial sums into."""
+@contextlib.contextmanager
+def _workspace(device: torch.device, nbytes: int, kind: int = 0):
+    """A zero-initialised workspace per (device, stream) and kind, grown on demand (None for 0 bytes), held for the
+    launches of one call: they hand x or partial sums on through it, and those of another thread on the same stream must
+    not come between.  The kernels leave its counters at zero, so it is cleared only when it is (re)allocated.  kind 1: the
+    decode plans of the tiled family with halved tiles, whose kernel keeps ALL their bytes zero between launches (the slots
+    through which the two halves of a tile meet); they do not share the workspace other plans pack x or partial sums into."""
+    if not nbytes:
+        yield None
+        return
     key = (device.index, torch.cuda.current_stream(device).cuda_stream, kind)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
+    ws = _workspaces.setdefault(key, _Workspace())
+    with ws.busy:
+        if ws.bytes is None or ws.bytes.numel() < nbytes:
+            ws.bytes = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+        yield ws.bytes
 
 
 def gemm(x: torch.Tensor, qweight: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor,
@@ -102,8 +115,7 @@ def gemm(x: torch.Tensor, qweight: torch.Tensor, qzeros: torch.Tensor, scales: t
         return out
     if plan is None:
         plan = _lib.select(M, K, N, bits, group_size, g_idx is not None)
-    ws = _workspace(dev, plan.workspace_bytes) if plan.workspace_bytes else None
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _workspace(dev, plan.workspace_bytes) as ws:
         rc = _lib.lib().gptq_hip_gemm_plan(
             _ptr(x), _ptr(qweight), _ptr(qzeros), _ptr(scales), _ptr(g_idx), _ptr(bias), _ptr(out),
             _ptr(ws), ws.numel() if ws is not None else 0, M, K, N, bits, group_size,
@@ -159,8 +171,7 @@ def gemm_sorted(x: torch.Tensor, qweight_sorted: torch.Tensor, qzeros: torch.Ten
         # kernels that want x in the sorted order (STREAM, GROUPED with packed rows): a small pass puts it
         # behind what the plan itself uses
         ws_bytes = max(ws_bytes, _lib.lib().gptq_hip_sorted_workspace_bytes(M, K, N, bits, group_size))
-    ws = _workspace(dev, ws_bytes) if ws_bytes else None
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _workspace(dev, ws_bytes) as ws:
         rc = _lib.lib().gptq_hip_gemm_sorted(
             _ptr(x), _ptr(qweight_sorted), _ptr(qzeros), _ptr(scales), _ptr(kmap), _ptr(bias), _ptr(out),
             _ptr(ws), ws.numel() if ws is not None else 0, M, K, N, bits, group_size,
@@ -249,8 +260,7 @@ def gemm_tiled(x: torch.Tensor, qtile: torch.Tensor, sz: torch.Tensor, xsrc: Opt
     if plan is None:
         plan = _lib.select_tiled(M, K, N, bits, group_size)
     slots = bool(plan.flags & _lib.PLAN_PRIVATE_ZERO_WORKSPACE)   # (halved tiles: a workspace of their own)
-    ws = _workspace(dev, plan.workspace_bytes, 1 if slots else 0) if plan.workspace_bytes else None
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _workspace(dev, plan.workspace_bytes, 1 if slots else 0) as ws:
         rc = _lib.lib().gptq_hip_gemm_tiled(_ptr(x), _ptr(qtile), _ptr(sz), _ptr(xsrc), _ptr(kinv), _ptr(bias), _ptr(out),
                                             _ptr(ws), ws.numel() if ws is not None else 0, M, K, N, bits, group_size,
                                             ctypes.byref(plan), _stream(dev))
@@ -318,8 +328,7 @@ def gemm_tiled_transposed(gy: torch.Tensor, qtile_t: torch.Tensor, szt: torch.Te
         return out
     if plan is None:
         plan = _lib.select_tiled_transposed(M, K, N, bits, group_size)
-    ws = _workspace(dev, plan.workspace_bytes)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _workspace(dev, max(plan.workspace_bytes, 1)) as ws:
         rc = _lib.lib().gptq_hip_gemm_tiled_transposed(_ptr(gy), _ptr(qtile_t), _ptr(szt), _ptr(xsrc), _ptr(out), _ptr(ws),
                                                        ws.numel(), M, K, N, bits, group_size, ctypes.byref(plan),
                                                        _stream(dev))

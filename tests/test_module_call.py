@@ -3,7 +3,7 @@ same numbers, and the module's ways of being changed or watched still reach it."
 import pytest
 import torch
 
-from autogptq.tvm_amd import ops
+from autogptq.tvm_amd import _lib, ops
 from autogptq.tvm_amd.qlinear import QuantLinear
 from tests.parity_util import assert_tight, expected_output, layer
 
@@ -79,3 +79,42 @@ def test_hooks_replaced_buffers_and_instance_forward_are_seen(dev):
     assert torch.allclose(q(x).float(), 2 * first.float(), rtol=1e-3, atol=1e-3)
     q._buffers["scales"] = q.scales * 0            # swapped behind the module's back
     assert float(q(x).abs().max()) == 0.0
+
+
+def module_of(L, dev, **kw):
+    q = QuantLinear(L["bits"], L["group_size"], L["K"], L["N"], L.get("bias") is not None, **kw)
+    q.load_state_dict({k: L[k] for k in ("qweight", "qzeros", "scales", "g_idx", "bias") if L.get(k) is not None})
+    return q.to(dev)
+
+
+@pytest.mark.parametrize("way", ["operator", "front end", "gradient", "module"])
+def test_threads_on_one_stream_do_not_mix_their_launches(dev, way):
+    """A call of a pack pass, a product and a sum hands them x and partial sums through its stream's workspace: the launches
+    of another thread's call do not come between."""
+    import threading
+
+    M, K, N = 40, 2048, 1056
+    L = layer(4250, K, N, 4, 128, True, M=M)
+    q = module_of(L, dev)
+    qtile, sz, xsrc, kinv = q.prepare_tiled()
+    plan = _lib.select_tiled(M, K, N, 4, 128)
+    assert plan.workspace_bytes and q.prepare_transposed() is not None
+    call = {"operator": lambda t: torch.ops.gptq_hip.gemm_tiled(t, qtile, sz, xsrc, kinv, None, 4, 128),
+            "front end": lambda t: ops.gemm_tiled(t, qtile, sz, xsrc, kinv, None, 4, 128, plan=plan),
+            "gradient": q.grad_input, "module": q}[way]
+    width = N if way == "gradient" else K
+    xs = [torch.randn(M, width, dtype=torch.float16, device=dev) for _ in range(4)]
+    want = [call(x) for x in xs]
+    torch.cuda.synchronize()
+    wrong = [0] * len(xs)
+
+    def work(i):
+        got = [call(xs[i]) for _ in range(200)]        # (every thread on the same, the default, stream)
+        wrong[i] = sum(not torch.equal(y, want[i]) for y in got)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(xs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == [0] * len(xs)
