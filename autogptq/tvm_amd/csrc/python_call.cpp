@@ -44,14 +44,25 @@ bool takes(const Bound &q, const Tensor &x)
            x.size(-1) == q.K && x.numel() == (int64_t)q.M * q.K && x.is_contiguous() && x.get_device() == q.a.get_device();
 }
 
+// Lets other Python threads run meanwhile: an allocation or a launch can wait for the GPU, and waits for the lock of a
+// workspace whose holder may itself be waiting for the interpreter (an allocator that records Python stacks).
+struct WithoutInterpreter {
+    PyThreadState *const state = PyEval_SaveThread();
+    ~WithoutInterpreter() { PyEval_RestoreThread(state); }
+};
+
 PyObject *apply(const Bound &q, const Tensor &x)
 {
-    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    c10::SmallVector<int64_t, 6> sizes(x.sizes().begin(), x.sizes().end());
-    sizes.back() = q.N;
-    Tensor y(at::detail::empty_cuda(sizes, at::kHalf, x.device(), std::nullopt));
-    void *stream = (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device()).stream();
-    raise(q.launch(x, y.data_ptr(), stream), "gptq_hip product", q.M, q.K, q.N, q.bits, q.group_size);
+    Tensor y;
+    {
+        const WithoutInterpreter free;
+        const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+        c10::SmallVector<int64_t, 6> sizes(x.sizes().begin(), x.sizes().end());
+        sizes.back() = q.N;
+        y = at::detail::empty_cuda(sizes, at::kHalf, x.device(), std::nullopt);
+        void *stream = (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device()).stream();
+        raise(q.launch(x, y.data_ptr(), stream), "gptq_hip product", q.M, q.K, q.N, q.bits, q.group_size);
+    }
     return THPVariable_Wrap(std::move(y));
 }
 

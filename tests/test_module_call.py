@@ -118,3 +118,40 @@ def test_threads_on_one_stream_do_not_mix_their_launches(dev, way):
     for t in threads:
         t.join()
     assert wrong == [0] * len(xs)
+
+
+def test_other_threads_run_while_a_call_allocates_and_launches(dev):
+    """The call gives the interpreter free around its allocation and launch.  The switch interval is far beyond the test, so
+    that another thread advances only where the call itself lets it; the emptied cache makes the allocation a long one."""
+    import sys
+    import threading
+    import time
+
+    L = layer(4200, 512, 16384, 4, 128, False, M=64)
+    q, x = module_of(L, dev), L["x"].to(dev)
+    for _ in range(3):
+        y = q(x)
+    beat, stop = [0], threading.Event()
+
+    def run():
+        while not stop.is_set():
+            beat[0] += 1
+            time.sleep(0)
+
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(60.0)
+    advanced = 0
+    t = threading.Thread(target=run)
+    t.start()
+    try:
+        for _ in range(50):
+            y = None
+            torch.cuda.empty_cache()
+            before = beat[0]
+            y = q(x)
+            advanced += beat[0] != before
+    finally:
+        stop.set()
+        sys.setswitchinterval(interval)
+        t.join()
+    assert advanced > 0 and y is not None
