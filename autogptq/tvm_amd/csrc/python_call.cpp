@@ -37,11 +37,12 @@ struct BoundCall {
 
 PyTypeObject *g_bound_type = nullptr;
 
-// an x that q takes as it is: fp16, dense rows of K, M of them in all
+// an x that q takes as it is: fp16, dense rows of K, M of them in all, and aligned for the kernels' 16-byte loads
 bool takes(const Bound &q, const Tensor &x)
 {
-    return x.is_cuda() && x.layout() == at::kStrided && x.scalar_type() == at::kHalf && x.dim() >= 1 &&
-           x.size(-1) == q.K && x.numel() == (int64_t)q.M * q.K && x.is_contiguous() && x.get_device() == q.a.get_device();
+    return x.is_cuda() && x.layout() == at::kStrided && x.has_storage() && x.scalar_type() == at::kHalf && x.dim() >= 1 &&
+           x.size(-1) == q.K && x.numel() == (int64_t)q.M * q.K && x.is_contiguous() && x.get_device() == q.a.get_device() &&
+           (uintptr_t)x.data_ptr() % 16 == 0;
 }
 
 // Lets other Python threads run meanwhile: an allocation or a launch can wait for the GPU, and waits for the lock of a
@@ -113,7 +114,7 @@ PyObject *bound_call(PyObject *self, PyObject *args, PyObject *kwargs)
     const Tensor x = THPVariable_Unpack(PyTuple_GET_ITEM(args, 0));
     TORCH_CHECK(x.is_cuda() && x.device() == q.a.device(), "x is on ", x.device(), ", the layer on ", q.a.device(),
                 ": the GPTQ kernels run on a ROCm GPU only and there is no CPU fallback");
-    TORCH_CHECK(takes(q, x), "x must be a contiguous fp16 tensor of ", q.M, " rows of ", q.K);
+    TORCH_CHECK(takes(q, x), "x must be a contiguous fp16 tensor, 16-byte aligned, of ", q.M, " rows of ", q.K);
     return apply(q, x);
     END_HANDLE_TH_ERRORS
 }

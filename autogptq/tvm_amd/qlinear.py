@@ -19,6 +19,11 @@ from . import _lib, ops
 from .pack import pack_qweight, pack_qzeros, tiled_qualifies
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """``t``, or a copy of it where the kernels' 16-byte loads ask for one (a contiguous view at an odd offset)."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 class _ProductWithInputGrad(torch.autograd.Function):
     """The product with a gradient for x (the packed weights are constants): grad_x = grad_y @ W^T, which
     is what the reference's Triton back end offers for training on top of quantised layers
@@ -215,6 +220,7 @@ class QuantLinear(nn.Module):
             gy = gy.half()
         if not gy.is_contiguous():
             gy = gy.contiguous()
+        gy = _aligned(gy)
         M = gy.size(0)
         # The panel kernel where the library says so; else the matmul kernel's transposed form below the switch.  Measured on
         # MI355X (us, eager, int4 with an activation order; the latter against dequant + library GEMM):
@@ -417,7 +423,7 @@ class QuantLinear(nn.Module):
         M = x2.shape[0]
         if M == 0:
             return x2.new_empty((0, self.outfeatures))
-        return self._routed(M)[3](x2)
+        return self._routed(M)[3](_aligned(x2))
 
     def dequantize(self) -> torch.Tensor:
         """fp16 [infeatures, outfeatures], the weight the reference materialises on every call."""

@@ -155,3 +155,24 @@ def test_other_threads_run_while_a_call_allocates_and_launches(dev):
         sys.setswitchinterval(interval)
         t.join()
     assert advanced > 0 and y is not None
+
+
+@pytest.mark.parametrize("M", [1, 8, 40, 1300])
+def test_rows_at_an_odd_offset_are_taken(dev, M):
+    """A contiguous view of a larger tensor need not be aligned for the kernels' 16-byte loads: on every route, and as a
+    gradient."""
+    K, N = 2048, 4128
+    L = layer(9710, K, N, 4, 128, True, M=M, bias=True)
+    q, x = module_of(L, dev), L["x"].to(dev)
+    want = q(x)
+    gy = torch.randn(M, N, generator=torch.Generator().manual_seed(3)).half().to(dev)
+    want_t = q.grad_input(gy)
+    for offset in (1, 4):
+        odd = torch.empty(M * K + 8, dtype=torch.float16, device=dev)[offset:offset + M * K].view(M, K).copy_(x)
+        assert odd.data_ptr() % 16 and odd.is_contiguous()
+        assert torch.equal(q(odd), want) and torch.equal(q(odd.view(M, 1, K)).view(M, N), want)
+        odd_t = torch.empty(M * N + 8, dtype=torch.float16, device=dev)[offset:offset + M * N].view(M, N).copy_(gy)
+        assert torch.equal(q.grad_input(odd_t), want_t)
+        xg = odd.clone().requires_grad_(True)
+        q(xg).backward(odd_t)
+        assert torch.equal(xg.grad, want_t)
