@@ -130,7 +130,17 @@ PyType_Spec bound_spec = {"gptq_hip_call.BoundCall", sizeof(BoundCall), 0, Py_TP
 PyTypeObject *g_module_type = nullptr;   // the class the function was installed on; a subclass takes the ordinary way
 PyObject *g_nn_module = nullptr;         // torch.nn.Module
 PyObject *g_global_hooks[4] = {};        // the four dicts of hooks on every module
-PyObject *s_call, *s_routes, *s_buffers, *s_forward, *s_hooks[4], *s_watched[4], *s_compiled;
+PyObject *g_forward = nullptr, *g_nn_call = nullptr, *g_nn_call_impl = nullptr, *g_own_call = nullptr;   // the methods that the function stands for
+PyObject *s_call, *s_call_impl, *s_routes, *s_buffers, *s_forward, *s_hooks[4], *s_watched[4], *s_compiled;
+
+// whether a call of a module would still run them: none replaced or added on the class or on nn.Module
+bool methods_untouched()
+{
+    PyObject *own = g_module_type->tp_dict, *nn = ((PyTypeObject *)g_nn_module)->tp_dict;
+    return PyDict_GetItem(own, s_forward) == g_forward && PyDict_GetItem(nn, s_call) == g_nn_call &&
+           PyDict_GetItem(nn, s_call_impl) == g_nn_call_impl && PyDict_GetItem(own, s_call) == g_own_call &&
+           !PyDict_GetItem(own, s_call_impl);
+}
 
 // The bound product of a call of `self` with x (a new reference), or nullptr where the ordinary way has to decide.
 PyObject *route_of(PyObject *self, const Tensor &x)
@@ -147,7 +157,8 @@ PyObject *route_of(PyObject *self, const Tensor &x)
         if (!h || !PyDict_Check(h) || PyDict_GET_SIZE(h) != 0) return nullptr;
     }
     // (a forward set on the instance, as offload hooks do, or a compiled call)
-    if (PyDict_GetItem(dict, s_forward) || PyDict_GetItem(dict, s_compiled)) return nullptr;
+    if (PyDict_GetItem(dict, s_forward) || PyDict_GetItem(dict, s_call_impl) || PyDict_GetItem(dict, s_compiled)) return nullptr;
+    if (!methods_untouched()) return nullptr;
     PyObject *routes = PyDict_GetItem(dict, s_routes), *buffers = PyDict_GetItem(dict, s_buffers);
     if (!routes || !PyDict_Check(routes) || !buffers || !PyDict_Check(buffers)) return nullptr;
     PyObject *rows = PyLong_FromLongLong((long long)(x.numel() / x.size(-1)));
@@ -218,8 +229,17 @@ PyObject *install(PyObject *, PyObject *cls)
         }
     }
     if (!(g_nn_module = PyObject_GetAttrString(mod.get(), "Module"))) return nullptr;
+    g_forward = PyDict_GetItem(((PyTypeObject *)cls)->tp_dict, s_forward);
+    g_nn_call = PyDict_GetItem(((PyTypeObject *)g_nn_module)->tp_dict, s_call);
+    g_nn_call_impl = PyDict_GetItem(((PyTypeObject *)g_nn_module)->tp_dict, s_call_impl);
+    if (!g_forward || !g_nn_call || !g_nn_call_impl) {
+        PyErr_SetString(PyExc_TypeError, "a class with a forward of its own, derived from nn.Module, is expected");
+        return nullptr;
+    }
+    for (PyObject *method : {g_forward, g_nn_call, g_nn_call_impl}) Py_INCREF(method);
     THPObjectPtr descr(PyDescr_NewMethod((PyTypeObject *)cls, &module_call_def));
     if (!descr || PyObject_SetAttr(cls, s_call, descr.get()) != 0) return nullptr;
+    g_own_call = descr.release();
     Py_INCREF(cls);
     g_module_type = (PyTypeObject *)cls;
     Py_RETURN_NONE;
@@ -235,6 +255,7 @@ PyMODINIT_FUNC PyInit_gptq_hip_call()
 {
     auto intern = [](const char *s) { return PyUnicode_InternFromString(s); };
     s_call = intern("__call__"), s_routes = intern("_routes"), s_buffers = intern("_buffers"), s_forward = intern("forward");
+    s_call_impl = intern("_call_impl");
     s_compiled = intern("_compiled_call_impl");
     static const char *const hooks[4] = {"_backward_hooks", "_backward_pre_hooks", "_forward_hooks", "_forward_pre_hooks"};
     static const char *const watched[4] = {"qweight", "qzeros", "scales", "g_idx"};

@@ -176,3 +176,33 @@ def test_rows_at_an_odd_offset_are_taken(dev, M):
         xg = odd.clone().requires_grad_(True)
         q(xg).backward(odd_t)
         assert torch.equal(xg.grad, want_t)
+
+
+def python_frames(fn):
+    """The names of the Python functions that a call of ``fn`` enters."""
+    import sys
+
+    names = []
+    sys.setprofile(lambda frame, event, arg: event == "call" and names.append(frame.f_code.co_name))
+    try:
+        fn()
+    finally:
+        sys.setprofile(None)
+    return names
+
+
+def test_methods_replaced_on_the_classes_are_seen(dev, monkeypatch):
+    L = layer(4160, 512, 96, 4, 128, True, M=2)
+    q, x = module_of(L, dev), L["x"].to(dev)
+    first = q(x)
+    call = lambda: q(x)
+    for owner, name in ((QuantLinear, "forward"), (QuantLinear, "__call__"), (QuantLinear, "_call_impl"),
+                        (torch.nn.Module, "__call__"), (torch.nn.Module, "_call_impl")):
+        original, seen = getattr(owner, name), []
+        with monkeypatch.context() as m:
+            m.setattr(owner, name, lambda self, *a: (seen.append(name), original(self, *a))[1])
+            assert torch.equal(q(x), first) and seen == [name]
+        assert torch.equal(q(x), first) and seen == [name]
+        assert python_frames(call) == ["<lambda>"]            # untouched again: the call in C
+    q._call_impl = lambda *a: "instance"
+    assert q(x) == "instance"
