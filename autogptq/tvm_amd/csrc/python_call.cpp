@@ -1,8 +1,8 @@
-// The module call from Python, in C: ``QuantLinear.__call__`` for the common case, and the bound product it runs.
+// The module call from Python, in C: what calling a ``QuantLinear`` does in the common case, and the bound product it runs.
 //
-// An eager decode step is a chain of calls of a few microseconds each; the kernel of one takes 4 to 7 us, and so
-// did nothing but the way to it: nn.Module.__call__, forward's reshapes of a 3-D input, the crossing into a TorchScript
-// class and the dispatcher's at::empty together took 7 us of host time on top of the 2.4 us of the launch itself.
+// An eager decode step is a chain of calls of a few microseconds each: the kernel of one takes 4 to 7 us.  The way to it
+// alone (nn.Module.__call__, forward's reshapes of a 3-D input, the crossing into a TorchScript class, the dispatcher's
+// at::empty) took 7 us of host time on top of the 2.4 us of the launch itself.
 // Here the call is one C function of the type: it looks the bound product of the row count up in the module's routes,
 // checks that the module and its buffers are as they were when the route was decided, allocates y in the shape of x
 // and launches.  Measured (one row, 4096 x 4096, us of host time per call of a 3-D x): 9.6 before, 3.8 now.
@@ -105,19 +105,7 @@ void bound_dealloc(PyObject *self)
     Py_DECREF(type);
 }
 
-PyObject *bound_call(PyObject *self, PyObject *args, PyObject *kwargs)
-{
-    HANDLE_TH_ERRORS
-    const Bound &q = ((BoundCall *)self)->q;
-    TORCH_CHECK(PyTuple_GET_SIZE(args) == 1 && (!kwargs || PyDict_GET_SIZE(kwargs) == 0) && THPVariable_Check(PyTuple_GET_ITEM(args, 0)),
-                "one tensor is expected");
-    const Tensor x = THPVariable_Unpack(PyTuple_GET_ITEM(args, 0));
-    TORCH_CHECK(x.is_cuda() && x.device() == q.a.device(), "x is on ", x.device(), ", the layer on ", q.a.device(),
-                ": the GPTQ kernels run on a ROCm GPU only and there is no CPU fallback");
-    TORCH_CHECK(takes(q, x), "x must be a contiguous fp16 tensor, 16-byte aligned, of ", q.M, " rows of ", q.K);
-    return apply(q, x);
-    END_HANDLE_TH_ERRORS
-}
+PyObject *bound_call(PyObject *self, PyObject *args, PyObject *kwargs);
 
 PyType_Slot bound_slots[] = {{Py_tp_new, (void *)bound_new},
                              {Py_tp_dealloc, (void *)bound_dealloc},
@@ -126,11 +114,15 @@ PyType_Slot bound_slots[] = {{Py_tp_new, (void *)bound_new},
                              {0, nullptr}};
 PyType_Spec bound_spec = {"gptq_hip_call.BoundCall", sizeof(BoundCall), 0, Py_TPFLAGS_DEFAULT, bound_slots};
 
-// ---- QuantLinear.__call__
+// ---- the call of a QuantLinear
+// The function stands in the type's tp_call slot, beside the methods: QuantLinear.__call__ is still nn.Module's, for tracers
+// and compilers that follow the methods.  Python fills the slot anew, with the ordinary call, whenever a __call__ is set on
+// the class or on nn.Module; the first product called the ordinary way after that was undone brings the function back.
 PyTypeObject *g_module_type = nullptr;   // the class the function was installed on; a subclass takes the ordinary way
+ternaryfunc g_ordinary = nullptr;        // Python's own function of the slot: looks __call__ up and calls it
 PyObject *g_nn_module = nullptr;         // torch.nn.Module
 PyObject *g_global_hooks[4] = {};        // the four dicts of hooks on every module
-PyObject *g_forward = nullptr, *g_nn_call = nullptr, *g_nn_call_impl = nullptr, *g_own_call = nullptr;   // the methods that the function stands for
+PyObject *g_forward = nullptr, *g_nn_call = nullptr, *g_nn_call_impl = nullptr;   // the methods that the function stands for
 PyObject *s_call, *s_call_impl, *s_routes, *s_buffers, *s_forward, *s_hooks[4], *s_watched[4], *s_compiled;
 
 // whether a call of a module would still run them: none replaced or added on the class or on nn.Module
@@ -138,8 +130,7 @@ bool methods_untouched()
 {
     PyObject *own = g_module_type->tp_dict, *nn = ((PyTypeObject *)g_nn_module)->tp_dict;
     return PyDict_GetItem(own, s_forward) == g_forward && PyDict_GetItem(nn, s_call) == g_nn_call &&
-           PyDict_GetItem(nn, s_call_impl) == g_nn_call_impl && PyDict_GetItem(own, s_call) == g_own_call &&
-           !PyDict_GetItem(own, s_call_impl);
+           PyDict_GetItem(nn, s_call_impl) == g_nn_call_impl && !PyDict_GetItem(own, s_call) && !PyDict_GetItem(own, s_call_impl);
 }
 
 // The bound product of a call of `self` with x (a new reference), or nullptr where the ordinary way has to decide.
@@ -186,29 +177,37 @@ PyObject *route_of(PyObject *self, const Tensor &x)
     return fn;
 }
 
-PyObject *module_call(PyObject *self, PyObject *const *args, Py_ssize_t nargs, PyObject *kwnames)
+PyObject *module_call(PyObject *self, PyObject *args, PyObject *kwargs)
 {
     HANDLE_TH_ERRORS
-    if (nargs == 1 && !kwnames && Py_TYPE(self) == g_module_type && THPVariable_CheckExact(args[0])) {
-        const Tensor &x = THPVariable_Unpack(args[0]);
+    if (PyTuple_GET_SIZE(args) == 1 && (!kwargs || PyDict_GET_SIZE(kwargs) == 0) && Py_TYPE(self) == g_module_type &&
+        THPVariable_CheckExact(PyTuple_GET_ITEM(args, 0))) {
+        const Tensor &x = THPVariable_Unpack(PyTuple_GET_ITEM(args, 0));
         if (PyObject *fn = route_of(self, x)) {
             const THPObjectPtr hold(fn);
             return apply(((BoundCall *)fn)->q, x);
         }
     }
-    THPObjectPtr ordinary(PyObject_GetAttr(g_nn_module, s_call));
-    if (!ordinary) return nullptr;
-    c10::SmallVector<PyObject *, 8> all{self};
-    const Py_ssize_t n = nargs + (kwnames ? PyTuple_GET_SIZE(kwnames) : 0);
-    all.append(args, args + n);
-    return PyObject_Vectorcall(ordinary.get(), all.data(), (size_t)(nargs + 1), kwnames);
+    return g_ordinary(self, args, kwargs);
     END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef module_call_def = {"__call__", (PyCFunction)(void (*)(void))module_call, METH_FASTCALL | METH_KEYWORDS,
-                               "The module call: the bound product of x's row count where one is known, else nn.Module.__call__."};
+PyObject *bound_call(PyObject *self, PyObject *args, PyObject *kwargs)
+{
+    HANDLE_TH_ERRORS
+    if (g_module_type && g_module_type->tp_call == g_ordinary && methods_untouched()) g_module_type->tp_call = module_call;
+    const Bound &q = ((BoundCall *)self)->q;
+    TORCH_CHECK(PyTuple_GET_SIZE(args) == 1 && (!kwargs || PyDict_GET_SIZE(kwargs) == 0) && THPVariable_Check(PyTuple_GET_ITEM(args, 0)),
+                "one tensor is expected");
+    const Tensor x = THPVariable_Unpack(PyTuple_GET_ITEM(args, 0));
+    TORCH_CHECK(x.is_cuda() && x.device() == q.a.device(), "x is on ", x.device(), ", the layer on ", q.a.device(),
+                ": the GPTQ kernels run on a ROCm GPU only and there is no CPU fallback");
+    TORCH_CHECK(takes(q, x), "x must be a contiguous fp16 tensor, 16-byte aligned, of ", q.M, " rows of ", q.K);
+    return apply(q, x);
+    END_HANDLE_TH_ERRORS
+}
 
-// install(cls): gives cls the function above as its __call__
+// install(cls): makes module_call what runs when an instance of cls is called
 PyObject *install(PyObject *, PyObject *cls)
 {
     HANDLE_TH_ERRORS
@@ -237,16 +236,17 @@ PyObject *install(PyObject *, PyObject *cls)
         return nullptr;
     }
     for (PyObject *method : {g_forward, g_nn_call, g_nn_call_impl}) Py_INCREF(method);
-    THPObjectPtr descr(PyDescr_NewMethod((PyTypeObject *)cls, &module_call_def));
-    if (!descr || PyObject_SetAttr(cls, s_call, descr.get()) != 0) return nullptr;
-    g_own_call = descr.release();
     Py_INCREF(cls);
     g_module_type = (PyTypeObject *)cls;
+    if (g_module_type->tp_call != module_call) {
+        g_ordinary = g_module_type->tp_call;
+        g_module_type->tp_call = module_call;
+    }
     Py_RETURN_NONE;
     END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef functions[] = {{"install", install, METH_O, "Gives a QuantLinear class its __call__."}, {nullptr, nullptr, 0, nullptr}};
+PyMethodDef functions[] = {{"install", install, METH_O, "Makes the call in C the one of a QuantLinear class."}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "gptq_hip_call", "the QuantLinear call in C", -1, functions};
 
 }  // namespace

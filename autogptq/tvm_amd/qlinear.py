@@ -404,8 +404,8 @@ class QuantLinear(nn.Module):
         return r
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        # (the common case, a contiguous fp16 x whose row count was seen before, does not come here: __call__ is a C
-        # function that runs the bound product itself)
+        # (the common case, a contiguous fp16 x whose row count was seen before, does not come here: the call of the module
+        # is a C function that runs the bound product itself)
         out_shape = x.shape[:-1] + (self.outfeatures,)
         x2 = x.reshape(-1, x.shape[-1])
         if x2.dtype != torch.float16:

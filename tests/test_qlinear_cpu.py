@@ -135,3 +135,14 @@ def test_the_product_is_handed_aligned_rows():
         rows = x[offset:offset + 8 * 64].view(8, 64)
         assert torch.equal(q(rows), rows[:, :32])
         assert seen[-1].data_ptr() % 16 == 0 and (offset or seen[-1].data_ptr() == rows.data_ptr())
+
+
+def test_compilers_see_the_methods_of_a_module():
+    """The call in C stands beside the methods: a module whose product can be traced compiles as one graph."""
+    q = QuantLinear(4, 32, 64, 32, False)
+    q._product = lambda x2: x2[:, :32] * 2
+    net = torch.nn.Sequential(q, torch.nn.ReLU())
+    x = torch.randn(3, 64).half()
+    want = net(x)
+    assert torch.equal(torch.compile(net, backend="eager", fullgraph=True)(x), want)
+    assert QuantLinear.__call__ is torch.nn.Module.__call__
