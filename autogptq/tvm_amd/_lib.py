@@ -84,7 +84,7 @@ class Plan(ctypes.Structure):
 PLAN_PRIVATE_ZERO_WORKSPACE = 1
 PANEL_TRANSPOSED, PANEL_ACT_ORDER = 1, 2
 
-COPY_CHECKPOINT, COPY_SORTED, COPY_TILED = 1, 2, 4
+COPY_CHECKPOINT, COPY_SORTED, COPY_TILED, COPY_TILED_PANEL = 1, 2, 4, 8
 ROUTE_CHECKPOINT, ROUTE_SORTED, ROUTE_TILED, ROUTE_LIBRARY = 0, 1, 2, 3
 PROBE_EMPTY, PROBE_STREAM, PROBE_MIXED = 0, 1, 2
 ROUTE_NAMES = {ROUTE_CHECKPOINT: "plain", ROUTE_SORTED: "sorted", ROUTE_TILED: "tiled", ROUTE_LIBRARY: "library"}
@@ -244,7 +244,7 @@ def select_route(M: int, K: int, N: int, bits: int, group_size: int, act_order: 
                  copies: int = COPY_CHECKPOINT | COPY_SORTED | COPY_TILED, switch_rows=None) -> Route:
     """Which copy of a layer a call with M rows runs on, and the plan there (gptq_hip_select_route).
     ``switch_rows``: (tiled, checkpoint, checkpoint with an activation order) rows from which the library GEMM
-    takes over, 0 = never; None = the library's defaults."""
+    takes over, 0 = never; None = the library's defaults.  ``COPY_TILED_PANEL`` lets the answer be the panel kernel."""
     route = Route()
     sw = None if switch_rows is None else (ctypes.c_int * 3)(*[int(v or 0) for v in switch_rows])
     rc = lib().gptq_hip_select_route(M, K, N, bits, group_size, int(bool(act_order)), copies, sw, ctypes.byref(route))

@@ -67,9 +67,9 @@ int Bound::choose()
 {
     int rc = GPTQ_HIP_ERR_UNSUPPORTED;
     if (kind == 2) {
-        // long prompts: the panel kernel where the library says it is the faster one, else the family's own plan
-        rc = gptq_hip_select_panel(M, K, N, bits, group_size, has(d) ? GPTQ_HIP_PANEL_ACT_ORDER : 0, 0, 0, &plan);
-        if (rc == GPTQ_HIP_ERR_UNSUPPORTED) rc = gptq_hip_select_tiled(M, K, N, bits, group_size, &plan);
+        gptq_hip_route route;
+        rc = gptq_hip_select_route(M, K, N, bits, group_size, has(d), GPTQ_HIP_COPY_TILED | GPTQ_HIP_COPY_TILED_PANEL, nullptr, &route);
+        plan = route.plan;
     } else {
         rc = gptq_hip_select(M, K, N, bits, group_size, kind == 0 && has(d), &plan);
     }

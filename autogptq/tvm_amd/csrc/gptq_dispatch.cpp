@@ -875,6 +875,8 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
     if (M < 1 || K < 32 || N < 32 || K % 32 != 0 || N % 32 != 0) return GPTQ_HIP_ERR_BAD_ARG;
     if (group_size == 0 || group_size < -1) return GPTQ_HIP_ERR_BAD_ARG;
     const unsigned all = GPTQ_HIP_COPY_CHECKPOINT | GPTQ_HIP_COPY_SORTED | GPTQ_HIP_COPY_TILED;
+    const bool panels = copies & GPTQ_HIP_COPY_TILED_PANEL;
+    copies &= ~(unsigned)GPTQ_HIP_COPY_TILED_PANEL;
     if (copies == 0 || (copies & ~all)) return GPTQ_HIP_ERR_BAD_ARG;
     static const int kDefaultSwitch[3] = {1152, 1024, 640};
     const int *sw = switch_rows ? switch_rows : kDefaultSwitch;
@@ -892,9 +894,18 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
         route->copy = GPTQ_HIP_ROUTE_TILED;
         return true;
     };
+    auto take_panel = [&]() {
+        if (!panels || !tiled_ok || gptq_hip_select_panel(M, K, N, bits, group_size, act_order ? GPTQ_HIP_PANEL_ACT_ORDER : 0, 0, 0,
+                                                          &route->plan) != GPTQ_HIP_OK) {
+            memset(&route->plan, 0, sizeof(route->plan));
+            return false;
+        }
+        route->copy = GPTQ_HIP_ROUTE_TILED;
+        return true;
+    };
     if (copies == GPTQ_HIP_COPY_TILED) {
         // the tiled copy is all the layer has: every M runs there
-        if (tiled_ok && take_tiled()) return GPTQ_HIP_OK;
+        if (take_panel() || (tiled_ok && take_tiled())) return GPTQ_HIP_OK;
         return GPTQ_HIP_ERR_UNSUPPORTED;
     }
     bool tiled = false;
@@ -904,12 +915,18 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
     } else if (tiled_ok && tiled_wins(M, K, N, act, bits, one_group)) {
         tiled = true;
     }
-    int threshold = sw[0];
-    if (threshold && !tiled) {   // off the tiled copy the library GEMM wins earlier
-        if (sw[1] && sw[1] < threshold) threshold = sw[1];
-        if (act && sw[2] && sw[2] < threshold) threshold = sw[2];
+    int which = 0;
+    if (sw[0] && !tiled) {   // off the tiled copy the library GEMM wins earlier
+        if (sw[1] && sw[1] < sw[which]) which = 1;
+        if (act && sw[2] && sw[2] < sw[which]) which = 2;
     }
-    if (threshold && M >= threshold) return GPTQ_HIP_OK;
+    // The measured rows stand between the library and the kernels below; the panel kernel beats dequant + library on both
+    // sides of them (2000 rows of 9216 x 9216 315 us against 410, 2048 rows of 4096 x 4096 61 against 90).  A caller's
+    // own row count is a wish, and comes first.
+    const bool past = sw[which] && M >= sw[which];
+    if (past && sw[which] != kDefaultSwitch[which]) return GPTQ_HIP_OK;
+    if (take_panel()) return GPTQ_HIP_OK;
+    if (past) return GPTQ_HIP_OK;
     if (tiled && take_tiled()) return GPTQ_HIP_OK;
     if (!fused_bits) return GPTQ_HIP_OK;
     if ((copies & GPTQ_HIP_COPY_SORTED) && act && M <= gptq::kSortedMaxRows &&

@@ -230,7 +230,8 @@ def gemm_tiled(x: torch.Tensor, qtile: torch.Tensor, sz: torch.Tensor, xsrc: Opt
                kinv: Optional[torch.Tensor], bias: Optional[torch.Tensor], bits: int, group_size: int,
                plan: Optional[_lib.Plan] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y[M, N] fp16 = x[M, K] @ W (+ bias) on a layer in the tiled format (``tile_prepare``); x and y in the
-    layer's own channel order; ``xsrc = kinv = None`` means no activation order."""
+    layer's own channel order; ``xsrc = kinv = None`` means no activation order.  ``plan=None``: the library's choice
+    for a layer with this copy alone (gptq_hip_select_route)."""
     _need_gpu("x", x, torch.float16)
     _need_gpu("qtile", qtile, torch.int32)
     _need_gpu("sz", sz, torch.int32)
@@ -258,7 +259,8 @@ def gemm_tiled(x: torch.Tensor, qtile: torch.Tensor, sz: torch.Tensor, xsrc: Opt
     if M == 0:
         return out
     if plan is None:
-        plan = _lib.select_tiled(M, K, N, bits, group_size)
+        plan = _lib.select_route(M, K, N, bits, group_size, xsrc is not None,
+                                 copies=_lib.COPY_TILED | _lib.COPY_TILED_PANEL).plan
     slots = bool(plan.flags & _lib.PLAN_PRIVATE_ZERO_WORKSPACE)   # (halved tiles: a workspace of their own)
     with torch.cuda.device(dev), _workspace(dev, plan.workspace_bytes, 1 if slots else 0) as ws:
         rc = _lib.lib().gptq_hip_gemm_tiled(_ptr(x), _ptr(qtile), _ptr(sz), _ptr(xsrc), _ptr(kinv), _ptr(bias), _ptr(out),
@@ -327,7 +329,8 @@ def gemm_tiled_transposed(gy: torch.Tensor, qtile_t: torch.Tensor, szt: torch.Te
     if M == 0:
         return out
     if plan is None:
-        plan = _lib.select_tiled_transposed(M, K, N, bits, group_size)
+        plan = (_lib.select_panel(M, K, N, bits, group_size, xsrc is not None, transposed=True)
+                or _lib.select_tiled_transposed(M, K, N, bits, group_size))
     with torch.cuda.device(dev), _workspace(dev, max(plan.workspace_bytes, 1)) as ws:
         rc = _lib.lib().gptq_hip_gemm_tiled_transposed(_ptr(gy), _ptr(qtile_t), _ptr(szt), _ptr(xsrc), _ptr(out), _ptr(ws),
                                                        ws.numel(), M, K, N, bits, group_size, ctypes.byref(plan),

@@ -46,7 +46,9 @@ class QuantLinear(nn.Module):
     FUSED_BITS = (3, 4)             # those the kernels on the checkpoint layout cover; 2 and 8 run fused on the
                                     # tiled format only (else as dequant + library GEMM)
 
-    def __init__(self, bits, groupsize, infeatures, outfeatures, bias, kernel_switch_threshold=1152,
+    SWITCH_ROWS, GRAD_SWITCH_ROWS = 1152, 384   # the measured defaults of the two switches to the library GEMM
+
+    def __init__(self, bits, groupsize, infeatures, outfeatures, bias, kernel_switch_threshold=SWITCH_ROWS,
                  sort_for_decode=True, tile_for_prefill=True):
         super().__init__()
         if bits not in self.SUPPORTED_BITS:
@@ -67,8 +69,9 @@ class QuantLinear(nn.Module):
         #   * kernels on the checkpoint layout (layers off the tiled route): contiguous groups 124 vs 139 us
         #     at 768 rows, 152 vs 146 at 1024; activation order 126 vs 130 at 640 rows, 139 vs 133 at 768.
         #     Hence 1024 and 640 there.
-        # 0 or None disables the switch.  (It stands between the matmul kernels and the library: calls that the panel
-        # kernel is the fastest for, see _route, run there on both sides of it.)
+        # 0 or None disables the switch.  The measured default stands between the kernels above and the library: calls
+        # that the panel kernel is the fastest for run there on both sides of it.  Any other value sends every
+        # call of that many rows to the library, as in the reference.
         self.kernel_switch_threshold = kernel_switch_threshold
         self.plain_switch_threshold = 1024
         self.act_order_switch_threshold = 640
@@ -96,7 +99,8 @@ class QuantLinear(nn.Module):
         self.tile_for_prefill = tile_for_prefill
         self._tiled = None    # (key, (qtile, sz, xsrc, kinv) or None)
         self._tiled_t = None  # (key, (qtile_t, szt, xsrc) or None): the copy the gradient for x runs on
-        self.grad_switch_threshold = 384   # rows of grad_y from which the gradient for x takes the library GEMM
+        # rows of grad_y from which the gradient for x takes the library GEMM (default and own values as above)
+        self.grad_switch_threshold = self.GRAD_SWITCH_ROWS
         self._compact = False
         self._routes = {}     # M -> (watched buffers, sum of their versions, path name, fn(x2)): see _route
 
@@ -225,15 +229,18 @@ class QuantLinear(nn.Module):
         # The panel kernel where the library says so; else the matmul kernel's transposed form below the switch.  Measured on
         # MI355X (us, eager, int4 with an activation order; the latter against dequant + library GEMM):
         # 4096 x 11008: 22 / 64 at 16 rows, 37 / 90 at 128; 11008 x 4096: 35 / 66 at 128; 4096 x 4096: 27 / 44 at 128.
-        threshold = self.kernel_switch_threshold
-        if threshold:
-            threshold = min(threshold, self.grad_switch_threshold)
         gx = None
         if self.tile_for_prefill and gy.is_cuda and M > 0:
             K, N, bits, gs = self.infeatures, self.outfeatures, self.bits, self.groupsize
+            past, asked = False, False
+            if self.kernel_switch_threshold and self.grad_switch_threshold:
+                for rows, default in ((self.kernel_switch_threshold, self.SWITCH_ROWS),
+                                      (self.grad_switch_threshold, self.GRAD_SWITCH_ROWS)):
+                    if M >= rows:
+                        past, asked = True, asked or rows != default
             plan = (_lib.select_panel(M, K, N, bits, gs, self._kernel_g_idx() is not None, transposed=True)
-                    if tiled_qualifies(K, N, bits, gs) else None)
-            if plan is not None or not (threshold and M >= threshold):
+                    if not asked and tiled_qualifies(K, N, bits, gs) else None)
+            if plan is not None or not past:
                 t = self.prepare_transposed()
                 if t is not None:
                     gx = ops.gemm_tiled_transposed(gy, t[0], t[1], t[2], K, bits, gs, plan=plan)
@@ -310,8 +317,7 @@ class QuantLinear(nn.Module):
 
     def _route(self, M):
         """(what, fn): the product for M rows as one call fn(x2), and the name of the path it takes: "tiled",
-        "sorted", "plain" (the checkpoint's own tensors) or "library" (past the switch: the panel kernel on the tiled copy, or
-        where that does not cover the call the dequant kernel + library GEMM).  Decided
+        "sorted", "plain" (the checkpoint's own tensors) or "library" (the dequant kernel + library GEMM).  Decided
         once per row count and state of the buffers; the operators are torch.ops.gptq_hip.* (csrc/binding.cpp)."""
         t = torch.ops.gptq_hip
         bits, gs, bias = self.bits, self.groupsize, self.bias
@@ -348,26 +354,16 @@ class QuantLinear(nn.Module):
         if self.sort_for_decode and self.bits in self.FUSED_BITS:
             copies |= _lib.COPY_SORTED
         if self.tile_for_prefill:
-            copies |= _lib.COPY_TILED
+            copies |= _lib.COPY_TILED | _lib.COPY_TILED_PANEL
         switch_rows = (self.kernel_switch_threshold or 0,
                        self.plain_switch_threshold if self.kernel_switch_threshold else 0,
                        self.act_order_switch_threshold if self.kernel_switch_threshold else 0)
-        # Long prompts and training batches run on the tiled copy wherever its panel kernel is the faster one, whatever the
-        # rule below names (it beats the dequant kernel with the library GEMM at every size measured: 2000 rows of 9216 x 9216
-        # 315 us against 410, 2048 rows of 4096 x 4096 61 against 90).
-        panel = None
-        if self.tile_for_prefill and _lib.select_panel(M, K, N, bits, gs, g is not None) is not None:
-            tiled = self.prepare_tiled()
-            if tiled is not None:
-                panel = bind(2, tiled[0], tiled[1], None, *((tiled[2], tiled[3]) if g is not None else (None, None)))
         while True:
             r = _lib.select_route(M, K, N, bits, gs, g is not None, copies, switch_rows)
-            if panel is not None:
-                return "library" if r.copy == _lib.ROUTE_LIBRARY else "tiled", panel
             if r.copy == _lib.ROUTE_TILED:
                 tiled = self.prepare_tiled()
                 if tiled is None:
-                    copies &= ~_lib.COPY_TILED
+                    copies &= ~(_lib.COPY_TILED | _lib.COPY_TILED_PANEL)
                     continue
                 xsrc, kinv = (tiled[2], tiled[3]) if g is not None else (None, None)
                 return "tiled", bind(2, tiled[0], tiled[1], None, xsrc, kinv)

@@ -253,7 +253,8 @@ def build_case(name: str, dev, kernel: int = 0, split_k: int = 0, waves_n: int =
     }
     act = lay.mapped and prepared != "sorted"   # the sorted copy is planned like contiguous groups
     if prepared == "tiled":
-        plan = _lib.select_tiled(M, K, N, bits, gs)
+        plan = _lib.select_route(M, K, N, bits, gs, lay.mapped,
+                                 copies=_lib.COPY_TILED | _lib.COPY_TILED_PANEL).plan
     elif prepared == "sorted" and not (kernel or split_k or waves_n):
         plan = ops.sorted_plan(M, K, N, bits, gs)
     elif kernel or split_k or waves_n:
@@ -306,7 +307,8 @@ def prepared_mode(name: str):
     from autogptq.tvm_amd import _lib
 
     bits, K, N, gs, desc_act, M = WORKLOADS[name]
-    r = _lib.select_route(M, K, N, bits, gs, desc_act, switch_rows=(0, 0, 0))
+    copies = _lib.COPY_CHECKPOINT | _lib.COPY_SORTED | _lib.COPY_TILED | _lib.COPY_TILED_PANEL
+    r = _lib.select_route(M, K, N, bits, gs, desc_act, copies, switch_rows=(0, 0, 0))
     return {_lib.ROUTE_TILED: "tiled", _lib.ROUTE_SORTED: "sorted"}.get(r.copy)
 
 
@@ -554,7 +556,8 @@ def run_transposed(args, dev):
         szt = t if c == 0 else szt
     gy_cpu = torch.randn(M, N, generator=torch.Generator().manual_seed(7)).half()
     gy, gx = gy_cpu.to(dev), torch.empty((M, K), dtype=torch.float16, device=dev)
-    plan = _lib.select_tiled_transposed(M, K, N, bits, gs)
+    plan = (_lib.select_panel(M, K, N, bits, gs, desc_act, transposed=True)
+            or _lib.select_tiled_transposed(M, K, N, bits, gs))
     ws = torch.zeros(max(plan.workspace_bytes, 16), dtype=torch.uint8, device=dev)
     lib = _lib.lib()
     vp = ctypes.c_void_p

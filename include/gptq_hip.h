@@ -223,7 +223,8 @@ int gptq_hip_select_tiled(int M, int K, int N, int bits, int group_size, gptq_hi
 
 /* The plan of the PANEL kernel on the same copy, or (flags: transposed) on the transposed copy below, for
  * gptq_hip_gemm_tiled / gptq_hip_gemm_tiled_transposed.  row_tiles and split_k: 0 = the planner's choice; with both 0 it answers
- * GPTQ_HIP_ERR_UNSUPPORTED where the family's other kernels are faster.  No counterpart in the reference. */
+ * GPTQ_HIP_ERR_UNSUPPORTED where the family's other kernels are faster (gptq_hip_select_route asks it in that way).  No
+ * counterpart in the reference. */
 enum {
     GPTQ_HIP_PANEL_TRANSPOSED = 1,
     GPTQ_HIP_PANEL_ACT_ORDER = 2   /* the layer has an activation order: the workspace holds x (or gx) in the copy's order */
@@ -240,7 +241,8 @@ int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int group_size, 
 /*
  * y = x @ W (+ bias) on a layer in the tiled format, any M; replaces the same handler call as gptq_hip_gemm
  * (pycuda_warpper.py:138, qlinear_tvm.py:123,150).  x and y are in the layer's own channel order (xsrc = kinv =
- * NULL means no activation order; pass both or neither).  plan: NULL = gptq_hip_select_tiled.  workspace:
+ * NULL means no activation order; pass both or neither).  plan: NULL = what gptq_hip_select_route names for a layer
+ * with this copy alone, PANEL included; where the workspace does not hold that plan's bytes, gptq_hip_select_tiled.  workspace:
  * plan.workspace_bytes (none for most decode plans).  Decode plans: one launch; matmul plans: two
  * (pack pass, matmul); one more when the plan splits K.  A plan whose flags hold
  * GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE wants ALL bytes of its workspace zero at the first call and leaves them zero
@@ -265,7 +267,8 @@ int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint32_t *sz, co
  * gptq_hip_tile_prepare_transposed writes both (two launches).  xsrc: the map of gptq_hip_tile_prepare (the channel at
  * each sorted position), NULL without an activation order; gy and gx are in the layer's own channel order.  The
  * weights are formed exactly as in the forward product (fp16(scale * (q - zero)), one rounding), sums are fp32.
- * plan: NULL = gptq_hip_select_tiled_transposed.  workspace: plan.workspace_bytes, zeroed once.
+ * plan: NULL = gptq_hip_select_panel (transposed) where that names a plan and the workspace holds its bytes, else
+ * gptq_hip_select_tiled_transposed.  workspace: plan.workspace_bytes, zeroed once.
  */
 size_t gptq_hip_tiled_transposed_bytes(int K, int N, int bits);
 size_t gptq_hip_tiled_transposed_table_bytes(int K, int N, int group_size);
@@ -285,17 +288,21 @@ int gptq_hip_gemm_tiled_transposed(const void *gy, const void *qtile_t, const ui
  *                CHECKPOINT = qweight / qzeros / scales / g_idx as loaded (gptq_hip_gemm_plan), SORTED = the
  *                channel-sorted copy (gptq_hip_sort_channels, gptq_hip_gemm_sorted), TILED = the tiled format
  *                (gptq_hip_tile_prepare, gptq_hip_gemm_tiled).  TILED alone describes a layer that keeps only its
- *                tiled copy: every M then runs there.
+ *                tiled copy: every M then runs there.  TILED_PANEL, beside TILED: the answer may be a plan of the PANEL
+ *                kernel on that copy, wherever gptq_hip_select_panel says that it is the faster one
  *   switch_rows  rows of x from which the caller prefers W from gptq_hip_dequant and its own fp16 GEMM (what the
  *                reference does from kernel_switch_threshold rows, auto_gptq/nn_modules/qlinear.py:25,198): three
  *                values, for calls on the tiled copy, on the checkpoint tensors, and on the checkpoint tensors of a
- *                layer with an activation order; 0 = never.  NULL = the measured defaults {1152, 1024, 640}.
+ *                layer with an activation order; 0 = never.  NULL = the measured defaults {1152, 1024, 640}.  A default
+ *                is where the library product overtakes the other kernels, and with TILED_PANEL says nothing about the
+ *                PANEL kernel, which is the faster one on both sides of it; a value of the caller's own (one
+ *                that is not the default in its place) sends every call from that many rows to the library
  * route->copy names the entry point (GPTQ_HIP_ROUTE_LIBRARY: no fused kernel; dequant + library GEMM) and
  * route->plan is the plan to hand to it (zeroed for LIBRARY).  A SORTED or TILED answer for a copy that turns out not
  * to exist (gptq_hip_sort_channels / gptq_hip_tile_prepare refused the layer's contents) is retried with that bit
  * cleared.
  */
-enum { GPTQ_HIP_COPY_CHECKPOINT = 1, GPTQ_HIP_COPY_SORTED = 2, GPTQ_HIP_COPY_TILED = 4 };
+enum { GPTQ_HIP_COPY_CHECKPOINT = 1, GPTQ_HIP_COPY_SORTED = 2, GPTQ_HIP_COPY_TILED = 4, GPTQ_HIP_COPY_TILED_PANEL = 8 };
 enum { GPTQ_HIP_ROUTE_CHECKPOINT = 0, GPTQ_HIP_ROUTE_SORTED = 1, GPTQ_HIP_ROUTE_TILED = 2, GPTQ_HIP_ROUTE_LIBRARY = 3 };
 typedef struct gptq_hip_route {
     int copy;           /* GPTQ_HIP_ROUTE_* */

@@ -109,7 +109,7 @@ def test_module_runs_long_batches_and_their_gradient_on_the_panel_kernel(dev, de
     q = QuantLinear(4, gs, K, N, True)
     q.load_state_dict({k: L[k] for k in ("qweight", "qzeros", "scales", "g_idx", "bias")})
     q = q.to(dev)
-    assert q.route(M) == "library" and q._tiled[1] is not None        # past the switch, on the tiled copy all the same
+    assert q.route(M) == "tiled" and q._tiled[1] is not None          # past the measured switch to the library all the same
     x = L["x"].to(dev).requires_grad_(True)
     y = q(x)
     assert_close(y.detach(), expected_output(L), "module")
@@ -138,3 +138,110 @@ def test_panel_plans_cover_the_problem(bits):
     assert _lib.select_panel(512, 4096, 11008, bits, 16, True) is None
     with pytest.raises(_lib.GptqHipError):
         _lib.select_panel(512, 4096, 11008, 5, 128, True)
+
+
+# ---- where a call comes to run on the panel kernel: one rule (gptq_hip_select_route), whoever asks
+ALL = _lib.COPY_CHECKPOINT | _lib.COPY_SORTED | _lib.COPY_TILED | _lib.COPY_TILED_PANEL
+
+
+def test_the_route_names_the_panel_kernel_where_it_is_offered_and_faster():
+    K, N = 4096, 11008
+    for M in (1, 8, 64, 256, 700, 1151, 1152, 4096):
+        for act in (False, True):
+            panel = _lib.select_panel(M, K, N, 4, 128, act)
+            before = _lib.select_route(M, K, N, 4, 128, act)
+            for copies in (ALL, _lib.COPY_TILED | _lib.COPY_TILED_PANEL):
+                r = _lib.select_route(M, K, N, 4, 128, act, copies)
+                if panel is not None:
+                    assert r.copy == _lib.ROUTE_TILED and r.plan.as_dict() == panel.as_dict(), (M, act)
+                elif copies == ALL:
+                    assert (r.copy, r.plan.as_dict()) == (before.copy, before.plan.as_dict()), (M, act)
+            assert before.plan.kernel != _lib.KERNEL_PANEL               # only where the caller asks for it
+    assert _lib.select_panel(700, K, N, 4, 128, True) is not None
+    # groups that the format does not cover, and a layer without a tiled copy
+    assert _lib.select_route(700, K, N, 4, 16, False, ALL).plan.kernel == _lib.KERNEL_STREAM
+    r = _lib.select_route(700, K, N, 4, 128, False, ALL & ~_lib.COPY_TILED)
+    assert r.plan.kernel == _lib.KERNEL_STREAM
+    with pytest.raises(_lib.GptqHipError):
+        _lib.select_route(700, K, N, 4, 128, False, _lib.COPY_TILED_PANEL)
+
+
+def test_a_caller_s_own_switch_rows_come_before_the_panel_kernel():
+    K, N, M = 4096, 11008, 2000
+    assert _lib.select_panel(M, K, N, 4, 128, True) is not None
+    route = lambda rows, m=M, k=K, n=N, act=True: _lib.select_route(m, k, n, 4, 128, act, ALL, rows).copy
+    for rows in (None, (1152, 1024, 640), (0, 0, 0), (3000, 1024, 640)):
+        assert route(rows) == _lib.ROUTE_TILED, rows
+    for rows in ((1000, 1024, 640), (2000, 0, 0)):
+        assert route(rows) == _lib.ROUTE_LIBRARY, rows
+    assert route((2000, 1024, 640), m=1999) == _lib.ROUTE_TILED
+    # a layer whose long batches the rule has on the checkpoint tensors: their switch counts there
+    K, N = 28672, 8192
+    assert _lib.select_panel(M, K, N, 4, 128, True) is not None
+    assert _lib.select_route(600, K, N, 4, 128, True).copy == _lib.ROUTE_CHECKPOINT
+    assert route((1152, 1024, 640), k=K, n=N) == route((0, 0, 0), k=K, n=N) == _lib.ROUTE_TILED
+    assert route((1152, 1024, 900), k=K, n=N) == route((1152, 800, 640), k=K, n=N, act=False) == _lib.ROUTE_LIBRARY
+
+
+@pytest.mark.gpu
+def test_module_switches_to_the_library_where_it_is_told_to(dev):
+    K, N, M = 2048, 4128, 1300
+    L = layer(9720, K, N, 4, 128, True, M=M, bias=True)
+    own = {"kernel_switch_threshold": 1000}
+    tensors = {k: L[k] for k in ("qweight", "qzeros", "scales", "g_idx", "bias")}
+    gy = torch.randn(M, N, generator=torch.Generator().manual_seed(4)).half().to(dev)
+    x = L["x"].to(dev)
+    for kw, path in ((own, "library"), ({}, "tiled"), ({"kernel_switch_threshold": 0}, "tiled")):
+        q = QuantLinear(4, 128, K, N, True, **kw)
+        q.load_state_dict(tensors)
+        q = q.to(dev)
+        assert q.route(M) == path and (q._tiled is None) == (path == "library")
+        assert_tight(q(x), expected_output(L), f"{kw}")
+        gx = q.grad_input(gy)
+        assert (q._tiled_t is None) == (path == "library")
+        assert_tight(gx, gy.float().cpu() @ expected_weight(L).float().t(), f"gradient, {kw}")
+    q = QuantLinear(4, 128, K, N, True)
+    q.load_state_dict(tensors)
+    q = q.to(dev)
+    q.grad_switch_threshold = 200
+    q.grad_input(gy)
+    assert q._tiled_t is None and q.route(M) == "tiled"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_every_entry_without_a_plan_takes_the_same_kernel(dev, desc_act):
+    M, K, N, bits, gs = 1300, 2048, 4128, 4, 128
+    L = layer(9721, K, N, bits, gs, desc_act, M=M)
+    D = to_dev(L, dev)
+    panel, panel_t = (_lib.select_panel(M, K, N, bits, gs, desc_act, t) for t in (False, True))
+    assert panel is not None and panel_t is not None
+    want = forward(D, panel)
+    gy = torch.randn(M, N, generator=torch.Generator().manual_seed(5)).half().to(dev)
+    want_t = transposed(D, gy, panel_t)
+    assert_tight(want, expected_output(L), "panel")
+    assert torch.equal(forward(D, None), want) and torch.equal(transposed(D, gy, None), want_t)
+    qtile, sz, xsrc, kinv = ops.tile_prepare(D["qweight"], D["qzeros"], D["scales"], D["g_idx"] if desc_act else None, bits, gs)
+    qtile_t, szt = ops.tile_prepare_transposed(D["qweight"], D["qzeros"], D["scales"], xsrc if desc_act else None, bits, gs)
+    if not desc_act:
+        xsrc = kinv = None
+    assert torch.equal(torch.ops.gptq_hip.gemm_tiled(D["x"], qtile, sz, xsrc, kinv, None, bits, gs), want)
+    # the C entries, and with a workspace sized for the matmul kernel's plan: that one runs then
+    lib, ptr, null = _lib.lib(), ops._ptr, ctypes.c_void_p(None)
+    tiled, tiled_t = _lib.select_tiled(M, K, N, bits, gs), _lib.select_tiled_transposed(M, K, N, bits, gs)
+    sizes = [max(panel.workspace_bytes, panel_t.workspace_bytes, 16), 16384 + 16, max(tiled.workspace_bytes, tiled_t.workspace_bytes)]
+    for nbytes in sizes:
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
+        y, gx = torch.zeros_like(want), torch.zeros_like(want_t)
+        rc = lib.gptq_hip_gemm_tiled(ptr(D["x"]), ptr(qtile), ptr(sz), ptr(xsrc), ptr(kinv), null, ptr(y), ptr(ws), nbytes, M, K, N,
+                                     bits, gs, None, ops._stream(dev))
+        fits = nbytes >= panel.workspace_bytes
+        assert rc == (_lib.OK if fits or nbytes >= tiled.workspace_bytes else _lib.ERR_WORKSPACE), nbytes
+        if rc == _lib.OK:
+            assert torch.equal(y, want if fits else forward(D, tiled))
+        rc = lib.gptq_hip_gemm_tiled_transposed(ptr(gy), ptr(qtile_t), ptr(szt), ptr(xsrc), ptr(gx), ptr(ws), nbytes, M, K, N, bits, gs,
+                                                None, ops._stream(dev))
+        fits = nbytes >= panel_t.workspace_bytes
+        assert rc == (_lib.OK if fits or nbytes >= tiled_t.workspace_bytes else _lib.ERR_WORKSPACE), nbytes
+        if rc == _lib.OK:
+            assert torch.equal(gx, want_t if fits else transposed(D, gy, tiled_t))

@@ -89,7 +89,10 @@ def unrounded_output(L, x):
 def run_tiled(D, prep, x=None, plan=None):
     qtile, sz, xsrc, kinv = prep
     act = D["desc_act"]
-    return ops.gemm_tiled(D["x"] if x is None else x, qtile, sz, xsrc if act else None, kinv if act else None,
+    x = D["x"] if x is None else x
+    if plan is None and x.shape[0] > 0:      # this family's own plan (long batches left to the library run on the panel kernel)
+        plan = _lib.select_tiled(x.shape[0], D["K"], D["N"], D["bits"], D["group_size"])
+    return ops.gemm_tiled(x, qtile, sz, xsrc if act else None, kinv if act else None,
                           D.get("bias"), D["bits"], D["group_size"], plan=plan)
 
 
@@ -672,8 +675,9 @@ def test_quantlinear_takes_the_route_the_library_names(dev, bits, K, N, gs, desc
     """QuantLinear asks gptq_hip_select_route which copy a call runs on; the path it reports is that answer."""
     L = layer(1910 + bits, K, N, bits, gs, desc_act, M=1)
     q = module_of(L, dev)
+    copies = _lib.COPY_CHECKPOINT | _lib.COPY_SORTED | _lib.COPY_TILED | _lib.COPY_TILED_PANEL   # what a module offers
     for M in (1, 2, 4, 8, 16, 17, 64, 128, 300, 700, 1100, 1200):
-        r = _lib.select_route(M, K, N, bits, gs, desc_act and gs != -1)
+        r = _lib.select_route(M, K, N, bits, gs, desc_act and gs != -1, copies)
         assert q.route(M) == _lib.ROUTE_NAMES[r.copy], (M, q.route(M), r.copy)
     # swapping a buffer behind the module's back (what offload hooks do) makes it decide again, on the new tensor
     x = torch.randn(3, K, dtype=torch.float16, device=dev)

@@ -37,6 +37,8 @@ def grad_rows(seed, M, N):
 
 def run_t(D, prep, gy, plan=None):
     qtile_t, szt, xsrc = prep
+    if plan is None and gy.shape[0] > 0:     # this family's own plan (long batches left to the library run on the panel kernel)
+        plan = _lib.select_tiled_transposed(gy.shape[0], D["K"], gy.shape[1], D["bits"], D["group_size"])
     return ops.gemm_tiled_transposed(gy, qtile_t, szt, xsrc, D["K"], D["bits"], D["group_size"], plan=plan)
 
 
