@@ -312,8 +312,8 @@ static int run_panel(const void *x, const void *qtile, const uint32_t *sz, const
                      void *workspace, size_t workspace_bytes, int M, int K, int N, int bits, int gs, bool trans,
                      const gptq_hip_plan &plan, void *stream)
 {
-    const int S_total = ((trans ? N : K) + 63) / 64, cols = trans ? K : N, rt = plan.row_tiles;
-    if (rt < 1 || rt > gptq::kPanelMaxTiles) return GPTQ_HIP_ERR_UNSUPPORTED;
+    const int red = trans ? N : K, S_total = (red + 63) / 64, cols = trans ? K : N, rt = plan.row_tiles;
+    if (rt < 1 || rt > gptq::kPanelMaxTiles || !gptq::panel_addresses(rt, red)) return GPTQ_HIP_ERR_UNSUPPORTED;
     if (plan.waves_n != 4 || plan.waves_k != gptq::panel_waves_k(rt) || plan.block != 256 * plan.waves_k || plan.split_k < 1 || plan.k_chunk < 1 || plan.m_blocks < 1 ||
         plan.grid_x != (cols + gptq::kPanelCols - 1) / gptq::kPanelCols || plan.grid_y != plan.split_k ||
         plan.grid_z != plan.m_blocks || plan.m_blocks != (M + 32 * rt - 1) / (32 * rt) ||

@@ -723,7 +723,7 @@ extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_si
         if (M <= gptq::kDecodeMaxRows && rt == 0 && split == 0) return GPTQ_HIP_ERR_UNSUPPORTED;   // (the decode kernels' rows)
         double best = 1e30;
         for (int r = 1; r <= gptq::kPanelMaxTiles; r++) {
-            if (row_tiles ? r != row_tiles : r > 1 && 32 * (r - 1) >= M) continue;
+            if ((row_tiles ? r != row_tiles : r > 1 && 32 * (r - 1) >= M) || !gptq::panel_addresses(r, red)) continue;
             const long long tiles = (long long)col_wgs * ceil_div(M, 32 * r);
             for (int s = 1; s <= 8; s++) {
                 if (split_k ? s != split_k : s > 1 && (S_total / s < 6 || tiles * s > 768 || s * out_elems > 48e6)) continue;
@@ -747,7 +747,7 @@ extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_si
                 return GPTQ_HIP_ERR_UNSUPPORTED;
         }
     }
-    if (rt > gptq::kPanelMaxTiles) return GPTQ_HIP_ERR_UNSUPPORTED;
+    if (rt > gptq::kPanelMaxTiles || !gptq::panel_addresses(rt, red)) return GPTQ_HIP_ERR_UNSUPPORTED;
     const int m_blocks = ceil_div(M, 32 * rt);
     plan->kernel = GPTQ_HIP_KERNEL_PANEL;
     plan->row_tiles = rt;

@@ -287,6 +287,8 @@ constexpr int panel_lds_bytes(int bits, int rt)
     const int turn = (panel_waves_k(rt) - 1) * 65536 + 4 * panel_waves_k(rt) * 32 * 272;
     return stages > turn ? stages : turn;
 }
+// The kernel addresses the rows of a workgroup with 31 bits (bit 31 of an offset marks what lies outside)
+constexpr bool panel_addresses(int rt, int red) { return 32LL * rt * red * 2 < (1LL << 31); }
 // rows x channels from which the transposed product puts its result's channels in order in a pass (2.5 us and 0.9 us per
 // million, against 3.7 us per million for scattered stores)
 inline bool panel_scatters(int M, int K) { return (long long)M * K >= (1LL << 20); }

@@ -245,3 +245,23 @@ def test_every_entry_without_a_plan_takes_the_same_kernel(dev, desc_act):
         assert rc == (_lib.OK if fits or nbytes >= tiled_t.workspace_bytes else _lib.ERR_WORKSPACE), nbytes
         if rc == _lib.OK:
             assert torch.equal(gx, want_t if fits else transposed(D, gy, tiled_t))
+
+
+def test_plans_keep_within_the_kernel_s_addresses():
+    # the rows of a workgroup are addressed with 31 bits: wider reductions take fewer rows, or none at all
+    M, K = 256, 32
+    for N, most in ((1 << 20, 8), (1 << 22, 7), (1 << 23, 3), (1 << 24, 1), (1 << 25, 0)):
+        for rt in range(1, 9):
+            p = _lib.select_panel(M, K, N, 4, 32, False, True, rt, 1)
+            assert (p is not None) == (rt <= most), (N, rt)
+            assert _lib.select_panel(M, K, N, 4, 32, False, False, rt, 1) is not None    # (its reduction is K)
+        p = _lib.select_panel(M, K, N, 4, 32, False, True)
+        assert p is None or p.row_tiles <= most
+    # and a plan from elsewhere is refused before anything runs
+    N = 1 << 24
+    lib, fake, null = _lib.lib(), ctypes.c_void_p(0x1000), ctypes.c_void_p(None)
+    p = _lib.select_panel(M, K, N, 4, 32, False, True, 1, 1)
+    p.row_tiles, p.m_blocks, p.grid_z = 2, M // 64, M // 64
+    p.lds_bytes = _lib.select_panel(M, K, 1 << 20, 4, 32, False, True, 2, 1).lds_bytes
+    rc = lib.gptq_hip_gemm_tiled_transposed(fake, fake, fake, null, fake, null, 0, M, K, N, 4, 32, ctypes.byref(p), null)
+    assert rc == _lib.ERR_UNSUPPORTED
