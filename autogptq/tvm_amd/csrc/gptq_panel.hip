@@ -232,7 +232,16 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
     };
     const uint32_t part = (uint32_t)kw * PART;
     const uint32_t a_dst = part + (uint32_t)nw * (RT * 1024u), b_dst = part + B_OFF + (uint32_t)(nw * CT * BL), s_dst = part + S_OFF + (uint32_t)(nw * CT * 256);
-    const uint32_t l_words = lane * (BITS == 2 ? 4u : (BITS == 3 ? 12u : 16u)), l4 = lane * 4u;
+    const uint32_t l_words = lane * (BITS == 2 ? 4u : (BITS == 3 ? 12u : 16u));
+    // A block past the range brings no scales either: zeros times its weights have to be zero, and they are not where a weight
+    // is infinite.
+    uint32_t t_off = lane * 4u;
+    auto cut_scales = [&](int S) {
+        if (S >= S_end) {
+            asm volatile("");
+            (TRANS ? t_off : g_off) |= 0x80000000u;
+        }
+    };
 
     // request d of a step: x of block Sa to the stage at byte `sa`, words and scales of block Sb to the one at `sb`
     auto request = [&](auto d_c, uint32_t sa, int Sa, uint32_t sb, int Sb, auto &&go) {
@@ -244,7 +253,7 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
                q_base[i] + (uint32_t)Sb * (uint32_t)BW + e * (bytes * 64));
         } else if constexpr (d < NLB) {
             constexpr int i = d - CT * NB;
-            go(std::integral_constant<int, 4>{}, sb + s_dst, i * 256, TRANS ? l4 : g_off, sr,
+            go(std::integral_constant<int, 4>{}, sb + s_dst, i * 256, TRANS ? t_off : g_off, sr,
                TRANS ? s_base[i] + (uint32_t)Sb * 256u : s_base[i]);
         } else {
             constexpr int i = d - NLB;
@@ -271,11 +280,13 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
 
     // words and scales run one block further ahead than x: they are in registers a step before they are used
     const int S_wave = S_begin + kw;
+    cut_scales(S_wave);
     request_now(std::integral_constant<int, 0>{}, std::integral_constant<int, NLB>{}, 0, 0, 0, min(S_wave, S_last));
 #pragma unroll
     for (int u = 0; u < STAGES - 1; u++) {
         next_group();
         cut(S_wave + KW * u);
+        cut_scales(S_wave + KW * (u + 1));
         request_now(std::integral_constant<int, 0>{}, std::integral_constant<int, NL>{}, u * STAGE, min(S_wave + KW * u, S_last),
                     (u + 1) * STAGE, min(S_wave + KW * (u + 1), S_last));
     }
@@ -356,6 +367,8 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
                     next_group();
                 } else if constexpr (m == 1) {
                     cut(Su);
+                } else if constexpr (m == 2) {
+                    cut_scales(Su + KW);
                 }
                 if constexpr (m == MEET * NC) wait_and_meet<(STAGES - 2) * NL>();   // x of the next block is in LDS, this one's has been read
                 constexpr int d0 = g * NL / MEET, d1 = (g + 1) * NL / MEET;

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from autogptq.tvm_amd import _lib, ops
+from autogptq.tvm_amd.pack import pack_qweight, pack_qzeros
 from autogptq.tvm_amd.qlinear import QuantLinear
 from tests.parity_util import assert_close, assert_tight, expected_output, expected_weight, layer, to_dev
 
@@ -265,3 +266,84 @@ def test_plans_keep_within_the_kernel_s_addresses():
     p.lds_bytes = _lib.select_panel(M, K, 1 << 20, 4, 32, False, True, 2, 1).lds_bytes
     rc = lib.gptq_hip_gemm_tiled_transposed(fake, fake, fake, null, fake, null, 0, M, K, N, 4, 32, ctypes.byref(p), null)
     assert rc == _lib.ERR_UNSUPPORTED
+
+
+# ---- infinities and NaN in the weights, x and the gradient
+def with_weights(L, columns, codes, scale):
+    """L with its columns' weights scale * (codes - 1)."""
+    for n in columns:
+        L["codes"][:, n], L["zeros"][:, n], L["scales"][:, n] = codes, 1, scale
+    L["qweight"] = torch.from_numpy(pack_qweight(L["codes"].numpy(), L["bits"]))
+    L["qzeros"] = torch.from_numpy(pack_qzeros(L["zeros"].numpy(), L["bits"]))
+    return L
+
+
+def assert_same_specials(got, want, what):
+    got, want = got.float().cpu(), want.float()
+    special = ~torch.isfinite(want.half().float())
+    assert torch.equal(torch.nan_to_num(got[special], nan=1.5), torch.nan_to_num(want.half().float()[special], nan=1.5)), what
+    assert_tight(got[~special], want[~special], what)
+
+
+# An odd count of blocks: of the two wave groups (up to four row tiles) the second walks a block past its range, whose x is zero
+# and whose weights must not count.  k, n: the one infinite weight of its column, in the last block, before it, in the first one
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("desc_act", [False, True])
+@pytest.mark.parametrize("K", [192, 320, 352])
+def test_panel_infinite_weights(dev, bits, desc_act, K):
+    N, gs, M = 96, 32, 70
+    for position in (K - 1, K - 70, 3):
+        L = layer(9800 + K, K, N, bits, gs, desc_act, M=M)
+        k = int(torch.argsort(L["g_idx"].long(), stable=True)[position])
+        codes = torch.ones(K, dtype=torch.int32)
+        codes[k] = 3                                    # 2 x 60000 does not fit fp16; the other weights of the column are zero
+        with_weights(L, (5,), codes, 60000.0)
+        W = expected_weight(L).float()
+        assert torch.isinf(W).sum() == 1 and not torch.isnan(W).any()
+        D = to_dev(L, dev)
+        want = L["x"].float() @ W
+        for rt, split in ((1, 1), (2, 1), (4, 1), (5, 1), (8, 1), (2, 2), (3, 3)):
+            y = forward(D, _lib.select_panel(M, K, N, bits, gs, desc_act, False, rt, split))
+            assert_same_specials(y, want, f"int{bits} K={K} act={desc_act} position {position} row tiles {rt} ranges {split}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("desc_act", [False, True])
+@pytest.mark.parametrize("N", [96, 160, 192])
+def test_panel_infinite_weights_transposed(dev, bits, desc_act, N):
+    K, gs, M = 256, 64, 70
+    gy = torch.randn(M, N, generator=torch.Generator().manual_seed(1)).half()
+    for n in (N - 1, 3):
+        codes = torch.ones(K, dtype=torch.int32)
+        codes[77] = 3
+        L = with_weights(layer(9900 + N, K, N, bits, gs, desc_act, M=M), (n,), codes, 60000.0)
+        D = to_dev(L, dev)
+        want = gy.float() @ expected_weight(L).float().t()
+        for rt, split in ((1, 1), (2, 1), (4, 1), (5, 1), (8, 1), (2, 2)):
+            gx = transposed(D, gy.to(dev), _lib.select_panel(M, K, N, bits, gs, desc_act, True, rt, split))
+            assert_same_specials(gx, want, f"transposed int{bits} N={N} act={desc_act} column {n} row tiles {rt} ranges {split}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_panel_special_values_stay_in_their_rows_and_columns(dev, bits, desc_act):
+    # rows of x (of the gradient) with an infinity, both, a NaN; columns with a scale of infinity and of NaN; ragged tiles
+    K, N, gs, M = 352, 160, 32, 77
+    L = layer(9950, K, N, bits, gs, desc_act, M=M)
+    gy = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).half()
+    inf, nan = float("inf"), float("nan")
+    for rows in (L["x"], gy):
+        rows[3, 5], rows[40, 0], rows[40, -1], rows[76, -2] = inf, inf, -inf, nan
+    L["scales"][2, 7], L["scales"][-1, 100] = inf, nan
+    D, W = to_dev(L, dev), expected_weight(L).float()
+    want, want_t = L["x"].float() @ W, gy.float() @ W.t()
+    assert torch.isfinite(want).sum() == (M - 3) * (N - 2)
+    for rt, split in ((1, 1), (2, 1), (3, 2), (5, 1), (8, 2)):
+        what = f"int{bits} act={desc_act} row tiles {rt} ranges {split}"
+        y = forward(D, _lib.select_panel(M, K, N, bits, gs, desc_act, False, rt, split))
+        assert_same_specials(y, want, what)
+        gx = transposed(D, gy.to(dev), _lib.select_panel(M, K, N, bits, gs, desc_act, True, rt, split))
+        assert_same_specials(gx, want_t, "transposed " + what)
