@@ -140,9 +140,9 @@ class QuantLinear(nn.Module):
             ref = torch.arange(self.infeatures, device=g.device, dtype=torch.int64) // self.groupsize
             contiguous = bool(torch.equal(g.to(torch.int64), ref))
             if not contiguous:
-                lo, hi = int(g.min()), int(g.max())
-                if lo < 0 or hi >= self.scales.shape[0]:
-                    raise ValueError(f"g_idx values must lie in [0, {self.scales.shape[0]}), found [{lo}, {hi}]")
+                lo, hi, groups = int(g.min()), int(g.max()), math.ceil(self.infeatures / self.groupsize)
+                if lo < 0 or hi >= groups:
+                    raise ValueError(f"g_idx values must lie in [0, {groups}), found [{lo}, {hi}]")
             self._g_state = (key, contiguous)
         if self._g_state[1]:
             return None

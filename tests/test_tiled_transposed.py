@@ -229,3 +229,20 @@ def test_module_gradient_runs_fused(dev, bits, desc_act):
     L2 = layer(3720 + bits, K, N, bits, gs, desc_act, bias=True)
     q2.load_state_dict({k: L2[k] for k in ("qweight", "qzeros", "scales", "g_idx", "bias")})
     assert_tight(q2.grad_input(gy.to(dev)), gy.float() @ expected_weight(L2).float().t(), "gradient after reload")
+
+
+@pytest.mark.parametrize("M", [8, 1300])
+def test_a_copied_compact_layer_keeps_its_gradient(dev, M):
+    """A compact layer that was copied or moved looks at its g_idx again, and has no scales left to count its groups by."""
+    import copy
+
+    K, N = 2048, 4128
+    L = layer(3800, K, N, 4, 128, True, M=M)
+    q = QuantLinear(4, 128, K, N, False)
+    q.load_state_dict({k: L[k] for k in ("qweight", "qzeros", "scales", "g_idx")})
+    q = q.to(dev)
+    assert q.prepare_transposed() is not None and q.compact()
+    clone = copy.deepcopy(q)
+    gy = grad_rows(3801, M, N).to(dev)
+    assert torch.equal(clone.grad_input(gy), q.grad_input(gy))
+    assert_tight(q.grad_input(gy), gy.float().cpu() @ expected_weight(L).float().t(), "compact layer")
