@@ -85,7 +85,7 @@ class QuantLinear(nn.Module):
             self.register_buffer("bias", torch.zeros((outfeatures,), dtype=torch.float16))
         else:
             self.bias = None
-        self._g_state = None  # (g_idx identity, contiguous?) cached by _kernel_g_idx
+        self._g_state = None  # (g_idx identity, contiguous?, groups of equal size?) cached by _kernel_g_idx
         # Activation-order layers: on the first decode-size call (up to 16 rows of x), keep a second
         # copy of qweight with the input channels sorted by group (plus a [K] int32 map), which the
         # decode kernel reads faster than it can follow g_idx.  Costs the layer's packed size again in
@@ -133,17 +133,22 @@ class QuantLinear(nn.Module):
     # ------------------------------------------------------------------ forward
     def _kernel_g_idx(self):
         """``None`` when ``g_idx`` is the contiguous ``k // groupsize`` (lets the kernels skip the
-        gather), else the tensor.  Checked once per distinct g_idx storage."""
+        gather), else the tensor.  Checked once per distinct g_idx storage: the first call of a layer waits for the GPU
+        here, once for all that its routes and copies want to know of g_idx."""
         g = self.g_idx
         key = (g.data_ptr(), g._version, g.device)
         if self._g_state is None or self._g_state[0] != key:
-            ref = torch.arange(self.infeatures, device=g.device, dtype=torch.int64) // self.groupsize
-            contiguous = bool(torch.equal(g.to(torch.int64), ref))
+            K, gs = self.infeatures, self.groupsize
+            groups = math.ceil(K / gs)
+            host = g.detach().cpu().numpy()     # (some tens of KB; a dozen small kernels for the same answers take longer)
+            contiguous = np.array_equal(host, np.repeat(np.arange(groups, dtype=np.int32), gs)[:K])
+            whole = K % gs == 0
             if not contiguous:
-                lo, hi, groups = int(g.min()), int(g.max()), math.ceil(self.infeatures / self.groupsize)
+                lo, hi = int(host.min()), int(host.max())
                 if lo < 0 or hi >= groups:
                     raise ValueError(f"g_idx values must lie in [0, {groups}), found [{lo}, {hi}]")
-            self._g_state = (key, contiguous)
+                whole = bool((np.bincount(host, minlength=groups) == gs).all())
+            self._g_state = (key, contiguous, whole)
         if self._g_state[1]:
             return None
         if not g.is_contiguous() or g.data_ptr() % 16 != 0 or g.dtype != torch.int32:
@@ -167,24 +172,24 @@ class QuantLinear(nn.Module):
             self._sorted = (key, tensors)
         return self._sorted[1]
 
-    def _whole_groups(self, g):
+    def _whole_groups(self):
         """The one check the preparation kernels cannot make: every group holds exactly ``groupsize`` channels."""
-        K, gs = self.infeatures, self.groupsize
-        counts = torch.bincount(g.to(torch.int64), minlength=K // gs)
-        return counts.numel() == K // gs and bool((counts == gs).all())
+        self._kernel_g_idx()
+        return self._g_state[2]
 
     def _sort_on_gpu(self, q, g):
         """``pack.sort_channels_by_group`` through the library's own kernels (gptq_hip_sort_channels)."""
         K, gs = self.infeatures, self.groupsize
         klane = 8 if self.bits == 4 else 32
-        if K >= 65536 or K % gs != 0 or gs % klane != 0 or not self._whole_groups(g):
+        if K >= 65536 or K % gs != 0 or gs % klane != 0 or not self._whole_groups():
             return None
         return ops.sort_channels(q, g, self.bits, self.groupsize)
 
     def prepare_tiled(self):
         """Builds (once per distinct storage of the packed tensors) the layer in the tiled format; returns
         ``(qtile, sz, xsrc, kinv)`` or None when the format does not cover the layer.  ``forward`` calls this
-        lazily; loaders may call it up front (it synchronises once, for the check of the group sizes)."""
+        lazily; loaders may call it up front (the first look at g_idx, for the check of the group sizes, waits for
+        the GPU)."""
         if self._compact:
             return self._tiled[1]
         g = self._kernel_g_idx()
@@ -194,7 +199,7 @@ class QuantLinear(nn.Module):
             tensors = None
             if (self.qweight.device.type == "cuda"
                     and tiled_qualifies(self.infeatures, self.outfeatures, self.bits, self.groupsize)
-                    and (g is None or self._whole_groups(g))):
+                    and (g is None or self._whole_groups())):
                 tensors = ops.tile_prepare(self.qweight, self.qzeros, self.scales, g, self.bits, self.groupsize)
             self._tiled = (key, tensors)
         return self._tiled[1]

@@ -5,7 +5,7 @@ import torch
 
 from autogptq.tvm_amd import _lib, ops
 from autogptq.tvm_amd.qlinear import QuantLinear
-from tests.parity_util import assert_tight, expected_output, layer
+from tests.parity_util import assert_tight, expected_output, expected_weight, layer
 
 pytestmark = pytest.mark.gpu
 
@@ -206,3 +206,24 @@ def test_methods_replaced_on_the_classes_are_seen(dev, monkeypatch):
         assert python_frames(call) == ["<lambda>"]            # untouched again: the call in C
     q._call_impl = lambda *a: "instance"
     assert q(x) == "instance"
+
+
+@pytest.mark.parametrize("M,desc_act", [(1, True), (9, True), (600, True), (600, False)])
+def test_the_first_call_of_a_layer_waits_for_the_gpu_once(dev, M, desc_act):
+    import warnings
+
+    L = layer(9730 + M, 2048, 4128, 4, 128, desc_act, M=M, bias=True)
+    q, x = module_of(L, dev), L["x"].to(dev).requires_grad_(True)
+    gy = torch.randn(M, 4128, device=dev, dtype=torch.float16)
+    torch.cuda.synchronize()
+    with warnings.catch_warnings(record=True) as seen:
+        warnings.simplefilter("always")
+        torch.cuda.set_sync_debug_mode("warn")
+        try:
+            y = q(x)
+            gx, = torch.autograd.grad(y, x, gy)
+        finally:
+            torch.cuda.set_sync_debug_mode("default")
+    assert sum("called a synchronizing" in str(w.message) for w in seen) == 1
+    assert_tight(y.detach(), expected_output(L), "first call")
+    assert_tight(gx, gy.float().cpu() @ expected_weight(L).float().t(), "first gradient")

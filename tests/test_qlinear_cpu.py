@@ -146,3 +146,24 @@ def test_compilers_see_the_methods_of_a_module():
     want = net(x)
     assert torch.equal(torch.compile(net, backend="eager", fullgraph=True)(x), want)
     assert QuantLinear.__call__ is torch.nn.Module.__call__
+
+
+def test_what_a_layer_finds_out_about_its_g_idx():
+    K, gs = 256, 64
+    order = torch.randperm(K, generator=torch.Generator().manual_seed(1))
+    contiguous = torch.arange(K, dtype=torch.int32) // gs
+    uneven = contiguous.clone()
+    uneven[-1] = 0
+    for g, none, whole in ((contiguous, True, True), (contiguous.flip(0).contiguous(), False, True), (contiguous[order], False, True),
+                           (uneven, False, False), (torch.zeros(K, dtype=torch.int32), False, False)):
+        q = QuantLinear(4, gs, K, 32, False)
+        q.g_idx = g
+        assert (q._kernel_g_idx() is None) == none and q._whole_groups() == whole
+    for bad, what in ((contiguous - 1, r"found \[-1, 2\]"), (contiguous + 1, r"in \[0, 4\), found \[1, 4\]")):
+        q.g_idx = bad
+        with pytest.raises(ValueError, match=what):
+            q._kernel_g_idx()
+    q = QuantLinear(4, 96, K, 32, False)            # a last group that is shorter
+    assert q._kernel_g_idx() is None and not q._whole_groups()
+    q = QuantLinear(4, -1, K, 32, False)
+    assert q._kernel_g_idx() is None and q._whole_groups()
