@@ -8,11 +8,13 @@
 // is a copy into LDS that the wave counts itself; they run a block further ahead than x, because their dequantisation is
 // spread between the matrix instructions of the step before.
 //
-// What bounds it (measured on MI355X, 4096 rows on 8192 x 28672 int4, RT = 8): the chip's power.  Matrix instructions alone
-// sustain 1840 TFLOP/s in the 16 x 16 x 32 shape and 1610 in the 32 x 32 x 16 one (which reads and writes each result twice
-// as often per product), hence the former; the kernel reaches 1400, dense library products of that size 1440 to 1480, and
-// taking out the requests or the dequantisation gives back what their share of the energy is (14 % and 17 % at RT = 4).
-// The matmul kernel of gptq_tiled.hip, whose workgroups share nothing, took 2050 us for what takes 1385 here.
+// What bounds it (MI355X, 4096 rows on 8192 x 28672 int4, RT = 8): the chip's power.
+// It runs at 1.56 of 2.4 GHz with the matrix pipes busy in 71 % of the cycles.  Matrix instructions alone sustain 1950 to 1990
+// TFLOP/s in the 16 x 16 x 32 shape and 1700 to 1750 in the 32 x 32 x 16 one (which reads and writes each result twice as often
+// per product), hence the former; on zeros, at full clock, both 2430 to 2460.  The kernel reaches 1320 to 1400, the dense library
+// product of that size 1210.  Taking out the requests of the walk or the dequantisation gives back 15 to 18 % and 13 % of the time
+// (RT = 4: 19 % and 16 %; three bits at RT = 5: 10 % and 26 %).
+// The matmul kernel of gptq_tiled.hip, whose workgroups share nothing, takes 2000 us for what takes 1410 here.
 // Below that, instruction issue: a wave alone on its SIMD issues an instruction per 5 clocks, so that two fit behind a
 // 16-clock matrix instruction.  RT = 8 has 2.3 of them per matrix instruction, RT = 4 has 3.7: up to four row tiles two
 // groups of four waves therefore take every other block each (two waves per SIMD, 256 registers each) and add up at the end.
@@ -536,7 +538,7 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
 
 // xs[m][p] = x[m][xsrc[p]]: the activations in the order of the tiled copy.  A workgroup takes ROWS rows and one of gridDim.y
 // parts of K: the rows go to LDS with coalesced loads, the gather reads LDS, and the index vectors are read once for all of
-// them (2048 x 4096: 6.5 us, 10 of its 33 MB of traffic per us; a pass that writes ready-made fragments took 21).
+// them (2048 x 4096: 7.4 to 9.8 us for 33 MB of traffic; a pass that writes ready-made fragments took 21).
 template <int ROWS>
 __global__ __launch_bounds__(256) void panel_gather_kernel(const _Float16 *__restrict__ x, const int32_t *__restrict__ xsrc,
                                                            _Float16 *__restrict__ xs, int M, int K)
@@ -563,7 +565,7 @@ __global__ __launch_bounds__(256) void panel_gather_kernel(const _Float16 *__res
 }
 
 // The way back for the transposed product: gx[m][xsrc[p]] = gs[m][p], or the sum of the K ranges' partial results.  A row is
-// put in order in LDS and leaves it in one piece (2048 x 4096: 6 us; stores of two bytes from the product itself cost 31).
+// put in order in LDS and leaves it in one piece (2048 x 4096: 6.1 to 8.3 us; stores of two bytes from the product itself cost 31).
 __global__ __launch_bounds__(256) void panel_scatter_kernel(const _Float16 *__restrict__ gs, const float *__restrict__ partial,
                                                             const int32_t *__restrict__ xsrc, _Float16 *__restrict__ gx, int M,
                                                             int K, int split)

@@ -58,9 +58,11 @@ enum {
                                    out evenly over grid_x workgroups of 16 waves, all of K staged per workgroup
                                    (k_chunk = blocks of 128 channels per unit and wave); chosen for layers of up to
                                    4096 columns and fewer than 4096 channels */
-    GPTQ_HIP_KERNEL_PANEL = 6 /* the same layer for long prompts and training batches: a workgroup of four waves takes
-                                   32 * row_tiles rows (shared in LDS) x 256 columns (64 per wave), k_chunk blocks of 64
-                                   channels; grid_x column and m_blocks row positions; split_k > 1 adds a reduce launch */
+    GPTQ_HIP_KERNEL_PANEL = 6 /* the same layer for long prompts and training batches: a workgroup takes 32 * row_tiles
+                                   (1..8) rows, shared in LDS, x 256 columns (waves_n = 4 waves of 64 each), k_chunk blocks of
+                                   64 channels; up to four row tiles two such groups of waves (waves_k = 2) take every
+                                   other block each.  grid_x column and m_blocks row positions; an activation order adds a
+                                   pass over x (or gx), split_k > 1 a reduce launch */
 };
 
 /* What the dispatcher decided for one problem; filled by gptq_hip_select. */
@@ -240,7 +242,8 @@ int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int group_size, 
 
 /*
  * y = x @ W (+ bias) on a layer in the tiled format, any M; replaces the same handler call as gptq_hip_gemm
- * (pycuda_warpper.py:138, qlinear_tvm.py:123,150).  x and y are in the layer's own channel order (xsrc = kinv =
+ * (pycuda_warpper.py:138, qlinear_tvm.py:123,150).  x is 16-byte aligned, y 8-byte aligned (gy and gx below likewise;
+ * GPTQ_HIP_ERR_BAD_ARG otherwise).  x and y are in the layer's own channel order (xsrc = kinv =
  * NULL means no activation order; pass both or neither).  plan: NULL = what gptq_hip_select_route names for a layer
  * with this copy alone, PANEL included; where the workspace does not hold that plan's bytes, gptq_hip_select_tiled.  workspace:
  * plan.workspace_bytes (none for most decode plans).  Decode plans: one launch; matmul plans: two
