@@ -10,6 +10,7 @@
 // zero-initialised tensor per (device, stream), grown on demand; the kernels leave its counters at zero.
 // Only the CUDA (= HIP on ROCm) dispatch key gets kernels; the CPU key gets functions that say so and raise.
 #include <ATen/ATen.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/custom_class.h>
@@ -95,6 +96,24 @@ int Bound::launch(const Tensor &x, void *y, void *stream) const
                                (const uint16_t *)ptr(e), ptr(bias), y, wsp, wsb, M, K, N, bits, group_size, &plan, stream);
 }
 
+Tensor dispatch(const Bound &q, const Tensor &x)
+{
+    auto op = [](const char *name) { return c10::Dispatcher::singleton().findSchemaOrThrow(name, ""); };
+    if (q.kind == 0) {
+        using Fn = Tensor(const Tensor &, const Tensor &, const Tensor &, const Tensor &, const OptTensor &, const OptTensor &, int64_t, int64_t);
+        static const auto gemm = op("gptq_hip::gemm").typed<Fn>();
+        return gemm.call(x, q.a, q.b, q.c, q.d, q.bias, q.bits, q.group_size);
+    }
+    if (q.kind == 1) {
+        using Fn = Tensor(const Tensor &, const Tensor &, const Tensor &, const Tensor &, const Tensor &, const OptTensor &, int64_t, int64_t);
+        static const auto gemm_sorted = op("gptq_hip::gemm_sorted").typed<Fn>();
+        return gemm_sorted.call(x, q.a, q.b, q.c, *q.d, q.bias, q.bits, q.group_size);
+    }
+    using Fn = Tensor(const Tensor &, const Tensor &, const Tensor &, const OptTensor &, const OptTensor &, const OptTensor &, int64_t, int64_t);
+    static const auto gemm_tiled = op("gptq_hip::gemm_tiled").typed<Fn>();
+    return gemm_tiled.call(x, q.a, q.b, q.d, q.e, q.bias, q.bits, q.group_size);
+}
+
 }  // namespace gptq_torch
 
 namespace {
@@ -160,7 +179,8 @@ Tensor gemm(const Tensor &x, const Tensor &qweight, const Tensor &qzeros, const 
     int rc = gptq_hip_select((int)s.M, (int)s.K, (int)s.N, (int)bits, (int)group_size, has(g_idx), &plan);
     raise(rc, "gptq_hip_gemm", s.M, s.K, s.N, bits, group_size);
     const WorkspaceLease ws(x, plan.workspace_bytes, stream);
-    rc = gptq_hip_gemm_plan(x.data_ptr(), (const int32_t *)qweight.data_ptr(), (const int32_t *)qzeros.data_ptr(),
+    const Tensor xa = aligned(x);
+    rc = gptq_hip_gemm_plan(xa.data_ptr(), (const int32_t *)qweight.data_ptr(), (const int32_t *)qzeros.data_ptr(),
                             scales.data_ptr(), (const int32_t *)ptr(g_idx), ptr(bias), y.data_ptr(),
                             ws.data(), ws.size(), (int)s.M,
                             (int)s.K, (int)s.N, (int)bits, (int)group_size, &plan, stream);
@@ -191,7 +211,8 @@ Tensor gemm_sorted(const Tensor &x, const Tensor &qweight_sorted, const Tensor &
     const size_t need_ws = std::max((size_t)plan.workspace_bytes,
                                     gptq_hip_sorted_workspace_bytes((int)s.M, (int)s.K, (int)s.N, (int)bits, (int)group_size));
     const WorkspaceLease ws(x, need_ws, stream);
-    rc = gptq_hip_gemm_sorted(x.data_ptr(), (const int32_t *)qweight_sorted.data_ptr(), (const int32_t *)qzeros.data_ptr(),
+    const Tensor xa = aligned(x);
+    rc = gptq_hip_gemm_sorted(xa.data_ptr(), (const int32_t *)qweight_sorted.data_ptr(), (const int32_t *)qzeros.data_ptr(),
                               scales.data_ptr(), (const int32_t *)kmap.data_ptr(), ptr(bias), y.data_ptr(),
                               ws.data(), ws.size(), (int)s.M,
                               (int)s.K, (int)s.N, (int)bits, (int)group_size, &plan, stream);
@@ -248,7 +269,7 @@ Tensor gemm_tiled(const Tensor &x, const Tensor &qtile, const Tensor &sz, const 
     void *stream = (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device()).stream();
     raise(q.choose(), "gptq_hip_gemm_tiled", q.M, q.K, q.N, bits, group_size);
     check_groups(q.K, sz, group_size);
-    raise(q.launch(x, y.data_ptr(), stream), "gptq_hip_gemm_tiled", q.M, q.K, q.N, bits, group_size);
+    raise(q.launch(aligned(x), y.data_ptr(), stream), "gptq_hip_gemm_tiled", q.M, q.K, q.N, bits, group_size);
     return y;
 }
 
@@ -330,7 +351,7 @@ struct Layer : torch::CustomClassHolder {
             Tensor y = at::empty({fast_rows, q.N}, x.options());
             const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
             void *stream = (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device()).stream();
-            raise(q.launch(x, y.data_ptr(), stream), "gptq_hip.Layer.forward", fast_rows, q.K, q.N, q.bits, q.group_size);
+            raise(q.launch(aligned(x), y.data_ptr(), stream), "gptq_hip.Layer.forward", fast_rows, q.K, q.N, q.bits, q.group_size);
             return y;
         }
         // the checked path; what it selects is what the operators select

@@ -17,6 +17,9 @@ using OptTensor = std::optional<Tensor>;
 inline const void *ptr(const OptTensor &t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
 inline bool has(const OptTensor &t) { return t.has_value() && t->defined(); }
 
+// x, or a copy of it where the kernels' 16-byte loads ask for one (a contiguous view at an odd offset)
+inline Tensor aligned(const Tensor &x) { return (uintptr_t)x.data_ptr() % 16 == 0 ? x : x.clone(); }
+
 void raise(int rc, const char *what, int64_t M, int64_t K, int64_t N, int64_t bits, int64_t gs);
 
 int workspace_kind(const gptq_hip_plan &plan);
@@ -56,6 +59,9 @@ struct Bound {
     // on that device, which is the current one.  A status of the library.
     int launch(const Tensor &x, void *y, void *stream) const;
 };
+
+// the same product as the operator torch.ops.gptq_hip.*, through the dispatcher
+Tensor dispatch(const Bound &q, const Tensor &x);
 
 // the operators' checks of a layer's tensors (devices, dtypes, shapes), once, when they are bound
 void check_bound(const Bound &q);

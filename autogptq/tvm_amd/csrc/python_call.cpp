@@ -200,10 +200,38 @@ PyObject *bound_call(PyObject *self, PyObject *args, PyObject *kwargs)
     TORCH_CHECK(PyTuple_GET_SIZE(args) == 1 && (!kwargs || PyDict_GET_SIZE(kwargs) == 0) && THPVariable_Check(PyTuple_GET_ITEM(args, 0)),
                 "one tensor is expected");
     const Tensor x = THPVariable_Unpack(PyTuple_GET_ITEM(args, 0));
+    // what is recorded or handled by something else (torch.jit.trace, dispatch modes, tensor subclasses) is the operator
+    if (!THPVariable_CheckExact(PyTuple_GET_ITEM(args, 0)) || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+        torch::jit::tracer::isTracing())
+        return THPVariable_Wrap(dispatch(q, x));
     TORCH_CHECK(x.is_cuda() && x.device() == q.a.device(), "x is on ", x.device(), ", the layer on ", q.a.device(),
                 ": the GPTQ kernels run on a ROCm GPU only and there is no CPU fallback");
-    TORCH_CHECK(takes(q, x), "x must be a contiguous fp16 tensor, 16-byte aligned, of ", q.M, " rows of ", q.K);
-    return apply(q, x);
+    const Tensor rows = x.is_contiguous() ? aligned(x) : x;
+    TORCH_CHECK(takes(q, rows), "x must be a contiguous fp16 tensor of ", q.M, " rows of ", q.K);
+    return apply(q, rows);
+    END_HANDLE_TH_ERRORS
+}
+
+// aside(fn, *args): fn(*args) hidden from torch.jit.trace and from dispatch modes.  A layer decides its routes and prepares its
+// copies so: a recording that holds the allocations of a copy, and not the kernels that fill it, replays on empty memory.
+PyObject *aside(PyObject *, PyObject *args)
+{
+    HANDLE_TH_ERRORS
+    if (PyTuple_GET_SIZE(args) < 1) {
+        PyErr_SetString(PyExc_TypeError, "a callable is expected");
+        return nullptr;
+    }
+    THPObjectPtr rest(PyTuple_GetSlice(args, 1, PyTuple_GET_SIZE(args)));
+    if (!rest) return nullptr;
+    PyObject *fn = PyTuple_GET_ITEM(args, 0);
+    if (!c10::impl::TorchDispatchModeTLS::any_modes_set() && !torch::jit::tracer::isTracing()) return PyObject_CallObject(fn, rest.get());
+    struct Untraced {
+        std::shared_ptr<torch::jit::tracer::TracingState> state = torch::jit::tracer::getTracingState();
+        Untraced() { torch::jit::tracer::setTracingState(nullptr); }
+        ~Untraced() { torch::jit::tracer::setTracingState(state); }
+    } untraced;
+    const c10::impl::ExcludeDispatchKeyGuard no_modes(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot}));
+    return PyObject_CallObject(fn, rest.get());
     END_HANDLE_TH_ERRORS
 }
 
@@ -246,7 +274,8 @@ PyObject *install(PyObject *, PyObject *cls)
     END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef functions[] = {{"install", install, METH_O, "Makes the call in C the one of a QuantLinear class."}, {nullptr, nullptr, 0, nullptr}};
+PyMethodDef functions[] = {{"aside", aside, METH_VARARGS, "aside(fn, *args): fn(*args), hidden from tracing and dispatch modes."},
+                           {"install", install, METH_O, "Makes the call in C the one of a QuantLinear class."}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "gptq_hip_call", "the QuantLinear call in C", -1, functions};
 
 }  // namespace

@@ -29,6 +29,11 @@ def _need_gpu(name: str, t: torch.Tensor, dtype: torch.dtype):
         raise ValueError(f"{name} must be contiguous")
 
 
+def aligned(t: torch.Tensor) -> torch.Tensor:
+    """``t``, or a copy of it where the kernels' 16-byte loads ask for one (a contiguous view at an odd offset)."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _stream(device: torch.device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
@@ -436,14 +441,14 @@ def _register_torch_ops():
                    "int bits, int group_size) -> Tensor")
         lib.define("dequant(Tensor qweight, Tensor qzeros, Tensor scales, Tensor? g_idx, int bits, int group_size) "
                    "-> Tensor")
-        lib.impl("gemm", lambda x, qw, qz, sc, g, b, bits, gs: gemm(x, qw, qz, sc, g, b, bits, gs), "CUDA")
-        lib.impl("gemm_sorted", lambda x, qw, qz, sc, km, b, bits, gs: gemm_sorted(x, qw, qz, sc, km, b, bits, gs), "CUDA")
-        lib.impl("gemm_tiled", lambda x, qt, sz, xs, ki, b, bits, gs: gemm_tiled(x, qt, sz, xs, ki, b, bits, gs), "CUDA")
+        lib.impl("gemm", lambda x, qw, qz, sc, g, b, bits, gs: gemm(aligned(x), qw, qz, sc, g, b, bits, gs), "CUDA")
+        lib.impl("gemm_sorted", lambda x, qw, qz, sc, km, b, bits, gs: gemm_sorted(aligned(x), qw, qz, sc, km, b, bits, gs), "CUDA")
+        lib.impl("gemm_tiled", lambda x, qt, sz, xs, ki, b, bits, gs: gemm_tiled(aligned(x), qt, sz, xs, ki, b, bits, gs), "CUDA")
         lib.impl("dequant", lambda qw, qz, sc, g, bits, gs: dequant(qw, qz, sc, g, bits, gs), "CUDA")
         # CPU tensors reach the same functions, whose first check raises ("no CPU fallback")
-        lib.impl("gemm", lambda x, qw, qz, sc, g, b, bits, gs: gemm(x, qw, qz, sc, g, b, bits, gs), "CPU")
-        lib.impl("gemm_sorted", lambda x, qw, qz, sc, km, b, bits, gs: gemm_sorted(x, qw, qz, sc, km, b, bits, gs), "CPU")
-        lib.impl("gemm_tiled", lambda x, qt, sz, xs, ki, b, bits, gs: gemm_tiled(x, qt, sz, xs, ki, b, bits, gs), "CPU")
+        lib.impl("gemm", lambda x, qw, qz, sc, g, b, bits, gs: gemm(aligned(x), qw, qz, sc, g, b, bits, gs), "CPU")
+        lib.impl("gemm_sorted", lambda x, qw, qz, sc, km, b, bits, gs: gemm_sorted(aligned(x), qw, qz, sc, km, b, bits, gs), "CPU")
+        lib.impl("gemm_tiled", lambda x, qt, sz, xs, ki, b, bits, gs: gemm_tiled(aligned(x), qt, sz, xs, ki, b, bits, gs), "CPU")
         lib.impl("dequant", lambda qw, qz, sc, g, bits, gs: dequant(qw, qz, sc, g, bits, gs), "CPU")
         keep.append(lib)
     meta = torch.library.Library("gptq_hip", "IMPL", "Meta")

@@ -19,11 +19,6 @@ from . import _lib, ops
 from .pack import pack_qweight, pack_qzeros, tiled_qualifies
 
 
-def _aligned(t: torch.Tensor) -> torch.Tensor:
-    """``t``, or a copy of it where the kernels' 16-byte loads ask for one (a contiguous view at an odd offset)."""
-    return t if t.data_ptr() % 16 == 0 else t.clone()
-
-
 class _ProductWithInputGrad(torch.autograd.Function):
     """The product with a gradient for x (the packed weights are constants): grad_x = grad_y @ W^T, which
     is what the reference's Triton back end offers for training on top of quantised layers
@@ -229,7 +224,7 @@ class QuantLinear(nn.Module):
             gy = gy.half()
         if not gy.is_contiguous():
             gy = gy.contiguous()
-        gy = _aligned(gy)
+        gy = ops.aligned(gy)
         M = gy.size(0)
         # The panel kernel where the library says so; else the matmul kernel's transposed form below the switch.  Measured on
         # MI355X (us, eager, int4 with an activation order; the latter against dequant + library GEMM):
@@ -398,7 +393,8 @@ class QuantLinear(nn.Module):
         r = self._routes.get(M)
         if r is not None and self._fresh(r):
             return r
-        what, fn = self._route(M)
+        # (a route is not part of what is being recorded, nor is a copy that it prepares)
+        what, fn = self._route(M) if ops.CALL is None else ops.CALL.aside(self._route, M)
         w = self._watched()               # (read after routing: the preparations may have re-made g_idx)
         r = (w, sum(t._version for t in w), what, fn)
         self._routes[M] = r
@@ -424,7 +420,7 @@ class QuantLinear(nn.Module):
         M = x2.shape[0]
         if M == 0:
             return x2.new_empty((0, self.outfeatures))
-        return self._routed(M)[3](_aligned(x2))
+        return self._routed(M)[3](x2)
 
     def dequantize(self) -> torch.Tensor:
         """fp16 [infeatures, outfeatures], the weight the reference materialises on every call."""

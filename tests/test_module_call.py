@@ -171,6 +171,9 @@ def test_rows_at_an_odd_offset_are_taken(dev, M):
         odd = torch.empty(M * K + 8, dtype=torch.float16, device=dev)[offset:offset + M * K].view(M, K).copy_(x)
         assert odd.data_ptr() % 16 and odd.is_contiguous()
         assert torch.equal(q(odd), want) and torch.equal(q(odd.view(M, 1, K)).view(M, N), want)
+        if q.route(M) == "tiled":
+            qtile, sz, xsrc, kinv = q.prepare_tiled()
+            assert torch.equal(torch.ops.gptq_hip.gemm_tiled(odd, qtile, sz, xsrc, kinv, q.bias, 4, 128), want)
         odd_t = torch.empty(M * N + 8, dtype=torch.float16, device=dev)[offset:offset + M * N].view(M, N).copy_(gy)
         assert torch.equal(q.grad_input(odd_t), want_t)
         xg = odd.clone().requires_grad_(True)
@@ -227,3 +230,51 @@ def test_the_first_call_of_a_layer_waits_for_the_gpu_once(dev, M, desc_act):
     assert sum("called a synchronizing" in str(w.message) for w in seen) == 1
     assert_tight(y.detach(), expected_output(L), "first call")
     assert_tight(gx, gy.float().cpu() @ expected_weight(L).float().t(), "first gradient")
+
+
+@pytest.mark.parametrize("bits,K,M,desc_act,path", [(4, 1024, 4, True, "tiled"), (3, 4224, 12, True, "sorted"), (4, 1024, 12, False, "plain")])
+@pytest.mark.parametrize("known", [False, True])
+def test_what_records_a_call_sees_the_operator(dev, bits, K, M, desc_act, path, known):
+    """torch.jit.trace, dispatch modes, make_fx and fake tensors get the operator of the route, whether the layer knows the row
+    count already or has its copies to prepare: not a constant, and no allocation without what fills it."""
+    import warnings
+
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    N = 416
+    L = layer(4300 + M, K, N, bits, 128, desc_act, M=M, bias=True)
+    x = L["x"].to(dev)
+    other = torch.randn_like(x)
+    one = module_of(L, dev)
+    first, want = one(x), one(other)
+
+    def module():
+        q = module_of(L, dev).eval()
+        if known:
+            assert q.route(M) == path and torch.equal(q(x), first) and torch.equal(q(x), first)
+        return q
+
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        traced = torch.jit.trace(module(), x, check_trace=False)
+    assert torch.equal(traced(other), want) and torch.equal(traced(x), first)
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    names, q = [], module()
+    with Seen():
+        assert torch.equal(q(x), first)
+    assert [n for n in names if n.startswith("gptq_hip.gemm")]
+    graph = make_fx(module())(x)
+    assert torch.equal(graph(other), want) and any(str(n.target).startswith("gptq_hip.gemm") for n in graph.graph.nodes)
+    q = module()
+    with FakeTensorMode(allow_non_fake_inputs=True) as fake:
+        assert q(fake.from_tensor(x)).shape == (M, N)
+    assert torch.equal(q(x), first)
+    with pytest.raises(RuntimeError):                       # (no rule for it, and never was one)
+        torch.func.vmap(module())(torch.stack((x, other)))

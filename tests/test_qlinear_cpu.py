@@ -125,18 +125,6 @@ def test_find_layers_matches_the_reference_helper_on_a_nested_model():
     assert find_layers(torch.nn.ReLU()) == {}
 
 
-def test_the_product_is_handed_aligned_rows():
-    """The kernels load 16 bytes at a time; a contiguous view at an odd offset of a larger tensor is copied first."""
-    q = QuantLinear(4, 32, 64, 32, False)
-    seen = []
-    q._routed = lambda M: (None, None, "plain", lambda x2: seen.append(x2) or x2[:, :32])
-    x = torch.randn(8 * 64 + 8).half()
-    for offset in range(8):
-        rows = x[offset:offset + 8 * 64].view(8, 64)
-        assert torch.equal(q(rows), rows[:, :32])
-        assert seen[-1].data_ptr() % 16 == 0 and (offset or seen[-1].data_ptr() == rows.data_ptr())
-
-
 def test_compilers_see_the_methods_of_a_module():
     """The call in C stands beside the methods: a module whose product can be traced compiles as one graph."""
     q = QuantLinear(4, 32, 64, 32, False)
