@@ -35,7 +35,8 @@ def aligned(t: torch.Tensor) -> torch.Tensor:
 
 
 def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    # (the raw handle: torch.compile, which runs this between two graphs, has no cuda_stream for the stream object it models)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(device.index))
 
 
 FUSED_BITS = (3, 4)        # widths the matmul kernels on the checkpoint layout (and its sorted copy) cover
@@ -85,7 +86,7 @@ def _workspace(device: torch.device, nbytes: int, kind: int = 0):
     if not nbytes:
         yield None
         return
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream, kind)
+    key = (device.index, _stream(device).value, kind)
     ws = _workspaces.setdefault(key, _Workspace())
     with ws.busy:
         if ws.bytes is None or ws.bytes.numel() < nbytes:

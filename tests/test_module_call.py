@@ -278,3 +278,20 @@ def test_what_records_a_call_sees_the_operator(dev, bits, K, M, desc_act, path, 
     assert torch.equal(q(x), first)
     with pytest.raises(RuntimeError):                       # (no rule for it, and never was one)
         torch.func.vmap(module())(torch.stack((x, other)))
+
+
+@pytest.mark.parametrize("known", [False, True])
+def test_compiled_models_run_the_layer_between_their_graphs(dev, known):
+    import warnings
+
+    L = layer(4350, 512, 96, 4, 128, True, M=4, bias=True)
+    q, x = module_of(L, dev).eval(), L["x"].to(dev)
+    net = torch.nn.Sequential(q, torch.nn.ReLU())
+    want = torch.relu(module_of(L, dev)(x))
+    if known:
+        assert torch.equal(net(x), want)
+    with warnings.catch_warnings(), torch.no_grad():
+        warnings.simplefilter("ignore")
+        compiled = torch.compile(net, backend="eager")
+        assert torch.equal(compiled(x), want) and torch.equal(compiled(2 * x), net(2 * x))
+    torch._dynamo.reset()
