@@ -705,6 +705,21 @@ double tiled_us(const gptq_hip_plan &p, int bits, bool transposed, double out_el
            (2.9 + 0.4 * act_order) * 1e-6 * in_elems;
 }
 
+// What both leave out and a short call is decided by, from 18900 calls of 9 to 64 rows drawn at random with their weights cold:
+// eight bits stream twice as long as the walk computes; a gradient with an activation order is put in order by a
+// workgroup per row, few of them for a long row; and the matmul kernel reads up to 16 rows of x in the layer's own order
+// itself, without its pack pass.  Calls that the choice makes slower by more than 3 %, without these / with them on another draw:
+// forward 9 to 16 rows 24 / 14 %, 17 to 64 rows 10 / 7 %, gradient 11 / 4 % and 7 / 4 % (15616 x 3008 at 8 bits, gradient of 18
+// rows: 26.6 us on the panel kernel, 19.2 on the other).
+double short_panel_us(double us, int K, int N, int bits, bool transposed, bool act_order)
+{
+    return us + (bits == 8 ? 0.06e-6 * K * (double)N : 0.0) + (transposed && act_order ? 1.6 + 0.27e-3 * K : 0.0);
+}
+double short_tiled_us(double us, int M, bool transposed, bool act_order)
+{
+    return us - (M <= 16 && !transposed && !act_order ? 2.0 : 0.0);
+}
+
 }  // namespace
 
 extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_size, unsigned flags, int row_tiles, int split_k,
@@ -741,10 +756,13 @@ extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_si
             const int rc = transposed ? gptq_hip_select_tiled_transposed(M, K, N, bits, group_size, &other)
                                       : gptq_hip_select_tiled(M, K, N, bits, group_size, &other);
             if (rc == GPTQ_HIP_OK && other.kernel != GPTQ_HIP_KERNEL_TILED) return GPTQ_HIP_ERR_UNSUPPORTED;
-            // (short prompts have other copies to run on, too: there the matmul kernel has to be clearly the slower one)
-            if (rc == GPTQ_HIP_OK &&
-                best > (M <= 128 ? 0.95 : 1.0) * tiled_us(other, bits, transposed, out_elems, (double)M * red, act))
-                return GPTQ_HIP_ERR_UNSUPPORTED;
+            if (rc == GPTQ_HIP_OK) {
+                const double tiled = tiled_us(other, bits, transposed, out_elems, (double)M * red, act);
+                // (short prompts have other copies to run on, too: there the matmul kernel has to be clearly the slower one)
+                if (best > (M <= 128 ? 0.95 : 1.0) * tiled) return GPTQ_HIP_ERR_UNSUPPORTED;
+                if (M <= 64 && short_panel_us(best, K, N, bits, transposed, act) > short_tiled_us(tiled, M, transposed, act))
+                    return GPTQ_HIP_ERR_UNSUPPORTED;
+            }
         }
     }
     if (rt > gptq::kPanelMaxTiles || !gptq::panel_addresses(rt, red)) return GPTQ_HIP_ERR_UNSUPPORTED;
@@ -925,7 +943,11 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
     // own row count is a wish, and comes first.
     const bool past = sw[which] && M >= sw[which];
     if (past && sw[which] != kDefaultSwitch[which]) return GPTQ_HIP_OK;
-    if (take_panel()) return GPTQ_HIP_OK;
+    // Up to 16 rows the kernels on the other copies, where the rule has them, keep their calls: against them it is 0.71 to 1.08 x
+    // as fast (0.92 on the mean) on drawn 3-bit layers without an activation order, level on 4-bit ones (0.85 to 1.32 x) and on 3-bit
+    // ones with an order (0.93 to 1.05 x), and no reason for another copy; on 4-bit layers with one it is ahead (0.86 to 1.38, 1.12).
+    const bool others = !tiled && M <= 16 && fused_bits && !(act && bits == 4) && (copies & (GPTQ_HIP_COPY_CHECKPOINT | GPTQ_HIP_COPY_SORTED));
+    if (!others && take_panel()) return GPTQ_HIP_OK;
     if (past) return GPTQ_HIP_OK;
     if (tiled && take_tiled()) return GPTQ_HIP_OK;
     if (!fused_bits) return GPTQ_HIP_OK;
@@ -944,6 +966,7 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
         memset(&route->plan, 0, sizeof(route->plan));
         if (rc != GPTQ_HIP_ERR_UNSUPPORTED) return rc;
     }
+    if (others && take_panel()) return GPTQ_HIP_OK;
     return GPTQ_HIP_OK;   // no fused kernel covers the call: dequant + library GEMM
 }
 

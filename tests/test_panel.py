@@ -347,3 +347,30 @@ def test_panel_special_values_stay_in_their_rows_and_columns(dev, bits, desc_act
         assert_same_specials(y, want, what)
         gx = transposed(D, gy.to(dev), _lib.select_panel(M, K, N, bits, gs, desc_act, True, rt, split))
         assert_same_specials(gx, want_t, "transposed " + what)
+
+
+def test_short_calls_stay_where_the_panel_kernel_is_behind():
+    # measured: gradients of few rows of long 8- and 2-bit layers with an activation order, few rows of x read without a pack pass
+    for M, K, N, bits, gs, act, tr in ((18, 15616, 3008, 8, 32, True, True), (35, 7168, 5504, 2, 32, True, True),
+                                       (12, 21632, 2112, 2, 32, True, True), (63, 3968, 12640, 8, 128, False, False)):
+        assert _lib.select_panel(M, K, N, bits, gs, act, tr) is None, (M, K, N, bits)
+    # clearly ahead: still there
+    for M, K, N, bits, gs, act, tr in ((36, 12672, 17152, 8, -1, False, False), (40, 4096, 11008, 4, 128, False, True),
+                                       (32, 36864, 9216, 3, -1, False, False)):
+        assert _lib.select_panel(M, K, N, bits, gs, act, tr) is not None, (M, K, N, bits)
+    # 9 to 16 rows: the sorted copy and the checkpoint tensors keep what the rule gives them, but for 4 bits with an order
+    seen = 0
+    for K, N in ((6784, 31616), (7552, 6816), (8192, 8192), (9856, 27232), (8192, 4096)):
+        for bits in (3, 4):
+            for act in (False, True):
+                for M in (9, 16):
+                    without = _lib.select_route(M, K, N, bits, 128, act)
+                    r = _lib.select_route(M, K, N, bits, 128, act, ALL)
+                    if without.copy in (_lib.ROUTE_CHECKPOINT, _lib.ROUTE_SORTED) and not (act and bits == 4):
+                        assert (r.copy, r.plan.as_dict()) == (without.copy, without.plan.as_dict()), (M, K, N, bits, act)
+                        seen += _lib.select_panel(M, K, N, bits, 128, act) is not None
+    assert seen > 0
+    # where those do not cover a call the panel kernel does (more groups than their tables hold)
+    assert _lib.select_route(12, 36864, 9216, 3, 32, True, copies=_lib.COPY_CHECKPOINT).copy == _lib.ROUTE_LIBRARY
+    r = _lib.select_route(12, 36864, 9216, 3, 32, True, copies=_lib.COPY_CHECKPOINT | _lib.COPY_TILED | _lib.COPY_TILED_PANEL)
+    assert r.copy == _lib.ROUTE_TILED
