@@ -710,7 +710,9 @@ double tiled_us(const gptq_hip_plan &p, int bits, bool transposed, double out_el
 // workgroup per row, few of them for a long row; and the matmul kernel reads up to 16 rows of x in the layer's own order
 // itself, without its pack pass.  Calls that the choice makes slower by more than 3 %, without these / with them on another draw:
 // forward 9 to 16 rows 24 / 14 %, 17 to 64 rows 10 / 7 %, gradient 11 / 4 % and 7 / 4 % (15616 x 3008 at 8 bits, gradient of 18
-// rows: 26.6 us on the panel kernel, 19.2 on the other).
+// rows: 26.6 us on the panel kernel, 19.2 on the other).  Forward the line lies at 128 rows (8 bits: a mean gain of 1.20 with
+// and without, 7 / 5 % slower; 128 rows of 4096 x 11008 33.5 us against 30.1), for the gradient at 64 (at 65 to 128 the terms
+// would give up more than they save: 1.29 / 1.26 at 8 bits with an activation order).
 double short_panel_us(double us, int K, int N, int bits, bool transposed, bool act_order)
 {
     return us + (bits == 8 ? 0.06e-6 * K * (double)N : 0.0) + (transposed && act_order ? 1.6 + 0.27e-3 * K : 0.0);
@@ -760,7 +762,7 @@ extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_si
                 const double tiled = tiled_us(other, bits, transposed, out_elems, (double)M * red, act);
                 // (short prompts have other copies to run on, too: there the matmul kernel has to be clearly the slower one)
                 if (best > (M <= 128 ? 0.95 : 1.0) * tiled) return GPTQ_HIP_ERR_UNSUPPORTED;
-                if (M <= 64 && short_panel_us(best, K, N, bits, transposed, act) > short_tiled_us(tiled, M, transposed, act))
+                if (M <= (transposed ? 64 : 128) && short_panel_us(best, K, N, bits, transposed, act) > short_tiled_us(tiled, M, transposed, act))
                     return GPTQ_HIP_ERR_UNSUPPORTED;
             }
         }

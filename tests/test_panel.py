@@ -352,7 +352,7 @@ def test_panel_special_values_stay_in_their_rows_and_columns(dev, bits, desc_act
 def test_short_calls_stay_where_the_panel_kernel_is_behind():
     # measured: gradients of few rows of long 8- and 2-bit layers with an activation order, few rows of x read without a pack pass
     for M, K, N, bits, gs, act, tr in ((18, 15616, 3008, 8, 32, True, True), (35, 7168, 5504, 2, 32, True, True),
-                                       (12, 21632, 2112, 2, 32, True, True), (63, 3968, 12640, 8, 128, False, False)):
+                                       (12, 21632, 2112, 2, 32, True, True), (128, 4096, 11008, 8, 128, True, False), (63, 3968, 12640, 8, 128, False, False)):
         assert _lib.select_panel(M, K, N, bits, gs, act, tr) is None, (M, K, N, bits)
     # clearly ahead: still there
     for M, K, N, bits, gs, act, tr in ((36, 12672, 17152, 8, -1, False, False), (40, 4096, 11008, 4, 128, False, True),
