@@ -53,10 +53,20 @@ int workspace_kind(const gptq_hip_plan &plan)
 WorkspaceLease::WorkspaceLease(const Tensor &like, size_t nbytes, void *stream, int kind)
 {
     if (nbytes == 0) return;
-    {
+    // (a thread finds the workspace that it used last without the map: entries are never removed)
+    struct Last {
+        int device = -1;
+        void *stream = nullptr;
+        Workspace *ws = nullptr;
+    };
+    static thread_local Last last[2];
+    Last &l = last[kind];
+    const int device = (int)like.get_device();
+    if (!l.ws || l.device != device || l.stream != stream) {
         const std::lock_guard<std::mutex> lock(g_ws_mutex);
-        ws = &g_ws[{(int)like.get_device(), stream, kind}];
+        l = {device, stream, &g_ws[{device, stream, kind}]};
     }
+    ws = l.ws;
     held = std::unique_lock<std::mutex>(ws->busy);
     if (!ws->bytes.defined() || (size_t)ws->bytes.numel() < nbytes) {
         const int64_t n = (int64_t)std::max(nbytes, (size_t)1 << 20);
