@@ -88,9 +88,11 @@ class QuantLinear(nn.Module):
         self.sort_for_decode = sort_for_decode
         self._sorted = None   # (key, (qweight_sorted, kmap) or None)
         # Every fused layer whose groups are whole multiples of 32 channels: on the first call with a row count
-        # the tiled kernels are faster at (the library's routing rule, gptq_hip_select_route), keep a copy of the layer in the order the matrix
-        # instructions consume (gptq_hip_tile_prepare).  Costs the layer's packed size again; False keeps
-        # the checkpoint's tensors (and the sorted copy) only.  compact() makes it the only copy.
+        # the tiled kernels are faster at (the library's routing rule, gptq_hip_select_route), keep a copy of the layer in
+        # the order the matrix instructions consume (gptq_hip_tile_prepare); the first gradient for x adds the transposed
+        # one.  Each costs the layer's packed size again, and the call that builds it its preparation (prepare_tiled /
+        # prepare_transposed do it up front); False keeps the checkpoint's tensors (and the sorted copy) only, and long
+        # batches then run as dequant + library GEMM.  compact() makes the tiled copy the only one.
         self.tile_for_prefill = tile_for_prefill
         self._tiled = None    # (key, (qtile, sz, xsrc, kinv) or None)
         self._tiled_t = None  # (key, (qtile_t, szt, xsrc) or None): the copy the gradient for x runs on
