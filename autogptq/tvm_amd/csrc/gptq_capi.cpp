@@ -319,7 +319,7 @@ static int run_panel(const void *x, const void *qtile, const uint32_t *sz, const
         plan.grid_z != plan.m_blocks || plan.m_blocks != (M + 32 * rt - 1) / (32 * rt) ||
         plan.split_k != (S_total + plan.k_chunk - 1) / plan.k_chunk || plan.lds_bytes != gptq::panel_lds_bytes(bits, rt))
         return GPTQ_HIP_ERR_BAD_ARG;
-    if ((long long)plan.grid_x * plan.m_blocks >= (1LL << 31)) return GPTQ_HIP_ERR_UNSUPPORTED;
+    if (!gptq::panel_launches((long long)plan.grid_x * plan.m_blocks, plan.block, trans && xsrc ? M : 0)) return GPTQ_HIP_ERR_UNSUPPORTED;
     if (plan.split_k > 1 && (long long)M * cols >= (1LL << 32)) return GPTQ_HIP_ERR_UNSUPPORTED;
     const size_t part = plan.split_k > 1 ? ((size_t)plan.split_k * M * cols * sizeof(float) + 255) / 256 * 256 : 0;
     // x in the order of the copy, or the transposed product's result before its channels are put in order

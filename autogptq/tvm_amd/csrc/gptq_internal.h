@@ -289,6 +289,11 @@ constexpr int panel_lds_bytes(int bits, int rt)
 }
 // The kernel addresses the rows of a workgroup with 31 bits (bit 31 of an offset marks what lies outside)
 constexpr bool panel_addresses(int rt, int red) { return 32LL * rt * red * 2 < (1LL << 31); }
+// and a launch has less than 2^32 threads, the pass that puts a gradient's rows in order included (256 for each of them)
+constexpr bool panel_launches(long long wgs, int block, long long ordered_rows)
+{
+    return wgs * block < (1LL << 32) && ordered_rows * 256 < (1LL << 32);
+}
 // rows x channels from which the transposed product puts its result's channels in order in a pass (2.5 us and 0.9 us per
 // million, against 3.7 us per million for scattered stores)
 inline bool panel_scatters(int M, int K) { return (long long)M * K >= (1LL << 20); }

@@ -374,3 +374,44 @@ def test_short_calls_stay_where_the_panel_kernel_is_behind():
     assert _lib.select_route(12, 36864, 9216, 3, 32, True, copies=_lib.COPY_CHECKPOINT).copy == _lib.ROUTE_LIBRARY
     r = _lib.select_route(12, 36864, 9216, 3, 32, True, copies=_lib.COPY_CHECKPOINT | _lib.COPY_TILED | _lib.COPY_TILED_PANEL)
     assert r.copy == _lib.ROUTE_TILED
+
+
+def test_plans_keep_within_a_launch():
+    # 2^32 threads: 256 per row of a gradient that is put in order, and the workgroups of the product
+    K, N = 64, 64
+    for M, act, tr, ok in (((1 << 24) - 1, True, True, True), (1 << 24, True, True, False), (1 << 24, True, False, True),
+                           (1 << 24, False, True, True), (1 << 30, False, False, False)):
+        p = _lib.select_panel(M, K, N, 4, 32, act, tr, 1 if M == 1 << 30 else 8, 1)
+        assert (p is not None) == ok, (M, act, tr)
+    fake, null = ctypes.c_void_p(0x1000), ctypes.c_void_p(None)
+    M = 1 << 24
+    p = _lib.select_panel(M, K, N, 4, 32, False, True, 8, 1)
+    rc = _lib.lib().gptq_hip_gemm_tiled_transposed(fake, fake, fake, fake, fake, fake, 1 << 40, M, K, N, 4, 32, ctypes.byref(p), null)
+    assert rc == _lib.ERR_UNSUPPORTED
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_panel_results_at_an_eight_byte_offset(dev, desc_act):
+    # y and gx are asked to be 8-byte aligned, the kernel stores 16 bytes at a time: a result that starts in between, and its guards
+    K, N, gs, bits = 2048, 544, 64, 4
+    for M in (70, 700):                          # (the gradient's channels put in order by the product itself, and in a pass)
+        L = layer(9960 + M, K, N, bits, gs, desc_act, M=M)
+        D = to_dev(L, dev)
+        gy = torch.randn(M, N, generator=torch.Generator().manual_seed(M)).half()
+        want, want_t = expected_output(L), gy.float() @ expected_weight(L).float().t()
+        g = D["g_idx"] if desc_act else None
+        xsrc = ops.tile_prepare(D["qweight"], D["qzeros"], D["scales"], g, bits, gs)[2] if desc_act else None
+        qtile_t, szt = ops.tile_prepare_transposed(D["qweight"], D["qzeros"], D["scales"], xsrc, bits, gs)
+        for rt, split in ((2, 1), (5, 1), (3, 2)):
+            for cols, ref, run in (
+                    (N, want, lambda out: forward(D, _lib.select_panel(M, K, N, bits, gs, desc_act, False, rt, split), out=out)),
+                    (K, want_t, lambda out: ops.gemm_tiled_transposed(
+                        gy.to(dev), qtile_t, szt, xsrc, K, bits, gs, out=out,
+                        plan=_lib.select_panel(M, K, N, bits, gs, desc_act, True, rt, split)))):
+                buf = torch.full((64 + M * cols + 64,), 1234.0, dtype=torch.float16, device=dev)
+                out = buf[60:60 + M * cols].view(M, cols)
+                assert out.data_ptr() % 16 == 8
+                run(out)
+                assert_tight(out, ref, f"M={M} columns={cols} row tiles {rt} ranges {split}")
+                assert bool((buf[:60] == 1234.0).all()) and bool((buf[60 + M * cols:] == 1234.0).all())
