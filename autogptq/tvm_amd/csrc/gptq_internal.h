@@ -192,10 +192,12 @@ inline bool tiled_qualifies(int K, int N, int bits, int gs)
 static const int kDecodeMaxRows = 8;      // rows the decode kernel of the tiled format takes (the 16-column kernel: 4)
 constexpr int kDecodeSelectRows = 4;   // rows up to which gptq_hip_select_tiled chooses it
 inline int tiled_decode_rows(int M) { return M <= 1 ? 1 : (M <= 2 ? 2 : (M <= 4 ? 4 : 8)); }
+// (four and eight rows: the zero point is taken off every code, so no sums of x are kept)
+constexpr bool tiled_decode_centred(int mr) { return mr >= 4; }
 inline int tiled_decode_lds_bytes(int mr, int span, int groups, int waves_k)
 {
     (void)groups;   // (the (scale, zero) words no longer pass through LDS)
-    return mr * span * 2 + 64 + (span / 32) * mr * 8 + waves_k * mr * 128;
+    return mr * span * 2 + 64 + (tiled_decode_centred(mr) ? 0 : (span / 32) * mr * 8) + waves_k * mr * 128;
 }
 // decode kernel with one workgroup per CU (16-column units, all of K staged): LDS of a workgroup that takes
 // `units_per_wg` units

@@ -21,15 +21,27 @@ namespace gptq {
 // and the instruction can broadcast the A operand of one block to the others (cbsz / abid): block b of the
 // half keeps positions 4 b .. 4 b + 3 in its A registers and the instruction for positions 4 i .. 4 i + 3
 // names block i, so x costs one 8-byte LDS read per lane and block.
-// Per weight the vector ALU only unpacks (2, 3, 4 bits).
+// One and two rows (2, 3, 4 bits): per weight the vector ALU only unpacks.
 // The codes enter as (base + q) with the bases of the register unpack; per block of 32 positions the
 // epilogue takes y += scale * (P - Bsum - zero * Xsum), with Xsum = sum x and Bsum = sum x * base of the
-// block computed once per workgroup when x is staged.  Like GROUPED, and unlike the TILED matmul, this
-// does not reproduce the fp16 rounding of each dequantised weight: products are exact, sums are fp32.
+// block computed once per workgroup when x is staged.
+// Four and eight rows: the codes enter as q - zero, (base + q) - (base + zero) in one packed subtraction per register
+// (exact: small integers), and the epilogue is y += scale * P.  The sums above cost vector instructions and LDS reads in
+// proportion to the rows, the subtraction does not: without / with it, us, no activation order: 4096 x 11008 int4 6.66 / 6.03 at
+// four rows, 8.53 / 7.55 at eight, 4096 x 4096 5.13 / 4.50 at four; one row 4.11 / 4.16, two rows 6.20 / 6.51 at 4096 x 11008.
+// (The sums' large terms no longer cancel in fp32, either.)
+// Either way, like GROUPED and unlike the TILED matmul, this does not reproduce the fp16 rounding of each dequantised
+// weight: products are exact, sums are fp32.
 // 8-bit layers instead dequantise every weight in registers, as the matmul does (tiled_decode_exact), and add
 // the products as they are.
 // x reaches LDS in position order: a layer with an activation order scatters it through kinv (16-bit
 // position per channel, one round trip; every workgroup walks all of x and keeps its K range).
+// Four and eight rows of such a layer lie position by position, the rows of a position side by side (PM): a channel is
+// one store of 8 or 16 bytes instead of one of two bytes per row (11008 channels x 8 rows: 1376 conflicting stores per
+// workgroup become 172), and the A operand, four positions of one row, comes out of a transposing read
+// (ds_read_b64_tr_b16: of each 16 lanes, lane 4 p + c fetches four values and lane 4 c + i receives value i of lanes c, 4 + c,
+// 8 + c, 12 + c).  11008 x 4096 int4 at eight rows 16.2 -> 10.1 us, 4096 x 11008 12.9 -> 7.8, 8192 x 8192 24.8 -> 14.5,
+// 4096 x 11008 at four rows 8.5 -> 7.1 (with the subtraction above).
 // ---------------------------------------------------------------------------------------------------
 struct DecodeParams {
     const _Float16 *x;      // [M, K]
@@ -63,9 +75,10 @@ struct DecodeTail {
     unsigned long long *slots;
 };
 
+// PM: x lies position by position in LDS (activation order, four or eight rows).
 // E: blocks of 64 positions that share one epilogue (1, or 2 when the groups are multiples of 128 channels and
 // every wave has an even number of blocks: both lane blocks of both blocks then lie in one group).
-template <int BITS, int MR, int KW, int E>
+template <int BITS, int MR, int KW, int E, bool PM>
 __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a_x, const uint16_t *a_kinv, const char *a_qtile,
                                                                const uint32_t *a_sz, int a_K, uint32_t a_m_steps, int a_T_total,
                                                                int a_grid_x, uint32_t a_lbg_magic, uint32_t a_flags,
@@ -82,6 +95,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     static_assert((MR == 1 || MR == 2 || MR == 4 || MR == 8) && (E == 1 || E == 2), "one or two sets of four rows");
     constexpr int RS = (MR + 3) / 4;   // sets of four rows: a matrix instruction takes four rows of x
     constexpr bool EXACT = tiled_decode_exact(BITS);
+    constexpr bool CENTRE = !EXACT && tiled_decode_centred(MR);
     constexpr int NT = 64 * KW;
     constexpr int PF = 2;              // blocks of weights per chunk
     // chunks in flight per wave.  A wave asks for a chunk when it has consumed one, so its walk is a chain of
@@ -118,12 +132,12 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     const int span = wg_steps * 64;                      // positions the workgroup stages
     const int p0 = S_wg * 64;                            // its first position
 
-    // LDS: x in position order [MR][span] fp16 | 64 zero bytes | block sums [span / 32][MR] (Xsum, Bsum) |
+    // LDS: x in position order [MR][span] fp16 (PM: [span][MR]) | 64 zero bytes | block sums [span / 32][MR] (Xsum, Bsum), none when CENTRE |
     //      partial results [KW][MR][32]
     _Float16 *xl = (_Float16 *)smem;
     const uint32_t zero_off = (uint32_t)MR * (uint32_t)span * 2u;
     f2 *xs = (f2 *)(smem + zero_off + 64);
-    const int lbs = span / 32;
+    const int lbs = tiled_decode_centred(MR) ? 0 : span / 32;
     float *red = (float *)(xs + (size_t)lbs * MR);
 
     // ---- 1. x and the map first (a wait for them would also wait for every older load: vector loads return
@@ -133,7 +147,9 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     //         for the word of a unit when it asks for the unit's weights and finds it when they are there.) -----
     // (without a map the channels of the range are the range itself)
     const int k8_lo = p.kinv ? 0 : p0 / 8, k8_hi = p.kinv ? p.K / 8 : min(p0 + span, p.K) / 8;
-    constexpr int QP = MR == 8 ? 1 : 2;  // passes over x kept in registers (eight rows: 32 registers a pass)
+    // passes over x kept in registers (eight rows: 32 registers a pass; a second one only shortens the way of workgroups of
+    // four waves without an activation order, 4096 x 11008 7.55 -> 7.29 us, and costs 0.2 to 0.5 us elsewhere)
+    constexpr int QP = MR == 8 && (PM || KW > 4) ? 1 : 2;
     u4 kq[QP];
     h8 xq[QP][MR];
 #pragma unroll
@@ -146,6 +162,21 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     // (a workgroup with a part of K, a half tile or one of several ranges, keeps the channels of its own range)
     const bool ranged = is_half || p.grid_y > 1;
     auto scatter8 = [&](int k, const u4 &kv, const h8 (&xv)[MR]) {
+        if constexpr (PM) {
+            // a channel's values of all rows in one store (8 or 16 bytes), put together from the rows' registers
+            typedef uint32_t row_words __attribute__((ext_vector_type(MR / 2)));
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const uint32_t pos = ((kv[e >> 1] >> (16 * (e & 1))) & 0xffffu) - (uint32_t)p0;
+                row_words v;
+#pragma unroll
+                for (int r = 0; r < MR / 2; r++)
+                    v[r] = __builtin_amdgcn_perm(__builtin_bit_cast(u4, xv[2 * r + 1])[e >> 1], __builtin_bit_cast(u4, xv[2 * r])[e >> 1],
+                                                 e & 1 ? 0x07060302u : 0x05040100u);
+                if (!ranged || pos < (uint32_t)span) *(row_words *)(smem + pos * (uint32_t)(2 * MR)) = v;
+            }
+            return;
+        }
         if (!p.kinv) {   // no activation order: the eight channels are eight consecutive positions, one store
             // (k8_lo .. k8_hi is the workgroup's own range here, a multiple of 8 away from p0)
 #pragma unroll
@@ -249,7 +280,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
         const int tail0 = max(p.K - p0, 0);
         for (int i = tail0 + tid; i < span; i += NT)
 #pragma unroll
-            for (int m = 0; m < MR; m++) xl[m * span + i] = (_Float16)0;
+            for (int m = 0; m < MR; m++) xl[PM ? MR * i + m : m * span + i] = (_Float16)0;
     }
 #pragma unroll
     for (int ps = 0; ps < QP; ps++) {
@@ -261,7 +292,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     //         unit's 32 E positions of that half; every wave for the units of its own slice (LDS serves one
     //         wave's accesses in order: no barrier needed).  Entry ((sb / E) * 2 + h) * MR + m, sb = the unit's
     //         first block inside the workgroup's range ------------------------------------------------------
-    if constexpr (!EXACT) {
+    if constexpr (!EXACT && !CENTRE) {
         // a lane sums 16 consecutive positions; a run of 32 positions (one half of one block) is two lanes,
         // a unit-half 2 E lanes: l, l + 1 (the other half of the run) and, E = 2, l + 4, l + 5 (the other block)
         const int sb0 = S_begin - S_wg;
@@ -319,26 +350,42 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     // the registers past M are never stored; one stride for all lanes keeps the block's offset an immediate)
     uint32_t x_base[RS];
 #pragma unroll
-    for (int rs = 0; rs < RS; rs++) x_base[rs] = (uint32_t)(min(4 * rs + row_i, p.M - 1) * span + 32 * h + 4 * lb8) * 2u;
-    constexpr uint32_t x_stride = 128u;
+    for (int rs = 0; rs < RS; rs++)
+        x_base[rs] = PM ? (uint32_t)((32 * h + 16 * ((lane >> 4) & 1) + 4 * (lane & 3) + ((lane >> 2) & 3)) * MR + 4 * rs) * 2u
+                        : (uint32_t)(min(4 * rs + row_i, p.M - 1) * span + 32 * h + 4 * lb8) * 2u;
+    constexpr uint32_t x_stride = PM ? 128u * MR : 128u;
     const uint32_t xs_lane = zero_off + 64u + (uint32_t)(h * MR) * 8u;   // sums of half h of unit 0
 
     // x of a block: this lane's four positions of row row_i; read one block ahead of its use
     auto load_x = [&](uint32_t sb, u2 (&xv)[RS]) {
 #pragma unroll
-        for (int rs = 0; rs < RS; rs++) xv[rs] = *(const u2 *)(smem + x_base[rs] + x_stride * sb);
+        for (int rs = 0; rs < RS; rs++) {
+            if constexpr (PM) {
+                typedef short s4 __attribute__((ext_vector_type(4)));
+                xv[rs] = __builtin_bit_cast(u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                    (__attribute__((address_space(3))) s4 *)(smem + x_base[rs] + x_stride * sb)));
+            } else {
+                xv[rs] = *(const u2 *)(smem + x_base[rs] + x_stride * sb);
+            }
+        }
     };
     f4 c0[RS], c1[RS];  // two chains per set of rows: a matrix instruction waits for the one it adds to
 #pragma unroll
     for (int rs = 0; rs < RS; rs++) c0[rs] = c1[rs] = (f4){0.f, 0.f, 0.f, 0.f};
     uint32_t szw = 0u;   // (scale, zero) word and sums of the unit in flight, read when the unit starts
     f2 xsv[MR];
+    h2 zb[TileCodec<BITS>::KINDS];   // CENTRE: (base + zero) of the unit, per register kind
     auto block = [&](auto uu_c, int S, const uint32_t (&wr)[BITS], uint32_t sr, const u2 (&xc)[RS], u2 (&xn)[RS]) {
         constexpr int uu = decltype(uu_c)::value;                 // block inside its unit
         const uint32_t sb = (uint32_t)(S - S_wg);                  // block inside the workgroup's range (wave-uniform)
         if constexpr (uu == 0) {
             szw = sr;   // the unit's (scale, zero) word, requested with its weights
-            if constexpr (!EXACT) {
+            if constexpr (CENTRE) {
+                const _Float16 z = as_h2(sr)[1];
+#pragma unroll
+                for (int k = 0; k < TileCodec<BITS>::KINDS; k++)
+                    zb[k] = (h2){z, z} + (h2){(_Float16)TileCodec<BITS>::base(2 * k), (_Float16)TileCodec<BITS>::base(2 * k + 1)};
+            } else if constexpr (!EXACT) {
                 const f2 *xb = (const f2 *)(smem + xs_lane + (sb / E) * (uint32_t)(2 * MR * 8));
 #pragma unroll
                 for (int m = 0; m < MR; m++) xsv[m] = xb[m];
@@ -350,6 +397,12 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
 #pragma unroll
         for (int j = 0; j < 4; j++) TileCodec<BITS>::operand(wr, j, q[j], mg);
         if constexpr (EXACT) tiled_dequant_exact<BITS>(q, szw);
+        if constexpr (CENTRE) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) q[j][r] = as_u32(as_h2(q[j][r]) - zb[r % TileCodec<BITS>::KINDS]);
+        }
 #pragma unroll
         for (int rs = 0; rs < RS; rs++) {
             if constexpr (uu == 0) {
@@ -367,6 +420,10 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
             if constexpr (EXACT) {
 #pragma unroll
                 for (int m = 0; m < MR; m++) ysum[m] += c0[m / 4][m % 4] + c1[m / 4][m % 4];
+            } else if constexpr (CENTRE) {
+                const float sc = (float)as_h2(szw)[0];
+#pragma unroll
+                for (int m = 0; m < MR; m++) ysum[m] += sc * (c0[m / 4][m % 4] + c1[m / 4][m % 4]);
             } else {
                 const h2 e = as_h2(szw);
                 const float sc = (float)e[0], zp = (float)e[1];
@@ -459,10 +516,10 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     }
 }
 
-template <int BITS, int MR, int KW, int E>
+template <int BITS, int MR, int KW, int E, bool PM>
 static int launch_decode_one(const DecodeParams &p, const gptq_hip_plan &plan, hipStream_t stream)
 {
-    auto kern = tiled_decode_kernel<BITS, MR, KW, E>;
+    auto kern = tiled_decode_kernel<BITS, MR, KW, E, PM>;
     if (plan.lds_bytes > 65536) {
         if (hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, plan.lds_bytes) != hipSuccess) {
             (void)hipGetLastError();
@@ -478,15 +535,15 @@ static int launch_decode_one(const DecodeParams &p, const gptq_hip_plan &plan, h
     return hipGetLastError() == hipSuccess ? GPTQ_HIP_OK : GPTQ_HIP_ERR_LAUNCH;
 }
 
-template <int BITS, int MR, int E>
+template <int BITS, int MR, int E, bool PM>
 static int launch_decode_kw(const DecodeParams &p, const gptq_hip_plan &plan, hipStream_t stream)
 {
     switch (plan.waves_k) {
-        case 4: return launch_decode_one<BITS, MR, 4, E>(p, plan, stream);
-        case 8: return launch_decode_one<BITS, MR, 8, E>(p, plan, stream);
+        case 4: return launch_decode_one<BITS, MR, 4, E, PM>(p, plan, stream);
+        case 8: return launch_decode_one<BITS, MR, 8, E, PM>(p, plan, stream);
         case 16:
             if constexpr (MR == 8) return GPTQ_HIP_ERR_UNSUPPORTED;   // (128 registers per lane do not hold two sets of rows)
-            else return launch_decode_one<BITS, MR, 16, E>(p, plan, stream);
+            else return launch_decode_one<BITS, MR, 16, E, PM>(p, plan, stream);
         default: return GPTQ_HIP_ERR_UNSUPPORTED;
     }
 }
@@ -530,7 +587,12 @@ int launch_tiled_decode(const void *x, const void *qtile, const uint32_t *sz, co
     // (halved tiles, grid_x > tiles: their waves walk the two even shares of k_chunk that the planner checked)
     const bool pairs = tiled_decode_pairs(group_size, plan.k_chunk);
 #define GPTQ_DECODE_CASE(B, R) \
-    if (bits == B && mr == R) rc = pairs ? launch_decode_kw<B, R, 2>(p, plan, stream) : launch_decode_kw<B, R, 1>(p, plan, stream)
+    if (bits == B && mr == R) {                                                                                            \
+        if (R >= 4 && kinv)                                                                                                \
+            rc = pairs ? launch_decode_kw<B, R, 2, (R >= 4)>(p, plan, stream) : launch_decode_kw<B, R, 1, (R >= 4)>(p, plan, stream); \
+        else                                                                                                               \
+            rc = pairs ? launch_decode_kw<B, R, 2, false>(p, plan, stream) : launch_decode_kw<B, R, 1, false>(p, plan, stream);       \
+    }
     GPTQ_DECODE_CASE(4, 1);
     GPTQ_DECODE_CASE(4, 2);
     GPTQ_DECODE_CASE(4, 4);

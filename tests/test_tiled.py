@@ -706,3 +706,30 @@ def test_tiled_decode_five_to_eight_rows(dev, bits, K, N, gs, M):
         assert_close(y, want, f"decode, two row sets: bits={bits} K={K} N={N} gs={gs} M={M} act={desc_act}")
         assert_tight(y, want, f"decode, two row sets: bits={bits} K={K} N={N} gs={gs} M={M} act={desc_act}")
         assert torch.equal(y, run_tiled(D, prep, plan=plan)), "two identical calls differ"
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("K,N,gs,split", [(32, 32, 32, 1), (96, 64, -1, 1), (1056, 96, 32, 1), (1024, 8224, 64, 1), (4160, 352, 32, 1),
+                                          (2048, 64, 128, 2)])
+@pytest.mark.parametrize("M", [3, 4, 5, 8])
+def test_tiled_decode_rows_side_by_side(dev, bits, K, N, gs, split, M):
+    """Three to eight rows of layers with an activation order lie position by position in LDS: half-empty last blocks, whole
+    and halved tiles, K in ranges (each keeps its own channels), rows past M; and what one row of x holds stays in its row."""
+    L = layer(2300 + K + M, K, N, bits, gs, True, M=M, bias=True)
+    D = to_dev(L, dev)
+    prep = prepare(D)
+    plan = _lib.select_tiled(M, K, N, bits, gs, decode=True)
+    if split > 1:
+        if M <= 4:
+            plan = tile_decode_plan(M, K, N, bits, gs)
+        assert plan.waves_n == 1 and plan.grid_x == N // 32
+        plan.split_k = plan.grid_y = split
+        plan.k_chunk = -(-(K // 64) // (split * plan.waves_k))
+        plan.workspace_bytes = 16384 + split * M * N * 4
+    y = run_tiled(D, prep, plan=plan)
+    assert_tight(y, expected_output(L), f"int{bits} {K}x{N} M={M}")
+    x = L["x"].clone()
+    x[1, K // 2] = float("inf")
+    y2 = run_tiled(D, prep, x=x.to(dev), plan=plan)
+    others = [m for m in range(M) if m != 1]
+    assert torch.equal(y2[others], y[others]) and not bool(torch.isfinite(y2[1]).any())
