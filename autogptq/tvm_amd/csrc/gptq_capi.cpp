@@ -352,6 +352,11 @@ extern "C" int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint3
         if (rc != GPTQ_HIP_OK || chosen.workspace_bytes > (workspace ? workspace_bytes : 0))
             rc = gptq_hip_select_tiled(M, K, N, bits, group_size, &chosen);
         if (rc != GPTQ_HIP_OK) return rc;
+        // row blocks need no workspace, but a call without the one that its size asks for stays refused
+        gptq_hip_plan blocks;
+        if (chosen.workspace_bytes <= (workspace && aligned(workspace, 16) ? workspace_bytes : 0) &&
+            gptq::select_row_blocks(M, K, N, bits, group_size, &blocks))
+            chosen = blocks;
         plan = &chosen;
     }
     if (plan->kernel == GPTQ_HIP_KERNEL_TILED_DECODE && plan->waves_n == 2) {
@@ -371,18 +376,22 @@ extern "C" int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint3
     if (plan->kernel == GPTQ_HIP_KERNEL_TILED_DECODE) {
         const int mr = plan->row_tiles, kw = plan->waves_k;
         const int S_all = (K + 63) / 64;
-        if (M > gptq::kDecodeMaxRows || mr != gptq::tiled_decode_rows(M)) return GPTQ_HIP_ERR_UNSUPPORTED;
+        const bool blocks = plan->m_blocks != 1 || mr == 16;   // row blocks of 8 or 16 rows
+        if (blocks ? (M > gptq::kRowBlocksMaxRows || (mr != 8 && mr != 16) || plan->m_blocks != (M + mr - 1) / mr)
+                   : (M > gptq::kDecodeMaxRows || mr != gptq::tiled_decode_rows(M)))
+            return GPTQ_HIP_ERR_UNSUPPORTED;
         // grid_x: a workgroup per tile, or the planner's halved tiles on top
         const int halved = plan->grid_x - N / 32;
-        if (halved != 0 && halved != gptq::tiled_decode_halved(N / 32, plan->k_chunk, plan->split_k, kw, S_all, gs))
+        if (halved != 0 && (blocks || halved != gptq::tiled_decode_halved(N / 32, plan->k_chunk, plan->split_k, kw, S_all, gs)))
             return GPTQ_HIP_ERR_BAD_ARG;
+        if (blocks && (plan->split_k != 1 || (kw != 4 && kw != 8))) return GPTQ_HIP_ERR_UNSUPPORTED;
         // a caller that runs halved tiles has to know what their workspace asks for
         if (halved != 0 && !(plan->flags & GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE)) return GPTQ_HIP_ERR_BAD_ARG;
         // and a plan that says so while it writes partial sums (K cut over workgroups, whole tiles) would leave them in
         // a workspace that has to stay zero
         if (halved == 0 && (plan->flags & GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE)) return GPTQ_HIP_ERR_BAD_ARG;
         if ((kw != 4 && kw != 8 && kw != 16) || plan->block != 64 * kw || plan->split_k < 1 || plan->k_chunk < 1 ||
-            plan->grid_y != plan->split_k || plan->grid_z != 1 ||
+            plan->grid_y != plan->split_k || plan->grid_z != plan->m_blocks ||
             (long long)plan->split_k * kw * plan->k_chunk < S_all ||
             (long long)(plan->split_k - 1) * kw * plan->k_chunk >= S_all)  // every workgroup starts inside K
             return GPTQ_HIP_ERR_BAD_ARG;

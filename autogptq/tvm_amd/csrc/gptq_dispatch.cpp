@@ -548,6 +548,39 @@ int tiled_ranges(int at, bool wide, long long tiles, int S_total, int kwv, doubl
 
 }  // namespace
 
+// 9 rows and more of a layer small enough: the decode kernel in blocks of 8 or 16 rows, a workgroup per column tile and
+// block, while those find a CU each and a block's x fits LDS (8 rows: K up to 9216, 16 rows: 4096).  A CU takes its x and
+// weights in at ~50 GB/s whatever the kernel; what this saves against the matmul kernel is the pack pass (a launch) and
+// the CUs that its 64 columns per workgroup leave idle.  us, graph replay, matmul or panel kernel / this (8 rows, else 16): 4096 x
+// 4096 int4 at 9 / 16 / 32 rows 11.6 / 10.4 / 12.5 and 6.0 / 6.1 / 8.1; 2048 x 2048 at 12 / 64 rows 8.8 / 8.5 and 4.2 / 5.5; 4096 x
+// 8192 at 16 rows 11.0-12.6 and 8.2-8.4; 8192 x 4096 at 16 rows 12.6, with an activation order 16.4, and 9.8, 10.0; 2048 x 4096
+// int8 at 32 rows 11.1 and 5.7.  One block more than CUs loses: every workgroup stages its x, and the second turn is as long as
+// the first (4096 x 11008 at 16 rows 11.5-13.1 and 14.0-14.6).
+// Four waves along K up to 1024 channels (1024 x 4096 at 32 rows 4.5 us, eight 5.1), eight beyond (2048 x 8192 at 16 rows 5.6, four 5.9).
+bool gptq::select_row_blocks(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
+{
+    if (M <= kDecodeMaxRows || M > kRowBlocksMaxRows) return false;
+    if (!tiled_qualifies(K, N, bits, group_size == -1 ? K : group_size)) return false;
+    const int tiles = N / 32, S_total = ceil_div(K, 64), kw = S_total <= 16 ? 4 : 8;
+    for (int mr = 8; mr <= 16; mr *= 2) {
+        const int z = ceil_div(M, mr), steps = ceil_div(S_total, kw);
+        const int lds = tiled_decode_lds_bytes(mr, steps * kw * 64, 0, kw);
+        if ((long long)tiles * z > kNumCUs || lds > 160 * 1024) continue;
+        memset(plan, 0, sizeof(*plan));
+        plan->kernel = GPTQ_HIP_KERNEL_TILED_DECODE;
+        plan->row_tiles = mr;
+        plan->m_blocks = plan->grid_z = z;
+        plan->waves_n = plan->split_k = plan->grid_y = 1;
+        plan->waves_k = kw;
+        plan->k_chunk = steps;
+        plan->grid_x = tiles;
+        plan->block = 64 * kw;
+        plan->lds_bytes = lds;
+        return true;
+    }
+    return false;
+}
+
 extern "C" int gptq_hip_select_tiled(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
 {
     // Up to four rows the decode kernels (one 4-row matrix instruction set per lane block); five to eight rows the
@@ -924,9 +957,14 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
         route->copy = GPTQ_HIP_ROUTE_TILED;
         return true;
     };
+    auto take_rows = [&]() {
+        if (!panels || !tiled_ok || !gptq::select_row_blocks(M, K, N, bits, group_size, &route->plan)) return false;
+        route->copy = GPTQ_HIP_ROUTE_TILED;
+        return true;
+    };
     if (copies == GPTQ_HIP_COPY_TILED) {
         // the tiled copy is all the layer has: every M runs there
-        if (take_panel() || (tiled_ok && take_tiled())) return GPTQ_HIP_OK;
+        if (take_rows() || take_panel() || (tiled_ok && take_tiled())) return GPTQ_HIP_OK;
         return GPTQ_HIP_ERR_UNSUPPORTED;
     }
     bool tiled = false;
@@ -949,7 +987,12 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
     // Up to 16 rows the kernels on the other copies, where the rule has them, keep their calls: against them it is 0.71 to 1.08 x
     // as fast (0.92 on the mean) on drawn 3-bit layers without an activation order, level on 4-bit ones (0.85 to 1.32 x) and on 3-bit
     // ones with an order (0.93 to 1.05 x), and no reason for another copy; on 4-bit layers with one it is ahead (0.86 to 1.38, 1.12).
-    const bool others = !tiled && M <= 16 && fused_bits && !(act && bits == 4) && (copies & (GPTQ_HIP_COPY_CHECKPOINT | GPTQ_HIP_COPY_SORTED));
+    const bool theirs = !tiled && M <= 16 && fused_bits && (copies & (GPTQ_HIP_COPY_CHECKPOINT | GPTQ_HIP_COPY_SORTED));
+    const bool others = theirs && !(act && bits == 4);
+    // Row blocks are ahead of the kernels on every copy (16 rows of 4096 x 4096 int4 with an activation order 6.0 us, 10.7 on the
+    // checkpoint tensors; without one 6.1 and 9.3); beyond 4096 channels they leave a layer that has other copies to those
+    // (8192 x 4096: 9.8 us against 11.5 to 12.5, for a copy more), and below 1024 columns, where a call costs its host time.
+    if (!past && (!theirs || (K <= 4096 && N >= 1024)) && take_rows()) return GPTQ_HIP_OK;
     if (!others && take_panel()) return GPTQ_HIP_OK;
     if (past) return GPTQ_HIP_OK;
     if (tiled && take_tiled()) return GPTQ_HIP_OK;

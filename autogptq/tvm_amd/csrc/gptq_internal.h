@@ -190,6 +190,7 @@ inline bool tiled_qualifies(int K, int N, int bits, int gs)
 // decode kernel on the tiled format: rows it is built for, and the LDS of a workgroup whose waves cover
 // `span` positions of `groups` groups
 static const int kDecodeMaxRows = 8;      // rows the decode kernel of the tiled format takes (the 16-column kernel: 4)
+constexpr int kRowBlocksMaxRows = 128;   // rows it takes in blocks of 8 or 16 along grid_z
 constexpr int kDecodeSelectRows = 4;   // rows up to which gptq_hip_select_tiled chooses it
 inline int tiled_decode_rows(int M) { return M <= 1 ? 1 : (M <= 2 ? 2 : (M <= 4 ? 4 : 8)); }
 // (four and eight rows: the zero point is taken off every code, so no sums of x are kept)
@@ -208,6 +209,8 @@ inline long long tiled_decode16_lds_bytes(int mr, int K, int groups, int units_p
     (void)groups;   // (the (scale, zero) words no longer pass through LDS)
     return mr * span * 2 + 64 + (span / 32) * mr * 8 + (long long)units_per_wg * 16 * mr * 256;
 }
+// the plan in row blocks, where it is the faster one (gptq_dispatch.cpp)
+bool select_row_blocks(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan);
 int launch_tile_prepare(const uint32_t *qweight, const uint32_t *qzeros, const void *scales, const int32_t *g_idx,
                         uint32_t *qtile, uint32_t *sz, int32_t *xsrc, uint16_t *kinv, int K, int N, int G, int bits,
                         int group_size, void *stream);

@@ -1,4 +1,4 @@
-// TILED family, the decode kernel with a workgroup per 32-column tile: up to four rows of x on the tiled format
+// TILED family, the decode kernel with a workgroup per 32-column tile: up to eight rows of x on the tiled format, more in blocks
 // (the format, its preparation and the matmul kernel for more rows are in gptq_tiled.hip; the decode kernel with
 // one workgroup per CU in gptq_tiled_decode16.hip).
 #include "gptq_tiled_common.h"
@@ -6,7 +6,7 @@
 namespace gptq {
 
 // ---------------------------------------------------------------------------------------------------
-// tiled_decode_kernel: M <= 4 rows of x on the tiled format.
+// tiled_decode_kernel: M <= 8 rows of x on the tiled format, or blocks of 8 or 16 rows (RB, blockIdx.z).
 //
 // A workgroup owns ONE column tile (32 columns) and one K range; its KW waves split that range.  With one
 // small workgroup per tile every CU gets work whatever N is (11008 columns: 344 workgroups of 4 waves,
@@ -75,10 +75,12 @@ struct DecodeTail {
     unsigned long long *slots;
 };
 
-// PM: x lies position by position in LDS (activation order, four or eight rows).
+// PM: x lies position by position in LDS (activation order, four rows and more).
+// RB: one of several row blocks.  From nine rows on the weights are formed as the matmul kernel forms them, rounded to fp16
+// (one packed multiplication more, and no epilogue per unit: the products of the whole walk add up in the result registers).
 // E: blocks of 64 positions that share one epilogue (1, or 2 when the groups are multiples of 128 channels and
 // every wave has an even number of blocks: both lane blocks of both blocks then lie in one group).
-template <int BITS, int MR, int KW, int E, bool PM>
+template <int BITS, int MR, int KW, int E, bool PM, bool RB>
 __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a_x, const uint16_t *a_kinv, const char *a_qtile,
                                                                const uint32_t *a_sz, int a_K, uint32_t a_m_steps, int a_T_total,
                                                                int a_grid_x, uint32_t a_lbg_magic, uint32_t a_flags,
@@ -92,9 +94,14 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     // groups = (K / 32) / (lane blocks per group), by the same multiply-high that maps a lane block to its group
     p.G = (int)(__umulhi((uint32_t)a_K >> 5, a_lbg_magic) + (p.lbg_add ? (uint32_t)a_K >> 5 : 0u));
     p.bias = t.bias, p.y = t.y, p.partial = t.partial, p.slots = t.slots;
-    static_assert((MR == 1 || MR == 2 || MR == 4 || MR == 8) && (E == 1 || E == 2), "one or two sets of four rows");
+    static_assert((MR == 1 || MR == 2 || MR == 4 || MR == 8 || MR == 16) && (E == 1 || E == 2), "up to four sets of four rows");
+    const int M_all = p.M, m0 = RB ? (int)blockIdx.z * MR : 0;   // RB: this workgroup's rows
+    if constexpr (RB) {
+        p.x += (size_t)m0 * p.K;
+        p.M = min(MR, M_all - m0);
+    }
     constexpr int RS = (MR + 3) / 4;   // sets of four rows: a matrix instruction takes four rows of x
-    constexpr bool EXACT = tiled_decode_exact(BITS);
+    constexpr bool EXACT = RB || tiled_decode_exact(BITS);
     constexpr bool CENTRE = !EXACT && tiled_decode_centred(MR);
     constexpr int NT = 64 * KW;
     constexpr int PF = 2;              // blocks of weights per chunk
@@ -118,7 +125,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     // The two halves of a tile meet through one 64-bit exchange per output (see the end of the kernel).
     const int n_halved = p.grid_x - p.T_total;           // e (0: no tile is halved)
     const int n_whole = p.T_total - n_halved;
-    const bool is_half = (int)blockIdx.x >= n_whole;
+    const bool is_half = !RB && (int)blockIdx.x >= n_whole;
     const int half_i = (int)blockIdx.x - n_whole;        // (halved tile, half) = (half_i / 2, half_i % 2)
     const int T = is_half ? n_whole + (half_i >> 1) : (int)blockIdx.x;
     const int split = is_half ? (half_i & 1) : (int)blockIdx.y;
@@ -149,7 +156,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     const int k8_lo = p.kinv ? 0 : p0 / 8, k8_hi = p.kinv ? p.K / 8 : min(p0 + span, p.K) / 8;
     // passes over x kept in registers (eight rows: 32 registers a pass; a second one only shortens the way of workgroups of
     // four waves without an activation order, 4096 x 11008 7.55 -> 7.29 us, and costs 0.2 to 0.5 us elsewhere)
-    constexpr int QP = MR == 8 && (PM || KW > 4) ? 1 : 2;
+    constexpr int QP = MR == 16 || (MR == 8 && (PM || KW > 4)) ? 1 : 2;
     u4 kq[QP];
     h8 xq[QP][MR];
 #pragma unroll
@@ -161,26 +168,27 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     }
     // (a workgroup with a part of K, a half tile or one of several ranges, keeps the channels of its own range)
     const bool ranged = is_half || p.grid_y > 1;
-    auto scatter8 = [&](int k, const u4 &kv, const h8 (&xv)[MR]) {
+    // the eight channels from k on, R rows of them from row r0 on
+    auto scatter8 = [&]<int R>(int k, const u4 &kv, const h8 (&xv)[R], int r0) {
         if constexpr (PM) {
             // a channel's values of all rows in one store (8 or 16 bytes), put together from the rows' registers
-            typedef uint32_t row_words __attribute__((ext_vector_type(MR / 2)));
+            typedef uint32_t row_words __attribute__((ext_vector_type(R / 2)));
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const uint32_t pos = ((kv[e >> 1] >> (16 * (e & 1))) & 0xffffu) - (uint32_t)p0;
                 row_words v;
 #pragma unroll
-                for (int r = 0; r < MR / 2; r++)
+                for (int r = 0; r < R / 2; r++)
                     v[r] = __builtin_amdgcn_perm(__builtin_bit_cast(u4, xv[2 * r + 1])[e >> 1], __builtin_bit_cast(u4, xv[2 * r])[e >> 1],
                                                  e & 1 ? 0x07060302u : 0x05040100u);
-                if (!ranged || pos < (uint32_t)span) *(row_words *)(smem + pos * (uint32_t)(2 * MR)) = v;
+                if (!ranged || pos < (uint32_t)span) *(row_words *)(smem + pos * (uint32_t)(2 * MR) + 2 * r0) = v;
             }
             return;
         }
         if (!p.kinv) {   // no activation order: the eight channels are eight consecutive positions, one store
             // (k8_lo .. k8_hi is the workgroup's own range here, a multiple of 8 away from p0)
 #pragma unroll
-            for (int m = 0; m < MR; m++) *(h8 *)(xl + m * span + (k - p0)) = xv[m];
+            for (int m = 0; m < R; m++) *(h8 *)(xl + (r0 + m) * span + (k - p0)) = xv[m];
             return;
         }
         if (!ranged) {   // the workgroup stages all of K: every position is its own, no test and no branch per channel
@@ -188,7 +196,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
             for (int e = 0; e < 8; e++) {
                 const uint32_t pos = (kv[e >> 1] >> (16 * (e & 1))) & 0xffffu;
 #pragma unroll
-                for (int m = 0; m < MR; m++) xl[(uint32_t)(m * span) + pos] = xv[m][e];
+                for (int m = 0; m < R; m++) xl[(uint32_t)((r0 + m) * span) + pos] = xv[m][e];
             }
             return;
         }
@@ -202,7 +210,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
             const int pl = pos - p0;
             const bool mine = (unsigned)pl < (unsigned)span;
 #pragma unroll
-            for (int m = 0; m < MR; m++) xl[mine ? (uint32_t)(m * span + pl) : dump] = xv[m][e];
+            for (int m = 0; m < R; m++) xl[mine ? (uint32_t)((r0 + m) * span + pl) : dump] = xv[m][e];
         }
     };
     // Long layers: the channels the register passes do not hold, a pass at a time, before the weights are asked for
@@ -212,28 +220,32 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     // the weight requests, or, with the loop behind them, a wait for all of them in front of the sums and the walk.
     for (int k8 = k8_lo + tid + QP * NT; k8 < k8_hi; k8 += NT) {
         const int k = 8 * k8;
+        constexpr int R = MR < 8 ? MR : 8;   // (eight rows at a time)
         u4 kv = {0u, 0u, 0u, 0u};
-        h8 xv[MR];
-        if (p.kinv) {   // the map and the rows of x, requested together
-            const void *ptr[MR + 1];
-            u4 v[MR + 1];
-            ptr[MR] = p.kinv + k;
 #pragma unroll
-            for (int m = 0; m < MR; m++) ptr[m] = p.x + (size_t)min(m, p.M - 1) * p.K + k;
-            LoadNow<MR + 1>::run(v, ptr);
-            kv = v[MR];
+        for (int r0 = 0; r0 < MR; r0 += R) {
+            h8 xv[R];
+            if (p.kinv && r0 == 0) {   // the map and the rows of x, requested together
+                const void *ptr[R + 1];
+                u4 v[R + 1];
+                ptr[R] = p.kinv + k;
 #pragma unroll
-            for (int m = 0; m < MR; m++) xv[m] = __builtin_bit_cast(h8, v[m]);
-        } else {
-            const void *ptr[MR];
-            u4 v[MR];
+                for (int m = 0; m < R; m++) ptr[m] = p.x + (size_t)min(m, p.M - 1) * p.K + k;
+                LoadNow<R + 1>::run(v, ptr);
+                kv = v[R];
 #pragma unroll
-            for (int m = 0; m < MR; m++) ptr[m] = p.x + (size_t)min(m, p.M - 1) * p.K + k;
-            LoadNow<MR>::run(v, ptr);
+                for (int m = 0; m < R; m++) xv[m] = __builtin_bit_cast(h8, v[m]);
+            } else {
+                const void *ptr[R];
+                u4 v[R];
 #pragma unroll
-            for (int m = 0; m < MR; m++) xv[m] = __builtin_bit_cast(h8, v[m]);
+                for (int m = 0; m < R; m++) ptr[m] = p.x + (size_t)min(r0 + m, p.M - 1) * p.K + k;
+                LoadNow<R>::run(v, ptr);
+#pragma unroll
+                for (int m = 0; m < R; m++) xv[m] = __builtin_bit_cast(h8, v[m]);
+            }
+            scatter8(k, kv, xv, r0);
         }
-        scatter8(k, kv, xv);
     }
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t b_lane = tile_lane_bytes<BITS>((uint32_t)lane);
@@ -285,7 +297,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
 #pragma unroll
     for (int ps = 0; ps < QP; ps++) {
         const int k8 = k8_lo + tid + ps * NT;
-        if (k8 < k8_hi) scatter8(8 * k8, kq[ps], xq[ps]);
+        if (k8 < k8_hi) scatter8(8 * k8, kq[ps], xq[ps], 0);
     }
     lds_barrier();
     // ---- 3. per epilogue unit (E blocks), half and row: Xsum = sum x, Bsum = sum x * base(position) over the
@@ -405,7 +417,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
         }
 #pragma unroll
         for (int rs = 0; rs < RS; rs++) {
-            if constexpr (uu == 0) {
+            if constexpr (uu == 0 && !RB) {
                 c0[rs] = (f4){0.f, 0.f, 0.f, 0.f};
                 c1[rs] = (f4){0.f, 0.f, 0.f, 0.f};
             }
@@ -417,7 +429,9 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
             }(std::make_integer_sequence<int, 4>{});
         }
         if constexpr (uu == E - 1) {
-            if constexpr (EXACT) {
+            if constexpr (RB) {
+                // (the products of all units add up in the result registers)
+            } else if constexpr (EXACT) {
 #pragma unroll
                 for (int m = 0; m < MR; m++) ysum[m] += c0[m / 4][m % 4] + c1[m / 4][m % 4];
             } else if constexpr (CENTRE) {
@@ -478,6 +492,10 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
         for (int j = 0; j < NCH; j++) chunk(c + RING + j * PF, w[j], szr[j], std::false_type{});
     }
 
+    if constexpr (RB) {
+#pragma unroll
+        for (int m = 0; m < MR; m++) ysum[m] = c0[m / 4][m % 4] + c1[m / 4][m % 4];
+    }
     // ---- 5. the two halves of a column (lanes n and n + 32), then the waves along K ---------------------
 #pragma unroll
     for (int m = 0; m < MR; m++) ysum[m] += __shfl_xor(ysum[m], 32);
@@ -486,12 +504,12 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
         for (int m = 0; m < MR; m++) red[(wave * MR + m) * 32 + n] = ysum[m];
     }
     lds_barrier();
-    if (tid < MR * 32) {
-        const int m = tid >> 5, nn = tid & 31;
+    for (int out = tid; out < MR * 32; out += NT) {
+        const int m = out >> 5, nn = out & 31;
         if (m < p.M) {
             float sum = 0.f;
             for (int k = 0; k < KW; k++) sum += red[(k * MR + m) * 32 + nn];
-            const size_t o = (size_t)m * p.N + 32 * T + nn;
+            const size_t o = (size_t)(m0 + m) * p.N + 32 * T + nn;
             if (is_half) {
                 // One 64-bit exchange per output carries the half's sum and a tag: the half that finds the slot
                 // empty leaves its sum there; the other finds it, adds (a + b = b + a: the result does not depend on
@@ -510,16 +528,16 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
                 if (p.bias) sum += (float)((const _Float16 *)p.bias)[32 * T + nn];
                 ((_Float16 *)p.y)[o] = (_Float16)sum;
             } else {
-                p.partial[(size_t)split * p.M * p.N + o] = sum;
+                p.partial[(size_t)split * M_all * p.N + o] = sum;
             }
         }
     }
 }
 
-template <int BITS, int MR, int KW, int E, bool PM>
+template <int BITS, int MR, int KW, int E, bool PM, bool RB>
 static int launch_decode_one(const DecodeParams &p, const gptq_hip_plan &plan, hipStream_t stream)
 {
-    auto kern = tiled_decode_kernel<BITS, MR, KW, E, PM>;
+    auto kern = tiled_decode_kernel<BITS, MR, KW, E, PM, RB>;
     if (plan.lds_bytes > 65536) {
         if (hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, plan.lds_bytes) != hipSuccess) {
             (void)hipGetLastError();
@@ -529,21 +547,21 @@ static int launch_decode_one(const DecodeParams &p, const gptq_hip_plan &plan, h
     if (plan.split_k != plan.grid_y || p.M > 255 || p.wave_steps >= (1 << 24)) return GPTQ_HIP_ERR_BAD_ARG;
     DecodeTail t;
     t.bias = p.bias, t.y = p.y, t.partial = p.partial, t.slots = p.slots;
-    hipLaunchKernelGGL(kern, dim3(plan.grid_x, plan.grid_y, 1), dim3(64 * KW), plan.lds_bytes, stream, p.x, p.kinv, p.qtile, p.sz,
+    hipLaunchKernelGGL(kern, dim3(plan.grid_x, plan.grid_y, plan.grid_z), dim3(64 * KW), plan.lds_bytes, stream, p.x, p.kinv, p.qtile, p.sz,
                        p.K, (uint32_t)p.M | ((uint32_t)p.wave_steps << 8), p.T_total, plan.grid_x, p.lbg_magic,
                        (uint32_t)p.lbg_add | ((uint32_t)p.split_k << 1), t);
     return hipGetLastError() == hipSuccess ? GPTQ_HIP_OK : GPTQ_HIP_ERR_LAUNCH;
 }
 
-template <int BITS, int MR, int E, bool PM>
+template <int BITS, int MR, int E, bool PM, bool RB = false>
 static int launch_decode_kw(const DecodeParams &p, const gptq_hip_plan &plan, hipStream_t stream)
 {
     switch (plan.waves_k) {
-        case 4: return launch_decode_one<BITS, MR, 4, E, PM>(p, plan, stream);
-        case 8: return launch_decode_one<BITS, MR, 8, E, PM>(p, plan, stream);
+        case 4: return launch_decode_one<BITS, MR, 4, E, PM, RB>(p, plan, stream);
+        case 8: return launch_decode_one<BITS, MR, 8, E, PM, RB>(p, plan, stream);
         case 16:
-            if constexpr (MR == 8) return GPTQ_HIP_ERR_UNSUPPORTED;   // (128 registers per lane do not hold two sets of rows)
-            else return launch_decode_one<BITS, MR, 16, E, PM>(p, plan, stream);
+            if constexpr (MR >= 8) return GPTQ_HIP_ERR_UNSUPPORTED;   // (128 registers per lane do not hold two sets of rows)
+            else return launch_decode_one<BITS, MR, 16, E, PM, RB>(p, plan, stream);
         default: return GPTQ_HIP_ERR_UNSUPPORTED;
     }
 }
@@ -581,7 +599,7 @@ int launch_tiled_decode(const void *x, const void *qtile, const uint32_t *sz, co
         const uint32_t groups = (uint32_t)(((unsigned long long)lbs * p.lbg_magic) >> 32) + (p.lbg_add ? lbs : 0u);
         if ((int)groups != G || N % 32 != 0) return GPTQ_HIP_ERR_UNSUPPORTED;
     }
-    const int mr = tiled_decode_rows(M);
+    const int mr = plan.row_tiles;
     int rc = GPTQ_HIP_ERR_UNSUPPORTED;
     // two blocks per epilogue where every unit of two blocks lies in one group
     // (halved tiles, grid_x > tiles: their waves walk the two even shares of k_chunk that the planner checked)
@@ -593,6 +611,24 @@ int launch_tiled_decode(const void *x, const void *qtile, const uint32_t *sz, co
         else                                                                                                               \
             rc = pairs ? launch_decode_kw<B, R, 2, false>(p, plan, stream) : launch_decode_kw<B, R, 1, false>(p, plan, stream);       \
     }
+    if (plan.m_blocks > 1 || mr == 16) {
+        auto rows = [&](auto bits_c, auto mr_c) {
+            constexpr int B = decltype(bits_c)::value, R = decltype(mr_c)::value;
+            if (plan.grid_x != p.T_total || plan.split_k != 1 || plan.waves_k > 8) return (int)GPTQ_HIP_ERR_UNSUPPORTED;   // (whole tiles, whole K)
+            return kinv ? launch_decode_kw<B, R, 1, true, true>(p, plan, stream) : launch_decode_kw<B, R, 1, false, true>(p, plan, stream);
+        };
+        auto go = [&](auto bits_c) {
+            return mr == 16 ? rows(bits_c, std::integral_constant<int, 16>{})
+                            : (mr == 8 ? rows(bits_c, std::integral_constant<int, 8>{}) : (int)GPTQ_HIP_ERR_UNSUPPORTED);
+        };
+        switch (bits) {
+            case 2: rc = go(std::integral_constant<int, 2>{}); break;
+            case 3: rc = go(std::integral_constant<int, 3>{}); break;
+            case 4: rc = go(std::integral_constant<int, 4>{}); break;
+            case 8: rc = go(std::integral_constant<int, 8>{}); break;
+            default: break;
+        }
+    } else {
     GPTQ_DECODE_CASE(4, 1);
     GPTQ_DECODE_CASE(4, 2);
     GPTQ_DECODE_CASE(4, 4);
@@ -609,6 +645,7 @@ int launch_tiled_decode(const void *x, const void *qtile, const uint32_t *sz, co
     GPTQ_DECODE_CASE(8, 2);
     GPTQ_DECODE_CASE(8, 4);
     GPTQ_DECODE_CASE(8, 8);
+    }
 #undef GPTQ_DECODE_CASE
     if (rc != GPTQ_HIP_OK) return rc;
     if (plan.split_k > 1) {

@@ -50,7 +50,8 @@ enum {
                                    workgroup of waves_k = 4 waves along K, m_blocks row blocks along grid_z
                                    (k_chunk = blocks of 64 channels per wave); x is pre-packed into the
                                    workspace; split_k > 1 adds a reduce launch */
-    GPTQ_HIP_KERNEL_TILED_DECODE = 5, /* the same layer for M <= 8 rows, x staged in LDS in the layer's sorted order,
+    GPTQ_HIP_KERNEL_TILED_DECODE = 5, /* the same layer for M <= 8 rows (small layers: up to 128, in m_blocks blocks of row_tiles = 8 or
+                                   16 rows along grid_z, on rounded weights), x staged in LDS in the layer's sorted order,
                                    scales applied per 32 or 64 channels; row_tiles = the rows the kernel is built
                                    for (1, 2, 4 or 8; 8 with waves_n = 1 and at most 8 waves only).  waves_n = 1: a workgroup per 32 columns, waves_k (4, 8 or 16)
                                    waves along K with k_chunk blocks of 64 channels each; split_k > 1 (an x that
@@ -245,7 +246,8 @@ int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int group_size, 
  * (pycuda_warpper.py:138, qlinear_tvm.py:123,150).  x is 16-byte aligned, y 8-byte aligned (gy and gx below likewise;
  * GPTQ_HIP_ERR_BAD_ARG otherwise).  x and y are in the layer's own channel order (xsrc = kinv =
  * NULL means no activation order; pass both or neither).  plan: NULL = what gptq_hip_select_route names for a layer
- * with this copy alone, PANEL included; where the workspace does not hold that plan's bytes, gptq_hip_select_tiled.  workspace:
+ * with this copy alone, PANEL included; where the workspace does not hold that plan's bytes, gptq_hip_select_tiled (row blocks
+ * run without a workspace, but a call is refused unless it brings the one its size asks for).  workspace:
  * plan.workspace_bytes (none for most decode plans).  Decode plans: one launch; matmul plans: two
  * (pack pass, matmul); one more when the plan splits K.  A plan whose flags hold
  * GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE wants ALL bytes of its workspace zero at the first call and leaves them zero

@@ -531,3 +531,28 @@ def test_matmul_plans_keep_the_measured_choices():
         p = _lib.select(M, K, N, bits, 128, False)
         assert (p.kernel, p.split_k) == (kernel, split), (M, K, N, bits, p.as_dict())
         assert p.grid_x * p.grid_y * p.grid_z <= 256
+
+
+@pytest.mark.parametrize("M,K,N,mr", [(9, 1024, 4096, 8), (16, 4096, 4096, 8), (17, 4096, 4096, 16), (16, 9216, 4096, 8), (16, 9248, 4096, 0),
+                                      (16, 4096, 8192, 16), (16, 4128, 8192, 0), (16, 4096, 8224, 0), (128, 512, 1024, 16), (129, 512, 32, 0)])
+def test_row_blocks_stay_within_one_turn_and_lds(M, K, N, mr):
+    """Small layers take 9 to 128 rows in blocks of 8 or 16 on the decode kernel while every block finds a CU and its x fits LDS."""
+    r = _lib.select_route(M, K, N, 4, 32, True, _lib.COPY_TILED | _lib.COPY_TILED_PANEL)
+    assert (r.plan.kernel == _lib.KERNEL_TILED_DECODE) == (mr > 0)
+    if mr:
+        p = r.plan
+        assert (p.row_tiles, p.m_blocks, p.grid_z) == (mr, -(-M // mr), -(-M // mr))
+        assert p.grid_x * p.grid_z <= 256 and p.lds_bytes <= 160 * 1024 and p.workspace_bytes == 0 and p.split_k == 1
+    # a caller's own row count for the library comes first
+    assert _lib.select_route(M, K, N, 4, 32, True, _lib.COPY_CHECKPOINT | _lib.COPY_TILED | _lib.COPY_TILED_PANEL,
+                             (9, 9, 9)).copy == _lib.ROUTE_LIBRARY
+
+
+def test_a_tiled_call_without_plan_and_workspace_stays_refused():
+    # (row blocks need none, but the sizes they take were always asked for one; checked before anything is launched)
+    fake, null = ctypes.c_void_p(0x1000), ctypes.c_void_p(None)
+    for M, K, N in ((40, 4096, 352), (9, 32, 32), (16, 4096, 4096), (128, 512, 1024)):
+        if _lib.select_panel(M, K, N, 4, 32, False) is None:
+            for ws, nbytes in ((null, 0), (fake, 4096)):
+                assert _lib.lib().gptq_hip_gemm_tiled(fake, fake, fake, null, null, null, fake, ws, nbytes, M, K, N, 4, 32, None,
+                                                      null) == _lib.ERR_WORKSPACE

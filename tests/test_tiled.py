@@ -733,3 +733,24 @@ def test_tiled_decode_rows_side_by_side(dev, bits, K, N, gs, split, M):
     y2 = run_tiled(D, prep, x=x.to(dev), plan=plan)
     others = [m for m in range(M) if m != 1]
     assert torch.equal(y2[others], y[others]) and not bool(torch.isfinite(y2[1]).any())
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("K,N,gs,M,mr", [(32, 32, 32, 9, 8), (1056, 96, 32, 13, 8), (1088, 2048, -1, 32, 8), (4096, 4096, 128, 16, 8),
+                                         (4096, 4128, 128, 16, 16), (2080, 8192, 32, 10, 16), (64, 1024, 64, 128, 16), (9216, 64, 512, 17, 8)])
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_tiled_row_blocks(dev, bits, K, N, gs, M, mr, desc_act):
+    """Nine rows and more of small layers: the decode kernel in blocks of 8 or 16 rows (the last one short), on rounded weights, and
+    what one row of x holds stays in its row."""
+    plan = _lib.select_route(M, K, N, bits, gs, desc_act, _lib.COPY_TILED | _lib.COPY_TILED_PANEL).plan
+    assert (plan.kernel, plan.row_tiles, plan.m_blocks) == (_lib.KERNEL_TILED_DECODE, mr, -(-M // mr))
+    L = layer(3300 + K + M, K, N, bits, gs, desc_act, M=M, bias=True)
+    D = to_dev(L, dev)
+    prep = prepare(D)
+    y = run_tiled(D, prep, plan=plan)
+    # (fp32 sums of the rounded weights, like the matmul kernel: the tight bound holds at every length)
+    assert_tight(y, expected_output(L), f"int{bits} {K}x{N} M={M}")
+    x = L["x"].clone()
+    x[M - 1, K // 2] = float("inf")
+    y2 = run_tiled(D, prep, x=x.to(dev), plan=plan)
+    assert torch.equal(y2[:-1], y[:-1]) and not bool(torch.isfinite(y2[-1]).all())
