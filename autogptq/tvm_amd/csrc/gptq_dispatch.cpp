@@ -396,18 +396,19 @@ extern "C" int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int g
     if (M > gptq::kDecodeMaxRows) return GPTQ_HIP_ERR_UNSUPPORTED;
     const int gs = group_size == -1 ? K : group_size;
     {
-        // Layers of up to 16 columns per CU (N <= 4096): one workgroup of sixteen waves per 16-column unit, all of
-        // K staged once per workgroup (waves_n = 2 marks this kernel), when that fits LDS.  Every CU then has
-        // work (a workgroup per 32-column tile leaves half of them idle): 11008 x 4096, one row, 9.0 / 9.3 us
-        // (int4 / int3) against 10.4 / 11.0; 4096 x 4096 5.3 against 5.4-5.5.  Wider layers would give a workgroup
-        // several units; there the kernel below is faster (4096 x 11008: 7.7 / 7.8 us against 9.0 / 9.3).
+        // Layers of up to 16 columns per CU (N <= 4096), one and two rows, 2560 to 4096 channels: one workgroup of sixteen
+        // waves per 16-column unit, all of K staged once per workgroup (waves_n = 2 marks this kernel), when that fits LDS.
+        // Every CU then has work, but its workgroups are long in starting and its items cost more: the kernel below with
+        // eight waves per tile takes everything else (us, this / that: 2048 x 4096 at one / two / four rows 4.4 / 4.9 / 5.7 and
+        // 3.5 / 3.7 / 4.1, 1024 x 1024 one row 3.8 and 3.5, 2560 x 2560 groups of 32 4.5 and 4.4, 3584 x 3072 at four rows 5.9 and 4.9;
+        // at one and two rows level or ahead beyond: 3584 x 1024 groups of 32 4.4 and 4.9, 3584 x 3072 two rows 5.0 and 5.1).
         const int mr = gptq::tiled_decode_rows(M);
         const int units = N / 16;
         const int nwg = units < gptq::kNumCUs ? units : gptq::kNumCUs;
         const int upw = ceil_div(units, nwg);
         const long long lds = gptq::tiled_decode16_lds_bytes(mr, K, K / gs, upw);
         // (long K: the kernel below with every tile halved, see tiled_decode_halves_all)
-        if (M <= 4 && upw == 1 && lds <= 128 * 1024 && !gptq::tiled_decode_halves_all(N / 32, ceil_div(K, 64))) {
+        if (M <= 2 && K > 2560 && upw == 1 && lds <= 128 * 1024 && !gptq::tiled_decode_halves_all(N / 32, ceil_div(K, 64))) {
             plan->kernel = GPTQ_HIP_KERNEL_TILED_DECODE;
             plan->row_tiles = mr;
             plan->m_blocks = 1;
@@ -430,7 +431,10 @@ extern "C" int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int g
         const int mr = gptq::tiled_decode_rows(M);
         const int tiles = N / 32;
         const int S_total = ceil_div(K, 64);
-        int kw = tiles * 4 >= 1024 ? 4 : (tiles * 8 >= 1024 ? 8 : 16);
+        int kw = tiles * 4 >= 1024 ? 4 : 8;
+        // up to 1024 channels four waves, but for one and two rows of 2 to 4 bits (1024 x 4096 int4 at four rows 3.3 us, eight waves
+        // 3.8; one row 3.6 and 3.5, int8 3.8 and 4.5; 1024 x 2048 at eight rows 3.5 and 3.9)
+        if (S_total <= 16 && (M > 2 || bits == 8)) kw = 4;
         // and enough of them that a wave walks about sixteen blocks at most: a wave issues one instruction per
         // four clocks, so a long K wants more, shorter waves.  One row, us, kw = 4 / 8 / 16: 8192 x 8192
         // 12.1 / 9.4 / 9.5, 5120 x 13824 10.9 / 9.4 / 11.6, 6144 x 16384 12.7 / 11.0 / 12.4, 9216 x 9216
@@ -470,7 +474,9 @@ extern "C" int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int g
             const int span = gptq::tiled_decode_span(halved, tiles, wave_steps, kw, gs);
             const int groups = (span - 1) / gs + 2 < ceil_div(K, gs) ? (span - 1) / gs + 2 : ceil_div(K, gs);
             const int lds = gptq::tiled_decode_lds_bytes(mr, span, groups, kw);
-            if (lds > 128 * 1024) continue;
+            // (all of the LDS where every workgroup has a CU to itself anyway: an uncut K saves the reduce pass, 8192 x 8192 at
+            // eight rows 13.1 -> 9.8 us, with an activation order 13.9 -> 10.4, 16384 x 8192 at four rows 19.6 -> 15.9)
+            if (lds > ((tiles + halved) * split <= gptq::kNumCUs ? 160 : 128) * 1024) continue;
             if (split > 1 && (long long)M * N >= (1LL << 32)) return GPTQ_HIP_ERR_UNSUPPORTED;
             plan->kernel = GPTQ_HIP_KERNEL_TILED_DECODE;
             plan->row_tiles = mr;
@@ -581,14 +587,20 @@ bool gptq::select_row_blocks(int M, int K, int N, int bits, int group_size, gptq
     return false;
 }
 
+// Five to eight rows on the decode kernel: K up to 11008, and longer layers of few columns, which the matmul kernel cuts into many
+// K ranges (us at 5 to 8 rows, matmul / decode kernel: 14336 x 4096 int4 13.7 / 9.8, with an activation order 20.6 / 10.6, 12288 x 1024
+// 15.0 / 9.9, 16384 x 4096 14.7 / 12.2, 17408 x 2048 int3 21.6 / 12.7, 20480 x 2048 24.0 / 13.5, 20480 x 1024 19.1 / 10.6; 20480 x 4096 17.3 /
+// 18.0 and 16384 x 8192 21.6 / 23.8 stay).
+static bool decode_takes(int K, int N) { return K <= 11008 || (K <= 18432 && N <= 4096) || (K <= 20480 && N <= 2048); }
+
 extern "C" int gptq_hip_select_tiled(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
 {
     // Up to four rows the decode kernels (one 4-row matrix instruction set per lane block); five to eight rows the
     // workgroup-per-tile decode kernel with two sets, for K up to 11008 (us at 5 / 8 rows, int4, against the matmul
     // kernel with one 32-row tile: 4096 x 11008 9.0 / 9.4 against 9.6 / 9.7, with an activation order 12.7 / 13.2
     // against 14.0 / 14.2; 11008 x 4096 9.9 / 10.3 against 16.7 / 17.2, with an activation order 15.1 / 15.8 against
-    // 18.9 / 19.4; 4096 x 4096 7.2 / 7.8 against 9.4 / 9.5; longer K was not measured: eight staged rows of x).
-    if (M >= 1 && (M <= gptq::kDecodeSelectRows || (M <= gptq::kDecodeMaxRows && K <= 11008))) {
+    // 18.9 / 19.4; 4096 x 4096 7.2 / 7.8 against 9.4 / 9.5), and beyond for narrow layers (decode_takes).
+    if (M >= 1 && (M <= gptq::kDecodeSelectRows || (M <= gptq::kDecodeMaxRows && decode_takes(K, N)))) {
         const int rc = gptq_hip_select_tiled_decode(M, K, N, bits, group_size, plan);
         if (rc != GPTQ_HIP_ERR_UNSUPPORTED || !plan) return rc;
     }
@@ -871,7 +883,7 @@ bool tiled_wins(int M, int K, int N, bool act_order, int bits, bool one_group)
         if (K > 32768) return false;
         return K <= 6656 || (K <= 11008 && N <= 8192);
     }
-    if (M <= 8 && K <= 11008) return true;   // the decode kernel with two sets of rows (below)
+    if (M <= 8 && decode_takes(K, N)) return true;   // the decode kernel with two sets of rows (below)
     if (M <= 16) {
         // (without an activation order and K beyond 4096, against the STREAM kernel that reads x itself, 9 / 16 rows:
         // 13824 x 5120 12.4 / 15.2 against 15.9 / 18.1, 5120 x 13824 10.0 / 14.1 against 13.1 / 15.1, 11008 x 11008 19.3 / 24.9
