@@ -190,6 +190,9 @@ inline bool tiled_qualifies(int K, int N, int bits, int gs)
 // decode kernel on the tiled format: rows it is built for, and the LDS of a workgroup whose waves cover
 // `span` positions of `groups` groups
 static const int kDecodeMaxRows = 8;      // rows the decode kernel of the tiled format takes (the 16-column kernel: 4)
+// channels up to which five to eight rows run on the products of the codes, scaled per group; the weights of longer layers are
+// rounded first, as the matmul kernel that used to take them does (the two differ by the rounding of the weights, 1.7e-4)
+constexpr int kDecodeUnroundedK = 11008;
 constexpr int kRowBlocksMaxRows = 128;   // rows it takes in blocks of 8 or 16 along grid_z
 constexpr int kDecodeSelectRows = 4;   // rows up to which gptq_hip_select_tiled chooses it
 inline int tiled_decode_rows(int M) { return M <= 1 ? 1 : (M <= 2 ? 2 : (M <= 4 ? 4 : 8)); }

@@ -76,8 +76,9 @@ struct DecodeTail {
 };
 
 // PM: x lies position by position in LDS (activation order, four rows and more).
-// RB: one of several row blocks.  From nine rows on the weights are formed as the matmul kernel forms them, rounded to fp16
-// (one packed multiplication more, and no epilogue per unit: the products of the whole walk add up in the result registers).
+// RB: row blocks along blockIdx.z, on weights formed as the matmul kernel forms them, rounded to fp16 (one packed multiplication
+// more, and no epilogue per unit: the products of the whole walk add up in the result registers).  Nine rows and more, and
+// eight rows of layers beyond kDecodeUnroundedK channels, run so.
 // E: blocks of 64 positions that share one epilogue (1, or 2 when the groups are multiples of 128 channels and
 // every wave has an even number of blocks: both lane blocks of both blocks then lie in one group).
 template <int BITS, int MR, int KW, int E, bool PM, bool RB>
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     // The two halves of a tile meet through one 64-bit exchange per output (see the end of the kernel).
     const int n_halved = p.grid_x - p.T_total;           // e (0: no tile is halved)
     const int n_whole = p.T_total - n_halved;
-    const bool is_half = !RB && (int)blockIdx.x >= n_whole;
+    const bool is_half = (int)blockIdx.x >= n_whole;
     const int half_i = (int)blockIdx.x - n_whole;        // (halved tile, half) = (half_i / 2, half_i % 2)
     const int T = is_half ? n_whole + (half_i >> 1) : (int)blockIdx.x;
     const int split = is_half ? (half_i & 1) : (int)blockIdx.y;
@@ -611,10 +612,9 @@ int launch_tiled_decode(const void *x, const void *qtile, const uint32_t *sz, co
         else                                                                                                               \
             rc = pairs ? launch_decode_kw<B, R, 2, false>(p, plan, stream) : launch_decode_kw<B, R, 1, false>(p, plan, stream);       \
     }
-    if (plan.m_blocks > 1 || mr == 16) {
+    if (plan.m_blocks > 1 || mr == 16 || (mr == 8 && K > kDecodeUnroundedK)) {
         auto rows = [&](auto bits_c, auto mr_c) {
             constexpr int B = decltype(bits_c)::value, R = decltype(mr_c)::value;
-            if (plan.grid_x != p.T_total || plan.split_k != 1 || plan.waves_k > 8) return (int)GPTQ_HIP_ERR_UNSUPPORTED;   // (whole tiles, whole K)
             return kinv ? launch_decode_kw<B, R, 1, true, true>(p, plan, stream) : launch_decode_kw<B, R, 1, false, true>(p, plan, stream);
         };
         auto go = [&](auto bits_c) {

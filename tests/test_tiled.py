@@ -754,3 +754,20 @@ def test_tiled_row_blocks(dev, bits, K, N, gs, M, mr, desc_act):
     x[M - 1, K // 2] = float("inf")
     y2 = run_tiled(D, prep, x=x.to(dev), plan=plan)
     assert torch.equal(y2[:-1], y[:-1]) and not bool(torch.isfinite(y2[-1]).all())
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("K,N,gs", [(11040, 64, 32), (14336, 96, 128), (18432, 64, 1024), (20480, 64, 128)])
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_tiled_decode_long_narrow_layers(dev, bits, K, N, gs, desc_act):
+    """Five to eight rows beyond 11008 channels: on the decode kernel (halved tiles, K in ranges) and on rounded weights, so that the
+    tight bound holds at these lengths."""
+    for M in (5, 8):
+        L = layer(4400 + K + M, K, N, bits, gs, desc_act, M=M, bias=True)
+        D = to_dev(L, dev)
+        prep = prepare(D)
+        plan = _lib.select_tiled(M, K, N, bits, gs)
+        assert plan.kernel == _lib.KERNEL_TILED_DECODE and plan.row_tiles == 8
+        y = run_tiled(D, prep, plan=plan)
+        assert_tight(y, expected_output(L), f"int{bits} {K}x{N} M={M}")
+        assert torch.equal(y, run_tiled(D, prep, plan=plan)), "two identical calls differ"
