@@ -292,7 +292,7 @@ constexpr int panel_lds_bytes(int bits, int rt)
 {
     // (or what the result is added up and turned around in)
     const int stages = panel_stages(bits, rt) * panel_waves_k(rt) * panel_block_bytes(bits, rt);
-    const int turn = (panel_waves_k(rt) - 1) * 65536 + 4 * panel_waves_k(rt) * 32 * 272;
+    const int turn = panel_waves_k(rt) == 2 ? 8 * rt * 4096 : 4 * 4 * 4096;
     return stages > turn ? stages : turn;
 }
 // The kernel addresses the rows of a workgroup with 31 bits (bit 31 of an offset marks what lies outside)

@@ -193,13 +193,14 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
 
     // x: request i of this wave brings rows 8 (nw RT + i) .. + 7 of the block, 128 bytes each (rows past M lie outside the
     // buffer and read as zeros).  LDS keeps a row's eight 16-byte octets at octet ^ f(row), f = (row & 7) ^ ((row >> 3) & 1):
-    // the reads of a fragment (16 rows x 4 octets) then spread over all banks.
+    // the reads of a fragment (16 rows x 4 octets) then spread over all banks.  The second wave group swaps the halves of a row
+    // tile (16 rows each): see the result.
     uint32_t xo[RT];
 #pragma unroll
     for (int i = 0; i < RT; i++) {
         const int blk = nw * RT + i;
         const int oct = (lane & 7) ^ (lane >> 3) ^ (blk & 1);
-        xo[i] = (uint32_t)(8 * blk + (lane >> 3)) * (uint32_t)ldx * 2u + (uint32_t)oct * 16u;
+        xo[i] = (uint32_t)(8 * (blk ^ (2 * kw)) + (lane >> 3)) * (uint32_t)ldx * 2u + (uint32_t)oct * 16u;
     }
     // a block past the workgroup's range (a walk of an odd count of blocks), and the half of a last block that lies past K,
     // are sent out of the buffer's range as well
@@ -422,9 +423,14 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
     // ---- the result ----
     // (the compiler does not know of the matrix instructions in flight: their results want 18 cycles)
     asm volatile("s_nop 15\n\ts_nop 7\n\ts_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    // Two wave groups add up in LDS, two row tiles at a time: each hands the other the tile that the other finishes.  A
-    // finished tile (32 rows x 64 columns) is turned around in LDS of the wave's own and stored in rows.
-    unsigned char *give = smem + w * 8192, *take = smem + (w ^ NW) * 8192, *mine = smem + (KW - 1) * 65536 + w * (32 * 272);
+    // In pieces of 16 rows x 64 columns, RT of them per wave: two wave groups add up in LDS, each wave hands over every other
+    // piece (acc[2 rt + 1]; the second group holds the halves of a row tile the other way round, so that it keeps what the first hands
+    // over); a group alone finishes all 2 RT.  A finished piece is turned around in LDS of the wave's own and stored
+    // in rows.  (One exchange, the same code for both groups and each with half of the work, where the groups took turns at whole row
+    // tiles, an exchange per two of them: 333 rows of 5120 x 3424 int8 27.5 -> 27.0 us, 701 of 7936 x 1600 33.8 -> 33.0, 1000 of 8192 x 8192
+    // 113.4 -> 111.8; a quarter of a row per four lanes, stored without turning the piece, was slower than before.)
+    constexpr int SLOT = 4096;
+    unsigned char *give = smem + w * (RT * SLOT), *take = KW == 2 ? smem + (w ^ NW) * (RT * SLOT) : smem + w * (4 * SLOT);
     const int c8 = (lane & 7) * 8, T8 = T0 + (c8 >> 5);
     f4 bias[NC];
 #pragma unroll
@@ -444,96 +450,76 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
         for (int e = 0; e < 8; e++) to[e] = min(max(to[e], 0), N - 1);
     }
     _Float16 *y = (_Float16 *)t.y;
-    auto finish = [&](auto rt_c) {
-        constexpr int rt = decltype(rt_c)::value;
-        f4 sum[2][NC];
+    if constexpr (KW == 2) {
 #pragma unroll
-        for (int e = 0; e < 2; e++)
+        for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-            for (int c = 0; c < NC; c++)
-                sum[e][c] = acc[2 * rt + e][c] + (KW == 2 ? *(const f4 *)(take + (e * NC + c) * 1024 + lane * 16) + bias[c] : bias[c]);
-        if (t.split_k > 1) {
-#pragma unroll
-            for (int e = 0; e < 2; e++)
-#pragma unroll
-                for (int c = 0; c < NC; c++) *(f4 *)(mine + (16 * e + i16) * 272 + (16 * c + 4 * q4) * 4) = sum[e][c];
-            const int c4 = (lane & 15) * 4, T4 = T0 + (c4 >> 5);
-#pragma unroll
-            for (int it = 0; it < 8; it++) {
-                const int m = 4 * it + (lane >> 4), row = row0 + 32 * rt + m;
-                const f4 v = *(const f4 *)(mine + m * 272 + c4 * 4);
-                if (row < M && T4 < T_total)
-                    *(f4 *)(t.partial + ((size_t)split * M + row) * (size_t)N + 32 * T4 + (c4 & 31)) = v;
-            }
-            return;
-        }
-#pragma unroll
-        for (int e = 0; e < 2; e++)
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                h4 o;
-#pragma unroll
-                for (int v = 0; v < 4; v++) o[v] = (_Float16)sum[e][c][v];
-                *(h4 *)(mine + (16 * e + i16) * 144 + (16 * c + 4 * q4) * 2) = o;
-            }
-#pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const int m = 8 * it + (lane >> 3), row = row0 + 32 * rt + m;
-            const h8 v = *(const h8 *)(mine + m * 144 + c8 * 2);
-            if (row < M && T8 < T_total) {
-                if (TRANS && t.out_map) {
-#pragma unroll
-                    for (int e = 0; e < 8; e++) y[(size_t)row * N + to[e]] = v[e];
-                } else {
-                    *(h8 *)(y + (size_t)row * N + 32 * T8 + (c8 & 31)) = v;
-                }
-            }
-        }
-    };
-    auto hand_over = [&](auto rt_c) {
-        constexpr int rt = decltype(rt_c)::value;
-#pragma unroll
-        for (int e = 0; e < 2; e++)
-#pragma unroll
-            for (int c = 0; c < NC; c++) *(f4 *)(give + (e * NC + c) * 1024 + lane * 16) = acc[2 * rt + e][c];
-    };
-    // (the results stay in the accumulation registers until their turn: all of them at once would spill)
-    auto keep = [&](auto rt_c) {
-        constexpr int rt = decltype(rt_c)::value;
-#pragma unroll
-        for (int e = 0; e < 2; e++)
-#pragma unroll
-            for (int c = 0; c < NC; c++) panel_pin(acc[2 * rt + e][c]);
-    };
-    if constexpr (KW == 1) {
-        [&]<int... R>(std::integer_sequence<int, R...>) {
-            ([&] {
-                keep(std::integral_constant<int, R>{});
-                finish(std::integral_constant<int, R>{});
-                __builtin_amdgcn_sched_barrier(0);
-            }(), ...);
-        }(std::make_integer_sequence<int, RT>{});
-    } else {
-        [&]<int... P>(std::integer_sequence<int, P...>) {
-            ([&] {
-                constexpr auto first = std::integral_constant<int, 2 * P>{};
-                constexpr auto second = std::integral_constant<int, 2 * P + 1 < RT ? 2 * P + 1 : 2 * P>{};
-                keep(first);
-                keep(second);
-                if (P > 0) __syncthreads();   // the last hand-over has been read
-                if (kw == 1)
-                    hand_over(first);
-                else if (second > first)
-                    hand_over(second);
-                __syncthreads();
-                if (kw == 0)
-                    finish(first);
-                else if (second > first)
-                    finish(second);
-                __builtin_amdgcn_sched_barrier(0);
-            }(), ...);
-        }(std::make_integer_sequence<int, (RT + 1) / 2>{});
+            for (int c = 0; c < NC; c++) *(f4 *)(give + rt * SLOT + c * 1024 + lane * 16) = acc[2 * rt + 1][c];
+        __syncthreads();
     }
+    // two pieces at a time: rows row0 + 16 mt .. + 15 (the second group's, 16 further on)
+    constexpr int PIECES = KW == 2 ? RT : 2 * RT;
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        ([&] {
+            constexpr int n = 2 * I + 1 < PIECES ? 2 : 1;
+            unsigned char *slot[2];
+            f4 sum[2][NC];
+            int first[2];
+#pragma unroll
+            for (int e = 0; e < n; e++) {
+                const int mt = KW == 2 ? 2 * (2 * I + e) : 2 * I + e;
+                slot[e] = take + (KW == 2 ? 2 * I + e : (2 * I + e) % 4) * SLOT;
+                first[e] = row0 + 16 * mt + (KW == 2 ? 16 * kw : 0);
+#pragma unroll
+                for (int c = 0; c < NC; c++) panel_pin(acc[mt][c]);   // (the others stay in the accumulation registers until their turn)
+#pragma unroll
+                for (int c = 0; c < NC; c++)
+                    sum[e][c] = acc[mt][c] + (KW == 2 ? *(const f4 *)(slot[e] + c * 1024 + lane * 16) + bias[c] : bias[c]);
+            }
+            if (t.split_k > 1) {
+                // (16 bytes of a row at place ^ row)
+                const int c4 = (lane & 15) * 4, T4 = T0 + (c4 >> 5);
+#pragma unroll
+                for (int e = 0; e < n; e++)
+#pragma unroll
+                    for (int c = 0; c < NC; c++) *(f4 *)(slot[e] + i16 * 256 + ((4 * c + q4) ^ i16) * 16) = sum[e][c];
+#pragma unroll
+                for (int e = 0; e < n; e++)
+#pragma unroll
+                    for (int it = 0; it < 4; it++) {
+                        const int m = 4 * it + (lane >> 4), row = first[e] + m;
+                        const f4 v = *(const f4 *)(slot[e] + m * 256 + ((lane & 15) ^ m) * 16);
+                        if (row < M && T4 < T_total) *(f4 *)(t.partial + ((size_t)split * M + row) * (size_t)N + 32 * T4 + (c4 & 31)) = v;
+                    }
+            } else {
+#pragma unroll
+                for (int e = 0; e < n; e++)
+#pragma unroll
+                    for (int c = 0; c < NC; c++) {
+                        h4 o;
+#pragma unroll
+                        for (int v = 0; v < 4; v++) o[v] = (_Float16)sum[e][c][v];
+                        *(h4 *)(slot[e] + i16 * 144 + (16 * c + 4 * q4) * 2) = o;
+                    }
+#pragma unroll
+                for (int e = 0; e < n; e++)
+#pragma unroll
+                    for (int it = 0; it < 2; it++) {
+                        const int m = 8 * it + (lane >> 3), row = first[e] + m;
+                        const h8 v = *(const h8 *)(slot[e] + m * 144 + c8 * 2);
+                        if (row < M && T8 < T_total) {
+                            if (TRANS && t.out_map) {
+#pragma unroll
+                                for (int k = 0; k < 8; k++) y[(size_t)row * N + to[k]] = v[k];
+                            } else {
+                                *(h8 *)(y + (size_t)row * N + 32 * T8 + (c8 & 31)) = v;
+                            }
+                        }
+                    }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }(), ...);
+    }(std::make_integer_sequence<int, (PIECES + 1) / 2>{});
 }
 
 // xs[m][p] = x[m][xsrc[p]]: the activations in the order of the tiled copy.  A workgroup takes ROWS rows and one of gridDim.y
