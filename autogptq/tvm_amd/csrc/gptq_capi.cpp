@@ -319,11 +319,16 @@ static int run_panel(const void *x, const void *qtile, const uint32_t *sz, const
         plan.grid_z != plan.m_blocks || plan.m_blocks != (M + 32 * rt - 1) / (32 * rt) ||
         plan.split_k != (S_total + plan.k_chunk - 1) / plan.k_chunk || plan.lds_bytes != gptq::panel_lds_bytes(bits, rt))
         return GPTQ_HIP_ERR_BAD_ARG;
-    if (!gptq::panel_launches((long long)plan.grid_x * plan.m_blocks, plan.block, trans && xsrc ? M : 0)) return GPTQ_HIP_ERR_UNSUPPORTED;
+    // K ranges for the row blocks from main on only
+    const int main = gptq::panel_main_blocks(plan);
+    if (plan.flags & ((1 << gptq::kPanelMainShift) - 1) || (main > 0 && (plan.split_k == 1 || main >= plan.m_blocks))) return GPTQ_HIP_ERR_BAD_ARG;
+    const int rows = M - 32 * rt * main;   // (of the tail; all of them without main blocks)
+    if (!gptq::panel_launches((long long)plan.grid_x * (main + (long long)(plan.m_blocks - main) * plan.split_k), plan.block, trans && xsrc ? M : 0))
+        return GPTQ_HIP_ERR_UNSUPPORTED;
     if (plan.split_k > 1 && (long long)M * cols >= (1LL << 32)) return GPTQ_HIP_ERR_UNSUPPORTED;
-    const size_t part = plan.split_k > 1 ? ((size_t)plan.split_k * M * cols * sizeof(float) + 255) / 256 * 256 : 0;
+    const size_t part = plan.split_k > 1 ? ((size_t)plan.split_k * rows * cols * sizeof(float) + 255) / 256 * 256 : 0;
     // x in the order of the copy, or the transposed product's result before its channels are put in order
-    const size_t xb = xsrc && (!trans || (plan.split_k == 1 && gptq::panel_scatters(M, K))) ? (size_t)M * K * 2 : 0;
+    const size_t xb = xsrc && (!trans || main > 0 || (plan.split_k == 1 && gptq::panel_scatters(M, K))) ? (size_t)M * K * 2 : 0;
     if (part + xb > 0 && (!workspace || !aligned(workspace, 16) || workspace_bytes < gptq::kCounterBytes + part + xb))
         return GPTQ_HIP_ERR_WORKSPACE;
     char *ws = (char *)workspace + gptq::kCounterBytes;

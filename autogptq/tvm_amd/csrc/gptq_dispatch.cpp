@@ -738,6 +738,17 @@ double panel_us(int rt, int split, int chunk, long long wgs, int bits, double ou
     return 4.8 + full * turn(256) + (last ? turn((double)last) : 0.0) + (split > 1 ? 2.2 + 0.86e-6 * split * out_elems : 0.0);
 }
 
+// The same where the first `main` row blocks take all of K in whole turns and the rest is cut into ranges: the CUs that the last
+// whole turn leaves idle begin with the ranges.
+double panel_tail_us(int rt, int S_total, int chunk, int split, int col_wgs, int main, int tail, int bits, double tail_elems)
+{
+    const double whole = panel_us(rt, 1, S_total, 256, bits, 0) - 4.8, part = panel_us(rt, 1, chunk, 256, bits, 0) - 4.8;
+    const long long wgs = (long long)col_wgs * main, full = (wgs + 255) / 256, idle = full * 256 - wgs;
+    const long long left = (long long)col_wgs * tail * split - idle * (long long)(whole / part);
+    const double rest = left <= 0 ? 0 : panel_us(rt, 1, chunk, left, bits, 0) - 4.8;
+    return 4.8 + full * whole + rest + 2.2 + 0.86e-6 * split * tail_elems;
+}
+
 // The same for the matmul kernel's plan (the tables above), 9 % rms over the same layers.
 double tiled_us(const gptq_hip_plan &p, int bits, bool transposed, double out_elems, double in_elems, bool act_order)
 {
@@ -780,7 +791,7 @@ extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_si
     const int red = transposed ? N : K, cols = transposed ? K : N;
     const int S_total = ceil_div(red, 64), col_wgs = ceil_div(cols, gptq::kPanelCols);
     const double out_elems = (double)M * cols;
-    int rt = row_tiles, split = split_k;
+    int rt = row_tiles, split = split_k, main = 0;
     if (rt == 0 || split == 0) {
         if (M <= gptq::kDecodeMaxRows && rt == 0 && split == 0) return GPTQ_HIP_ERR_UNSUPPORTED;   // (the decode kernels' rows)
         double best = 1e30;
@@ -796,6 +807,29 @@ extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_si
             }
         }
         if (rt == 0 || split == 0) return GPTQ_HIP_ERR_UNSUPPORTED;
+        // More than a turn of the chip: whole turns, and the last row blocks in K ranges that fill one turn more.  2000 rows of
+        // 9216 x 9216 int3 (36 column positions): 13 blocks of 160 rows are 468 workgroups, 310 us; 8 of 256 rows are 288, 252 of them
+        // uncut and the last block in seven ranges 278.  Rarely the best plan by more than a little (7 % of 121 drawn calls of more than a turn
+        // gain over 3 %), hence the margin.
+        if (row_tiles == 0 && split_k == 0) {
+            double best_tail = 0.97 * best;
+            for (int r = 1; r <= gptq::kPanelMaxTiles; r++) {
+                const int blocks = ceil_div(M, 32 * r);
+                if (!gptq::panel_addresses(r, red)) continue;
+                const long long most = ((long long)col_wgs * blocks - 1) / 256;   // whole turns (one or two fewer for a longer tail)
+                for (long long turns = most > 2 ? most - 2 : 1; turns <= most; turns++) {
+                    const int m = (int)(turns * 256 / col_wgs);
+                    if (m < 1 || m >= blocks || m >= 1 << 20) continue;
+                    const double elems = (double)(M - 32 * r * m) * cols;
+                    for (int s = 2; s <= 8; s++) {
+                        const int chunk = ceil_div(S_total, s);
+                        if (S_total / s < 6 || ceil_div(S_total, chunk) != s || s * elems > 48e6) continue;
+                        const double us = panel_tail_us(r, S_total, chunk, s, col_wgs, m, blocks - m, bits, elems);
+                        if (us < best_tail) best = best_tail = us, rt = r, split = s, main = m;
+                    }
+                }
+            }
+        }
         if (row_tiles == 0 && split_k == 0) {
             // an activation order: a pass that puts x (or the result) in the layer's order
             if (act) best += transposed ? 2.5 + 0.9e-6 * M * K : 3.5 + 0.7e-6 * M * K;
@@ -814,7 +848,8 @@ extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_si
     }
     if (rt > gptq::kPanelMaxTiles || !gptq::panel_addresses(rt, red)) return GPTQ_HIP_ERR_UNSUPPORTED;
     const int m_blocks = ceil_div(M, 32 * rt);
-    if (!gptq::panel_launches((long long)col_wgs * m_blocks, 256 * gptq::panel_waves_k(rt), transposed && act ? M : 0)) return GPTQ_HIP_ERR_UNSUPPORTED;
+    if (!gptq::panel_launches((long long)col_wgs * (main + (long long)(m_blocks - main) * split), 256 * gptq::panel_waves_k(rt), transposed && act ? M : 0))
+        return GPTQ_HIP_ERR_UNSUPPORTED;
     plan->kernel = GPTQ_HIP_KERNEL_PANEL;
     plan->row_tiles = rt;
     plan->m_blocks = m_blocks;
@@ -827,8 +862,9 @@ extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_si
     plan->grid_z = m_blocks;
     plan->block = 256 * gptq::panel_waves_k(rt);
     plan->lds_bytes = gptq::panel_lds_bytes(bits, rt);
+    plan->flags = main << gptq::kPanelMainShift;
     size_t ws = gptq::kCounterBytes;
-    if (plan->split_k > 1) ws += ((size_t)plan->split_k * M * cols * sizeof(float) + 255) / 256 * 256;
+    if (plan->split_k > 1) ws += ((size_t)plan->split_k * (M - 32 * rt * main) * cols * sizeof(float) + 255) / 256 * 256;
     if (act) ws += ((size_t)M * K * 2 + 255) / 256 * 256;   // x, or the transposed product's result, in the copy's order
     plan->workspace_bytes = plan->split_k > 1 || act ? ws : 0;
     return GPTQ_HIP_OK;

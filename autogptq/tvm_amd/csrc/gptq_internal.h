@@ -302,6 +302,9 @@ constexpr bool panel_launches(long long wgs, int block, long long ordered_rows)
 {
     return wgs * block < (1LL << 32) && ordered_rows * 256 < (1LL << 32);
 }
+// row blocks of a plan with K ranges that take all of K, ahead of the ones that are cut (in the upper bits of the plan's flags)
+constexpr int kPanelMainShift = 8;
+inline int panel_main_blocks(const gptq_hip_plan &plan) { return (int)((unsigned)plan.flags >> kPanelMainShift); }
 // rows x channels from which the transposed product puts its result's channels in order in a pass (2.5 us and 0.9 us per
 // million, against 3.7 us per million for scattered stores)
 inline bool panel_scatters(int M, int K) { return (long long)M * K >= (1LL << 20); }

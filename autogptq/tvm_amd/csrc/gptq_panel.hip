@@ -27,11 +27,26 @@ namespace gptq {
 struct PanelTail {
     const void *bias;        // fp16 [N] or nullptr
     void *y;                 // fp16 [M, N]
-    float *partial;          // [split_k][M][N] when split_k > 1
+    float *partial;          // [split_k][rows of the tail][N] when split_k > 1
     const int32_t *out_map;  // TRANS: channel of result column p (nullptr = identity)
     uint32_t q_bytes, s_bytes;
-    int split_k, col_wgs, row_wgs, tiles_per_group, lb_per_group, G;
+    int col_wgs, main_rbs, tail_rbs, split_k, tail_steps, lb_per_group, G;
+    // what the divisors of the first addresses are multiplied by instead (panel_div)
+    uint32_t column_group_magic, tail_magic, lb_magic, tile_magic;
+    uint32_t step_groups, step_rem;   // 2 x wave groups of lane blocks: whole groups, and the rest
 };
+
+// n / d by one multiplication, magic = floor(2^32 / d) + 1: exact while n d < 2^32 (e = d magic - 2^32 <= d adds less than 1 / d).
+// 0 stands for d = 1; the host takes 1 for sizes beyond, which are divided.
+static uint32_t panel_magic(unsigned long long most, uint32_t d)
+{
+    return d <= 1 ? 0u : (most * d < (1ull << 32) ? (uint32_t)((1ull << 32) / d) + 1u : 1u);
+}
+__device__ __forceinline__ uint32_t panel_div(uint32_t n, uint32_t d, uint32_t magic)
+{
+    if (magic == 1u) return n / d;
+    return magic ? __umulhi(n, magic) : n;
+}
 
 // A request brings 1 KB (or 256 bytes) from a buffer into LDS: lane i's 16 (4) bytes land at lds + off + 16 i (4 i).  Inline
 // assembly, so that the compiler does not wait for every outstanding request before each read of LDS; the kernel counts
@@ -143,7 +158,7 @@ constexpr int panel_pieces(int i, int all, int first)
 
 template <int BITS, int RT, bool TRANS>
 __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _Float16 *x, const char *qtile, const uint32_t *sz, int M, int ldx,
-                                                       int N, int S_total, int T_total, int wg_steps, const PanelTail t)
+                                                       int N, int S_total, int T_total, const PanelTail t)
 {
     using Codec = TileCodec<BITS>;
     constexpr int KINDS = Codec::KINDS;
@@ -169,19 +184,27 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
     const int kw = w / NW, nw = w % NW;
     const int i16 = lane & 15, q4 = lane >> 4;
 
+    // The first main_rbs row blocks take all of K each, the tail_rbs after them K in split_k ranges: whole turns of the chip,
+    // and what is left of the rows spread over one turn more.
     // XCD-aware order: workgroups are dealt to the XCDs round robin, so id % 8 names the XCD; each takes a
     // contiguous run of the tile order, in which groups of four row blocks walk the columns together
-    int rb, cb;
+    int rb, cb, split = 0;
+    const int n_main = t.col_wgs * t.main_rbs;
+    const bool tail_wg = (int)blockIdx.x >= n_main;
+    const bool ranges = tail_wg && t.split_k > 1;
     {
-        const int nwg = t.col_wgs * t.row_wgs, id = blockIdx.x;
-        const int q = nwg / 8, r = nwg % 8, xcd = id % 8, i = id / 8;
-        const int lin = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + i;
-        const int per = 4 * t.col_wgs, grp = lin / per, in = lin - grp * per;
-        const int rows = min(4, t.row_wgs - 4 * grp);
-        cb = in / rows;
-        rb = 4 * grp + (in - cb * rows);
+        const uint32_t row_wgs = tail_wg ? t.tail_rbs : t.main_rbs, nwg = t.col_wgs * row_wgs;
+        uint32_t id = blockIdx.x - (tail_wg ? n_main : 0);
+        if (ranges) split = (int)panel_div(id, nwg, t.tail_magic), id -= split * nwg;
+        const uint32_t q = nwg / 8, r = nwg % 8, xcd = id % 8, i = id / 8;
+        const uint32_t lin = xcd * q + min(xcd, r) + i;
+        const uint32_t per = 4 * t.col_wgs, grp = panel_div(lin, per, t.column_group_magic), in = lin - grp * per;
+        const uint32_t rows = min(4u, row_wgs - 4 * grp);
+        const uint32_t c = rows == 4 ? in / 4 : (rows == 3 ? in / 3 : (rows == 2 ? in / 2 : in));
+        cb = (int)c;
+        rb = (int)(4 * grp + (in - c * rows)) + (tail_wg ? t.main_rbs : 0);
     }
-    const int split = blockIdx.y;
+    const int wg_steps = tail_wg ? t.tail_steps : S_total;
     const int row0 = rb * 32 * RT;
     const int T0 = cb * NW * CT + nw * CT;
     const int S_begin = split * wg_steps, S_last = S_total - 1;
@@ -220,13 +243,14 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
     for (int i = 0; i < CT; i++) {
         const int T = min(T0 + i, T_total - 1);   // (a missing tile repeats the last one; it is never stored)
         q_base[i] = (uint32_t)T * (uint32_t)S_total * (uint32_t)BW;
-        s_base[i] = TRANS ? (uint32_t)(T / t.tiles_per_group) * (uint32_t)S_total * 256u : 128u * (uint32_t)T;
+        s_base[i] = TRANS ? panel_div((uint32_t)T, (uint32_t)t.lb_per_group, t.tile_magic) * (uint32_t)S_total * 256u : 128u * (uint32_t)T;
     }
     // the group of this lane's half of the block requested next, as an offset into sz; a step moves on by 2 KW runs of 32 positions
     const uint32_t row_bytes = 4u * (uint32_t)N, lbg = (uint32_t)t.lb_per_group;
     const uint32_t lb0 = 2u * (uint32_t)(S_begin + kw) + (uint32_t)(lane >> 5);
-    uint32_t g_off = (lb0 / lbg) * row_bytes + (uint32_t)(lane & 31) * 4u, g_rem = lb0 % lbg;
-    const uint32_t g_skip = 2u * KW / lbg * row_bytes, g_inc = 2u * KW % lbg;
+    const uint32_t g0 = panel_div(lb0, lbg, t.lb_magic);
+    uint32_t g_off = g0 * row_bytes + (uint32_t)(lane & 31) * 4u, g_rem = lb0 - g0 * lbg;
+    const uint32_t g_skip = t.step_groups * row_bytes, g_inc = t.step_rem;
     auto next_group = [&]() {
         g_rem += g_inc;
         const bool over = g_rem >= lbg;
@@ -436,7 +460,7 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
 #pragma unroll
     for (int c = 0; c < NC; c++) {
         bias[c] = (f4){0.f, 0.f, 0.f, 0.f};
-        if (!TRANS && t.bias && t.split_k == 1) {
+        if (!TRANS && t.bias && !ranges) {
             const h4 v = *(const h4 *)((const _Float16 *)t.bias + 32 * min(T0 + (c >> 1), T_total - 1) + 16 * (c & 1) + 4 * q4);
             bias[c] = (f4){(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
         }
@@ -476,8 +500,9 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
                 for (int c = 0; c < NC; c++)
                     sum[e][c] = acc[mt][c] + (KW == 2 ? *(const f4 *)(slot[e] + c * 1024 + lane * 16) + bias[c] : bias[c]);
             }
-            if (t.split_k > 1) {
+            if (ranges) {
                 // (16 bytes of a row at place ^ row)
+                const int tail0 = 32 * RT * t.main_rbs;
                 const int c4 = (lane & 15) * 4, T4 = T0 + (c4 >> 5);
 #pragma unroll
                 for (int e = 0; e < n; e++)
@@ -489,7 +514,7 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
                     for (int it = 0; it < 4; it++) {
                         const int m = 4 * it + (lane >> 4), row = first[e] + m;
                         const f4 v = *(const f4 *)(slot[e] + m * 256 + ((lane & 15) ^ m) * 16);
-                        if (row < M && T4 < T_total) *(f4 *)(t.partial + ((size_t)split * M + row) * (size_t)N + 32 * T4 + (c4 & 31)) = v;
+                        if (row < M && T4 < T_total) *(f4 *)(t.partial + ((size_t)split * (M - tail0) + (row - tail0)) * (size_t)N + 32 * T4 + (c4 & 31)) = v;
                     }
             } else {
 #pragma unroll
@@ -550,11 +575,11 @@ __global__ __launch_bounds__(256) void panel_gather_kernel(const _Float16 *__res
     }
 }
 
-// The way back for the transposed product: gx[m][xsrc[p]] = gs[m][p], or the sum of the K ranges' partial results.  A row is
+// The way back for the transposed product: gx[m][xsrc[p]] = gs[m][p], or, from row tail0 on, the sum of the K ranges' partial results.  A row is
 // put in order in LDS and leaves it in one piece (2048 x 4096: 6.1 to 8.3 us; stores of two bytes from the product itself cost 31).
 __global__ __launch_bounds__(256) void panel_scatter_kernel(const _Float16 *__restrict__ gs, const float *__restrict__ partial,
                                                             const int32_t *__restrict__ xsrc, _Float16 *__restrict__ gx, int M,
-                                                            int K, int split)
+                                                            int K, int split, int tail0)
 {
     const int row = blockIdx.x;
     _Float16 *xl = (_Float16 *)smem;
@@ -562,10 +587,10 @@ __global__ __launch_bounds__(256) void panel_scatter_kernel(const _Float16 *__re
         const int4 u = *(const int4 *)(xsrc + 8 * o), v = *(const int4 *)(xsrc + 8 * o + 4);
         const int idx[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
         h8 g;
-        if (partial) {
+        if (partial && row >= tail0) {
             f4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
             for (int s = 0; s < split; s++) {
-                const f4 *p = (const f4 *)(partial + ((size_t)s * M + row) * K + 8 * o);
+                const f4 *p = (const f4 *)(partial + ((size_t)s * (M - tail0) + (row - tail0)) * K + 8 * o);
                 a += p[0], b += p[1];
             }
 #pragma unroll
@@ -606,11 +631,11 @@ static int launch_panel_gather(const void *x, const int32_t *xsrc, void *xs, int
 }
 
 static int launch_panel_scatter(const void *gs, const float *partial, const int32_t *xsrc, void *gx, int M, int K, int split,
-                                hipStream_t stream)
+                                int tail0, hipStream_t stream)
 {
     if (!allow_lds(panel_scatter_kernel, K * 2)) return GPTQ_HIP_ERR_LAUNCH;
     hipLaunchKernelGGL(panel_scatter_kernel, dim3(M), dim3(256), K * 2, stream, (const _Float16 *)gs, partial, xsrc,
-                       (_Float16 *)gx, M, K, split);
+                       (_Float16 *)gx, M, K, split, tail0);
     return hipGetLastError() == hipSuccess ? GPTQ_HIP_OK : GPTQ_HIP_ERR_LAUNCH;
 }
 
@@ -621,8 +646,8 @@ static int launch_panel_one(const _Float16 *x, const char *qtile, const uint32_t
     auto kern = panel_kernel<BITS, RT, TRANS>;
     const int lds = panel_lds_bytes(BITS, RT);
     if (!allow_lds(kern, lds)) return GPTQ_HIP_ERR_LAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)plan.grid_x * (unsigned)plan.m_blocks, plan.split_k), dim3(256 * panel_waves_k(RT)), lds, stream, x, qtile,
-                       sz, M, ldx, N, S_total, T_total, plan.k_chunk, t);
+    hipLaunchKernelGGL(kern, dim3((unsigned)t.col_wgs * ((unsigned)t.main_rbs + (unsigned)t.tail_rbs * (unsigned)t.split_k)), dim3(256 * panel_waves_k(RT)), lds,
+                       stream, x, qtile, sz, M, ldx, N, S_total, T_total, t);
     return hipGetLastError() == hipSuccess ? GPTQ_HIP_OK : GPTQ_HIP_ERR_LAUNCH;
 }
 
@@ -667,8 +692,14 @@ int launch_panel(const void *x, const void *qtile, const uint32_t *sz, const int
     t.G = K / group_size;
     t.q_bytes = (uint32_t)((unsigned long long)T_total * S_total * 256 * bits);
     t.s_bytes = trans ? (uint32_t)t.G * (uint32_t)S_total * 256u : (uint32_t)t.G * (uint32_t)N * 4u;
-    t.split_k = plan.split_k, t.col_wgs = plan.grid_x, t.row_wgs = plan.m_blocks;
-    t.tiles_per_group = t.lb_per_group = group_size / 32;
+    const int main_rbs = plan.split_k > 1 ? panel_main_blocks(plan) : 0, tail0 = 32 * plan.row_tiles * main_rbs;
+    t.col_wgs = plan.grid_x, t.main_rbs = main_rbs, t.tail_rbs = plan.m_blocks - main_rbs, t.split_k = plan.split_k, t.tail_steps = plan.k_chunk;
+    t.lb_per_group = group_size / 32;
+    const uint32_t lbg = (uint32_t)t.lb_per_group, pair = 2u * panel_waves_k(plan.row_tiles), tail_wgs = (uint32_t)(t.col_wgs * t.tail_rbs);
+    const unsigned long long wgs = (unsigned long long)t.col_wgs * plan.m_blocks;
+    t.column_group_magic = panel_magic(wgs, 4u * t.col_wgs), t.tail_magic = panel_magic((unsigned long long)tail_wgs * t.split_k, tail_wgs);
+    t.lb_magic = panel_magic(2ull * S_total + 64, lbg), t.tile_magic = panel_magic(T_total, lbg);
+    t.step_groups = pair / lbg, t.step_rem = pair % lbg;
     int rc = GPTQ_HIP_ERR_BAD_ARG;
     auto go = [&](auto bits_c) {
         constexpr int B = decltype(bits_c)::value;
@@ -683,8 +714,9 @@ int launch_panel(const void *x, const void *qtile, const uint32_t *sz, const int
         default: break;
     }
     if (rc != GPTQ_HIP_OK) return rc;
-    if (scatter) return launch_panel_scatter(xs, plan.split_k > 1 ? partial : nullptr, xsrc, y, M, K, plan.split_k, stream);
-    return plan.split_k > 1 ? launch_tiled_reduce(partial, bias, y, M, N_out, plan.split_k, nullptr, stream) : GPTQ_HIP_OK;
+    if (scatter) return launch_panel_scatter(xs, plan.split_k > 1 ? partial : nullptr, xsrc, y, M, K, plan.split_k, tail0, stream);
+    if (plan.split_k == 1) return GPTQ_HIP_OK;
+    return launch_tiled_reduce(partial, bias, (_Float16 *)y + (size_t)tail0 * N_out, M - tail0, N_out, plan.split_k, nullptr, stream);
 }
 
 }  // namespace gptq

@@ -79,7 +79,8 @@ typedef struct gptq_hip_plan {
     int grid_x, grid_y, grid_z;
     int block;              /* threads per workgroup */
     int lds_bytes;          /* dynamic LDS per workgroup */
-    int flags;              /* GPTQ_HIP_PLAN_* bits */
+    int flags;              /* GPTQ_HIP_PLAN_* bits (below 256); PANEL with split_k > 1: flags / 256 row blocks at the head take all of K,
+                               the ranges (split_k, k_chunk) are those of the blocks after them */
     size_t workspace_bytes; /* 0 when the plan needs none (e.g. GROUPED with split_k == 1) */
 } gptq_hip_plan;
 

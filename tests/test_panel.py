@@ -415,3 +415,45 @@ def test_panel_results_at_an_eight_byte_offset(dev, desc_act):
                 run(out)
                 assert_tight(out, ref, f"M={M} columns={cols} row tiles {rt} ranges {split}")
                 assert bool((buf[:60] == 1234.0).all()) and bool((buf[60 + M * cols:] == 1234.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("desc_act", [False, True])
+@pytest.mark.parametrize("bits,K,N,M,rt,split,main", [(4, 1600, 800, 500, 2, 3, 4), (3, 1056, 544, 330, 4, 2, 1), (8, 832, 288, 1100, 8, 2, 4),
+                                                      (2, 800, 1312, 353, 5, 2, 2), (4, 2048, 320, 97, 1, 5, 3)])
+def test_panel_ranges_for_the_last_row_blocks_only(dev, desc_act, bits, K, N, M, rt, split, main):
+    """The first `main` row blocks take all of K, the ones after them are cut into ranges: both products, the result's channels put in
+    order from both kinds of rows; and nothing outside of the result is written."""
+    gs = 32
+    L = layer(9990 + rt, K, N, bits, gs, desc_act, M=M, bias=True)
+    D = to_dev(L, dev)
+
+    def plan(tr):
+        p = _lib.select_panel(M, K, N, bits, gs, desc_act, tr, rt, split)
+        assert p.split_k == split and p.m_blocks > main
+        p.flags = main << 8
+        return p
+
+    want = expected_output(L)
+    buf = torch.full((64 + M * N + 64,), 1234.0, dtype=torch.float16, device=dev)
+    y = buf[64:64 + M * N].view(M, N)
+    forward(D, plan(False), out=y)
+    assert_tight(y, want, f"int{bits} rt={rt} ranges {split} after {main} blocks")
+    assert bool((buf[:64] == 1234.0).all()) and bool((buf[64 + M * N:] == 1234.0).all())
+    gy = torch.randn(M, N, generator=torch.Generator().manual_seed(M)).half()
+    gx = transposed(D, gy.to(dev), plan(True))
+    assert_tight(gx, gy.float() @ expected_weight(L).float().t(), f"transposed int{bits} rt={rt} ranges {split} after {main} blocks")
+
+
+def test_panel_plans_with_ranges_for_the_last_blocks():
+    # 36 column positions: eight blocks of 256 rows are a turn and an eighth of the chip
+    p = _lib.select_panel(2000, 9216, 9216, 3, -1, False)
+    main = p.flags >> 8
+    assert 0 < main < p.m_blocks and p.split_k > 1 and p.flags & 255 == 0 and main * p.grid_x <= 256
+    assert p.workspace_bytes == 16384 + p.split_k * (2000 - 32 * p.row_tiles * main) * 9216 * 4
+    fake, null = ctypes.c_void_p(0x1000), ctypes.c_void_p(None)
+    for flags, split in ((p.m_blocks << 8, p.split_k), (main << 8 | 1, p.split_k), (1 << 8, 1)):
+        q = _lib.select_panel(2000, 9216, 9216, 3, -1, False, False, p.row_tiles, split)
+        q.flags = flags
+        assert _lib.lib().gptq_hip_gemm_tiled(fake, fake, fake, null, null, null, fake, fake, 1 << 40, 2000, 9216, 9216, 3, -1,
+                                              ctypes.byref(q), null) == _lib.ERR_BAD_ARG
