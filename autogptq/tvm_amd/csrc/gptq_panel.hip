@@ -557,10 +557,21 @@ __global__ __launch_bounds__(256) void panel_gather_kernel(const _Float16 *__res
     const int row0 = blockIdx.x * ROWS, rows = min(ROWS, M - row0);
     _Float16 *xl = (_Float16 *)smem;
     const u4 *src = (const u4 *)(x + (size_t)row0 * K);
-    for (int i = threadIdx.x; i < rows * (K / 8); i += 256) ((u4 *)xl)[i] = src[i];
+    // the first index vectors, and four requests of x at a time: one after the other they are a chain of latencies
+    const int o0 = blockIdx.y * 256 + threadIdx.x, oc = min(o0, K / 8 - 1), all = rows * (K / 8);
+    int4 u = *(const int4 *)(xsrc + 8 * oc), v = *(const int4 *)(xsrc + 8 * oc + 4);
+    for (int i = threadIdx.x; i < all; i += 1024) {
+        u4 q[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (i + 256 * j < all) q[j] = src[i + 256 * j];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (i + 256 * j < all) ((u4 *)xl)[i + 256 * j] = q[j];
+    }
     __syncthreads();
-    for (int o = blockIdx.y * 256 + threadIdx.x; o < K / 8; o += 256 * gridDim.y) {
-        const int4 u = *(const int4 *)(xsrc + 8 * o), v = *(const int4 *)(xsrc + 8 * o + 4);
+    for (int o = o0; o < K / 8; o += 256 * gridDim.y) {
+        if (o > o0) u = *(const int4 *)(xsrc + 8 * o), v = *(const int4 *)(xsrc + 8 * o + 4);
         int idx[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int e = 0; e < 8; e++) idx[e] = min(max(idx[e], 0), K - 1);   // a bad map must not fault

@@ -573,10 +573,12 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
     }
 }
 
-// y = fp16(sum over split of partial[split] (+ bias)), four columns per thread, in split order.
+// y = fp16(sum over split of partial[split] (+ bias)), four columns per thread, in split order.  S: the ranges, all requested together
+// (0: any number, one after the other; 150 rows of 18944 x 2048 int3 in six ranges 38.5 -> 36.8 us a call, 64 of 16384 x 4096 21.9 -> 21.2).
+template <int S>
 __global__ __launch_bounds__(256) void tiled_reduce_kernel(const float *__restrict__ partial, const _Float16 *bias,
                                                            _Float16 *__restrict__ y, int M, int N, int split_k,
-                                                           const int32_t *__restrict__ out_map = nullptr)
+                                                           const int32_t *__restrict__ out_map)
 {
     const uint32_t q = blockIdx.x * 256u + threadIdx.x;
     const uint32_t nq = (uint32_t)N / 4u;
@@ -588,7 +590,17 @@ __global__ __launch_bounds__(256) void tiled_reduce_kernel(const float *__restri
         const h4 b4 = *(const h4 *)(bias + c);
         sum = (f4){(float)b4[0], (float)b4[1], (float)b4[2], (float)b4[3]};
     }
-    for (int s = 0; s < split_k; s++) sum += *(const f4 *)(partial + ((size_t)s * M + row) * N + c);
+    const float *src = partial + (size_t)row * N + c;
+    const size_t range = (size_t)M * N;
+    if constexpr (S > 0) {
+        f4 part[S];
+#pragma unroll
+        for (int s = 0; s < S; s++) part[s] = *(const f4 *)(src + s * range);
+#pragma unroll
+        for (int s = 0; s < S; s++) sum += part[s];
+    } else {
+        for (int s = 0; s < split_k; s++) sum += *(const f4 *)(src + s * range);
+    }
     if (out_map) {   // the transposed product: column c is a sorted position, its channel is out_map[c]
         const int4 dst = *(const int4 *)(out_map + c);
         const int d[4] = {dst.x, dst.y, dst.z, dst.w};
@@ -606,8 +618,20 @@ int launch_tiled_reduce(const float *partial, const void *bias, void *y, int M, 
                         hipStream_t stream)
 {
     const uint32_t quads = (uint32_t)M * ((uint32_t)N / 4u);
-    hipLaunchKernelGGL(tiled_reduce_kernel, dim3((quads + 255u) / 256u), dim3(256), 0, stream, partial,
-                       (const _Float16 *)bias, (_Float16 *)y, M, N, split_k, out_map);
+    auto go = [&](auto ranges) {
+        hipLaunchKernelGGL(tiled_reduce_kernel<decltype(ranges)::value>, dim3((quads + 255u) / 256u), dim3(256), 0, stream, partial,
+                           (const _Float16 *)bias, (_Float16 *)y, M, N, split_k, out_map);
+    };
+    switch (split_k) {
+        case 2: go(std::integral_constant<int, 2>{}); break;
+        case 3: go(std::integral_constant<int, 3>{}); break;
+        case 4: go(std::integral_constant<int, 4>{}); break;
+        case 5: go(std::integral_constant<int, 5>{}); break;
+        case 6: go(std::integral_constant<int, 6>{}); break;
+        case 7: go(std::integral_constant<int, 7>{}); break;
+        case 8: go(std::integral_constant<int, 8>{}); break;
+        default: go(std::integral_constant<int, 0>{});
+    }
     return hipGetLastError() == hipSuccess ? GPTQ_HIP_OK : GPTQ_HIP_ERR_LAUNCH;
 }
 
@@ -723,10 +747,7 @@ int launch_tiled(const void *x, const void *qtile, const uint32_t *sz, const int
     }
     if (rc != GPTQ_HIP_OK) return rc;
     if (plan.split_k > 1) {
-        const uint32_t quads = (uint32_t)M * ((uint32_t)N / 4u);
-        hipLaunchKernelGGL(tiled_reduce_kernel, dim3((quads + 255u) / 256u), dim3(256), 0, stream, partial,
-                           (const _Float16 *)bias, (_Float16 *)y, M, N, plan.split_k);
-        if (hipGetLastError() != hipSuccess) return GPTQ_HIP_ERR_LAUNCH;
+        return launch_tiled_reduce(partial, bias, y, M, N, plan.split_k, nullptr, stream);
     }
     return GPTQ_HIP_OK;
 }
@@ -896,10 +917,7 @@ int launch_tiled_t(const void *gy, const void *qtile_t, const uint32_t *szt, con
 #undef GPTQ_TILED_T_CASE
     if (rc != GPTQ_HIP_OK) return rc;
     if (plan.split_k > 1) {
-        const uint32_t quads = (uint32_t)M * ((uint32_t)K / 4u);
-        hipLaunchKernelGGL(tiled_reduce_kernel, dim3((quads + 255u) / 256u), dim3(256), 0, stream, partial,
-                           (const _Float16 *)nullptr, (_Float16 *)gx, M, K, plan.split_k, xsrc);
-        if (hipGetLastError() != hipSuccess) return GPTQ_HIP_ERR_LAUNCH;
+        return launch_tiled_reduce(partial, nullptr, gx, M, K, plan.split_k, xsrc, stream);
     }
     return GPTQ_HIP_OK;
 }

@@ -771,3 +771,18 @@ def test_tiled_decode_long_narrow_layers(dev, bits, K, N, gs, desc_act):
         y = run_tiled(D, prep, plan=plan)
         assert_tight(y, expected_output(L), f"int{bits} {K}x{N} M={M}")
         assert torch.equal(y, run_tiled(D, prep, plan=plan)), "two identical calls differ"
+
+
+@pytest.mark.parametrize("split", [2, 3, 4, 5, 6, 7, 8, 9])
+def test_tiled_reduce_every_count_of_ranges(dev, split):
+    """The pass that adds K ranges up asks for two to eight of them together and walks more: every count, the last one short."""
+    M, K, N, gs = 37, 64 * 4 * 9 - 32, 96, 32
+    L = layer(5200 + split, K, N, 4, gs, True, M=M, bias=True)
+    D = to_dev(L, dev)
+    plan = _lib.select_tiled(M, K, N, 4, gs)
+    plan.k_chunk = -(-36 // (plan.waves_k * split))
+    plan.split_k = plan.grid_y = split
+    part = (split * M * N * 4 + 255) // 256 * 256
+    plan.workspace_bytes = 16384 + part + split * plan.waves_k * plan.k_chunk * 4 * plan.row_tiles * plan.m_blocks * 1024
+    y = run_tiled(D, prepare(D), plan=plan)
+    assert_tight(y, expected_output(L), f"{split} ranges")
