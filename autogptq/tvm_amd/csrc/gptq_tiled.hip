@@ -162,8 +162,11 @@ int launch_tile_prepare(const uint32_t *qweight, const uint32_t *qzeros, const v
 // 64 lanes x 16 bytes; lane (m = lane % 32, h = lane / 32) holds x[32 rt + m][xsrc[64 S + 32 h + 8 j + e]],
 // e = 0..7.  Rows past M and positions past K are zeros; blocks up to S_pack are written (the kernel's
 // waves walk whole ranges, and their refills run a ring past the end).
-// One workgroup per row: the row goes to LDS with coalesced loads and the gather through xsrc reads LDS
-// (lanes that gather from global memory with one row per lane touch 64 cache lines per instruction).
+// One workgroup per row, or several (grid_y) with a part of the octets each while the rows are few: the row goes to LDS with
+// coalesced loads and the gather through xsrc reads LDS (lanes that gather from global memory with one row per lane touch 64
+// cache lines per instruction).  What bounds it is latency: a thread has two octets at most where a part of the row per workgroup
+// allows that, and asks for four vectors of x at a time (us a call, a workgroup per row / this: 16 rows of 11008 x 4096 17.4 / 15.1, 48 of
+// 12288 x 5120 int3 22.7 / 20.3, 32 and 128 of 4096 x 11008 13.3 / 13.0 and 25.3 / 25.0).
 // ---------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void tile_pack_x_kernel(const _Float16 *__restrict__ x, const int32_t *__restrict__ xsrc,
                                                           char *__restrict__ xpack, int M, int K, int Kp, int rt_total,
@@ -176,18 +179,30 @@ __global__ __launch_bounds__(256) void tile_pack_x_kernel(const _Float16 *__rest
     const bool live = row < M;
     const _Float16 *xr = x + (size_t)row * K;
     const int octets = S_pack * 8;
+    const int o0 = blockIdx.y * 256 + tid, step = 256 * gridDim.y;
     int4 ia[2], ib[2];  // the map entries of this thread's first two octets, requested before the row is staged
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-        const int p0 = min(8 * (tid + 256 * i), Kp - 8);
+        const int p0 = min(8 * (o0 + step * i), Kp - 8);
         ia[i] = xsrc ? *(const int4 *)(xsrc + p0) : make_int4(0, 0, 0, 0);
         ib[i] = xsrc ? *(const int4 *)(xsrc + p0 + 4) : make_int4(0, 0, 0, 0);
     }
     if (live && xsrc) {
-        for (int i = tid; i < K / 8; i += 256) ((u4 *)xl)[i] = ((const u4 *)xr)[i];
+        if (K <= 4096)   // (one or two vectors per thread: short rows lose 0.1 to 0.2 us on the tests below)
+            for (int i = tid; i < K / 8; i += 256) ((u4 *)xl)[i] = ((const u4 *)xr)[i];
+        else
+        for (int i = tid; i < K / 8; i += 1024) {
+            u4 q[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (i + 256 * j < K / 8) q[j] = ((const u4 *)xr)[i + 256 * j];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (i + 256 * j < K / 8) ((u4 *)xl)[i + 256 * j] = q[j];
+        }
     }
     __syncthreads();
-    for (int o = tid, it = 0; o < octets; o += 256, it++) {
+    for (int o = o0, it = 0; o < octets; o += step, it++) {
         const int p0 = 8 * o;
         const int S = p0 >> 6, h = (p0 >> 5) & 1, j = (p0 >> 3) & 3;
         h8 v = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -213,6 +228,13 @@ __global__ __launch_bounds__(256) void tile_pack_x_kernel(const _Float16 *__rest
         }
         *(h8 *)(xpack + ((size_t)(4 * S + j) * rt_total + rt) * 1024 + (h * 32 + m) * 16) = v;
     }
+}
+
+// workgroups per row of the pack pass: an octet per thread while that is at most two workgroups per CU
+static int pack_parts(int rows, int S_pack)
+{
+    const int most = (S_pack * 8 + 255) / 256, room = 2 * kNumCUs / rows;
+    return room < 2 ? 1 : (room < most ? room : most);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -704,7 +726,7 @@ int launch_tiled(const void *x, const void *qtile, const uint32_t *sz, const int
                 return GPTQ_HIP_ERR_LAUNCH;
             }
         }
-        hipLaunchKernelGGL(tile_pack_x_kernel, dim3(32 * p.rt_total), dim3(256), pack_lds, stream, (const _Float16 *)x,
+        hipLaunchKernelGGL(tile_pack_x_kernel, dim3(32 * p.rt_total, pack_parts(32 * p.rt_total, S_pack)), dim3(256), pack_lds, stream, (const _Float16 *)x,
                            xsrc, xpack, M, K, Kp, p.rt_total, S_pack);
         if (hipGetLastError() != hipSuccess) return GPTQ_HIP_ERR_LAUNCH;
     }
@@ -896,7 +918,7 @@ int launch_tiled_t(const void *gy, const void *qtile_t, const uint32_t *szt, con
     p.x = nullptr;           // (the forward product's direct read of x: not used here)
     p.K = K;
     const int S_pack = tiled_pack_blocks(plan.split_k, plan.waves_k, plan.k_chunk);
-    hipLaunchKernelGGL(tile_pack_x_kernel, dim3(32 * p.rt_total), dim3(256), 0, stream, (const _Float16 *)gy,
+    hipLaunchKernelGGL(tile_pack_x_kernel, dim3(32 * p.rt_total, pack_parts(32 * p.rt_total, S_pack)), dim3(256), 0, stream, (const _Float16 *)gy,
                        (const int32_t *)nullptr, xpack, M, N, Np, p.rt_total, S_pack);
     if (hipGetLastError() != hipSuccess) return GPTQ_HIP_ERR_LAUNCH;
     int rc = GPTQ_HIP_ERR_UNSUPPORTED;

@@ -786,3 +786,14 @@ def test_tiled_reduce_every_count_of_ranges(dev, split):
     plan.workspace_bytes = 16384 + part + split * plan.waves_k * plan.k_chunk * 4 * plan.row_tiles * plan.m_blocks * 1024
     y = run_tiled(D, prepare(D), plan=plan)
     assert_tight(y, expected_output(L), f"{split} ranges")
+
+
+@pytest.mark.parametrize("K", [32, 2048, 2080, 4096, 4128, 8192, 12320])
+@pytest.mark.parametrize("M,desc_act", [(9, True), (33, False), (70, True)])
+def test_tiled_pack_pass_in_parts_of_a_row(dev, K, M, desc_act):
+    """The pass that writes x's fragments takes a row in one to eight parts: a part's last octets, the padding behind K, short last rows."""
+    L = layer(5300 + K + M, K, 64, 4, 32, desc_act, M=M, bias=True)
+    D = to_dev(L, dev)
+    plan = _lib.select_tiled(M, K, 64, 4, 32)
+    assert plan.kernel == _lib.KERNEL_TILED
+    assert_tight(run_tiled(D, prepare(D), plan=plan), expected_output(L), f"K={K} M={M} act={desc_act}")
