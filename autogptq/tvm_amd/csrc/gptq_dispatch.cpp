@@ -597,9 +597,9 @@ extern "C" int gptq_hip_select_tiled(int M, int K, int N, int bits, int group_si
 {
     // Up to four rows the decode kernels (one 4-row matrix instruction set per lane block); five to eight rows the
     // workgroup-per-tile decode kernel with two sets, for K up to 11008 (us at 5 / 8 rows, int4, against the matmul
-    // kernel with one 32-row tile: 4096 x 11008 9.0 / 9.4 against 9.6 / 9.7, with an activation order 12.7 / 13.2
-    // against 14.0 / 14.2; 11008 x 4096 9.9 / 10.3 against 16.7 / 17.2, with an activation order 15.1 / 15.8 against
-    // 18.9 / 19.4; 4096 x 4096 7.2 / 7.8 against 9.4 / 9.5), and beyond for narrow layers (decode_takes).
+    // kernel with one 32-row tile: 4096 x 11008 7.4 / 7.4 against 9.6 / 9.7, with an activation order 7.9 / 7.8
+    // against 14.0 / 14.2; 11008 x 4096 7.8 / 7.9 against 16.7 / 17.2, with an activation order 9.6 / 9.9 against
+    // 18.9 / 19.4; 4096 x 4096 4.7 / 4.8 against 9.4 / 9.5), and beyond for narrow layers (decode_takes).
     if (M >= 1 && (M <= gptq::kDecodeSelectRows || (M <= gptq::kDecodeMaxRows && decode_takes(K, N)))) {
         const int rc = gptq_hip_select_tiled_decode(M, K, N, bits, group_size, plan);
         if (rc != GPTQ_HIP_ERR_UNSUPPORTED || !plan) return rc;
@@ -729,7 +729,8 @@ namespace {
 // 4000 measurements (3 to 8 sizes of M each on sixteen layers of 1024 to 32768 columns, both products, all widths, one to eight
 // row tiles, one to eight K ranges): 8 % rms, and the plan it names best is 1 % slower than the fastest one on average.  What
 // a step costs besides its matrix instructions (the constant of the first line) is the dequantisation, which every workgroup
-// does for its columns; a turn that is not full runs at a higher clock.
+// does for its columns; a turn that is not full runs at a higher clock.  On 1900 calls drawn since, with the plans of whole turns
+// and K ranges among the choices, the plan named is 1.8 % (forward) and 2.4 % (gradient) slower than the fastest one on the mean.
 double panel_us(int rt, int split, int chunk, long long wgs, int bits, double out_elems)
 {
     const double step = (rt <= 4 ? 0.295 + 0.100 * rt : 0.281 + 0.131 * rt) + (bits == 8 ? 0.01 : (bits == 3 ? 0.07 : 0.0));
@@ -874,8 +875,8 @@ namespace {
 
 // Where the tiled kernels were measured faster than the ones that read the checkpoint layout or its channel-sorted
 // copy, on MI355X with the weights cold (us per call, graph replay, group size 128 unless said):
-//   * up to 4 rows, layers of up to 4096 columns (decode kernel with a workgroup per 16 columns, or every tile in two
-//     halves along K from 4096 channels): always.  4096 x 4096: 4.1-4.2 at one row, 5.2 at four, against 6.8-7.5
+//   * up to 4 rows, layers of up to 4096 columns (decode kernel with a workgroup per tile, per half of one along K from 4096
+//     channels, or per 16 columns): always.  4096 x 4096: 4.1-4.2 at one row, 5.2 at four, against 6.8-7.5
 //     and 7.8-10.5; 11008 x 4096: int4 9.0-9.4 / 11.5 against 13.5 / 15.3, int3 8.7 / 11.1 against 10.9 / 15.2;
 //   * up to 4 rows, wider layers (a workgroup per 32 columns): K = 4096: one and two rows always, three and four up
 //     to 16384 columns (4096 x 11008 with an activation order, one / two / four rows: int4 7.8 / 8.1 / 9.8 against
@@ -886,10 +887,10 @@ namespace {
 //     up to 11008 for layers of up to 8192 columns (beyond, the four staged rows of x cost more than they save:
 //     8192 x 28672 41.9 against 30.4);
 //   * 5 to 8 rows, K up to 11008: the decode kernel with two sets of four rows (5 / 8 rows, int4 / int3, against the
-//     better of the other copies: 4096 x 11008 with an activation order 12.7 / 13.2 and 12.8 / 13.3 against 13.4 / 13.6
-//     and 12.5 / 12.6 on the sorted copy, without one 9.0 / 9.4 against 9.6 / 9.7 on the matmul kernel; 11008 x 4096 with
-//     an activation order 15.1 / 15.8 and 15.3 / 16.1 against 15.8 / 16.0 and 16.4 / 16.9, without one 9.9 / 10.3 against
-//     13.1; 4096 x 4096 7.2 / 7.8 against 9.9, with an activation order 9.5 / 10.2 against 10.9 (int3 12.3));
+//     better of the other copies: 4096 x 11008 with an activation order 7.9 / 7.8 and 7.9 / 8.2 against 13.4 / 13.6
+//     and 12.5 / 12.6 on the sorted copy, without one 7.4 / 7.4 against 9.6 / 9.7 on the matmul kernel; 11008 x 4096 with
+//     an activation order 9.6 / 9.9 and 9.1 / 9.6 against 15.8 / 16.0 and 16.4 / 16.9, without one 7.8 / 7.9 against
+//     13.1; 4096 x 4096 4.7 / 4.8 against 9.9, with an activation order 5.5 / 5.4 against 10.9 (int3 12.3));
 //   * 5 to 16 rows otherwise: only layers without an activation order, K up to 4096 and more than 4096 columns (the matmul
 //     kernel then reads x itself, one launch: 4096 x 11008 int4, 5 / 8 / 16 rows: 10.6 / 10.7 / 11.5 against 11.2 /
 //     11.3 / 12.5; int3 from nine rows); with an activation order the pack pass makes it 14.6 against 13.4 at 8 rows;
@@ -947,6 +948,19 @@ bool tiled_wins(int M, int K, int N, bool act_order, int bits, bool one_group)
     // the longer layers are level or behind: 28672 x 8192 167 / 169 against 164 / 169, 13824 x 5120 at 192 rows 54.7
     // against 46.3)
     return K <= 8192 || (M <= 256 && (K <= 11008 || act_order || (one_group && N <= 16384)));
+}
+
+// Three and four rows of layers past that table that would run on GROUPED, since the decode kernel takes the zero point off the codes
+// and stages an activation order in whole positions (us, against GROUPED on the better of the other copies: 8192 x 28672 int4 25.4 /
+// 24.1 with / without an order against 30.1 / 27.7, int3 21.8 / 20.2 against 33.3 / 30.9; 11008 x 11008 int3 16.2 / 13.8 against 25.6 / 23.0;
+// 4096 x 22016 8.6-10.5 against 13.6-15.9; 2048 x 33632 int3 7.7 against 14.6; 1792 x 19968 6.0 against 12.5; 2816 x 32608 11.7 against 23.0).  Both scale the
+// exact products of the codes group by group.  Layers whose small groups or length put them on STREAM stay there, though they would gain as
+// much (13824 x 5120 11 against 17): it multiplies the weights as the reference rounds them, and the two differ by that rounding, 1.7e-4.
+bool decode_wins_past_table(int M, int K, int N, int bits, int group_size)
+{
+    gptq_hip_plan other;
+    return (M == 3 || M == 4) && K <= 19712 && gptq_hip_select(M, K, N, bits, group_size, 0, &other) == GPTQ_HIP_OK &&
+           other.kernel == GPTQ_HIP_KERNEL_GROUPED;
 }
 
 // The plan gptq_hip_gemm_sorted runs for M rows of a layer whose channels were sorted by group, if that path covers
@@ -1019,8 +1033,8 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
     if (!fused_bits) {
         if (!tiled_ok) return GPTQ_HIP_OK;   // 2 and 8 bits have no other fused kernels: the library
         tiled = true;
-    } else if (tiled_ok && tiled_wins(M, K, N, act, bits, one_group)) {
-        tiled = true;
+    } else if (tiled_ok && (tiled_wins(M, K, N, act, bits, one_group) || (panels && decode_wins_past_table(M, K, N, bits, group_size)))) {
+        tiled = true;   // (the rows past the table like the panel kernel: for hosts that set the bit)
     }
     int which = 0;
     if (sw[0] && !tiled) {   // off the tiled copy the library GEMM wins earlier
@@ -1038,9 +1052,10 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
     const bool theirs = !tiled && M <= 16 && fused_bits && (copies & (GPTQ_HIP_COPY_CHECKPOINT | GPTQ_HIP_COPY_SORTED));
     const bool others = theirs && !(act && bits == 4);
     // Row blocks are ahead of the kernels on every copy (16 rows of 4096 x 4096 int4 with an activation order 6.0 us, 10.7 on the
-    // checkpoint tensors; without one 6.1 and 9.3); beyond 4096 channels they leave a layer that has other copies to those
-    // (8192 x 4096: 9.8 us against 11.5 to 12.5, for a copy more), and below 1024 columns, where a call costs its host time.
-    if (!past && (!theirs || (K <= 4096 && N >= 1024)) && take_rows()) return GPTQ_HIP_OK;
+    // checkpoint tensors; without one 6.1 and 9.3; 4352 x 1408 int3 7.1 and 12.8, 6656 x 4096 int3 9.0 and 12.9, 7680 x 1536 int3 one group 9.6
+    // and 12.5); from 8192 channels they leave a layer that has other copies to those (8192 x 4096: 9.8 us against 11.5 to 12.5, for a
+    // copy more), and below 1024 columns, where a call costs its host time.
+    if (!past && (!theirs || (K < 8192 && N >= 1024)) && take_rows()) return GPTQ_HIP_OK;
     if (!others && take_panel()) return GPTQ_HIP_OK;
     if (past) return GPTQ_HIP_OK;
     if (tiled && take_tiled()) return GPTQ_HIP_OK;

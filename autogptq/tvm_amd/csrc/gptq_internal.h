@@ -250,7 +250,8 @@ inline bool tiled_decode_can_halve(int wave_steps, int split_k, int waves_k, int
 // 4.13 / 5.58 / 7.10; 4096 x 1024 3.48 / 4.70 / 6.23 against 4.04 / 5.49 / 7.06; 6144 x 4096 4.79 / 6.04 / 7.87 against 5.45 /
 // 7.21 / 8.52; 11008 x 4096 int3 8.4 / 11.2 against 9.6 / 13.6 at one / four rows.  At 2048 channels the halves are four
 // blocks per wave: 2048 x 4096 3.93 / 5.17 / 6.31 against 3.98 / 5.33 / 5.72, 2048 x 2048 3.78 / 5.03 / 6.25 against
-// 3.79 / 5.19 / 5.66: level up to four rows, a loss at eight, so shorter layers stay with the 16-column kernel).
+// 3.79 / 5.19 / 5.66: level up to four rows, a loss at eight, so shorter layers keep whole tiles of eight waves, one and two
+// rows of more than 2560 channels the 16-column kernel).
 inline bool tiled_decode_halves_all(int tiles, int S_total) { return 2 * tiles <= kNumCUs && S_total >= 64; }
 inline int tiled_decode_halved(int tiles, int wave_steps, int split_k, int waves_k, int S_total, int group_size)
 {

@@ -413,6 +413,7 @@ int launch_tiled_decode16(const void *x, const void *qtile, const uint32_t *sz, 
     int rc = GPTQ_HIP_ERR_UNSUPPORTED;
     // contiguous ranges per wave when a wave has more than two items (a long K, or several units per workgroup)
     const bool contig = (long long)((p.units + plan.grid_x - 1) / plan.grid_x) * p.V_total > 32;
+    // (four rows: plans of callers that kept them; the planner names this kernel for one and two)
 #define GPTQ_DECODE16_CASE(B, R)                                                                              \
     if (bits == B && mr == R)                                                                                 \
         rc = g128 ? (contig ? launch_decode16_one<B, R, true, true>(p, plan, stream)                          \

@@ -57,8 +57,8 @@ enum {
                                    waves along K with k_chunk blocks of 64 channels each; split_k > 1 (an x that
                                    does not fit LDS) adds a reduce launch.  waves_n = 2: units of 16 columns dealt
                                    out evenly over grid_x workgroups of 16 waves, all of K staged per workgroup
-                                   (k_chunk = blocks of 128 channels per unit and wave); chosen for layers of up to
-                                   4096 columns and fewer than 4096 channels */
+                                   (k_chunk = blocks of 128 channels per unit and wave); chosen for one and two
+                                   rows of layers of up to 4096 columns and more than 2560, fewer than 4096 channels */
     GPTQ_HIP_KERNEL_PANEL = 6 /* the same layer for long prompts and training batches: a workgroup takes 32 * row_tiles
                                    (1..8) rows, shared in LDS, x 256 columns (waves_n = 4 waves of 64 each), k_chunk blocks of
                                    64 channels; up to four row tiles two such groups of waves (waves_k = 2) take every

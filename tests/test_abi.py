@@ -548,6 +548,22 @@ def test_row_blocks_stay_within_one_turn_and_lds(M, K, N, mr):
                              (9, 9, 9)).copy == _lib.ROUTE_LIBRARY
 
 
+def test_three_and_four_rows_past_the_table_run_on_the_decode_kernel_where_it_is_ahead():
+    """With the bit that offers the newer plans; hosts that do not set it get the answers they got, and layers on STREAM stay there."""
+    old = _lib.COPY_CHECKPOINT | _lib.COPY_SORTED | _lib.COPY_TILED
+    for K, N, bits, gs, ahead in ((8192, 28672, 4, 128, True), (4096, 16384, 4, 128, True), (2048, 33632, 3, 64, True), (11008, 11008, 3, 128, True),
+                                  (11008, 11008, 4, 128, False), (8192, 28672, 4, 32, False), (28672, 8192, 4, 128, False)):
+        for M, act in ((3, False), (3, True), (4, False), (4, True)):
+            r, before = _lib.select_route(M, K, N, bits, gs, act, old | _lib.COPY_TILED_PANEL), _lib.select_route(M, K, N, bits, gs, act, old)
+            assert before.copy != _lib.ROUTE_TILED and (before.plan.kernel == _lib.KERNEL_GROUPED) == ahead
+            if ahead:
+                assert r.copy == _lib.ROUTE_TILED and r.plan.as_dict() == _lib.select_tiled(M, K, N, bits, gs).as_dict()
+            else:
+                assert (r.copy, r.plan.as_dict()) == (before.copy, before.plan.as_dict())
+    r = _lib.select_route(12, 7680, 1536, 3, -1, False, old | _lib.COPY_TILED_PANEL)   # (row blocks below 8192 channels)
+    assert r.copy == _lib.ROUTE_TILED and r.plan.row_tiles == 8
+
+
 def test_a_tiled_call_without_plan_and_workspace_stays_refused():
     # (row blocks need none, but the sizes they take were always asked for one; checked before anything is launched)
     fake, null = ctypes.c_void_p(0x1000), ctypes.c_void_p(None)
