@@ -352,16 +352,11 @@ extern "C" int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint3
     if (!gptq::tiled_qualifies(K, N, bits, gs)) return GPTQ_HIP_ERR_UNSUPPORTED;
     if ((long long)((K + 63) / 64 * 64) * N * bits / 8 >= (1LL << 32)) return GPTQ_HIP_ERR_UNSUPPORTED;
     gptq_hip_plan chosen;
+    int clear = 0;   // the slots of halved tiles
     if (!plan) {
-        int rc = gptq_hip_select_panel(M, K, N, bits, group_size, xsrc ? GPTQ_HIP_PANEL_ACT_ORDER : 0, 0, 0, &chosen);
-        if (rc != GPTQ_HIP_OK || chosen.workspace_bytes > (workspace ? workspace_bytes : 0))
-            rc = gptq_hip_select_tiled(M, K, N, bits, group_size, &chosen);
+        const int rc = gptq::gptq_tiled_default_plan(M, K, N, bits, group_size, xsrc != nullptr,
+                                                     workspace && aligned(workspace, 16) ? workspace_bytes : 0, &chosen, &clear);
         if (rc != GPTQ_HIP_OK) return rc;
-        // row blocks need no workspace, but a call without the one that its size asks for stays refused
-        gptq_hip_plan blocks;
-        if (chosen.workspace_bytes <= (workspace && aligned(workspace, 16) ? workspace_bytes : 0) &&
-            gptq::select_row_blocks(M, K, N, bits, group_size, &blocks))
-            chosen = blocks;
         plan = &chosen;
     }
     if (plan->kernel == GPTQ_HIP_KERNEL_TILED_DECODE && plan->waves_n == 2) {
@@ -414,9 +409,13 @@ extern "C" int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint3
         }
         unsigned long long *slots = nullptr;
         if (halved > 0) {
-            const size_t need = gptq::kCounterBytes + gptq::tiled_decode_slot_bytes(halved, mr);
-            if (!workspace || !aligned(workspace, 16) || workspace_bytes < need) return GPTQ_HIP_ERR_WORKSPACE;
+            const size_t bytes = gptq::tiled_decode_slot_bytes(halved, mr);
+            if (!workspace || !aligned(workspace, 16) || workspace_bytes < gptq::kCounterBytes + bytes) return GPTQ_HIP_ERR_WORKSPACE;
             slots = (unsigned long long *)((char *)workspace + gptq::kCounterBytes);
+            if (clear) {
+                const int rc = gptq::launch_fill_zero(slots, bytes, stream);
+                if (rc != GPTQ_HIP_OK) return rc;
+            }
         }
         return gptq::launch_tiled_decode(x, qtile, sz, kinv, bias, y, part, slots, M, K, N, G_all, bits, gs, *plan, stream);
     }

@@ -389,7 +389,9 @@ static int tiled_args_ok(int M, int K, int N, int bits, int group_size, gptq_hip
     return GPTQ_HIP_OK;
 }
 
-extern "C" int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
+// settled: within the bounds that tell which kind of workspace a call without a plan asks for (gptq_tiled_default_plan): 128 KB of LDS,
+// sums of x counted in for every number of rows.
+static int plan_tiled_decode(int M, int K, int N, int bits, int group_size, bool settled, gptq_hip_plan *plan)
 {
     const int ok = tiled_args_ok(M, K, N, bits, group_size, plan);
     if (ok != GPTQ_HIP_OK) return ok;
@@ -476,7 +478,9 @@ extern "C" int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int g
             const int lds = gptq::tiled_decode_lds_bytes(mr, span, groups, kw);
             // (all of the LDS where every workgroup has a CU to itself anyway: an uncut K saves the reduce pass, 8192 x 8192 at
             // eight rows 13.1 -> 9.8 us, with an activation order 13.9 -> 10.4, 16384 x 8192 at four rows 19.6 -> 15.9)
-            if (lds > ((tiles + halved) * split <= gptq::kNumCUs ? 160 : 128) * 1024) continue;
+            if (settled ? lds + (gptq::tiled_decode_centred(mr) ? (span / 32) * mr * 8 : 0) > 128 * 1024
+                        : lds > ((tiles + halved) * split <= gptq::kNumCUs ? 160 : 128) * 1024)
+                continue;
             if (split > 1 && (long long)M * N >= (1LL << 32)) return GPTQ_HIP_ERR_UNSUPPORTED;
             plan->kernel = GPTQ_HIP_KERNEL_TILED_DECODE;
             plan->row_tiles = mr;
@@ -501,6 +505,11 @@ extern "C" int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int g
         }
         return GPTQ_HIP_ERR_UNSUPPORTED;
     }
+}
+
+extern "C" int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
+{
+    return plan_tiled_decode(M, K, N, bits, group_size, false, plan);
 }
 
 namespace {
@@ -593,15 +602,15 @@ bool gptq::select_row_blocks(int M, int K, int N, int bits, int group_size, gptq
 // 18.0 and 16384 x 8192 21.6 / 23.8 stay).
 static bool decode_takes(int K, int N) { return K <= 11008 || (K <= 18432 && N <= 4096) || (K <= 20480 && N <= 2048); }
 
-extern "C" int gptq_hip_select_tiled(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
+static int plan_tiled(int M, int K, int N, int bits, int group_size, bool settled, gptq_hip_plan *plan)
 {
     // Up to four rows the decode kernels (one 4-row matrix instruction set per lane block); five to eight rows the
     // workgroup-per-tile decode kernel with two sets, for K up to 11008 (us at 5 / 8 rows, int4, against the matmul
     // kernel with one 32-row tile: 4096 x 11008 7.4 / 7.4 against 9.6 / 9.7, with an activation order 7.9 / 7.8
     // against 14.0 / 14.2; 11008 x 4096 7.8 / 7.9 against 16.7 / 17.2, with an activation order 9.6 / 9.9 against
     // 18.9 / 19.4; 4096 x 4096 4.7 / 4.8 against 9.4 / 9.5), and beyond for narrow layers (decode_takes).
-    if (M >= 1 && (M <= gptq::kDecodeSelectRows || (M <= gptq::kDecodeMaxRows && decode_takes(K, N)))) {
-        const int rc = gptq_hip_select_tiled_decode(M, K, N, bits, group_size, plan);
+    if (M >= 1 && (M <= gptq::kDecodeSelectRows || (M <= gptq::kDecodeMaxRows && (settled ? K <= 11008 : decode_takes(K, N))))) {
+        const int rc = plan_tiled_decode(M, K, N, bits, group_size, settled, plan);
         if (rc != GPTQ_HIP_ERR_UNSUPPORTED || !plan) return rc;
     }
     const int ok = tiled_args_ok(M, K, N, bits, group_size, plan);
@@ -668,6 +677,34 @@ extern "C" int gptq_hip_select_tiled(int M, int K, int N, int bits, int group_si
     ws += (size_t)gptq::tiled_pack_blocks(split, kwv, wave_steps) * 4 * (size_t)(at * rw * m_blocks) * 1024;
     plan->workspace_bytes = ws;
     return GPTQ_HIP_OK;
+}
+
+extern "C" int gptq_hip_select_tiled(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
+{
+    return plan_tiled(M, K, N, bits, group_size, false, plan);
+}
+
+// The plan of a gptq_hip_gemm_tiled call that names none and brings `have` bytes of workspace.  Most plans want zeros in the first 16 KB of
+// theirs only; halved tiles want all of it zero and for themselves, and in a workspace that something else has written they add
+// what they find there to the result.  A caller that names no plan has not read that, so a size whose plan was not of that kind
+// (five to eight rows beyond 11008 channels, three and four of long layers: the settled bounds) does not ask for it: *clear says that
+// the call clears the slots itself, with one launch more.
+extern "C" int gptq::gptq_tiled_default_plan(int M, int K, int N, int bits, int group_size, int act_order, size_t have, gptq_hip_plan *plan,
+                                             int *clear)
+{
+    *clear = 0;
+    int rc = gptq_hip_select_panel(M, K, N, bits, group_size, act_order ? GPTQ_HIP_PANEL_ACT_ORDER : 0, 0, 0, plan);
+    if (rc != GPTQ_HIP_OK || plan->workspace_bytes > have) rc = gptq_hip_select_tiled(M, K, N, bits, group_size, plan);
+    if (rc != GPTQ_HIP_OK) return rc;
+    // row blocks need no workspace, but a call without the one that its size asks for stays refused
+    gptq_hip_plan other;
+    if (plan->workspace_bytes <= have && select_row_blocks(M, K, N, bits, group_size, &other)) *plan = other;
+    if (plan->kernel == GPTQ_HIP_KERNEL_TILED_DECODE && (plan->flags & GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE) &&
+        plan_tiled(M, K, N, bits, group_size, true, &other) == GPTQ_HIP_OK && !(other.flags & GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE)) {
+        *clear = plan->workspace_bytes <= have;
+        if (!*clear) *plan = other;   // (three rows in two K ranges: 12 bytes a column, the slots take 32)
+    }
+    return rc;
 }
 
 // The transposed product gx[M, K] = gy[M, N] @ W^T on the matmul kernel: the reduction runs over the layer's N

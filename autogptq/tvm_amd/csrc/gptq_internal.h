@@ -214,6 +214,9 @@ inline long long tiled_decode16_lds_bytes(int mr, int K, int groups, int units_p
 }
 // the plan in row blocks, where it is the faster one (gptq_dispatch.cpp)
 bool select_row_blocks(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan);
+// the plan of a gptq_hip_gemm_tiled call that names none, and whether the call clears the slots of its halved tiles (the tests ask, too)
+extern "C" int gptq_tiled_default_plan(int M, int K, int N, int bits, int group_size, int act_order, size_t have, gptq_hip_plan *plan,
+                                       int *clear);
 int launch_tile_prepare(const uint32_t *qweight, const uint32_t *qzeros, const void *scales, const int32_t *g_idx,
                         uint32_t *qtile, uint32_t *sz, int32_t *xsrc, uint16_t *kinv, int K, int N, int G, int bits,
                         int group_size, void *stream);

@@ -237,9 +237,9 @@ int gptq_hip_select_panel(int M, int K, int N, int bits, int group_size, unsigne
                           gptq_hip_plan *plan);
 
 /* The plan of the family's decode kernel (GPTQ_HIP_KERNEL_TILED_DECODE), M <= 8 rows (GPTQ_HIP_ERR_UNSUPPORTED
- * above); gptq_hip_select_tiled chooses it by itself up to 4 rows, and up to 8 for K <= 11008, the matmul kernel above.  No counterpart in the reference, whose
- * GEMV handler takes one row (pycuda_warpper.py:150-152).  Plans with halved tiles carry
- * GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE. */
+ * above); gptq_hip_select_tiled chooses it by itself up to 4 rows, and up to 8 for K <= 11008, for K <= 18432 with N <= 4096 and for
+ * K <= 20480 with N <= 2048, the matmul kernel above.  No counterpart in the reference, whose GEMV handler takes one row (pycuda_warpper.py:150-152).
+ * Plans with halved tiles carry GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE. */
 int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan);
 
 /*
@@ -253,7 +253,9 @@ int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int group_size, 
  * (pack pass, matmul); one more when the plan splits K.  A plan whose flags hold
  * GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE wants ALL bytes of its workspace zero at the first call and leaves them zero
  * (the two halves of a tile that is halved along K meet in 64-bit slots behind the counters): give such plans a
- * workspace of their own, which no other entry point writes between the calls.
+ * workspace of their own, which no other entry point writes between the calls.  A call without a plan asks for that only up
+ * to four rows, for 5 to 8 rows up to K = 11008, and never where x needs more than 128 KB of LDS; for the other sizes that run on halved
+ * tiles it clears the slots itself, and ordinary scratch is enough.
  */
 int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint32_t *sz, const int32_t *xsrc, const uint16_t *kinv,
                         const void *bias, void *y, void *workspace, size_t workspace_bytes, int M, int K, int N,

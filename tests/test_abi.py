@@ -572,3 +572,28 @@ def test_a_tiled_call_without_plan_and_workspace_stays_refused():
             for ws, nbytes in ((null, 0), (fake, 4096)):
                 assert _lib.lib().gptq_hip_gemm_tiled(fake, fake, fake, null, null, null, fake, ws, nbytes, M, K, N, 4, 32, None,
                                                       null) == _lib.ERR_WORKSPACE
+
+
+def default_plan(M, K, N, bits, gs, act, have):
+    """The plan of a gptq_hip_gemm_tiled call that names none and brings ``have`` bytes of workspace, and whether it clears its slots."""
+    plan, clear = _lib.Plan(), ctypes.c_int(-1)
+    rc = _lib.lib().gptq_tiled_default_plan(M, K, N, bits, gs, int(act), ctypes.c_size_t(have), ctypes.byref(plan), ctypes.byref(clear))
+    assert rc == _lib.OK
+    return plan, bool(clear.value)
+
+
+def test_calls_without_a_plan_keep_the_kind_of_workspace_their_size_asked_for():
+    """Halved tiles need a workspace that is zero and their own; the first 16 KB suffice everywhere else, and a caller that names no plan
+    may have packed x behind them.  Sizes that ran on other plans clear the slots; the ones that always ran on halved tiles do not."""
+    private = _lib.PLAN_PRIVATE_ZERO_WORKSPACE
+    for M, K, N, gs in ((8, 14336, 4096, 128), (5, 11040, 64, 32), (6, 18432, 64, 1024), (8, 17408, 64, 128), (3, 14112, 8320, 32),
+                        (4, 27392, 2240, 128), (5, 6720, 8320, 32)):
+        for bits in (2, 3, 4, 8):
+            for act in (False, True):
+                plan, clear = default_plan(M, K, N, bits, gs, act, 1 << 40)
+                assert plan.flags == private and clear, (M, K, N, bits)
+    for M, K, N, gs in ((1, 4096, 11008, 128), (8, 4096, 11008, 128), (8, 11008, 4096, 128), (1, 27392, 2240, 32), (4, 4096, 4096, -1)):
+        plan, clear = default_plan(M, K, N, 4, gs, False, 1 << 40)
+        assert plan.flags == private and not clear
+    for M, K, N in ((1, 1024, 1024), (16, 4096, 4096), (40, 4096, 11008), (2000, 9216, 9216)):
+        assert not default_plan(M, K, N, 4, 128, False, 1 << 40)[1]

@@ -797,3 +797,19 @@ def test_tiled_pack_pass_in_parts_of_a_row(dev, K, M, desc_act):
     plan = _lib.select_tiled(M, K, 64, 4, 32)
     assert plan.kernel == _lib.KERNEL_TILED
     assert_tight(run_tiled(D, prepare(D), plan=plan), expected_output(L), f"K={K} M={M} act={desc_act}")
+
+
+@pytest.mark.parametrize("M,K,N,gs", [(8, 14336, 96, 128), (3, 27392, 64, 128)])
+def test_tiled_calls_without_a_plan_run_on_used_scratch(dev, M, K, N, gs):
+    """A call that names no plan, on a workspace whose first 16 KB are zero and whose other bytes an earlier call has written."""
+    L = layer(5400 + K, K, N, 4, gs, True, M=M, bias=True)
+    D = to_dev(L, dev)
+    qtile, sz, xsrc, kinv = prepare(D)
+    ws = torch.randint(0, 255, (64 << 20,), dtype=torch.uint8, device=dev, generator=torch.Generator(dev).manual_seed(1))
+    ws[:16384] = 0
+    p = lambda t: ctypes.c_void_p(t.data_ptr())   # noqa: E731
+    for _ in range(2):
+        y = torch.zeros((M, N), dtype=torch.float16, device=dev)
+        assert _lib.lib().gptq_hip_gemm_tiled(p(D["x"]), p(qtile), p(sz), p(xsrc), p(kinv), p(D["bias"]), p(y), p(ws), ws.numel(), M, K, N, 4, gs,
+                                              None, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == _lib.OK
+        assert_tight(y, expected_output(L), f"M={M} K={K}")
