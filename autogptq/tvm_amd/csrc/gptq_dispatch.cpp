@@ -693,8 +693,8 @@ extern "C" int gptq::gptq_tiled_default_plan(int M, int K, int N, int bits, int 
                                              int *clear)
 {
     *clear = 0;
-    int rc = gptq_hip_select_panel(M, K, N, bits, group_size, act_order ? GPTQ_HIP_PANEL_ACT_ORDER : 0, 0, 0, plan);
-    if (rc != GPTQ_HIP_OK || plan->workspace_bytes > have) rc = gptq_hip_select_tiled(M, K, N, bits, group_size, plan);
+    int rc = gptq_panel_plan_within(M, K, N, bits, group_size, act_order ? GPTQ_HIP_PANEL_ACT_ORDER : 0, have, plan);
+    if (rc != GPTQ_HIP_OK) rc = gptq_hip_select_tiled(M, K, N, bits, group_size, plan);
     if (rc != GPTQ_HIP_OK) return rc;
     // row blocks need no workspace, but a call without the one that its size asks for stays refused
     gptq_hip_plan other;
@@ -818,8 +818,9 @@ double short_tiled_us(double us, int M, bool transposed, bool act_order)
 
 }  // namespace
 
-extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_size, unsigned flags, int row_tiles, int split_k,
-                                     gptq_hip_plan *plan)
+// tails: plans may cut K for the last row blocks only
+static int plan_panel(int M, int K, int N, int bits, int group_size, unsigned flags, int row_tiles, int split_k, bool tails,
+                      gptq_hip_plan *plan)
 {
     const int ok = tiled_args_ok(M, K, N, bits, group_size, plan);
     if (ok != GPTQ_HIP_OK) return ok;
@@ -849,7 +850,7 @@ extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_si
         // 9216 x 9216 int3 (36 column positions): 13 blocks of 160 rows are 468 workgroups, 310 us; 8 of 256 rows are 288, 252 of them
         // uncut and the last block in seven ranges 278.  Rarely the best plan by more than a little (7 % of 121 drawn calls of more than a turn
         // gain over 3 %), hence the margin.
-        if (row_tiles == 0 && split_k == 0) {
+        if (row_tiles == 0 && split_k == 0 && tails) {
             double best_tail = 0.97 * best;
             for (int r = 1; r <= gptq::kPanelMaxTiles; r++) {
                 const int blocks = ceil_div(M, 32 * r);
@@ -906,6 +907,23 @@ extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_si
     if (act) ws += ((size_t)M * K * 2 + 255) / 256 * 256;   // x, or the transposed product's result, in the copy's order
     plan->workspace_bytes = plan->split_k > 1 || act ? ws : 0;
     return GPTQ_HIP_OK;
+}
+
+extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_size, unsigned flags, int row_tiles, int split_k,
+                                     gptq_hip_plan *plan)
+{
+    return plan_panel(M, K, N, bits, group_size, flags, row_tiles, split_k, true, plan);
+}
+
+// The PANEL plan of a call that names none and brings `have` bytes of workspace.  K ranges for the last row blocks take up to
+// 192 MB for their partial sums, where the plan without them may need none: it is the next choice, ahead of the matmul kernel's.
+extern "C" int gptq::gptq_panel_plan_within(int M, int K, int N, int bits, int group_size, unsigned flags, size_t have, gptq_hip_plan *plan)
+{
+    for (const bool tails : {true, false}) {
+        const int rc = plan_panel(M, K, N, bits, group_size, flags, 0, 0, tails, plan);
+        if (rc == GPTQ_HIP_OK ? plan->workspace_bytes <= have : rc != GPTQ_HIP_ERR_UNSUPPORTED) return rc;
+    }
+    return GPTQ_HIP_ERR_UNSUPPORTED;
 }
 
 namespace {

@@ -247,7 +247,8 @@ int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int group_size, 
  * (pycuda_warpper.py:138, qlinear_tvm.py:123,150).  x is 16-byte aligned, y 8-byte aligned (gy and gx below likewise;
  * GPTQ_HIP_ERR_BAD_ARG otherwise).  x and y are in the layer's own channel order (xsrc = kinv =
  * NULL means no activation order; pass both or neither).  plan: NULL = what gptq_hip_select_route names for a layer
- * with this copy alone, PANEL included; where the workspace does not hold that plan's bytes, gptq_hip_select_tiled (row blocks
+ * with this copy alone, PANEL included; where the workspace does not hold that plan's bytes, the PANEL plan without ranges for the
+ * last row blocks, then gptq_hip_select_tiled (row blocks
  * run without a workspace, but a call is refused unless it brings the one its size asks for).  workspace:
  * plan.workspace_bytes (none for most decode plans).  Decode plans: one launch; matmul plans: two
  * (pack pass, matmul); one more when the plan splits K.  A plan whose flags hold
@@ -275,8 +276,8 @@ int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint32_t *sz, co
  * gptq_hip_tile_prepare_transposed writes both (two launches).  xsrc: the map of gptq_hip_tile_prepare (the channel at
  * each sorted position), NULL without an activation order; gy and gx are in the layer's own channel order.  The
  * weights are formed exactly as in the forward product (fp16(scale * (q - zero)), one rounding), sums are fp32.
- * plan: NULL = gptq_hip_select_panel (transposed) where that names a plan and the workspace holds its bytes, else
- * gptq_hip_select_tiled_transposed.  workspace: plan.workspace_bytes, zeroed once.
+ * plan: NULL = gptq_hip_select_panel (transposed) where that names a plan and the workspace holds its bytes, with or without ranges
+ * for the last row blocks, else gptq_hip_select_tiled_transposed.  workspace: plan.workspace_bytes, zeroed once.
  */
 size_t gptq_hip_tiled_transposed_bytes(int K, int N, int bits);
 size_t gptq_hip_tiled_transposed_table_bytes(int K, int N, int group_size);

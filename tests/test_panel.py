@@ -457,3 +457,19 @@ def test_panel_plans_with_ranges_for_the_last_blocks():
         q.flags = flags
         assert _lib.lib().gptq_hip_gemm_tiled(fake, fake, fake, null, null, null, fake, fake, 1 << 40, 2000, 9216, 9216, 3, -1,
                                               ctypes.byref(q), null) == _lib.ERR_BAD_ARG
+
+
+def test_calls_without_the_workspace_of_the_last_blocks_keep_the_panel_kernel():
+    # ranges for the last row blocks want memory that the plan without them does not: calls without it run on that one
+    lib, p = _lib.lib(), _lib.Plan()
+    for tr, M, K, N, bits, gs in ((False, 2000, 9216, 9216, 3, -1), (False, 4096, 12544, 16704, 3, 32), (True, 2000, 9216, 9216, 3, -1)):
+        full = _lib.select_panel(M, K, N, bits, gs, False, tr)
+        assert full.flags >> 8 > 0 and full.split_k > 1 and full.workspace_bytes > 1 << 20
+        for have, ranges in ((0, False), (full.workspace_bytes - 1, False), (full.workspace_bytes, True)):
+            rc = lib.gptq_panel_plan_within(M, K, N, bits, gs, _lib.PANEL_TRANSPOSED if tr else 0, ctypes.c_size_t(have), ctypes.byref(p))
+            assert rc == _lib.OK and p.kernel == _lib.KERNEL_PANEL and p.workspace_bytes <= have
+            assert (p.as_dict() == full.as_dict()) if ranges else (p.flags == 0 and p.split_k == 1)
+            if not tr:
+                q, clear = _lib.Plan(), ctypes.c_int()
+                assert lib.gptq_tiled_default_plan(M, K, N, bits, gs, 0, ctypes.c_size_t(have), ctypes.byref(q), ctypes.byref(clear)) == _lib.OK
+                assert q.as_dict() == p.as_dict()
