@@ -597,3 +597,18 @@ def test_calls_without_a_plan_keep_the_kind_of_workspace_their_size_asked_for():
         assert plan.flags == private and not clear
     for M, K, N in ((1, 1024, 1024), (16, 4096, 4096), (40, 4096, 11008), (2000, 9216, 9216)):
         assert not default_plan(M, K, N, 4, 128, False, 1 << 40)[1]
+
+
+def test_calls_without_a_plan_are_refused_by_one_rule():
+    """What gptq_hip_select_tiled asks for is what a call has to bring, decode plans and row blocks alike, unless a PANEL plan takes it."""
+    runs = refused = 0
+    for M in (1, 2, 3, 4, 5, 8, 9, 16, 40, 128):
+        for K, N, gs in ((8192, 8192, 128), (16384, 8192, -1), (4096, 4096, 128), (4096, 11008, 32), (14336, 4096, 128), (512, 1024, 64), (28672, 8192, 128)):
+            need = _lib.select_tiled(M, K, N, 4, gs).workspace_bytes
+            for have in (0, need - 1, need):
+                if have < 0 or _lib.lib().gptq_panel_plan_within(M, K, N, 4, gs, 0, ctypes.c_size_t(have), ctypes.byref(_lib.Plan())) == _lib.OK:
+                    continue
+                plan, _ = default_plan(M, K, N, 4, gs, False, have)
+                assert (plan.workspace_bytes <= have) == (have >= need), (M, K, N, have)
+                runs, refused = runs + (have >= need), refused + (have < need)
+    assert runs > 60 and refused > 60
