@@ -101,6 +101,9 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
         p.x += (size_t)m0 * p.K;
         p.M = min(MR, M_all - m0);
     }
+    // the channel map: four rows and more come with one exactly where their x lies position by position (the launcher's choice), so that
+    // nothing is built for the other case (kept as a test at run time it cost the variants without a map 10 to 80 registers)
+    const bool mapped = MR >= 4 ? PM : p.kinv != nullptr;
     constexpr int RS = (MR + 3) / 4;   // sets of four rows: a matrix instruction takes four rows of x
     constexpr bool EXACT = RB || tiled_decode_exact(BITS);
     constexpr bool CENTRE = !EXACT && tiled_decode_centred(MR);
@@ -154,7 +157,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     //         workgroup at the barrier until the last of them had arrived, 0.6-0.9 us after x; a wave now asks
     //         for the word of a unit when it asks for the unit's weights and finds it when they are there.) -----
     // (without a map the channels of the range are the range itself)
-    const int k8_lo = p.kinv ? 0 : p0 / 8, k8_hi = p.kinv ? p.K / 8 : min(p0 + span, p.K) / 8;
+    const int k8_lo = mapped ? 0 : p0 / 8, k8_hi = mapped ? p.K / 8 : min(p0 + span, p.K) / 8;
     // passes over x kept in registers (eight rows: 32 registers a pass; a second one only shortens the way of workgroups of
     // four waves without an activation order, 4096 x 11008 7.55 -> 7.29 us, and costs 0.2 to 0.5 us elsewhere)
     constexpr int QP = MR == 16 || (MR == 8 && (PM || KW > 4)) ? 1 : 2;
@@ -163,7 +166,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
 #pragma unroll
     for (int ps = 0; ps < QP; ps++) {
         const int k = 8 * min(k8_lo + tid + ps * NT, k8_hi - 1);  // (clamped: the pass is skipped below when outside)
-        kq[ps] = p.kinv ? *(const u4 *)(p.kinv + k) : (u4){0u, 0u, 0u, 0u};
+        kq[ps] = mapped ? *(const u4 *)(p.kinv + k) : (u4){0u, 0u, 0u, 0u};
 #pragma unroll
         for (int m = 0; m < MR; m++) xq[ps][m] = *(const h8 *)(p.x + (size_t)min(m, p.M - 1) * p.K + k);
     }
@@ -186,7 +189,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
             }
             return;
         }
-        if (!p.kinv) {   // no activation order: the eight channels are eight consecutive positions, one store
+        if (!mapped) {   // no activation order: the eight channels are eight consecutive positions, one store
             // (k8_lo .. k8_hi is the workgroup's own range here, a multiple of 8 away from p0)
 #pragma unroll
             for (int m = 0; m < R; m++) *(h8 *)(xl + (r0 + m) * span + (k - p0)) = xv[m];
@@ -226,7 +229,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
 #pragma unroll
         for (int r0 = 0; r0 < MR; r0 += R) {
             h8 xv[R];
-            if (p.kinv && r0 == 0) {   // the map and the rows of x, requested together
+            if (mapped && r0 == 0) {   // the map and the rows of x, requested together
                 const void *ptr[R + 1];
                 u4 v[R + 1];
                 ptr[R] = p.kinv + k;

@@ -38,3 +38,16 @@ def test_hot_path_kernels_do_not_spill():
         assert r.get("vgpr_spill", 0) == 0 and r.get("scratch", 0) == 0, (name, r)   # every shipped kernel
         if "stream_kernel" in name or "stream_direct" in name or "grouped_kernel" in name:
             assert r.get("occupancy", 0) >= 2, (name, r)   # two waves per SIMD is what these designs assume
+
+
+def test_decode_kernels_keep_their_scalars_in_registers():
+    """What a variant of the decode kernel cannot reach must not be built into it: the channel-by-channel staging, once behind a test at
+    run time, cost the variants of eight and sixteen rows without a map 21 to 105 spilled scalar registers."""
+    if not os.path.exists(build.REPORT):
+        pytest.skip("library was built without the resource report")
+    with open(build.REPORT) as f:
+        report = json.load(f)
+    decode = {n: r for n, r in report.items() if "tiled_decode_kernel" in n}
+    assert len(decode) > 100
+    for name, r in decode.items():
+        assert r["sgpr_spill"] == 0, (name, r)
