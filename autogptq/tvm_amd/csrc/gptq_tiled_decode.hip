@@ -256,7 +256,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     constexpr uint32_t BLOCK_BYTES = 256u * BITS;
     // the tile as a buffer: the lane's offset in a vector register, the block's in a scalar one.  Blocks requested
     // past the wave's range (ahead of the walk, never multiplied) are the next wave's; past the end of the tile:
-    // its last block again (the padding of K past the wave's range: multiplied by zeros of x)
+    // its last block again (never multiplied either)
     const __amdgpu_buffer_rsrc_t tile = tile_buffer(p.qtile + (size_t)T * (size_t)p.S_total * BLOCK_BYTES,
                                                     (uint32_t)p.S_total * BLOCK_BYTES);
     const int S_last = p.S_total - 1;
@@ -275,7 +275,11 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
         const uint32_t l0 = 2u * (uint32_t)min(S_begin + i, S_last);
         const uint32_t g0 = group_of(l0);
         uint32_t off = sz_lane;
-        if constexpr (E == 1) off += h ? (group_of(l0 + 1u) - g0) * row_bytes : 0u;   // the two halves of a block may differ
+        if constexpr (E == 1) {   // the two halves of a block may differ; one past K has no scale (zero, from behind the buffer): its
+            // zeros of x times an infinite weight of the last group would be NaN
+            const uint32_t next = l0 + 1u < (uint32_t)p.K >> 5 ? (group_of(l0 + 1u) - g0) * row_bytes : 0xffffff80u;
+            off += h ? next : 0u;
+        }
         sr = __builtin_amdgcn_raw_buffer_load_b32(szb, off, g0 * row_bytes, 0);
     };
     auto load_chunk = [&](int i, uint32_t (&wc)[PF][BITS], uint32_t (&sc)[UPC]) {
@@ -452,14 +456,15 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
         }
     };
 
-    // Chunks of PF blocks, NCH in flight; x rides one block ahead in two register sets.  Blocks past the end
-    // of K inside a wave's range are harmless (their x and sums are zeros), blocks past the range are skipped.
+    // Chunks of PF blocks, NCH in flight; x rides one block ahead in two register sets.  Blocks past the end of K or of the
+    // wave's range are skipped.
+    const int todo = max(min(ws, p.S_total - S_begin), 0);   // (paired blocks: even, like both of these)
     u2 xr[2][RS];
     load_x((uint32_t)(S_begin - S_wg), xr[0]);
     auto chunk = [&](int c, uint32_t (&wc)[PF][BITS], const uint32_t (&sc)[UPC], auto all_c) {
         constexpr bool ALL = decltype(all_c)::value;
         [&]<int... U>(std::integer_sequence<int, U...>) {
-            ((ALL || c + U < ws
+            ((ALL || c + U < todo
                   ? block(std::integral_constant<int, U % E>{}, S_begin + c + U, wc[U], sc[U / E], xr[U & 1], xr[(U + 1) & 1])
                   : (void)0),
              ...);
@@ -467,7 +472,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     };
     int c = 0;
     // steady state: every chunk consumed is replaced by the one a ring further on, which lies inside the range
-    for (; c + 2 * RING <= ws; c += RING) {
+    for (; c + 2 * RING <= todo; c += RING) {
 #pragma unroll
         for (int j = 0; j < NCH; j++) {
             chunk(c + j * PF, w[j], szr[j], std::true_type{});
@@ -476,7 +481,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    if (ws - c == RING) {   // exactly what is in flight is left: no more requests, no tests
+    if (todo - c == RING) {   // exactly what is in flight is left: no more requests, no tests
 #pragma unroll
         for (int j = 0; j < NCH; j++) chunk(c + j * PF, w[j], szr[j], std::true_type{});
     } else {
@@ -484,7 +489,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
         // stands behind a test (the compiler would no longer know how many are outstanding, and wait for all of them
         // at every chunk): a chunk past the end of the range asks for the range's last chunk again, which the
         // cache has, and is not multiplied.
-        const int last_chunk = max((ws - 1) / PF * PF, 0);
+        const int last_chunk = max((todo - 1) / PF * PF, 0);
 #pragma unroll
         for (int j = 0; j < NCH; j++) {
             chunk(c + j * PF, w[j], szr[j], std::false_type{});

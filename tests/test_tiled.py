@@ -813,3 +813,39 @@ def test_tiled_calls_without_a_plan_run_on_used_scratch(dev, M, K, N, gs):
         assert _lib.lib().gptq_hip_gemm_tiled(p(D["x"]), p(qtile), p(sz), p(xsrc), p(kinv), p(D["bias"]), p(y), p(ws), ws.numel(), M, K, N, 4, gs,
                                               None, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == _lib.OK
         assert_tight(y, expected_output(L), f"M={M} K={K}")
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("K,N,gs", [(96, 96, 32), (352, 96, 32), (1152, 96, 128), (1280, 8224, 128), (4128, 96, 32), (14400, 64, 64)])
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_tiled_decode_infinite_weights_of_the_last_group(dev, bits, K, N, gs, desc_act):
+    """The waves of the decode kernel walk past K where it is no whole number of their blocks: x is zero there, and an infinite weight
+    (a scale of infinity, or one times codes beyond fp16) must not count."""
+    top = (1 << bits) - 1
+    for M in (1, 2, 4, 8, 12, 40):
+        if M > 8 and K > 9216:
+            continue
+        L = layer(5500 + K, K, N, bits, gs, desc_act, M=M)
+        L["x"] = L["x"].abs()
+        L["scales"][-1, 5] = float("inf")
+        L["codes"][:, 5], L["zeros"][:, 5] = top, 1
+        L["qweight"] = torch.from_numpy(pack.pack_qweight(L["codes"].numpy(), bits))
+        L["qzeros"] = torch.from_numpy(pack.pack_qzeros(L["zeros"].numpy(), bits))
+        want = expected_output(L)
+        assert bool((torch.isinf(want).sum(1) == 1).all()) and bool(torch.isinf(want[:, 5]).all())
+        D = to_dev(L, dev)
+        prep = prepare(D)
+        plans = [_lib.select_route(M, K, N, bits, gs, desc_act, _lib.COPY_TILED | _lib.COPY_TILED_PANEL).plan]
+        if plans[0].row_tiles == 8 and plans[0].m_blocks > 1:
+            p = _lib.select_route(M, K, N, bits, gs, desc_act, _lib.COPY_TILED | _lib.COPY_TILED_PANEL).plan
+            span = p.waves_k * p.k_chunk * 64
+            p.row_tiles, p.m_blocks, p.grid_z, p.lds_bytes = 16, -(-M // 16), -(-M // 16), 16 * span * 2 + 64 + p.waves_k * 16 * 128
+            if p.lds_bytes <= 160 * 1024:
+                plans.append(p)
+        for plan in plans:
+            if plan.kernel != _lib.KERNEL_TILED_DECODE or plan.waves_n == 2:
+                continue
+            y = run_tiled(D, prep, plan=plan).float().cpu()
+            assert bool((y[:, 5] == float("inf")).all()), (M, plan.as_dict())
+            y[:, 5] = want[:, 5] = 0.0
+            assert_tight(y, want, f"M={M} rows built for {plan.row_tiles}")
