@@ -198,6 +198,11 @@ constexpr int kDecodeSelectRows = 4;   // rows up to which gptq_hip_select_tiled
 inline int tiled_decode_rows(int M) { return M <= 1 ? 1 : (M <= 2 ? 2 : (M <= 4 ? 4 : 8)); }
 // (four and eight rows: the zero point is taken off every code, so no sums of x are kept)
 constexpr bool tiled_decode_centred(int mr) { return mr >= 4; }
+// one and two rows of small layers as well (figures at the kernel), with the LDS of the others
+constexpr bool tiled_decode_centres(int mr, int K, int N, int waves_k)
+{
+    return tiled_decode_centred(mr) || (K <= 2560 && N <= 4096 && waves_k <= 8);
+}
 inline int tiled_decode_lds_bytes(int mr, int span, int groups, int waves_k)
 {
     (void)groups;   // (the (scale, zero) words no longer pass through LDS)

@@ -21,7 +21,7 @@ namespace gptq {
 // and the instruction can broadcast the A operand of one block to the others (cbsz / abid): block b of the
 // half keeps positions 4 b .. 4 b + 3 in its A registers and the instruction for positions 4 i .. 4 i + 3
 // names block i, so x costs one 8-byte LDS read per lane and block.
-// One and two rows (2, 3, 4 bits): per weight the vector ALU only unpacks.
+// One and two rows (2, 3, 4 bits), but for small layers: per weight the vector ALU only unpacks.
 // The codes enter as (base + q) with the bases of the register unpack; per block of 32 positions the
 // epilogue takes y += scale * (P - Bsum - zero * Xsum), with Xsum = sum x and Bsum = sum x * base of the
 // block computed once per workgroup when x is staged.
@@ -29,7 +29,12 @@ namespace gptq {
 // (exact: small integers), and the epilogue is y += scale * P.  The sums above cost vector instructions and LDS reads in
 // proportion to the rows, the subtraction does not: without / with it, us, no activation order: 4096 x 11008 int4 6.66 / 6.03 at
 // four rows, 8.53 / 7.55 at eight, 4096 x 4096 5.13 / 4.50 at four; one row 4.11 / 4.16, two rows 6.20 / 6.51 at 4096 x 11008.
-// (The sums' large terms no longer cancel in fp32, either.)
+// (The sums' large terms no longer cancel in fp32, either: error against 64 bits 8e-8 of the result, 4e-6 to 2.5e-5 with the sums.)
+// So do one and two rows of layers of up to 2560 channels and 4096 columns (tiled_decode_centres), where there are few weights to
+// take it off: with the sums, whose pairs of blocks would make the error 1.4 times that of the 16-column kernel, which ran these layers
+// (1024 x 1024 int4 7.7e-6, 5.5e-6 there; this form 7.7e-8), / this form, us: 1024 x 1024 one / two rows 3.52 / 2.95 and 3.55 / 3.06, groups of 32 3.77 /
+// 3.42, 2048 x 4096 3.29 / 3.31 and 3.50 / 3.44, 2560 x 2560 with an activation order 4.12 / 3.94, 2560 x 4096 two rows of groups of 32 4.58 /
+// 4.33; 4096 x 4096 level, 4096 x 11008 with an activation order 6.27 / 6.63.
 // Either way, like GROUPED and unlike the TILED matmul, this does not reproduce the fp16 rounding of each dequantised
 // weight: products are exact, sums are fp32.
 // 8-bit layers instead dequantise every weight in registers, as the matmul does (tiled_decode_exact), and add
@@ -81,7 +86,8 @@ struct DecodeTail {
 // eight rows of layers beyond kDecodeUnroundedK channels, run so.
 // E: blocks of 64 positions that share one epilogue (1, or 2 when the groups are multiples of 128 channels and
 // every wave has an even number of blocks: both lane blocks of both blocks then lie in one group).
-template <int BITS, int MR, int KW, int E, bool PM, bool RB>
+// C: the zero point is taken off every code (CENTRE; four rows and more always are built so).
+template <int BITS, int MR, int KW, int E, bool PM, bool RB, bool C>
 __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a_x, const uint16_t *a_kinv, const char *a_qtile,
                                                                const uint32_t *a_sz, int a_K, uint32_t a_m_steps, int a_T_total,
                                                                int a_grid_x, uint32_t a_lbg_magic, uint32_t a_flags,
@@ -106,7 +112,8 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     const bool mapped = MR >= 4 ? PM : p.kinv != nullptr;
     constexpr int RS = (MR + 3) / 4;   // sets of four rows: a matrix instruction takes four rows of x
     constexpr bool EXACT = RB || tiled_decode_exact(BITS);
-    constexpr bool CENTRE = !EXACT && tiled_decode_centred(MR);
+    static_assert(C || !tiled_decode_centred(MR), "one and two rows only keep sums of x");
+    constexpr bool CENTRE = !EXACT && C;
     constexpr int NT = 64 * KW;
     constexpr int PF = 2;              // blocks of weights per chunk
     // chunks in flight per wave.  A wave asks for a chunk when it has consumed one, so its walk is a chain of
@@ -148,7 +155,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     _Float16 *xl = (_Float16 *)smem;
     const uint32_t zero_off = (uint32_t)MR * (uint32_t)span * 2u;
     f2 *xs = (f2 *)(smem + zero_off + 64);
-    const int lbs = tiled_decode_centred(MR) ? 0 : span / 32;
+    const int lbs = C ? 0 : span / 32;
     float *red = (float *)(xs + (size_t)lbs * MR);
 
     // ---- 1. x and the map first (a wait for them would also wait for every older load: vector loads return
@@ -545,10 +552,10 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     }
 }
 
-template <int BITS, int MR, int KW, int E, bool PM, bool RB>
+template <int BITS, int MR, int KW, int E, bool PM, bool RB, bool C>
 static int launch_decode_one(const DecodeParams &p, const gptq_hip_plan &plan, hipStream_t stream)
 {
-    auto kern = tiled_decode_kernel<BITS, MR, KW, E, PM, RB>;
+    auto kern = tiled_decode_kernel<BITS, MR, KW, E, PM, RB, C>;
     if (plan.lds_bytes > 65536) {
         if (hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, plan.lds_bytes) != hipSuccess) {
             (void)hipGetLastError();
@@ -564,15 +571,16 @@ static int launch_decode_one(const DecodeParams &p, const gptq_hip_plan &plan, h
     return hipGetLastError() == hipSuccess ? GPTQ_HIP_OK : GPTQ_HIP_ERR_LAUNCH;
 }
 
-template <int BITS, int MR, int E, bool PM, bool RB = false>
+template <int BITS, int MR, int E, bool PM, bool RB = false, bool C = tiled_decode_centred(MR)>
 static int launch_decode_kw(const DecodeParams &p, const gptq_hip_plan &plan, hipStream_t stream)
 {
     switch (plan.waves_k) {
-        case 4: return launch_decode_one<BITS, MR, 4, E, PM, RB>(p, plan, stream);
-        case 8: return launch_decode_one<BITS, MR, 8, E, PM, RB>(p, plan, stream);
+        case 4: return launch_decode_one<BITS, MR, 4, E, PM, RB, C>(p, plan, stream);
+        case 8: return launch_decode_one<BITS, MR, 8, E, PM, RB, C>(p, plan, stream);
         case 16:
-            if constexpr (MR >= 8) return GPTQ_HIP_ERR_UNSUPPORTED;   // (128 registers per lane do not hold two sets of rows)
-            else return launch_decode_one<BITS, MR, 16, E, PM, RB>(p, plan, stream);
+            // (128 registers per lane do not hold two sets of rows)
+            if constexpr (MR >= 8 || (C && MR < 4)) return GPTQ_HIP_ERR_UNSUPPORTED;
+            else return launch_decode_one<BITS, MR, 16, E, PM, RB, C>(p, plan, stream);
         default: return GPTQ_HIP_ERR_UNSUPPORTED;
     }
 }
@@ -615,9 +623,13 @@ int launch_tiled_decode(const void *x, const void *qtile, const uint32_t *sz, co
     // two blocks per epilogue where every unit of two blocks lies in one group
     // (halved tiles, grid_x > tiles: their waves walk the two even shares of k_chunk that the planner checked)
     const bool pairs = tiled_decode_pairs(group_size, plan.k_chunk);
+    const bool centred = tiled_decode_centres(mr, K, N, plan.waves_k);   // (8 bits round every weight: one form)
 #define GPTQ_DECODE_CASE(B, R) \
     if (bits == B && mr == R) {                                                                                            \
-        if (R >= 4 && kinv)                                                                                                \
+        if (R < 4 && B != 8 && centred)                                                                                    \
+            rc = pairs ? launch_decode_kw<B, R, 2, false, false, (R >= 4 || B != 8)>(p, plan, stream)                      \
+                       : launch_decode_kw<B, R, 1, false, false, (R >= 4 || B != 8)>(p, plan, stream);                     \
+        else if (R >= 4 && kinv)                                                                                                \
             rc = pairs ? launch_decode_kw<B, R, 2, (R >= 4)>(p, plan, stream) : launch_decode_kw<B, R, 1, (R >= 4)>(p, plan, stream); \
         else                                                                                                               \
             rc = pairs ? launch_decode_kw<B, R, 2, false>(p, plan, stream) : launch_decode_kw<B, R, 1, false>(p, plan, stream);       \

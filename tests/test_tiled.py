@@ -849,3 +849,21 @@ def test_tiled_decode_infinite_weights_of_the_last_group(dev, bits, K, N, gs, de
             assert bool((y[:, 5] == float("inf")).all()), (M, plan.as_dict())
             y[:, 5] = want[:, 5] = 0.0
             assert_tight(y, want, f"M={M} rows built for {plan.row_tiles}")
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("K,N,gs", [(32, 32, 32), (512, 1024, -1), (1024, 1024, 128), (1056, 96, 32), (2048, 4096, 128), (2560, 96, 512)])
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_tiled_decode_small_layers_sum_without_the_bases(dev, bits, K, N, gs, desc_act):
+    """Up to eight rows of small layers: fp32 sums of scale * (q - zero) * x, not of the codes with the large bases of the unpack, whose
+    cancellation costs 4e-6 to 2e-5.  The bias takes the fp16 of the exact result off, so that y holds the sums' own error: with about
+    sixteen roundings of 2^-24 one after the other, 1e-6 of the result."""
+    L = layer(5600 + K, K, N, bits, gs, desc_act, M=1)
+    exact = unrounded_output(L, L["x"])
+    L["bias"] = -exact[0].half()
+    rest = exact + L["bias"].double()
+    D = to_dev(L, dev)
+    prep = prepare(D)
+    for M in (1, 2, 4, 8):
+        y = run_tiled(D, prep, x=D["x"].expand(M, K).contiguous())
+        assert float((y.double().cpu() - rest).norm() / (M ** 0.5 * exact.norm())) < 1e-6, M
