@@ -1005,19 +1005,6 @@ bool tiled_wins(int M, int K, int N, bool act_order, int bits, bool one_group)
     return K <= 8192 || (M <= 256 && (K <= 11008 || act_order || (one_group && N <= 16384)));
 }
 
-// Three and four rows of layers past that table that would run on GROUPED, since the decode kernel takes the zero point off the codes
-// and stages an activation order in whole positions (us, against GROUPED on the better of the other copies: 8192 x 28672 int4 25.4 /
-// 24.1 with / without an order against 30.1 / 27.7, int3 21.8 / 20.2 against 33.3 / 30.9; 11008 x 11008 int3 16.2 / 13.8 against 25.6 / 23.0;
-// 4096 x 22016 8.6-10.5 against 13.6-15.9; 2048 x 33632 int3 7.7 against 14.6; 1792 x 19968 6.0 against 12.5; 2816 x 32608 11.7 against 23.0).  Both scale the
-// exact products of the codes group by group.  Layers whose small groups or length put them on STREAM stay there, though they would gain as
-// much (13824 x 5120 11 against 17): it multiplies the weights as the reference rounds them, and the two differ by that rounding, 1.7e-4.
-bool decode_wins_past_table(int M, int K, int N, int bits, int group_size)
-{
-    gptq_hip_plan other;
-    return (M == 3 || M == 4) && K <= 19712 && gptq_hip_select(M, K, N, bits, group_size, 0, &other) == GPTQ_HIP_OK &&
-           other.kernel == GPTQ_HIP_KERNEL_GROUPED;
-}
-
 // The plan gptq_hip_gemm_sorted runs for M rows of a layer whose channels were sorted by group, if that path covers
 // the problem: the GROUPED family, or up to kSortedMaxRows rows on the STREAM kernel that reads x itself behind the
 // pass that reorders x (that pass costs a launch, ~2 us: int3 gains 2-4 us over the per-weight lookups of the
@@ -1032,6 +1019,22 @@ bool sorted_plan(int M, int K, int N, int bits, int group_size, gptq_hip_plan *p
     if (plan->kernel == GPTQ_HIP_KERNEL_STREAM && M <= gptq::kSortedMaxRows && plan->row_tiles == 1)
         return bits == 3 || (long long)K * N >= (1LL << 25);
     return false;
+}
+
+// Three and four rows of layers past that table that would run on GROUPED, since the decode kernel takes the zero point off the codes
+// and stages an activation order in whole positions (us, against GROUPED on the better of the other copies: 8192 x 28672 int4 25.4 /
+// 24.1 with / without an order against 30.1 / 27.7, int3 21.8 / 20.2 against 33.3 / 30.9; 11008 x 11008 int3 16.2 / 13.8 against 25.6 / 23.0;
+// 4096 x 22016 8.6-10.5 against 13.6-15.9; 2048 x 33632 int3 7.7 against 14.6; 1792 x 19968 6.0 against 12.5; 2816 x 32608 11.7 against 23.0).  Both scale the
+// exact products of the codes group by group.  Layers whose small groups or length put them on STREAM stay there, though they would gain as
+// much (13824 x 5120 11 against 17): it multiplies the weights as the reference rounds them, and the two differ by that rounding, 1.7e-4.
+// The plan asked for is the one that the call would have on the copies on offer: without the sorted copy an activation order is STREAM's.
+bool decode_wins_past_table(int M, int K, int N, int bits, int group_size, bool act, unsigned copies)
+{
+    if (M != 3 && M != 4) return false;
+    gptq_hip_plan other;
+    if ((copies & GPTQ_HIP_COPY_SORTED) && act && sorted_plan(M, K, N, bits, group_size, &other)) return other.kernel == GPTQ_HIP_KERNEL_GROUPED;
+    return (copies & GPTQ_HIP_COPY_CHECKPOINT) && gptq_hip_select(M, K, N, bits, group_size, act, &other) == GPTQ_HIP_OK &&
+           other.kernel == GPTQ_HIP_KERNEL_GROUPED;
 }
 
 }  // namespace
@@ -1088,7 +1091,7 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
     if (!fused_bits) {
         if (!tiled_ok) return GPTQ_HIP_OK;   // 2 and 8 bits have no other fused kernels: the library
         tiled = true;
-    } else if (tiled_ok && (tiled_wins(M, K, N, act, bits, one_group) || (panels && decode_wins_past_table(M, K, N, bits, group_size)))) {
+    } else if (tiled_ok && (tiled_wins(M, K, N, act, bits, one_group) || (panels && decode_wins_past_table(M, K, N, bits, group_size, act, copies)))) {
         tiled = true;   // (the rows past the table like the panel kernel: for hosts that set the bit)
     }
     int which = 0;

@@ -612,3 +612,23 @@ def test_calls_without_a_plan_are_refused_by_one_rule():
                 assert (plan.workspace_bytes <= have) == (have >= need), (M, K, N, have)
                 runs, refused = runs + (have >= need), refused + (have < need)
     assert runs > 60 and refused > 60
+
+
+def test_three_and_four_rows_past_the_table_leave_no_stream_plan():
+    """What decides is the plan of the copies on offer: an activation order without the sorted copy runs on STREAM, whose rounded weights are
+    closer to the reference's than the decode kernel's products."""
+    moved = stayed = 0
+    panel = _lib.COPY_TILED | _lib.COPY_TILED_PANEL
+    for K, N, bits, gs in ((12288, 28672, 4, 256), (1024, 16384, 3, 32), (8192, 28672, 4, 128), (4096, 22016, 3, 128), (11008, 11008, 3, -1),
+                           (2048, 33632, 4, 64), (28672, 8192, 4, 128)):
+        for act in (False, True):
+            for M in (3, 4):
+                for kept in (_lib.COPY_CHECKPOINT, _lib.COPY_CHECKPOINT | _lib.COPY_SORTED, _lib.COPY_SORTED):
+                    without, r = _lib.select_route(M, K, N, bits, gs, act, kept | _lib.COPY_TILED), _lib.select_route(M, K, N, bits, gs, act, kept | panel)
+                    if without.copy != _lib.ROUTE_TILED and without.plan.kernel == _lib.KERNEL_GROUPED:
+                        assert r.copy == _lib.ROUTE_TILED and r.plan.kernel == _lib.KERNEL_TILED_DECODE
+                        moved += 1
+                    else:
+                        assert (r.copy, r.plan.as_dict()) == (without.copy, without.plan.as_dict()), (M, K, N, bits, gs, act, kept)
+                        stayed += without.plan.kernel == _lib.KERNEL_STREAM
+    assert moved > 20 and stayed > 10
