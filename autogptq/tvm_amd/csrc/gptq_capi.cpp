@@ -323,7 +323,7 @@ static int run_panel(const void *x, const void *qtile, const uint32_t *sz, const
     const int main = gptq::panel_main_blocks(plan);
     if (plan.flags & ((1 << gptq::kPanelMainShift) - 1) || (main > 0 && (plan.split_k == 1 || main >= plan.m_blocks))) return GPTQ_HIP_ERR_BAD_ARG;
     const int rows = M - 32 * rt * main;   // (of the tail; all of them without main blocks)
-    if (!gptq::panel_launches((long long)plan.grid_x * (main + (long long)(plan.m_blocks - main) * plan.split_k), plan.block, trans && xsrc ? M : 0))
+    if (!gptq::panel_launches(plan.grid_x, plan.m_blocks, main, plan.split_k, plan.block, trans && xsrc ? M : 0))
         return GPTQ_HIP_ERR_UNSUPPORTED;
     if (plan.split_k > 1 && (long long)M * cols >= (1LL << 32)) return GPTQ_HIP_ERR_UNSUPPORTED;
     const size_t part = plan.split_k > 1 ? ((size_t)plan.split_k * rows * cols * sizeof(float) + 255) / 256 * 256 : 0;

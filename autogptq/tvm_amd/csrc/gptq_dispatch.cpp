@@ -887,7 +887,7 @@ static int plan_panel(int M, int K, int N, int bits, int group_size, unsigned fl
     }
     if (rt > gptq::kPanelMaxTiles || !gptq::panel_addresses(rt, red)) return GPTQ_HIP_ERR_UNSUPPORTED;
     const int m_blocks = ceil_div(M, 32 * rt);
-    if (!gptq::panel_launches((long long)col_wgs * (main + (long long)(m_blocks - main) * split), 256 * gptq::panel_waves_k(rt), transposed && act ? M : 0))
+    if (!gptq::panel_launches(col_wgs, m_blocks, main, split, 256 * gptq::panel_waves_k(rt), transposed && act ? M : 0))
         return GPTQ_HIP_ERR_UNSUPPORTED;
     plan->kernel = GPTQ_HIP_KERNEL_PANEL;
     plan->row_tiles = rt;

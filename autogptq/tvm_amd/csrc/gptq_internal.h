@@ -308,10 +308,11 @@ constexpr int panel_lds_bytes(int bits, int rt)
 }
 // The kernel addresses the rows of a workgroup with 31 bits (bit 31 of an offset marks what lies outside)
 constexpr bool panel_addresses(int rt, int red) { return 32LL * rt * red * 2 < (1LL << 31); }
-// and a launch has less than 2^32 threads, the pass that puts a gradient's rows in order included (256 for each of them)
-constexpr bool panel_launches(long long wgs, int block, long long ordered_rows)
+// and a launch has less than 2^32 threads along its first dimension (K ranges of all rows lie along the second, those of the rows after
+// the first `main` blocks behind them), the pass that puts a gradient's rows in order included (256 for each of them)
+constexpr bool panel_launches(long long col_wgs, long long m_blocks, long long main, long long split_k, int block, long long ordered_rows)
 {
-    return wgs * block < (1LL << 32) && ordered_rows * 256 < (1LL << 32);
+    return col_wgs * (main > 0 ? main + (m_blocks - main) * split_k : m_blocks) * block < (1LL << 32) && ordered_rows * 256 < (1LL << 32);
 }
 // row blocks of a plan with K ranges that take all of K, ahead of the ones that are cut (in the upper bits of the plan's flags)
 constexpr int kPanelMainShift = 8;

@@ -188,14 +188,15 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
     // and what is left of the rows spread over one turn more.
     // XCD-aware order: workgroups are dealt to the XCDs round robin, so id % 8 names the XCD; each takes a
     // contiguous run of the tile order, in which groups of four row blocks walk the columns together
-    int rb, cb, split = 0;
+    // (K ranges of all rows lie along the grid's second dimension, those of the last row blocks behind the whole ones)
+    int rb, cb, split = blockIdx.y;
     const int n_main = t.col_wgs * t.main_rbs;
     const bool tail_wg = (int)blockIdx.x >= n_main;
     const bool ranges = tail_wg && t.split_k > 1;
     {
         const uint32_t row_wgs = tail_wg ? t.tail_rbs : t.main_rbs, nwg = t.col_wgs * row_wgs;
         uint32_t id = blockIdx.x - (tail_wg ? n_main : 0);
-        if (ranges) split = (int)panel_div(id, nwg, t.tail_magic), id -= split * nwg;
+        if (ranges && n_main > 0) split = (int)panel_div(id, nwg, t.tail_magic), id -= split * nwg;
         const uint32_t q = nwg / 8, r = nwg % 8, xcd = id % 8, i = id / 8;
         const uint32_t lin = xcd * q + min(xcd, r) + i;
         const uint32_t per = 4 * t.col_wgs, grp = panel_div(lin, per, t.column_group_magic), in = lin - grp * per;
@@ -657,8 +658,9 @@ static int launch_panel_one(const _Float16 *x, const char *qtile, const uint32_t
     auto kern = panel_kernel<BITS, RT, TRANS>;
     const int lds = panel_lds_bytes(BITS, RT);
     if (!allow_lds(kern, lds)) return GPTQ_HIP_ERR_LAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)t.col_wgs * ((unsigned)t.main_rbs + (unsigned)t.tail_rbs * (unsigned)t.split_k)), dim3(256 * panel_waves_k(RT)), lds,
-                       stream, x, qtile, sz, M, ldx, N, S_total, T_total, t);
+    const unsigned tail_wgs = (unsigned)t.col_wgs * (unsigned)t.tail_rbs, main_wgs = (unsigned)t.col_wgs * (unsigned)t.main_rbs;
+    const dim3 grid = main_wgs ? dim3(main_wgs + tail_wgs * (unsigned)t.split_k) : dim3(tail_wgs, (unsigned)t.split_k);
+    hipLaunchKernelGGL(kern, grid, dim3(256 * panel_waves_k(RT)), lds, stream, x, qtile, sz, M, ldx, N, S_total, T_total, t);
     return hipGetLastError() == hipSuccess ? GPTQ_HIP_OK : GPTQ_HIP_ERR_LAUNCH;
 }
 

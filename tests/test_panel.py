@@ -473,3 +473,11 @@ def test_calls_without_the_workspace_of_the_last_blocks_keep_the_panel_kernel():
                 q, clear = _lib.Plan(), ctypes.c_int()
                 assert lib.gptq_tiled_default_plan(M, K, N, bits, gs, 0, ctypes.c_size_t(have), ctypes.byref(q), ctypes.byref(clear)) == _lib.OK
                 assert q.as_dict() == p.as_dict()
+
+
+def test_plans_in_ranges_of_all_rows_keep_within_a_launch():
+    # the ranges lie along the grid's second dimension: what counts against 2^32 threads is one range's workgroups
+    for M, K, N, tr, rt, split, ok in ((1 << 25, 512, 64, False, 1, 8, True), (1 << 24, 4096, 128, False, 1, 16, True), ((1 << 28) - 32, 512, 32, False, 1, 8, True),
+                                       (1 << 28, 512, 32, False, 1, 8, False), (1 << 25, 64, 512, True, 1, 8, True)):
+        p = _lib.select_panel(M, K, N, 4, 32, False, tr, rt, split)
+        assert (p is not None) == ok and (not ok or p.split_k == split), (M, K, N)
