@@ -317,7 +317,8 @@ static int run_panel(const void *x, const void *qtile, const uint32_t *sz, const
     if (plan.waves_n != 4 || plan.waves_k != gptq::panel_waves_k(rt) || plan.block != 256 * plan.waves_k || plan.split_k < 1 || plan.k_chunk < 1 || plan.m_blocks < 1 ||
         plan.grid_x != (cols + gptq::kPanelCols - 1) / gptq::kPanelCols || plan.grid_y != plan.split_k ||
         plan.grid_z != plan.m_blocks || plan.m_blocks != (M + 32 * rt - 1) / (32 * rt) ||
-        plan.split_k != (S_total + plan.k_chunk - 1) / plan.k_chunk || plan.lds_bytes != gptq::panel_lds_bytes(bits, rt))
+        plan.split_k != (S_total + plan.k_chunk - 1) / plan.k_chunk ||
+        plan.lds_bytes < gptq::panel_lds_bytes(bits, rt) || plan.lds_bytes > 160 * 1024)   // (plans kept from a build that took more)
         return GPTQ_HIP_ERR_BAD_ARG;
     // K ranges for the row blocks from main on only
     const int main = gptq::panel_main_blocks(plan);

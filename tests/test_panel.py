@@ -481,3 +481,16 @@ def test_plans_in_ranges_of_all_rows_keep_within_a_launch():
                                        (1 << 28, 512, 32, False, 1, 8, False), (1 << 25, 64, 512, True, 1, 8, True)):
         p = _lib.select_panel(M, K, N, 4, 32, False, tr, rt, split)
         assert (p is not None) == ok and (not ok or p.split_k == split), (M, K, N)
+
+
+def test_plans_that_ask_for_more_lds_than_the_kernel_takes_are_accepted():
+    # (a plan kept from when the result took 132 KB to turn around; refused for its workspace only, so nothing is launched)
+    fake, null = ctypes.c_void_p(0x1000), ctypes.c_void_p(None)
+    for rt in (1, 2, 3):
+        p = _lib.select_panel(300, 2048, 512, 4, 128, False, False, rt, 2)
+        for lds, rc in ((p.lds_bytes, _lib.ERR_WORKSPACE), (135168, _lib.ERR_WORKSPACE), (p.lds_bytes - 4, _lib.ERR_BAD_ARG),
+                        (160 * 1024 + 4, _lib.ERR_BAD_ARG)):
+            p.lds_bytes = lds
+            assert _lib.lib().gptq_hip_gemm_tiled(fake, fake, fake, null, null, null, fake, null, 0, 300, 2048, 512, 4, 128, ctypes.byref(p),
+                                                  null) == rc, (rt, lds)
+            p = _lib.select_panel(300, 2048, 512, 4, 128, False, False, rt, 2)
