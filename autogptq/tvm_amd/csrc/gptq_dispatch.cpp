@@ -596,6 +596,20 @@ bool gptq::select_row_blocks(int M, int K, int N, int bits, int group_size, gptq
     return false;
 }
 
+// Nine to sixteen rows that the matmul kernel reads itself, without its pack pass, are its own again on long layers, whose K it cuts over CUs that
+// row blocks leave idle; with fewer bits or columns sooner (us at 9 / 16 rows, matmul / row blocks: 9216 x 64 int4 6.7 / 9.9 and 7.6 / 10.0,
+// 9216 x 2048 8.3 / 10.4 and 9.2 / 10.5, int3 7.5 / 10.7 and 8.1 / 10.8, 9216 x 4096 int4 10.4 / 10.9 and 11.6 / 10.8, int3 9.4 / 11.1 and
+// 10.7 / 11.2; 7680 x 2048 int4 8.3 / 9.0 and 9.0 / 9.0; 7168 x 2048 int4 8.7 / 8.5 and 9.9 / 8.5, int3 8.0 / 9.0 and 8.6 / 9.0; 8 bits 9216 x 64 7.0 /
+// 9.9, 9216 x 2048 9.9 / 10.5 and 10.8 / 10.6, 7680 x 1024 9.3 / 9.1 and 10.0 / 9.1; with a pack pass row blocks are level or ahead: 8704 x 2048 11.3 /
+// 10.1, 9216 x 512 with an activation order 10.7 / 10.7).
+static bool matmul_keeps(int M, int K, int N, int bits, int group_size, bool mapped)
+{
+    gptq_hip_plan plan;
+    if (K < 7168 || (bits >= 4 && (K == 7168 || N > (bits == 4 ? 2048 : 512)))) return false;
+    return gptq_hip_select_tiled(M, K, N, bits, group_size, &plan) == GPTQ_HIP_OK && plan.kernel == GPTQ_HIP_KERNEL_TILED &&
+           gptq::tiled_reads_x_directly(mapped, M, K, plan);
+}
+
 // Five to eight rows on the decode kernel: K up to 11008, and longer layers of few columns, which the matmul kernel cuts into many
 // K ranges (us at 5 to 8 rows, matmul / decode kernel: 14336 x 4096 int4 13.7 / 9.8, with an activation order 20.6 / 10.6, 12288 x 1024
 // 15.0 / 9.9, 16384 x 4096 14.7 / 12.2, 17408 x 2048 int3 21.6 / 12.7, 20480 x 2048 24.0 / 13.5, 20480 x 1024 19.1 / 10.6; 20480 x 4096 17.3 /
@@ -698,7 +712,9 @@ extern "C" int gptq::gptq_tiled_default_plan(int M, int K, int N, int bits, int 
     if (rc != GPTQ_HIP_OK) return rc;
     // row blocks need no workspace, but a call without the one that its size asks for stays refused
     gptq_hip_plan other;
-    if (plan->workspace_bytes <= have && select_row_blocks(M, K, N, bits, group_size, &other)) *plan = other;
+    if (plan->workspace_bytes <= have && !matmul_keeps(M, K, N, bits, group_size, act_order) &&
+        select_row_blocks(M, K, N, bits, group_size, &other))
+        *plan = other;
     if (plan->kernel == GPTQ_HIP_KERNEL_TILED_DECODE && (plan->flags & GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE) &&
         plan_tiled(M, K, N, bits, group_size, true, &other) == GPTQ_HIP_OK && !(other.flags & GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE)) {
         *clear = plan->workspace_bytes <= have;
@@ -1084,7 +1100,7 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
     };
     if (copies == GPTQ_HIP_COPY_TILED) {
         // the tiled copy is all the layer has: every M runs there
-        if (take_rows() || take_panel() || (tiled_ok && take_tiled())) return GPTQ_HIP_OK;
+        if ((!matmul_keeps(M, K, N, bits, group_size, act_order) && take_rows()) || take_panel() || (tiled_ok && take_tiled())) return GPTQ_HIP_OK;
         return GPTQ_HIP_ERR_UNSUPPORTED;
     }
     bool tiled = false;
@@ -1113,7 +1129,7 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
     // checkpoint tensors; without one 6.1 and 9.3; 4352 x 1408 int3 7.1 and 12.8, 6656 x 4096 int3 9.0 and 12.9, 7680 x 1536 int3 one group 9.6
     // and 12.5); from 8192 channels they leave a layer that has other copies to those (8192 x 4096: 9.8 us against 11.5 to 12.5, for a
     // copy more), and below 1024 columns, where a call costs its host time.
-    if (!past && (!theirs || (K < 8192 && N >= 1024)) && take_rows()) return GPTQ_HIP_OK;
+    if (!past && (theirs ? K < 8192 && N >= 1024 : !matmul_keeps(M, K, N, bits, group_size, act_order)) && take_rows()) return GPTQ_HIP_OK;
     if (!others && take_panel()) return GPTQ_HIP_OK;
     if (past) return GPTQ_HIP_OK;
     if (tiled && take_tiled()) return GPTQ_HIP_OK;

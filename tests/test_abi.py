@@ -632,3 +632,16 @@ def test_three_and_four_rows_past_the_table_leave_no_stream_plan():
                         assert (r.copy, r.plan.as_dict()) == (without.copy, without.plan.as_dict()), (M, K, N, bits, gs, act, kept)
                         stayed += without.plan.kernel == _lib.KERNEL_STREAM
     assert moved > 20 and stayed > 10
+
+
+def test_row_blocks_leave_long_layers_to_the_matmul_kernel_that_reads_x_itself():
+    tiled = _lib.COPY_TILED | _lib.COPY_TILED_PANEL
+    for M, K, N, bits, act, rows in ((9, 9216, 64, 4, False, False), (16, 9216, 2048, 4, False, False), (16, 9216, 4096, 3, False, False),
+                                     (9, 7680, 1024, 2, False, False), (9, 9216, 64, 8, False, False),
+                                     (9, 9216, 64, 4, True, True), (17, 9216, 64, 4, False, True), (9, 8704, 2048, 4, False, True),
+                                     (16, 9216, 4096, 4, False, True), (16, 9216, 1024, 8, False, True), (16, 6144, 64, 4, False, True)):
+        r = _lib.select_route(M, K, N, bits, 128, act, tiled)
+        assert (r.plan.kernel == _lib.KERNEL_TILED_DECODE) == rows, (M, K, N, bits, act)
+        assert default_plan(M, K, N, bits, 128, act, 1 << 40)[0].as_dict() == r.plan.as_dict()
+    # a layer with its other copies, which would run on those and not on the matmul kernel, keeps row blocks
+    assert _lib.select_route(12, 7680, 1536, 3, -1, False, _lib.COPY_CHECKPOINT | tiled).plan.kernel == _lib.KERNEL_TILED_DECODE
