@@ -401,9 +401,11 @@ static int plan_tiled_decode(int M, int K, int N, int bits, int group_size, bool
         // Layers of up to 16 columns per CU (N <= 4096), one and two rows, 2560 to 4096 channels: one workgroup of sixteen
         // waves per 16-column unit, all of K staged once per workgroup (waves_n = 2 marks this kernel), when that fits LDS.
         // Every CU then has work, but its workgroups are long in starting and its items cost more: the kernel below with
-        // eight waves per tile takes everything else (us, this / that: 2048 x 4096 at one / two / four rows 4.4 / 4.9 / 5.7 and
-        // 3.5 / 3.7 / 4.1, 1024 x 1024 one row 3.8 and 3.5, 2560 x 2560 groups of 32 4.5 and 4.4, 3584 x 3072 at four rows 5.9 and 4.9;
-        // at one and two rows level or ahead beyond: 3584 x 1024 groups of 32 4.4 and 4.9, 3584 x 3072 two rows 5.0 and 5.1).
+        // eight waves per tile takes everything else (us, this / that: 2048 x 4096 at one / two / four rows 4.2 / 4.7 / 5.5 and
+        // 3.2 / 3.4 / 3.9, 1024 x 1024 one row 3.9 and 3.1, 2560 x 2560 groups of 32 4.4 and 4.2, 3584 x 3072 at four rows 5.8 and 4.9).
+        // Beyond 2560 channels, at one and two rows, it is level or ahead with groups of 32 (3584 x 1024 4.2 / 4.8 and 4.6 / 4.9, 2592 x
+        // 4096 4.5 / 5.1 and 4.6 / 5.0); with groups of 128 it is behind (3072 x 4096 4.6 / 4.8 and 4.2 / 4.4, 3968 x 4096 int3 4.6 / 5.0 and 4.1 /
+        // 4.3), but its sums run over 32 positions where that one's pairs of blocks run over 64, with 1.4 times the error.
         const int mr = gptq::tiled_decode_rows(M);
         const int units = N / 16;
         const int nwg = units < gptq::kNumCUs ? units : gptq::kNumCUs;
@@ -434,8 +436,8 @@ static int plan_tiled_decode(int M, int K, int N, int bits, int group_size, bool
         const int tiles = N / 32;
         const int S_total = ceil_div(K, 64);
         int kw = tiles * 4 >= 1024 ? 4 : 8;
-        // up to 1024 channels four waves, but for one and two rows of 2 to 4 bits (1024 x 4096 int4 at four rows 3.3 us, eight waves
-        // 3.8; one row 3.6 and 3.5, int8 3.8 and 4.5; 1024 x 2048 at eight rows 3.5 and 3.9)
+        // up to 1024 channels four waves, but for one and two rows of 2 to 4 bits (1024 x 4096 int4 at four rows 3.0 us, eight waves
+        // 3.7; one row 3.6 and 3.3, int8 3.4 and 4.2; 1024 x 2048 at eight rows 3.4 and 3.7)
         if (S_total <= 16 && (M > 2 || bits == 8)) kw = 4;
         // and enough of them that a wave walks about sixteen blocks at most: a wave issues one instruction per
         // four clocks, so a long K wants more, shorter waves.  One row, us, kw = 4 / 8 / 16: 8192 x 8192
@@ -477,7 +479,7 @@ static int plan_tiled_decode(int M, int K, int N, int bits, int group_size, bool
             const int groups = (span - 1) / gs + 2 < ceil_div(K, gs) ? (span - 1) / gs + 2 : ceil_div(K, gs);
             const int lds = gptq::tiled_decode_lds_bytes(mr, span, groups, kw);
             // (all of the LDS where every workgroup has a CU to itself anyway: an uncut K saves the reduce pass, 8192 x 8192 at
-            // eight rows 13.1 -> 9.8 us, with an activation order 13.9 -> 10.4, 16384 x 8192 at four rows 19.6 -> 15.9)
+            // eight rows 13.1 -> 9.2 us, with an activation order 13.9 -> 9.8, 16384 x 8192 at four rows 19.6 -> 15.9)
             if (settled ? lds + (gptq::tiled_decode_centred(mr) ? (span / 32) * mr * 8 : 0) > 128 * 1024
                         : lds > ((tiles + halved) * split <= gptq::kNumCUs ? 160 : 128) * 1024)
                 continue;
@@ -567,11 +569,12 @@ int tiled_ranges(int at, bool wide, long long tiles, int S_total, int kwv, doubl
 // block, while those find a CU each and a block's x fits LDS (8 rows: K up to 9216, 16 rows: 4096).  A CU takes its x and
 // weights in at ~50 GB/s whatever the kernel; what this saves against the matmul kernel is the pack pass (a launch) and
 // the CUs that its 64 columns per workgroup leave idle.  us, graph replay, matmul or panel kernel / this (8 rows, else 16): 4096 x
-// 4096 int4 at 9 / 16 / 32 rows 11.6 / 10.4 / 12.5 and 6.0 / 6.1 / 8.1; 2048 x 2048 at 12 / 64 rows 8.8 / 8.5 and 4.2 / 5.5; 4096 x
-// 8192 at 16 rows 11.0-12.6 and 8.2-8.4; 8192 x 4096 at 16 rows 12.6, with an activation order 16.4, and 9.8, 10.0; 2048 x 4096
-// int8 at 32 rows 11.1 and 5.7.  One block more than CUs loses: every workgroup stages its x, and the second turn is as long as
-// the first (4096 x 11008 at 16 rows 11.5-13.1 and 14.0-14.6).
-// Four waves along K up to 1024 channels (1024 x 4096 at 32 rows 4.5 us, eight 5.1), eight beyond (2048 x 8192 at 16 rows 5.6, four 5.9).
+// 4096 int4 at 9 / 16 / 32 rows 9.1 / 10.3 / 11.7 and 5.9 / 6.0 / 8.0; 2048 x 2048 at 12 / 64 rows 7.3 / 9.0 and 4.1 / 5.3; 4096 x
+// 8192 at 16 rows 11.0-12.6 and 8.3-8.5; 8192 x 4096 at 16 rows 11.9, with an activation order 14.2, and 9.6, 10.0; 2048 x 4096
+// int8 at 32 rows 10.8 and 5.6; few workgroups: 3296 x 64 at 16 / 128 rows 8.6 / 9.1 and 5.4 / 5.4, 1024 x 32 at 128 rows 7.3 and 3.5.
+// One block more than CUs loses: every workgroup stages its x, and the second turn is as long as the first (4096 x 11008 at 16 rows
+// 11.4-12.7 and 13.7-14.3).
+// Four waves along K up to 1024 channels (1024 x 4096 at 32 rows 4.4 us, eight 5.1), eight beyond (2048 x 8192 at 16 rows 5.4, four 5.8).
 bool gptq::select_row_blocks(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
 {
     if (M <= kDecodeMaxRows || M > kRowBlocksMaxRows) return false;
@@ -611,18 +614,19 @@ static bool matmul_keeps(int M, int K, int N, int bits, int group_size, bool map
 }
 
 // Five to eight rows on the decode kernel: K up to 11008, and longer layers of few columns, which the matmul kernel cuts into many
-// K ranges (us at 5 to 8 rows, matmul / decode kernel: 14336 x 4096 int4 13.7 / 9.8, with an activation order 20.6 / 10.6, 12288 x 1024
-// 15.0 / 9.9, 16384 x 4096 14.7 / 12.2, 17408 x 2048 int3 21.6 / 12.7, 20480 x 2048 24.0 / 13.5, 20480 x 1024 19.1 / 10.6; 20480 x 4096 17.3 /
-// 18.0 and 16384 x 8192 21.6 / 23.8 stay).
+// K ranges (us at 8 rows, matmul / decode kernel: 14336 x 4096 int4 12.6 / 9.8, with an activation order 16.8 / 11.1, 16384 x 4096 13.5 /
+// 10.7, 17408 x 2048 int3 13.6 / 11.1, 20480 x 1024 16.4 / 10.5; level where the matmul kernel reads x itself: 12288 x 1024 8.0 / 8.0, 20480 x
+// 2048 10.7 / 10.6.  Beyond these LDS does not hold the longer half of x and K is cut as well: 20480 x 4096 15.6 / 18.7 and 16384 x 8192
+// 21.9 / 23.5 stay; 18432 channels are the longest of which eight rows of a half fit).
 static bool decode_takes(int K, int N) { return K <= 11008 || (K <= 18432 && N <= 4096) || (K <= 20480 && N <= 2048); }
 
 static int plan_tiled(int M, int K, int N, int bits, int group_size, bool settled, gptq_hip_plan *plan)
 {
     // Up to four rows the decode kernels (one 4-row matrix instruction set per lane block); five to eight rows the
     // workgroup-per-tile decode kernel with two sets, for K up to 11008 (us at 5 / 8 rows, int4, against the matmul
-    // kernel with one 32-row tile: 4096 x 11008 7.4 / 7.4 against 9.6 / 9.7, with an activation order 7.9 / 7.8
-    // against 14.0 / 14.2; 11008 x 4096 7.8 / 7.9 against 16.7 / 17.2, with an activation order 9.6 / 9.9 against
-    // 18.9 / 19.4; 4096 x 4096 4.7 / 4.8 against 9.4 / 9.5), and beyond for narrow layers (decode_takes).
+    // kernel with one 32-row tile: 4096 x 11008 7.3 / 7.6 against 9.7 / 9.9, with an activation order 7.8 / 7.9
+    // against 12.6 / 12.9; 11008 x 4096 7.7 / 7.7 against 13.9 / 14.1, with an activation order 9.4 / 9.7 against
+    // 14.4 / 14.8; 4096 x 4096 4.6 / 4.7 against 8.7 / 9.2), and beyond for narrow layers (decode_takes).
     if (M >= 1 && (M <= gptq::kDecodeSelectRows || (M <= gptq::kDecodeMaxRows && (settled ? K <= 11008 : decode_takes(K, N))))) {
         const int rc = plan_tiled_decode(M, K, N, bits, group_size, settled, plan);
         if (rc != GPTQ_HIP_ERR_UNSUPPORTED || !plan) return rc;
@@ -864,7 +868,7 @@ static int plan_panel(int M, int K, int N, int bits, int group_size, unsigned fl
         if (rt == 0 || split == 0) return GPTQ_HIP_ERR_UNSUPPORTED;
         // More than a turn of the chip: whole turns, and the last row blocks in K ranges that fill one turn more.  2000 rows of
         // 9216 x 9216 int3 (36 column positions): 13 blocks of 160 rows are 468 workgroups, 310 us; 8 of 256 rows are 288, 252 of them
-        // uncut and the last block in seven ranges 278.  Rarely the best plan by more than a little (7 % of 121 drawn calls of more than a turn
+        // uncut and the last block in seven ranges 276.  Rarely the best plan by more than a little (7 % of 121 drawn calls of more than a turn
         // gain over 3 %), hence the margin.
         if (row_tiles == 0 && split_k == 0 && tails) {
             double best_tail = 0.97 * best;
@@ -947,21 +951,20 @@ namespace {
 // Where the tiled kernels were measured faster than the ones that read the checkpoint layout or its channel-sorted
 // copy, on MI355X with the weights cold (us per call, graph replay, group size 128 unless said):
 //   * up to 4 rows, layers of up to 4096 columns (decode kernel with a workgroup per tile, per half of one along K from 4096
-//     channels, or per 16 columns): always.  4096 x 4096: 4.1-4.2 at one row, 5.2 at four, against 6.8-7.5
-//     and 7.8-10.5; 11008 x 4096: int4 9.0-9.4 / 11.5 against 13.5 / 15.3, int3 8.7 / 11.1 against 10.9 / 15.2;
+//     channels, or per 16 columns): always.  4096 x 4096: 4.0-4.2 at one row, 4.7-4.8 at four, against 6.8-7.5
+//     and 7.8-10.5; 11008 x 4096: int4 6.3 / 7.2 against 13.5 / 15.3, int3 5.8 / 6.4 against 10.9 / 15.2;
 //   * up to 4 rows, wider layers (a workgroup per 32 columns): K = 4096: one and two rows always, three and four up
-//     to 16384 columns (4096 x 11008 with an activation order, one / two / four rows: int4 7.8 / 8.1 / 9.8 against
-//     8.1 / 11.0 / 11.1, int3 7.3 / 7.7 / 9.7 against 7.7 / 10.2 / 10.3; 4096 x 22016 one row 9.7 / 10.3 against
-//     11.4 / 12.8).  Longer K, one and two rows: always (8192 x 8192 9.7 / 9.9 against 14.0 / 13.3, 8192 x 28672
+//     to 16384 columns (4096 x 11008 with an activation order, one / two / four rows: int4 6.4 / 6.7 / 7.2 against
+//     8.1 / 11.0 / 11.1, int3 5.8 / 6.5 / 6.8 against 7.7 / 10.2 / 10.3; 4096 x 22016 one row 9.7 / 10.3 against
+//     11.4 / 12.8).  Longer K, one and two rows: always (8192 x 8192 7.7 / 7.9 against 14.0 / 13.3, 8192 x 28672
 //     24.6 / 26.4 against 32.3 / 30.2, 28672 x 8192 25.1 / 31.7 against 50.1 / 39.2; 36864 x 9216 int3 with one
 //     group, K cut in six ranges: 26.7 against 37.3); three and four rows: K up to 6656, and
-//     up to 11008 for layers of up to 8192 columns (beyond, the four staged rows of x cost more than they save:
-//     8192 x 28672 41.9 against 30.4);
+//     up to 11008 for layers of up to 8192 columns (beyond, by the kernel that they would run on otherwise: decode_wins_past_table);
 //   * 5 to 8 rows, K up to 11008: the decode kernel with two sets of four rows (5 / 8 rows, int4 / int3, against the
-//     better of the other copies: 4096 x 11008 with an activation order 7.9 / 7.8 and 7.9 / 8.2 against 13.4 / 13.6
-//     and 12.5 / 12.6 on the sorted copy, without one 7.4 / 7.4 against 9.6 / 9.7 on the matmul kernel; 11008 x 4096 with
-//     an activation order 9.6 / 9.9 and 9.1 / 9.6 against 15.8 / 16.0 and 16.4 / 16.9, without one 7.8 / 7.9 against
-//     13.1; 4096 x 4096 4.7 / 4.8 against 9.9, with an activation order 5.5 / 5.4 against 10.9 (int3 12.3));
+//     better of the other copies: 4096 x 11008 with an activation order 7.8 / 7.9 and 7.9 / 8.1 against 13.4 / 13.6
+//     and 12.5 / 12.6 on the sorted copy, without one 7.3 / 7.6 against 9.7 / 9.9 on the matmul kernel; 11008 x 4096 with
+//     an activation order 9.4 / 9.7 and 9.0 / 9.4 against 15.8 / 16.0 and 16.4 / 16.9, without one 7.7 / 7.7 against
+//     13.1; 4096 x 4096 4.6 / 4.7 against 9.9, with an activation order 5.3 / 5.3 against 10.9 (int3 12.3));
 //   * 5 to 16 rows otherwise: only layers without an activation order, K up to 4096 and more than 4096 columns (the matmul
 //     kernel then reads x itself, one launch: 4096 x 11008 int4, 5 / 8 / 16 rows: 10.6 / 10.7 / 11.5 against 11.2 /
 //     11.3 / 12.5; int3 from nine rows); with an activation order the pack pass makes it 14.6 against 13.4 at 8 rows;
@@ -1038,8 +1041,8 @@ bool sorted_plan(int M, int K, int N, int bits, int group_size, gptq_hip_plan *p
 }
 
 // Three and four rows of layers past that table that would run on GROUPED, since the decode kernel takes the zero point off the codes
-// and stages an activation order in whole positions (us, against GROUPED on the better of the other copies: 8192 x 28672 int4 25.4 /
-// 24.1 with / without an order against 30.1 / 27.7, int3 21.8 / 20.2 against 33.3 / 30.9; 11008 x 11008 int3 16.2 / 13.8 against 25.6 / 23.0;
+// and stages an activation order in whole positions (us, against GROUPED on the better of the other copies: 8192 x 28672 int4 25.8 /
+// 23.7 with / without an order against 30.1 / 27.7, int3 21.8 / 20.2 against 33.3 / 30.9; 11008 x 11008 int3 16.2 / 13.4 against 25.6 / 23.0;
 // 4096 x 22016 8.6-10.5 against 13.6-15.9; 2048 x 33632 int3 7.7 against 14.6; 1792 x 19968 6.0 against 12.5; 2816 x 32608 11.7 against 23.0).  Both scale the
 // exact products of the codes group by group.  Layers whose small groups or length put them on STREAM stay there, though they would gain as
 // much (13824 x 5120 11 against 17): it multiplies the weights as the reference rounds them, and the two differ by that rounding, 1.7e-4.
@@ -1125,9 +1128,9 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
     // ones with an order (0.93 to 1.05 x), and no reason for another copy; on 4-bit layers with one it is ahead (0.86 to 1.38, 1.12).
     const bool theirs = !tiled && M <= 16 && fused_bits && (copies & (GPTQ_HIP_COPY_CHECKPOINT | GPTQ_HIP_COPY_SORTED));
     const bool others = theirs && !(act && bits == 4);
-    // Row blocks are ahead of the kernels on every copy (16 rows of 4096 x 4096 int4 with an activation order 6.0 us, 10.7 on the
-    // checkpoint tensors; without one 6.1 and 9.3; 4352 x 1408 int3 7.1 and 12.8, 6656 x 4096 int3 9.0 and 12.9, 7680 x 1536 int3 one group 9.6
-    // and 12.5); from 8192 channels they leave a layer that has other copies to those (8192 x 4096: 9.8 us against 11.5 to 12.5, for a
+    // Row blocks are ahead of the kernels on every copy (16 rows of 4096 x 4096 int4 with an activation order 6.1 us, 10.7 on the
+    // checkpoint tensors; without one 6.0 and 9.3; 4352 x 1408 int3 6.7 and 12.8, 6656 x 4096 int3 9.0 and 12.9, 7680 x 1536 int3 one group 9.1
+    // and 12.5); from 8192 channels they leave a layer that has other copies to those (8192 x 4096: 9.6 us against 11.5 to 12.5, for a
     // copy more), and below 1024 columns, where a call costs its host time.
     if (!past && (theirs ? K < 8192 && N >= 1024 : !matmul_keeps(M, K, N, bits, group_size, act_order)) && take_rows()) return GPTQ_HIP_OK;
     if (!others && take_panel()) return GPTQ_HIP_OK;

@@ -191,7 +191,9 @@ inline bool tiled_qualifies(int K, int N, int bits, int gs)
 // `span` positions of `groups` groups
 static const int kDecodeMaxRows = 8;      // rows the decode kernel of the tiled format takes (the 16-column kernel: 4)
 // channels up to which five to eight rows run on the products of the codes, scaled per group; the weights of longer layers are
-// rounded first, as the matmul kernel that used to take them does (the two differ by the rounding of the weights, 1.7e-4)
+// rounded first, as the reference rounds them and as the matmul kernel does, which those calls ran on: error against the reference's
+// weights in 64 bits 2.1e-4, 2.6e-4 with the products.  That is the line: no call's results are further off than they were.  (It costs
+// 0.5 to 0.7 us; shorter layers have run on the products since their rows came to this kernel.)
 constexpr int kDecodeUnroundedK = 11008;
 constexpr int kRowBlocksMaxRows = 128;   // rows it takes in blocks of 8 or 16 along grid_z
 constexpr int kDecodeSelectRows = 4;   // rows up to which gptq_hip_select_tiled chooses it
@@ -255,13 +257,14 @@ inline bool tiled_decode_can_halve(int wave_steps, int split_k, int waves_k, int
 // Layers of so few tiles that two workgroups per tile still find a CU each (N <= 4096), with K long enough for
 // two ranges (4096 channels): EVERY tile is halved, which gives every CU work like the 16-column kernel does, at
 // the lower cost per weight of this one (one / four / eight rows, us, against the 16-column kernel, which has no
-// eight-row form: there the comparison is with whole tiles.  4096 x 4096 int4 4.11 / 5.20 / 6.42 against 4.43 / 5.86 /
-// 7.29, int3 with an activation order 4.05 / 5.96 / 9.21 against 4.40 / 6.47 / 10.0; 4096 x 2048 3.59 / 4.81 / 6.32 against
-// 4.13 / 5.58 / 7.10; 4096 x 1024 3.48 / 4.70 / 6.23 against 4.04 / 5.49 / 7.06; 6144 x 4096 4.79 / 6.04 / 7.87 against 5.45 /
-// 7.21 / 8.52; 11008 x 4096 int3 8.4 / 11.2 against 9.6 / 13.6 at one / four rows.  At 2048 channels the halves are four
-// blocks per wave: 2048 x 4096 3.93 / 5.17 / 6.31 against 3.98 / 5.33 / 5.72, 2048 x 2048 3.78 / 5.03 / 6.25 against
-// 3.79 / 5.19 / 5.66: level up to four rows, a loss at eight, so shorter layers keep whole tiles of eight waves, one and two
-// rows of more than 2560 channels the 16-column kernel).
+// eight-row form: there the comparison is with whole tiles.  4096 x 4096 int4 4.23 / 4.76 / 4.63 against 4.68 / 5.97 /
+// 5.48, int3 with an activation order 4.19 / 4.66 / 5.10 against 4.53 / 6.59 / 5.33; 4096 x 2048 3.83 / 4.26 / 4.45 against
+// 4.39 / 5.74 / 5.39; 4096 x 1024 3.73 / 4.23 / 4.50 against 4.22 / 5.67 / 5.47; 6144 x 4096 4.87 / 5.44 / 5.70 against 5.39 /
+// 7.19 / 6.76; 11008 x 4096 int3 5.7 / 6.4 against 7.7 / 9.7 at one / four rows.  At 2048 channels the halves are two
+// blocks per wave and lose: 2048 x 4096 3.88 / 4.35 / 4.49 against 3.32 / 3.80 / 3.90, 2048 x 2048 at four / eight rows 4.00 / 4.25 against 3.58 /
+// 3.82 of whole tiles of eight waves, which shorter layers keep, one and two rows of more than 2560 channels the 16-column kernel.  Three
+// to eight rows from 3072 channels would gain: 3072 x 4096 4.41 / 4.60 against 4.53 / 4.88, 3584 x 2048 with an activation order 4.62 /
+// 5.03 against 5.10 / 5.60).
 inline bool tiled_decode_halves_all(int tiles, int S_total) { return 2 * tiles <= kNumCUs && S_total >= 64; }
 inline int tiled_decode_halved(int tiles, int wave_steps, int split_k, int waves_k, int S_total, int group_size)
 {

@@ -166,7 +166,7 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     // (without a map the channels of the range are the range itself)
     const int k8_lo = mapped ? 0 : p0 / 8, k8_hi = mapped ? p.K / 8 : min(p0 + span, p.K) / 8;
     // passes over x kept in registers (eight rows: 32 registers a pass; a second one only shortens the way of workgroups of
-    // four waves without an activation order, 4096 x 11008 7.55 -> 7.29 us, and costs 0.2 to 0.5 us elsewhere)
+    // four waves without an activation order, 4096 x 11008 7.55 -> 7.29 us, and costs up to 0.8 us elsewhere: 2048 x 4096 3.9 -> 4.7)
     constexpr int QP = MR == 16 || (MR == 8 && (PM || KW > 4)) ? 1 : 2;
     u4 kq[QP];
     h8 xq[QP][MR];
