@@ -489,7 +489,7 @@ extern "C" int gptq_hip_gemm_tiled_transposed(const void *gy, const void *qtile_
     gptq_hip_plan chosen;
     if (!plan) {
         int rc = gptq::gptq_panel_plan_within(M, K, N, bits, group_size, GPTQ_HIP_PANEL_TRANSPOSED | (xsrc ? GPTQ_HIP_PANEL_ACT_ORDER : 0),
-                                              workspace ? workspace_bytes : 0, &chosen);
+                                              workspace && aligned(workspace, 16) ? workspace_bytes : 0, &chosen);
         if (rc != GPTQ_HIP_OK)
             rc = gptq_hip_select_tiled_transposed(M, K, N, bits, group_size, &chosen);
         if (rc != GPTQ_HIP_OK) return rc;

@@ -494,3 +494,24 @@ def test_plans_that_ask_for_more_lds_than_the_kernel_takes_are_accepted():
             assert _lib.lib().gptq_hip_gemm_tiled(fake, fake, fake, null, null, null, fake, null, 0, 300, 2048, 512, 4, 128, ctypes.byref(p),
                                                   null) == rc, (rt, lds)
             p = _lib.select_panel(300, 2048, 512, 4, 128, False, False, rt, 2)
+
+
+@pytest.mark.gpu
+def test_gradients_without_ranges_need_no_aligned_workspace(dev):
+    # the plan with ranges for the last row blocks wants 16-byte aligned memory; a call whose memory is not runs on the plan that needs none
+    M, K, N, bits = 2000, 9216, 9216, 3
+    lib, ptr, null = _lib.lib(), ops._ptr, ctypes.c_void_p(None)
+    assert _lib.select_panel(M, K, N, bits, -1, False, True).workspace_bytes > 0
+    gen = torch.Generator(dev).manual_seed(3)
+    qtile_t = torch.randint(-2 ** 31, 2 ** 31 - 1, (lib.gptq_hip_tiled_transposed_bytes(K, N, bits) // 4,), dtype=torch.int32, device=dev, generator=gen)
+    szt = torch.tensor([0.01, 4.0], dtype=torch.float16, device=dev).view(torch.int32).repeat(
+        lib.gptq_hip_tiled_transposed_table_bytes(K, N, -1) // 4)
+    gy = torch.randn(M, N, dtype=torch.float16, device=dev, generator=gen)
+    memory = torch.zeros(1 << 26, dtype=torch.uint8, device=dev)
+    got = []
+    for ws, nbytes in ((null, 0), (ctypes.c_void_p(memory.data_ptr() + 8), memory.numel() - 8)):
+        gx = torch.zeros(M, K, dtype=torch.float16, device=dev)
+        assert lib.gptq_hip_gemm_tiled_transposed(ptr(gy), ptr(qtile_t), ptr(szt), null, ptr(gx), ws, nbytes, M, K, N, bits, -1, None,
+                                                  ops._stream(dev)) == _lib.OK
+        got.append(gx)
+    assert torch.equal(*got) and bool(got[0].any())
