@@ -868,13 +868,17 @@ static int plan_panel(int M, int K, int N, int bits, int group_size, unsigned fl
         if (rt == 0 || split == 0) return GPTQ_HIP_ERR_UNSUPPORTED;
         // More than a turn of the chip: whole turns, and the last row blocks in K ranges that fill one turn more.  2000 rows of
         // 9216 x 9216 int3 (36 column positions): 13 blocks of 160 rows are 468 workgroups, 310 us; 8 of 256 rows are 288, 252 of them
-        // uncut and the last block in seven ranges 276.  Rarely the best plan by more than a little (7 % of 121 drawn calls of more than a turn
-        // gain over 3 %), hence the margin.
+        // uncut and the last block in seven ranges 276.  Where the model gives such a plan a tenth, it is never behind: 64 of 220 drawn plans
+        // of this kind, 9 % faster on the mean, the least of them level.  Between 0.90 and 0.94 of the other plan's modelled time a fifth of
+        // 62 were 1 to 12 % slower (1676 rows of 11904 x 8992, gradient, 294 -> 330), and their partial sums take memory.  Nor do they
+        // leave one wave group (five row tiles and more) for two, where the model flatters the shorter blocks: 21 of 56 were slower, all of the
+        // 8-bit ones (506 rows of 7936 x 19392 165 -> 200).
         if (row_tiles == 0 && split_k == 0 && tails) {
-            double best_tail = 0.97 * best;
+            double best_tail = 0.9 * best;
+            const int groups = gptq::panel_waves_k(rt);
             for (int r = 1; r <= gptq::kPanelMaxTiles; r++) {
                 const int blocks = ceil_div(M, 32 * r);
-                if (!gptq::panel_addresses(r, red)) continue;
+                if (!gptq::panel_addresses(r, red) || gptq::panel_waves_k(r) > groups) continue;
                 const long long most = ((long long)col_wgs * blocks - 1) / 256;   // whole turns (one or two fewer for a longer tail)
                 for (long long turns = most > 2 ? most - 2 : 1; turns <= most; turns++) {
                     const int m = (int)(turns * 256 / col_wgs);
