@@ -311,8 +311,8 @@ constexpr int panel_lds_bytes(int bits, int rt)
 }
 // The kernel addresses the rows of a workgroup with 31 bits (bit 31 of an offset marks what lies outside)
 constexpr bool panel_addresses(int rt, int red) { return 32LL * rt * red * 2 < (1LL << 31); }
-// and a launch has less than 2^32 threads along its first dimension (K ranges of all rows lie along the second, those of the rows after
-// the first `main` blocks behind them), the pass that puts a gradient's rows in order included (256 for each of them)
+// and a launch has less than 2^32 threads, the pass that puts a gradient's rows in order included (256 for each of them).  Row blocks
+// that are all in K ranges can go in several launches (launch_panel), so their ranges do not count
 constexpr bool panel_launches(long long col_wgs, long long m_blocks, long long main, long long split_k, int block, long long ordered_rows)
 {
     return col_wgs * (main > 0 ? main + (m_blocks - main) * split_k : m_blocks) * block < (1LL << 32) && ordered_rows * 256 < (1LL << 32);

@@ -188,15 +188,14 @@ __global__ __launch_bounds__(256 * panel_waves_k(RT)) void panel_kernel(const _F
     // and what is left of the rows spread over one turn more.
     // XCD-aware order: workgroups are dealt to the XCDs round robin, so id % 8 names the XCD; each takes a
     // contiguous run of the tile order, in which groups of four row blocks walk the columns together
-    // (K ranges of all rows lie along the grid's second dimension, those of the last row blocks behind the whole ones)
-    int rb, cb, split = blockIdx.y;
+    int rb, cb, split = 0;
     const int n_main = t.col_wgs * t.main_rbs;
     const bool tail_wg = (int)blockIdx.x >= n_main;
     const bool ranges = tail_wg && t.split_k > 1;
     {
         const uint32_t row_wgs = tail_wg ? t.tail_rbs : t.main_rbs, nwg = t.col_wgs * row_wgs;
         uint32_t id = blockIdx.x - (tail_wg ? n_main : 0);
-        if (ranges && n_main > 0) split = (int)panel_div(id, nwg, t.tail_magic), id -= split * nwg;
+        if (ranges) split = (int)panel_div(id, nwg, t.tail_magic), id -= split * nwg;
         const uint32_t q = nwg / 8, r = nwg % 8, xcd = id % 8, i = id / 8;
         const uint32_t lin = xcd * q + min(xcd, r) + i;
         const uint32_t per = 4 * t.col_wgs, grp = panel_div(lin, per, t.column_group_magic), in = lin - grp * per;
@@ -658,9 +657,8 @@ static int launch_panel_one(const _Float16 *x, const char *qtile, const uint32_t
     auto kern = panel_kernel<BITS, RT, TRANS>;
     const int lds = panel_lds_bytes(BITS, RT);
     if (!allow_lds(kern, lds)) return GPTQ_HIP_ERR_LAUNCH;
-    const unsigned tail_wgs = (unsigned)t.col_wgs * (unsigned)t.tail_rbs, main_wgs = (unsigned)t.col_wgs * (unsigned)t.main_rbs;
-    const dim3 grid = main_wgs ? dim3(main_wgs + tail_wgs * (unsigned)t.split_k) : dim3(tail_wgs, (unsigned)t.split_k);
-    hipLaunchKernelGGL(kern, grid, dim3(256 * panel_waves_k(RT)), lds, stream, x, qtile, sz, M, ldx, N, S_total, T_total, t);
+    hipLaunchKernelGGL(kern, dim3((unsigned)t.col_wgs * ((unsigned)t.main_rbs + (unsigned)t.tail_rbs * (unsigned)t.split_k)), dim3(256 * panel_waves_k(RT)), lds,
+                       stream, x, qtile, sz, M, ldx, N, S_total, T_total, t);
     return hipGetLastError() == hipSuccess ? GPTQ_HIP_OK : GPTQ_HIP_ERR_LAUNCH;
 }
 
@@ -692,6 +690,22 @@ int launch_panel(const void *x, const void *qtile, const uint32_t *sz, const int
 {
     hipStream_t stream = (hipStream_t)stream_v;
     const int K_red = trans ? N : K, N_out = trans ? K : N;
+    // Workgroups that with all their ranges are past the 2^32 threads of a launch: so many row blocks at a time (ranges along a second
+    // dimension of the grid made every call of the kernel slower, 13 rows of 12640 x 30784 int3 51.6 -> 53.9 us, 1176 of 5120 x 3296 48.4 -> 49.1)
+    const unsigned long long block_threads = (unsigned long long)plan.grid_x * plan.split_k * plan.block;
+    const int most = (int)(((1ull << 32) - 1) / block_threads), block_rows = 32 * plan.row_tiles;
+    if (plan.m_blocks > most && panel_main_blocks(plan) == 0) {
+        for (int b = 0; b < plan.m_blocks; b += most) {
+            gptq_hip_plan part = plan;
+            part.m_blocks = part.grid_z = plan.m_blocks - b < most ? plan.m_blocks - b : most;
+            const size_t row0 = (size_t)b * block_rows;
+            const int rows = (int)((size_t)M - row0 < (size_t)most * block_rows ? M - row0 : (size_t)most * block_rows);
+            const int rc = launch_panel((const _Float16 *)x + row0 * K_red, qtile, sz, xsrc, bias, (_Float16 *)y + row0 * N_out,
+                                        xsrc ? (_Float16 *)xs + row0 * K : xs, partial, rows, K, N, bits, group_size, trans, part, stream_v);
+            if (rc != GPTQ_HIP_OK) return rc;
+        }
+        return GPTQ_HIP_OK;
+    }
     if (!trans && xsrc) {
         const int rc = launch_panel_gather(x, xsrc, xs, M, K, stream);
         if (rc != GPTQ_HIP_OK) return rc;

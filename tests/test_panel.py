@@ -476,7 +476,7 @@ def test_calls_without_the_workspace_of_the_last_blocks_keep_the_panel_kernel():
 
 
 def test_plans_in_ranges_of_all_rows_keep_within_a_launch():
-    # the ranges lie along the grid's second dimension: what counts against 2^32 threads is one range's workgroups
+    # past 2^32 threads with all their ranges the row blocks go in several launches: what counts is one range's workgroups
     for M, K, N, tr, rt, split, ok in ((1 << 25, 512, 64, False, 1, 8, True), (1 << 24, 4096, 128, False, 1, 16, True), ((1 << 28) - 32, 512, 32, False, 1, 8, True),
                                        (1 << 28, 512, 32, False, 1, 8, False), (1 << 25, 64, 512, True, 1, 8, True)):
         p = _lib.select_panel(M, K, N, 4, 32, False, tr, rt, split)
@@ -515,3 +515,29 @@ def test_gradients_without_ranges_need_no_aligned_workspace(dev):
                                                   ops._stream(dev)) == _lib.OK
         got.append(gx)
     assert torch.equal(*got) and bool(got[0].any())
+
+
+@pytest.mark.gpu
+def test_panel_ranges_past_the_threads_of_one_launch(dev):
+    # 2^32 threads with all eight ranges, so two launches, the second of a single row block.  Rows repeat, and so must the results
+    M, K, N, bits, gs, some = 1 << 25, 512, 32, 4, 32, 4096
+    if torch.cuda.mem_get_info(dev)[0] < 100 << 30:
+        pytest.skip("wants 70 GB")
+    L = layer(9871, K, N, bits, gs, False, M=some)
+    D = to_dev(L, dev)
+    qtile, sz, _, _ = ops.tile_prepare(D["qweight"], D["qzeros"], D["scales"], None, bits, gs)
+
+    def product(x):
+        plan, y = _lib.select_panel(x.shape[0], K, N, bits, gs, False, False, 1, 8), torch.zeros(x.shape[0], N, dtype=torch.float16, device=dev)
+        ws = torch.zeros(plan.workspace_bytes, dtype=torch.uint8, device=dev)
+        null = ctypes.c_void_p(None)
+        assert _lib.lib().gptq_hip_gemm_tiled(ops._ptr(x), ops._ptr(qtile), ops._ptr(sz), null, null, null, ops._ptr(y), ops._ptr(ws), ws.numel(),
+                                              x.shape[0], K, N, bits, gs, ctypes.byref(plan), ops._stream(dev)) == _lib.OK
+        return y
+
+    want = product(D["x"])
+    assert_tight(want, expected_output(L), "in one launch")
+    y = product(D["x"].repeat(M // some, 1))
+    assert bool((y.view(M // some, some, N) == want).all())
+    del y
+    torch.cuda.empty_cache()
