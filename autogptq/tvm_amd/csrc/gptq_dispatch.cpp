@@ -406,13 +406,17 @@ static int plan_tiled_decode(int M, int K, int N, int bits, int group_size, bool
         // Beyond 2560 channels, at one and two rows, it is level or ahead with groups of 32 (3584 x 1024 4.2 / 4.8 and 4.6 / 4.9, 2592 x
         // 4096 4.5 / 5.1 and 4.6 / 5.0); with groups of 128 it is behind (3072 x 4096 4.6 / 4.8 and 4.2 / 4.4, 3968 x 4096 int3 4.6 / 5.0 and 4.1 /
         // 4.3), but its sums run over 32 positions where that one's pairs of blocks run over 64, with 1.4 times the error.
+        // One row of 2 and 3 bits in groups of no whole 128 stays here from 2048 channels on already, where that kernel's waves have five blocks, one
+        // past what they ask for at first, and an epilogue for each (2304 x 1024 int3 groups of 64 with an activation order 3.85 and 4.11, 2496 x
+        // 2496 3.95 and 4.12, 2560 x 2560 int2 4.03 and 4.17; 4 bits and two rows are level or behind here, groups of 128 4 to 10 % behind).
         const int mr = gptq::tiled_decode_rows(M);
         const int units = N / 16;
         const int nwg = units < gptq::kNumCUs ? units : gptq::kNumCUs;
         const int upw = ceil_div(units, nwg);
         const long long lds = gptq::tiled_decode16_lds_bytes(mr, K, K / gs, upw);
         // (long K: the kernel below with every tile halved, see tiled_decode_halves_all)
-        if (M <= 2 && K > 2560 && upw == 1 && lds <= 128 * 1024 && !gptq::tiled_decode_halves_all(N / 32, ceil_div(K, 64))) {
+        const bool longer = K > 2560 || (K > 2048 && M == 1 && bits <= 3 && gs % 128 != 0);
+        if (M <= 2 && longer && upw == 1 && lds <= 128 * 1024 && !gptq::tiled_decode_halves_all(N / 32, ceil_div(K, 64))) {
             plan->kernel = GPTQ_HIP_KERNEL_TILED_DECODE;
             plan->row_tiles = mr;
             plan->m_blocks = 1;

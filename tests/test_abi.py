@@ -645,3 +645,10 @@ def test_row_blocks_leave_long_layers_to_the_matmul_kernel_that_reads_x_itself()
         assert default_plan(M, K, N, bits, 128, act, 1 << 40)[0].as_dict() == r.plan.as_dict()
     # a layer with its other copies, which would run on those and not on the matmul kernel, keeps row blocks
     assert _lib.select_route(12, 7680, 1536, 3, -1, False, _lib.COPY_CHECKPOINT | tiled).plan.kernel == _lib.KERNEL_TILED_DECODE
+
+
+def test_one_row_of_few_bits_in_small_groups_keeps_the_16_column_kernel():
+    for M, K, N, bits, gs, columns16 in ((1, 2080, 1024, 3, 32, True), (1, 2560, 4096, 2, 64, True), (1, 2560, 2560, 3, -1, False), (1, 2048, 1024, 3, 64, False),
+                                         (1, 2496, 2496, 4, 64, False), (2, 2496, 2496, 3, 64, False), (1, 2560, 1024, 3, 128, False),
+                                         (1, 2592, 1024, 4, 32, True), (3, 2592, 1024, 3, 32, False)):
+        assert (_lib.select_tiled(M, K, N, bits, gs).waves_n == 2) == columns16, (M, K, N, bits, gs)
