@@ -402,7 +402,7 @@ static int plan_tiled_decode(int M, int K, int N, int bits, int group_size, bool
         // waves per 16-column unit, all of K staged once per workgroup (waves_n = 2 marks this kernel), when that fits LDS.
         // Every CU then has work, but its workgroups are long in starting and its items cost more: the kernel below with
         // eight waves per tile takes everything else (us, this / that: 2048 x 4096 at one / two / four rows 4.2 / 4.7 / 5.5 and
-        // 3.2 / 3.4 / 3.9, 1024 x 1024 one row 3.9 and 3.1, 2560 x 2560 groups of 32 4.4 and 4.2, 3584 x 3072 at four rows 5.8 and 4.9).
+        // 3.2 / 3.4 / 3.5, 1024 x 1024 one row 3.9 and 2.7, 2560 x 2560 groups of 32 4.4 and 4.2, 3584 x 3072 at four rows 5.8 and 4.9).
         // Beyond 2560 channels, at one and two rows, it is level or ahead with groups of 32 (3584 x 1024 4.2 / 4.8 and 4.6 / 4.9, 2592 x
         // 4096 4.5 / 5.1 and 4.6 / 5.0); with groups of 128 it is behind (3072 x 4096 4.6 / 4.8 and 4.2 / 4.4, 3968 x 4096 int3 4.6 / 5.0 and 4.1 /
         // 4.3), but its sums run over 32 positions where that one's pairs of blocks run over 64, with 1.4 times the error.
@@ -440,8 +440,8 @@ static int plan_tiled_decode(int M, int K, int N, int bits, int group_size, bool
         const int tiles = N / 32;
         const int S_total = ceil_div(K, 64);
         int kw = tiles * 4 >= 1024 ? 4 : 8;
-        // up to 1024 channels four waves, but for one and two rows of 2 to 4 bits (1024 x 4096 int4 at four rows 3.0 us, eight waves
-        // 3.7; one row 3.6 and 3.3, int8 3.4 and 4.2; 1024 x 2048 at eight rows 3.4 and 3.7)
+        // up to 1024 channels four waves, but for one and two rows of 2 to 4 bits (1024 x 4096 int4 at four rows 2.9 us, eight waves
+        // 3.3; one row 3.2 and 3.0, int8 3.2 and 3.6; 1024 x 2048 at eight rows 3.2 and 3.4)
         if (S_total <= 16 && (M > 2 || bits == 8)) kw = 4;
         // and enough of them that a wave walks about sixteen blocks at most: a wave issues one instruction per
         // four clocks, so a long K wants more, shorter waves.  One row, us, kw = 4 / 8 / 16: 8192 x 8192
@@ -872,9 +872,9 @@ static int plan_panel(int M, int K, int N, int bits, int group_size, unsigned fl
         if (rt == 0 || split == 0) return GPTQ_HIP_ERR_UNSUPPORTED;
         // More than a turn of the chip: whole turns, and the last row blocks in K ranges that fill one turn more.  2000 rows of
         // 9216 x 9216 int3 (36 column positions): 13 blocks of 160 rows are 468 workgroups, 310 us; 8 of 256 rows are 288, 252 of them
-        // uncut and the last block in seven ranges 276.  Where the model gives such a plan a tenth, it is never behind: 64 of 220 drawn plans
-        // of this kind, 9 % faster on the mean, the least of them level.  Between 0.90 and 0.94 of the other plan's modelled time a fifth of
-        // 62 were 1 to 12 % slower (1676 rows of 11904 x 8992, gradient, 294 -> 330), and their partial sums take memory.  Nor do they
+        // uncut and the last block in seven ranges 276.  Where the model gives such a plan a tenth, two of 144 drawn ones were behind (by 1 and
+        // 4 %), all of them 8 % faster on the mean.  Between 0.90 and 0.94 of the other plan's modelled time a fifth of 62 were 1 to 12 %
+        // slower (1676 rows of 11904 x 8992, gradient, 294 -> 330), and their partial sums take memory.  Nor do they
         // leave one wave group (five row tiles and more) for two, where the model flatters the shorter blocks: 21 of 56 were slower, all of the
         // 8-bit ones (506 rows of 7936 x 19392 165 -> 200).
         if (row_tiles == 0 && split_k == 0 && tails) {

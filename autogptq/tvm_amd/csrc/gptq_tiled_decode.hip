@@ -34,7 +34,8 @@ namespace gptq {
 // take it off: with the sums, whose pairs of blocks would make the error 1.4 times that of the 16-column kernel, which ran these layers
 // (1024 x 1024 int4 7.7e-6, 5.5e-6 there; this form 7.7e-8), / this form, us: 1024 x 1024 one / two rows 3.52 / 2.95 and 3.55 / 3.06, groups of 32 3.77 /
 // 3.42, 2048 x 4096 3.29 / 3.31 and 3.50 / 3.44, 2560 x 2560 with an activation order 4.12 / 3.94, 2560 x 4096 two rows of groups of 32 4.58 /
-// 4.33; 4096 x 4096 level, 4096 x 11008 with an activation order 6.27 / 6.63.
+// 4.33; 4096 x 4096 level, 4096 x 11008 with an activation order 6.27 / 6.63; both before short ranges had a way without requests, with which
+// 1024 x 1024 takes 2.7 and 2.8).
 // Either way, like GROUPED and unlike the TILED matmul, this does not reproduce the fp16 rounding of each dequantised
 // weight: products are exact, sums are fp32.
 // 8-bit layers instead dequantise every weight in registers, as the matmul does (tiled_decode_exact), and add
