@@ -35,7 +35,7 @@ namespace gptq {
 // (1024 x 1024 int4 7.7e-6, 5.5e-6 there; this form 7.7e-8), / this form, us: 1024 x 1024 one / two rows 3.52 / 2.95 and 3.55 / 3.06, groups of 32 3.77 /
 // 3.42, 2048 x 4096 3.29 / 3.31 and 3.50 / 3.44, 2560 x 2560 with an activation order 4.12 / 3.94, 2560 x 4096 two rows of groups of 32 4.58 /
 // 4.33; 4096 x 4096 level, 4096 x 11008 with an activation order 6.27 / 6.63; both before short ranges had a way without requests, with which
-// 1024 x 1024 takes 2.7 and 2.8).
+// 1024 x 1024 takes 2.7 and 2.8.
 // Either way, like GROUPED and unlike the TILED matmul, this does not reproduce the fp16 rounding of each dequantised
 // weight: products are exact, sums are fp32.
 // 8-bit layers instead dequantise every weight in registers, as the matmul does (tiled_decode_exact), and add
@@ -167,8 +167,10 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     // (without a map the channels of the range are the range itself)
     const int k8_lo = mapped ? 0 : p0 / 8, k8_hi = mapped ? p.K / 8 : min(p0 + span, p.K) / 8;
     // passes over x kept in registers (eight rows: 32 registers a pass; a second one only shortens the way of workgroups of
-    // four waves without an activation order, 4096 x 11008 7.55 -> 7.29 us, and costs up to 0.8 us elsewhere: 2048 x 4096 3.9 -> 4.7)
-    constexpr int QP = MR == 16 || (MR == 8 && (PM || KW > 4)) ? 1 : 2;
+    // four waves without an activation order, 4096 x 11008 int4 7.55 -> 7.29 us, and costs up to 0.8 us elsewhere: 2048 x 4096 3.9 -> 4.7;
+    // with 8 bits it costs 2 to 9 % where workgroups share a CU or K is short, 2496 x 9792 8.45 us with it, 7.74 without, 1024 x 1024 3.44 and
+    // 3.23, and saves 1 to 4 % of 3008 to 4096 x 8192)
+    constexpr int QP = MR == 16 || (MR == 8 && (PM || KW > 4 || BITS == 8)) ? 1 : 2;
     u4 kq[QP];
     h8 xq[QP][MR];
 #pragma unroll
