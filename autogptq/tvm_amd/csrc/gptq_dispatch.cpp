@@ -614,7 +614,7 @@ static bool matmul_keeps(int M, int K, int N, int bits, int group_size, bool map
     gptq_hip_plan plan;
     if (K < 7168 || (bits >= 4 && (K == 7168 || N > (bits == 4 ? 2048 : 512)))) return false;
     return gptq_hip_select_tiled(M, K, N, bits, group_size, &plan) == GPTQ_HIP_OK && plan.kernel == GPTQ_HIP_KERNEL_TILED &&
-           gptq::tiled_reads_x_directly(mapped, M, K, plan);
+           M <= 16 && gptq::tiled_stages_x(mapped, plan);
 }
 
 // Five to eight rows on the decode kernel: K up to 11008, and longer layers of few columns, which the matmul kernel cuts into many

@@ -273,13 +273,19 @@ struct TiledParams {
 // per octet of columns; the workgroup copies the part of its tiles' groups and of its K range into LDS, and
 // every operand reads its 32 bytes from there, one operand ahead of the arithmetic.  The weights are formed
 // exactly as in the forward product.  The result's column p goes to channel out_map[p].
-// DIRECT: no pack pass.  Without an activation order position p is channel p, so lane (m, h) of fragment (S, j) finds
-// its eight values in row m of x at 64 S + 32 h + 8 j: sixteen bytes of a 128-byte line that the lane's other seven
-// fragments of the block share.  Rows past M read row M - 1 (a row of the result depends on its own row of x only,
-// and those rows are never stored), so a wave's load touches M lines; the launcher takes this form up to 16 rows
-// (4096 x 11008, us with / without the pack pass: 8 rows 14.0 / 10.7, 16 rows 14.5 / 11.5; with 32 distinct rows
-// per load 14.8 / 16.2, 64 rows 19 / 29.5: every lane then asks for a line of its own), and only when K is a whole
-// number of blocks that the waves' ranges cover exactly: there is no zero padding to read.
+// Without an activation order position p is channel p and the kernel reads x itself, with no pass and no launch before it, in one of two ways.
+// X_DIRECT: lane (m, h) of fragment (S, j) finds its eight values in row m of x at 64 S + 32 h + 8 j: sixteen bytes of a 128-byte line
+// that the lane's other seven fragments of the block share.  Rows past M read row M - 1 (a row of the result depends on its own row of x only,
+// and those rows are never stored), so a wave's load touches M lines; with 32 distinct rows every lane asks for a line of its own (4096 x 11008,
+// 64 rows 29.5 us, 19 with the pack pass).  Up to kTiledDirectRows rows, and only when K is a whole number of blocks that the waves' ranges cover
+// exactly: there is no zero padding to read.
+// X_STAGED: a request brings eight rows of a block, whole 128-byte lines, into the ring's registers; when its block is next they go to LDS,
+// to a place of the wave's own (no barrier; the area that the result tiles take at the end), and come back as fragments one step ahead of
+// the matrix instructions.  Eight LDS accesses per 32 rows and block stand for the pass, its launch gap and its write and read of x (us,
+// eager, pack pass / this: 55 rows of 18816 x 1056 int4 21.0 / 16.2, 20 of 9984 x 2912 13.4 / 11.1, 18 of 2240 x 30688 int3 14.3 / 12.7, 88 of
+// 1792 x 5600 9.9 / 8.9; the matmul kernel alone on x that is packed already, which computes nothing useful, 14.1 at the first).  Against
+// X_DIRECT (graph): 16 rows of 18432 x 23552 int8 106.4 / 88.8, 14 of 2048 x 32288 16.4 / 14.1, 16 of 2560 x 1344 8.9 / 8.2; 13 of 4352 x 7392 int2 10.3 /
+// 10.9, 10 of 15360 x 11328 27.4 / 30.6, 5 of 2304 x 15648 6.7 / 7.5: its requests and LDS accesses are for 32 rows always.
 // What the kernel needs before its first requests go out arrives as fourteen dwords that the dispatcher preloads
 // into scalar registers (this source is built with kernel-argument preloading), so that a wave does not begin by
 // waiting ~0.4 us for its argument segment: the source of the A operand (the packed fragments, or x itself for
@@ -294,11 +300,19 @@ struct TiledTail {
     int split_k, tiles_per_group;
 };
 
-template <int BITS, int AT, int RW, int KW, int RING, int CT, bool TRANS = false, bool DIRECT = false>
+// how the matmul kernel comes by x
+enum XMode {
+    X_PACKED,   // fragments that a pass before it wrote
+    X_DIRECT,   // from the rows of x, lane by lane
+    X_STAGED    // from the rows of x through LDS
+};
+
+template <int BITS, int AT, int RW, int KW, int RING, int CT, bool TRANS = false, XMode XM = X_PACKED>
 __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_src, const char *a_qtile, const uint32_t *a_sz,
                                                                   int a_wave_steps, int a_S_total, int a_T_total, int a_rt_total,
                                                                   int a_N, int a_M, int a_K, uint32_t a_groups, const TiledTail t)
 {
+    constexpr bool DIRECT = XM == X_DIRECT, STAGED = XM == X_STAGED;
     TiledParams p;
     p.xpack = a_src, p.x = (const _Float16 *)a_src, p.qtile = a_qtile, p.sz = a_sz;
     p.wave_steps = a_wave_steps, p.S_total = a_S_total, p.T_total = a_T_total, p.rt_total = a_rt_total;
@@ -349,8 +363,34 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
         for (int rt = 0; rt < AT; rt++)
             a_row[rt] = p.x + (size_t)min(32 * (rt0 + rt) + n, p.M - 1) * (size_t)p.K + 32 * h;
     }
+    // STAGED: request j of row tile rt brings rows 8 j .. + 7 of the block, 128 bytes each (eight lanes to a row).  Rows past M lie
+    // outside the buffer, the half of a last block past K is sent there, and blocks past K read from an empty one: zeros.
+    const int red_len = p.K;
+    const _Float16 *x_base = p.x + (size_t)(32 * rt0) * (size_t)red_len;
+    const uint32_t x_bytes = (uint32_t)max(min(p.M - 32 * rt0, 32 * AT), 0) * (uint32_t)red_len * 2u;
+    const uint32_t x_lane = (uint32_t)(lane >> 3) * (uint32_t)red_len * 2u + (uint32_t)(lane & 7) * 16u;
+    const int S_half = red_len % 64 != 0 ? S_last : -1;
+    const uint32_t x_cut = lane & 4 ? 0x80000000u : 0u;
+    // the wave's own two blocks in LDS, [row][octet ^ (row & 7)] of 16 bytes: neither the writes (eight rows of eight octets) nor the reads
+    // (32 rows, one octet of each half) meet on a bank
+    unsigned char *x_lds = smem + wave * (AT * 8192);
+    const uint32_t x_put = (uint32_t)(lane >> 3) * 128u + (uint32_t)(((lane & 7) ^ (lane >> 3)) * 16);
+    auto write_a = [&](int buf, int j, const h8 (&ar)[AT]) {
+#pragma unroll
+        for (int rt = 0; rt < AT; rt++) *(h8 *)(x_lds + (buf * AT + rt) * 4096 + j * 1024 + x_put) = ar[rt];
+    };
+    auto read_a = [&](int buf, int j, h8 (&fr)[AT]) {
+#pragma unroll
+        for (int rt = 0; rt < AT; rt++) fr[rt] = *(const h8 *)(x_lds + (buf * AT + rt) * 4096 + n * 128 + (((4 * h + j) ^ (n & 7)) * 16));
+    };
     auto load_a = [&](int S, int j, h8 (&ar)[AT]) {
-        if constexpr (DIRECT) {
+        if constexpr (STAGED) {
+            const __amdgpu_buffer_rsrc_t xb = tile_buffer((const char *)x_base, S <= S_last ? x_bytes : 0u);
+            const uint32_t at = x_lane | (S == S_half ? x_cut : 0u);
+#pragma unroll
+            for (int rt = 0; rt < AT; rt++)
+                ar[rt] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(xb, at + (uint32_t)(4 * rt + j) * (16u * (uint32_t)red_len), (uint32_t)S * 128u, 0));
+        } else if constexpr (DIRECT) {
             const int off = 64 * S + 8 * j;
 #pragma unroll
             for (int rt = 0; rt < AT; rt++) ar[rt] = *(const h8 *)(a_row[rt] + off);
@@ -381,10 +421,28 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
         const int S = next_block();
         S_of[u] = S;
         load_b(S, w[u], szr[u]);
-        if (TRANS || u == 0) {
+        if (TRANS || u == 0 || (STAGED && u == 1)) {
 #pragma unroll
             for (int j = 0; j < 4; j++) load_a(S, j, a[u][j]);
         }
+    }
+    // STAGED: x runs a block further ahead than the weights (its slot is free as soon as it is in LDS)
+    int x_ahead = ahead;
+    auto next_x = [&]() {
+        const int S = S_begin + x_ahead;
+        x_ahead = x_ahead + 1 == ws_n ? 0 : x_ahead + 1;
+        return S;
+    };
+    h8 fr[2][AT];
+    int buf = 0;
+    if constexpr (STAGED) {
+        const int S = next_x();
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            write_a(0, j, a[0][j]);
+            load_a(S, j, a[0][j]);
+        }
+        read_a(0, 0, fr[0]);
     }
     __builtin_amdgcn_sched_barrier(0);
     // TRANS: the (scale, base + zero) pairs of the workgroup's K range for the groups of its CT tiles -> LDS,
@@ -452,6 +510,7 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
         constexpr bool REFILL = decltype(refill_c)::value;
         constexpr bool FIRST = decltype(first_c)::value;   // the first block of the walk: asks for the other slots' A fragments
         const int S_refill = REFILL ? next_block() : 0;  // the block a ring ahead of this one in the walk
+        const int S_x = STAGED && REFILL ? next_x() : 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
 #pragma unroll
@@ -478,7 +537,35 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
                 }
 #pragma unroll
                 for (int rt = 0; rt < AT; rt++) {
-                    acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u][j][rt], bop, acc[rt][ct], 0, 0, 0);
+                    acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(STAGED ? fr[j & 1][rt] : a[u][j][rt], bop, acc[rt][ct], 0, 0, 0);
+                }
+                if constexpr (STAGED) {
+                    // the next fragments (of this block, or of the next one, whose rows have gone to LDS by then), the next block's
+                    // rows, and the requests for the slot that they leave
+                    constexpr int un = (u + 1) % RING;
+                    if (ct == 0) {
+                        read_a(j == 3 ? buf ^ 1 : buf, (j + 1) & 3, fr[(j + 1) & 1]);
+                    }
+                    if (ct == CT - 1) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (FIRST) {
+#pragma unroll
+                            for (int s = 2; s < RING; s++) load_a(S_of[s], j, a[s][j]);
+                        }
+                        if (j < 2) {
+#pragma unroll
+                            for (int i = 2 * j; i < 2 * j + 2; i++) {
+                                write_a(buf ^ 1, i, a[un][i]);
+                                if (REFILL) load_a(S_x, i, a[un][i]);
+                            }
+                        }
+                        if (REFILL && j == 3) {
+                            load_b(S_refill, w[u], szr[u]);
+                            S_of[u] = S_refill;
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    continue;
                 }
                 if (FIRST && ct == CT - 1) {
                     __builtin_amdgcn_sched_barrier(0);
@@ -497,6 +584,7 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
                 }
             }
         }
+        buf ^= 1;
     };
     // whole turns of the ring, then what is left without refills (no load sits behind a branch, and the loop
     // has no early exit: an exit into its latch would make the compiler wait at the head of every turn for
@@ -660,21 +748,21 @@ int launch_tiled_reduce(const float *partial, const void *bias, void *y, int M, 
 // the kernel's argument list from its parameter struct
 template <typename Kern>
 static int launch_gemm_kernel(Kern kern, dim3 grid, dim3 block, int lds_bytes, hipStream_t stream, const TiledParams &p,
-                              bool direct)
+                              bool from_x)
 {
     if (p.lb_per_group < 0 || p.lb_per_group > 0xfff || p.G < 0 || p.G >= (1 << 20)) return GPTQ_HIP_ERR_UNSUPPORTED;
     TiledTail t;
     t.bias = p.bias, t.y = p.y, t.partial = p.partial, t.szt = p.szt, t.out_map = p.out_map;
     t.split_k = p.split_k, t.tiles_per_group = p.tiles_per_group;
-    hipLaunchKernelGGL(kern, grid, block, lds_bytes, stream, direct ? (const char *)p.x : p.xpack, p.qtile, p.sz, p.wave_steps,
+    hipLaunchKernelGGL(kern, grid, block, lds_bytes, stream, from_x ? (const char *)p.x : p.xpack, p.qtile, p.sz, p.wave_steps,
                        p.S_total, p.T_total, p.rt_total, p.N, p.M, p.K, (uint32_t)p.lb_per_group | ((uint32_t)p.G << 12), t);
     return hipGetLastError() == hipSuccess ? GPTQ_HIP_OK : GPTQ_HIP_ERR_LAUNCH;
 }
 
-template <int BITS, int AT, int RW, int KW, int RING, int CT, bool DIRECT = false>
+template <int BITS, int AT, int RW, int KW, int RING, int CT, XMode XM = X_PACKED>
 static int launch_tiled_one(const TiledParams &p, const gptq_hip_plan &plan, hipStream_t stream)
 {
-    auto kern = tiled_gemm_kernel<BITS, AT, RW, KW, RING, CT, false, DIRECT>;
+    auto kern = tiled_gemm_kernel<BITS, AT, RW, KW, RING, CT, false, XM>;
     const int lds_bytes = tiled_lds_bytes(AT * RW, KW);
     if (plan.lds_bytes < lds_bytes || plan.waves_k != KW || plan.block != 64 * RW * KW) return GPTQ_HIP_ERR_BAD_ARG;
     if (lds_bytes > 65536) {
@@ -683,7 +771,7 @@ static int launch_tiled_one(const TiledParams &p, const gptq_hip_plan &plan, hip
             return GPTQ_HIP_ERR_LAUNCH;
         }
     }
-    return launch_gemm_kernel(kern, dim3(plan.grid_x, plan.grid_y, plan.grid_z), dim3(64 * RW * KW), lds_bytes, stream, p, DIRECT);
+    return launch_gemm_kernel(kern, dim3(plan.grid_x, plan.grid_y, plan.grid_z), dim3(64 * RW * KW), lds_bytes, stream, p, XM != X_PACKED);
 }
 
 // x is packed into the workspace, the matmul runs, and a reduce pass follows when K is split over workgroups.
@@ -717,7 +805,8 @@ int launch_tiled(const void *x, const void *qtile, const uint32_t *sz, const int
     const int S_pack = tiled_pack_blocks(plan.split_k, plan.waves_k, plan.k_chunk);
     // without an activation order the fragments can be read from x itself: one launch less
     const bool direct = tiled_reads_x_directly(xsrc != nullptr, M, K, plan);
-    if (!direct) {
+    const bool staged = !direct && tiled_stages_x(xsrc != nullptr, plan);
+    if (!direct && !staged) {
         const int pack_lds = xsrc ? K * 2 : 0;  // one row of x
         if (pack_lds > 65536) {
             if (hipFuncSetAttribute((const void *)tile_pack_x_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -736,10 +825,24 @@ int launch_tiled(const void *x, const void *qtile, const uint32_t *sz, const int
         rc = launch_tiled_one<B, A, 1, 4, tiled_ring(A), 2>(p, plan, stream)
     if (direct) {
         switch (bits) {
-            case 2: rc = launch_tiled_one<2, 1, 1, 4, tiled_ring(1), 2, true>(p, plan, stream); break;
-            case 3: rc = launch_tiled_one<3, 1, 1, 4, tiled_ring(1), 2, true>(p, plan, stream); break;
-            case 4: rc = launch_tiled_one<4, 1, 1, 4, tiled_ring(1), 2, true>(p, plan, stream); break;
-            case 8: rc = launch_tiled_one<8, 1, 1, 4, tiled_ring(1), 2, true>(p, plan, stream); break;
+            case 2: rc = launch_tiled_one<2, 1, 1, 4, tiled_ring(1), 2, X_DIRECT>(p, plan, stream); break;
+            case 3: rc = launch_tiled_one<3, 1, 1, 4, tiled_ring(1), 2, X_DIRECT>(p, plan, stream); break;
+            case 4: rc = launch_tiled_one<4, 1, 1, 4, tiled_ring(1), 2, X_DIRECT>(p, plan, stream); break;
+            case 8: rc = launch_tiled_one<8, 1, 1, 4, tiled_ring(1), 2, X_DIRECT>(p, plan, stream); break;
+            default: break;
+        }
+    } else if (staged) {
+        auto go = [&](auto bits_c) {
+            constexpr int B = decltype(bits_c)::value;
+            if (plan.row_tiles == 1) return launch_tiled_one<B, 1, 1, 4, tiled_ring(1), 2, X_STAGED>(p, plan, stream);
+            if (plan.row_tiles == 2) return launch_tiled_one<B, 2, 1, 4, tiled_ring(2), 2, X_STAGED>(p, plan, stream);
+            return launch_tiled_one<B, 4, 1, 4, tiled_ring(4), 2, X_STAGED>(p, plan, stream);
+        };
+        switch (bits) {
+            case 2: rc = go(std::integral_constant<int, 2>{}); break;
+            case 3: rc = go(std::integral_constant<int, 3>{}); break;
+            case 4: rc = go(std::integral_constant<int, 4>{}); break;
+            case 8: rc = go(std::integral_constant<int, 8>{}); break;
             default: break;
         }
     } else {
@@ -758,7 +861,7 @@ int launch_tiled(const void *x, const void *qtile, const uint32_t *sz, const int
     }
 #undef GPTQ_TILED_CASE
     // 128 x 128 per wave (waves_n = 2): a ring of two blocks
-    if (plan.row_tiles == 4 && plan.waves_n == 2) {
+    if (!direct && !staged && plan.row_tiles == 4 && plan.waves_n == 2) {
         switch (bits) {
             case 2: rc = launch_tiled_one<2, 4, 1, 4, 2, 4>(p, plan, stream); break;
             case 3: rc = launch_tiled_one<3, 4, 1, 4, 2, 4>(p, plan, stream); break;

@@ -250,8 +250,8 @@ int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int group_size, 
  * with this copy alone, PANEL included; where the workspace does not hold that plan's bytes, the PANEL plan without ranges for the
  * last row blocks, then gptq_hip_select_tiled.  A call that neither of these PANEL plans takes brings the workspace of
  * gptq_hip_select_tiled's plan, or is refused: also where it would run on row blocks, which need none.  workspace:
- * plan.workspace_bytes (none for most decode plans).  Decode plans: one launch; matmul plans: two
- * (pack pass, matmul); one more when the plan splits K.  A plan whose flags hold
+ * plan.workspace_bytes (none for most decode plans).  Decode plans: one launch; matmul plans: one without
+ * an activation order, two with one (pack pass, matmul) or with 128 columns per wave; one more when the plan splits K.  A plan whose flags hold
  * GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE wants ALL bytes of its workspace zero at the first call and leaves them zero
  * (the two halves of a tile that is halved along K meet in 64-bit slots behind the counters): give such plans a
  * workspace of their own, which no other entry point writes between the calls.  A call without a plan asks for that only up

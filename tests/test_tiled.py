@@ -167,6 +167,32 @@ def test_tiled_small_batches_read_x_without_the_pack_pass(dev, bits, K, N, gs):
 
 
 @pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("K,N,gs", [(32, 32, 32), (992, 96, 32), (1024, 416, 128), (4160, 160, -1)])
+@pytest.mark.parametrize("M,row_tiles", [(14, 1), (17, 1), (33, 1), (40, 2), (64, 2), (65, 4), (127, 4), (129, 4)])
+@pytest.mark.parametrize("split", [1, 3])
+def test_tiled_batches_bring_x_through_lds(dev, bits, K, N, gs, M, row_tiles, split):
+    # layers without an activation order: x comes through LDS, block by block.  Rows past M, the half of a last block past K, whole blocks
+    # past K (ranges that do not cover it evenly) and walks shorter than the ring.  The identity map forces the pack pass: same fragments,
+    # same order of the sums, so the two results are the same bits.
+    L = layer(2600 + bits + M, K, N, bits, gs, False, M=M, bias=True)
+    D = to_dev(L, dev)
+    plan = _lib.select_tiled(130, K, N, bits, gs)
+    assert plan.kernel == _lib.KERNEL_TILED
+    plan.row_tiles, plan.waves_n, plan.grid_x = row_tiles, 1, -(-N // 64)
+    plan.m_blocks = plan.grid_z = -(-M // (32 * row_tiles))
+    plan.lds_bytes = plan.waves_k * row_tiles * 2 * 4096
+    plan.k_chunk = -(-(-(-K // 64)) // (plan.waves_k * split))
+    plan.split_k, plan.grid_y = split, split
+    part = (split * M * N * 4 + 255) // 256 * 256 if split > 1 else 0
+    plan.workspace_bytes = 16384 + part + split * plan.waves_k * plan.k_chunk * 4 * plan.row_tiles * plan.m_blocks * 1024
+    qtile, sz, xsrc, kinv = prepare(D)
+    staged = ops.gemm_tiled(D["x"], qtile, sz, None, None, D["bias"], bits, gs, plan=plan)
+    packed = ops.gemm_tiled(D["x"], qtile, sz, xsrc, kinv, D["bias"], bits, gs, plan=plan)
+    assert_tight(staged, expected_output(L), f"M={M} K={K} split={split}")
+    assert torch.equal(staged, packed), f"M={M} K={K}: x through LDS and through the pack pass differ"
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
 @pytest.mark.parametrize("split", [1, 2, 3, 5])
 @pytest.mark.parametrize("M", [20, 130])
 def test_tiled_forced_split_k(dev, bits, split, M):
