@@ -603,7 +603,7 @@ bool gptq::select_row_blocks(int M, int K, int N, int bits, int group_size, gptq
     return false;
 }
 
-// Nine to sixteen rows that the matmul kernel reads itself, without its pack pass, are its own again on long layers, whose K it cuts over CUs that
+// Nine to sixteen rows that the matmul kernel reads itself, in ranges that cover K exactly, are its own again on long layers, whose K it cuts over CUs that
 // row blocks leave idle; with fewer bits or columns sooner (us at 9 / 16 rows, matmul / row blocks: 9216 x 64 int4 6.7 / 9.9 and 7.6 / 10.0,
 // 9216 x 2048 8.3 / 10.4 and 9.2 / 10.5, int3 7.5 / 10.7 and 8.1 / 10.8, 9216 x 4096 int4 10.4 / 10.9 and 11.6 / 10.8, int3 9.4 / 11.1 and
 // 10.7 / 11.2; 7680 x 2048 int4 8.3 / 9.0 and 9.0 / 9.0; 7168 x 2048 int4 8.7 / 8.5 and 9.9 / 8.5, int3 8.0 / 9.0 and 8.6 / 9.0; 8 bits 9216 x 64 7.0 /
@@ -614,7 +614,7 @@ static bool matmul_keeps(int M, int K, int N, int bits, int group_size, bool map
     gptq_hip_plan plan;
     if (K < 7168 || (bits >= 4 && (K == 7168 || N > (bits == 4 ? 2048 : 512)))) return false;
     return gptq_hip_select_tiled(M, K, N, bits, group_size, &plan) == GPTQ_HIP_OK && plan.kernel == GPTQ_HIP_KERNEL_TILED &&
-           M <= 16 && gptq::tiled_stages_x(mapped, plan);
+           M <= 16 && gptq::tiled_stages_x(mapped, plan) && gptq::tiled_covers_exactly(K, plan);
 }
 
 // Five to eight rows on the decode kernel: K up to 11008, and longer layers of few columns, which the matmul kernel cuts into many

@@ -167,11 +167,14 @@ inline int tiled_lds_bytes(int row_tiles, int waves_k) { return waves_k * row_ti
 // is a whole number of blocks that the waves' ranges cover exactly (no zero padding is read), else through LDS (figures at the kernel).
 // Plans of 128 columns per wave, for several blocks of 128 rows, keep the pass.
 constexpr int kTiledDirectRows = 13;
+inline bool tiled_covers_exactly(int K, const gptq_hip_plan &plan)
+{
+    return K % 64 == 0 && plan.split_k * plan.waves_k * plan.k_chunk == K / 64;
+}
 inline bool tiled_reads_x_directly(bool act_order, int M, int K, const gptq_hip_plan &plan)
 {
     return !act_order && M <= kTiledDirectRows && plan.kernel == GPTQ_HIP_KERNEL_TILED && plan.row_tiles == 1 &&
-           plan.m_blocks == 1 && plan.waves_n == 1 && K % 64 == 0 &&
-           plan.split_k * plan.waves_k * plan.k_chunk == K / 64;
+           plan.m_blocks == 1 && plan.waves_n == 1 && tiled_covers_exactly(K, plan);
 }
 inline bool tiled_stages_x(bool act_order, const gptq_hip_plan &plan)
 {
