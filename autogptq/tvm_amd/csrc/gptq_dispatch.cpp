@@ -718,8 +718,10 @@ extern "C" int gptq::gptq_tiled_default_plan(int M, int K, int N, int bits, int 
     int rc = gptq_panel_plan_within(M, K, N, bits, group_size, act_order ? GPTQ_HIP_PANEL_ACT_ORDER : 0, have, plan);
     if (rc != GPTQ_HIP_OK) rc = gptq_hip_select_tiled(M, K, N, bits, group_size, plan);
     if (rc != GPTQ_HIP_OK) return rc;
+    gptq_hip_plan other = *plan;
+    refine_short_plan(M, K, N, bits, group_size, act_order, &other);
+    if (plan->workspace_bytes <= have && other.workspace_bytes <= have) *plan = other;
     // row blocks need no workspace, but a call without the one that its size asks for stays refused
-    gptq_hip_plan other;
     if (plan->workspace_bytes <= have && !matmul_keeps(M, K, N, bits, group_size, act_order) &&
         select_row_blocks(M, K, N, bits, group_size, &other))
         *plan = other;
@@ -956,6 +958,105 @@ extern "C" int gptq::gptq_panel_plan_within(int M, int K, int N, int bits, int g
 
 namespace {
 
+// ---- Forward calls of 9 to 320 rows: matmul or PANEL plan by two models of both kernels, as they are called from a program (eager launches,
+// weights from memory), fitted to 58000 measurements of 1100 layers and row counts drawn at random (K of 1024 to 20480, N of 1024 to 32768, all
+// widths, with and without an activation order; 7.6 and 5.1 % rms, plans near the best one counting most). ----
+
+// A launch of the matmul kernel: turns of 256 workgroups, each as long as a wave's walk; two of one row tile share a CU (but for 8 bits, whose
+// registers fill it), which is what makes many short row blocks the better plan for narrow layers: a CU's second workgroup takes two thirds of
+// a turn and needs no pass that adds ranges up (2 us and the launch gap).
+double matmul_us(const gptq_hip_plan &p, int M, int K, int N, int bits, bool act)
+{
+    static const double kBlock[4] = {0.554, 0.723, 1.13, 1.83}, kTurn[4] = {1.72, 2.46, 4.03, 8.43}, kIdle[4] = {0.70, 0.70, 0.68, 0.36},
+                        kNext[4] = {0.70, 0.92, 0.89, 0.85};   // row tiles 1, 2, 4; 4 with 128 columns per wave
+    const int i = p.row_tiles == 1 ? 0 : (p.row_tiles == 2 ? 1 : (p.waves_n == 2 ? 3 : 2));
+    const double x_mb = 2e-6 * M * K;   // (beyond 3 MB the row blocks no longer find all of x in their chiplet's L2)
+    const double block = kBlock[i] * (bits == 8 ? 1.355 : (bits == 3 ? 0.854 : 1.0)) * (1 + 0.045 * (x_mb > 3 ? x_mb - 3 : 0));
+    auto turn = [&](double n) { return p.k_chunk * block * (kIdle[i] + (1 - kIdle[i]) * n / 256) + kTurn[i]; };
+    const long long wgs = (long long)p.grid_x * p.split_k * p.m_blocks, full = wgs / 256, last = wgs % 256;
+    double us = full * turn(256) + (last ? turn((double)last) : 0.0);
+    if (wgs > 256) us = turn(256) + (i == 0 && bits == 8 ? 1.0 : kNext[i]) * (us - turn(256));
+    return 1.92 + us + (p.split_k > 1 ? 2.18 + 1.477e-6 * p.split_k * M * N : 0.0) + (act ? 1.77 + 3.41e-6 * M * K : 0.0);
+}
+
+double panel_call_us(int rt, int split, int chunk, long long wgs, int M, int K, int N, int bits, bool act)
+{
+    const double step = (rt <= 4 ? 0.263 + 0.093 * rt : 0.299 + 0.113 * rt) + (bits == 8 ? 0.072 : (bits == 3 ? 0.096 : (bits == 2 ? 0.004 : 0.0)));
+    auto turn = [&](double n) { return chunk * step * (0.868 + 0.132 * n / 256) + 1.09 + 0.79 * rt; };
+    const long long full = wgs / 256, last = wgs % 256;
+    return 2.20 + full * turn(256) + (last ? turn((double)last) : 0.0) + (split > 1 ? 3.68 + 0.868e-6 * split * M * N : 0.0) +
+           (act ? 2.61 + 1.018e-6 * M * K : 0.0) + 0.0171e-6 * K * N * bits / 8 + 0.158e-6 * M * N;
+}
+
+// a plan of the matmul kernel with 64 columns per workgroup
+bool matmul_plan(int M, int K, int N, int bits, int group_size, int at, int split, gptq_hip_plan *plan)
+{
+    const int S_total = ceil_div(K, 64);
+    if (tiled_args_ok(M, K, N, bits, group_size, plan) != GPTQ_HIP_OK) return false;
+    plan->kernel = GPTQ_HIP_KERNEL_TILED;
+    plan->row_tiles = at;
+    plan->m_blocks = plan->grid_z = ceil_div(M, 32 * at);
+    plan->waves_n = 1;
+    plan->waves_k = 4;
+    plan->k_chunk = ceil_div(S_total, split * 4);
+    plan->split_k = plan->grid_y = ceil_div(S_total, plan->k_chunk * 4);
+    plan->grid_x = ceil_div(N / 32, 2);
+    plan->block = 256;
+    plan->lds_bytes = gptq::tiled_lds_bytes(at, 4);
+    plan->workspace_bytes = gptq::kCounterBytes + (plan->split_k > 1 ? ((size_t)plan->split_k * M * N * sizeof(float) + 255) / 256 * 256 : 0) +
+                            (size_t)gptq::tiled_pack_blocks(plan->split_k, 4, plan->k_chunk) * 4 * (size_t)(at * plan->m_blocks) * 1024;
+    return plan->split_k == split;
+}
+
+}  // namespace
+
+// The plan of a call that has one, PANEL or matmul, replaced by the one that the models name where they give it 7 % at least.  Without that
+// margin 5 % of the measured calls became slower by more than 3 % (the worst 1.2 x), with it 0.5 % (1.12 x).  On 1000 calls drawn since it
+// moves 155, which are 1.20 x as fast on the mean (us, eager, the pack pass gone in both where there is no activation order: 88 rows of 1024 x 3520 int3
+// 6.2 -> 5.1, 138 of 4096 x 1792 14.4 -> 10.7, 84 of 4288 x 3264 int4 13.8 -> 11.7, 104 of 1536 x 20576 22.8 -> 17.6; with an activation order 68 of
+// 5248 x 4576 20.8 -> 16.0, 86 of 8064 x 4384 29.4 -> 22.1, 199 of 1664 x 1216 11.3 -> 10.0).  With an activation order the pack pass is most of what a call
+// of up to 32 rows could lose or gain, and the mean of those was level (0.5 % at 17 to 32 rows, none below): they stay.  So do plans with whole row
+// blocks ahead of their ranges; calls past 320 rows and the gradient were not measured.
+void gptq::refine_short_plan(int M, int K, int N, int bits, int group_size, bool act, gptq_hip_plan *plan)
+{
+    if (M <= (act ? 32 : kDecodeMaxRows) || M > kShortPlanRows) return;
+    const bool panel = plan->kernel == GPTQ_HIP_KERNEL_PANEL;
+    if ((!panel && plan->kernel != GPTQ_HIP_KERNEL_TILED) || (panel && panel_main_blocks(*plan) != 0)) return;
+    const int S_total = ceil_div(K, 64), panel_cols = ceil_div(N, kPanelCols);
+    double best = 0.93 * (panel ? panel_call_us(plan->row_tiles, plan->split_k, plan->k_chunk, (long long)plan->grid_x * plan->m_blocks * plan->split_k,
+                                                M, K, N, bits, act)
+                                : matmul_us(*plan, M, K, N, bits, act));
+    gptq_hip_plan other, found;
+    bool better = false;
+    // (the partial tiles of a matmul plan stay within three times the packed weights, as in its own planner)
+    const long long cap = (3LL * K * bits) / (128LL * M);
+    for (int at = 1; at <= 4; at *= 2) {
+        const long long tiles = (long long)ceil_div(N / 32, 2) * ceil_div(M, 32 * at);
+        if ((at > 1 && 16 * at >= M) || tiles > 1100) continue;
+        for (int s = 1; s <= 12; s++) {
+            if (s > 1 && (s > cap || tiles * s > 520 || S_total / (4 * s) < (at == 1 ? 3 : 2))) break;
+            if (!matmul_plan(M, K, N, bits, group_size, at, s, &other)) continue;
+            const double us = matmul_us(other, M, K, N, bits, act);
+            if (us < best) best = us, found = other, better = true;
+        }
+    }
+    for (int rt = 1; rt <= kPanelMaxTiles && (rt == 1 || 32 * (rt - 1) < M); rt++) {
+        const long long tiles = (long long)panel_cols * ceil_div(M, 32 * rt);
+        if (tiles > 1100) continue;
+        for (int s = 1; s <= 8; s++) {
+            const int chunk = ceil_div(S_total, s);
+            if (s > 1 && (S_total / s < 6 || tiles * s > 520 || (double)s * M * N > 48e6)) break;
+            if (ceil_div(S_total, chunk) != s) continue;
+            const double us = panel_call_us(rt, s, chunk, tiles * s, M, K, N, bits, act);
+            if (us < best && gptq_hip_select_panel(M, K, N, bits, group_size, act ? GPTQ_HIP_PANEL_ACT_ORDER : 0, rt, s, &other) == GPTQ_HIP_OK)
+                best = us, found = other, better = true;
+        }
+    }
+    if (better) *plan = found;
+}
+
+namespace {
+
 // Where the tiled kernels were measured faster than the ones that read the checkpoint layout or its channel-sorted
 // copy, on MI355X with the weights cold (us per call, graph replay, group size 128 unless said):
 //   * up to 4 rows, layers of up to 4096 columns (decode kernel with a workgroup per tile, per half of one along K from 4096
@@ -1093,6 +1194,7 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
             return false;
         }
         route->copy = GPTQ_HIP_ROUTE_TILED;
+        if (panels) gptq::refine_short_plan(M, K, N, bits, group_size, act_order != 0, &route->plan);
         return true;
     };
     auto take_panel = [&]() {
@@ -1102,6 +1204,7 @@ extern "C" int gptq_hip_select_route(int M, int K, int N, int bits, int group_si
             return false;
         }
         route->copy = GPTQ_HIP_ROUTE_TILED;
+        gptq::refine_short_plan(M, K, N, bits, group_size, act_order != 0, &route->plan);
         return true;
     };
     auto take_rows = [&]() {

@@ -228,6 +228,9 @@ inline long long tiled_decode16_lds_bytes(int mr, int K, int groups, int units_p
 }
 // the plan in row blocks, where it is the faster one (gptq_dispatch.cpp)
 bool select_row_blocks(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan);
+// a matmul or PANEL plan of a forward call of 9 to kShortPlanRows rows, replaced where another one is clearly the faster (gptq_dispatch.cpp)
+constexpr int kShortPlanRows = 320;
+void refine_short_plan(int M, int K, int N, int bits, int group_size, bool act_order, gptq_hip_plan *plan);
 // the PANEL plan of a call that names none, if one fits its workspace;
 extern "C" int gptq_panel_plan_within(int M, int K, int N, int bits, int group_size, unsigned flags, size_t have, gptq_hip_plan *plan);
 // the plan of a gptq_hip_gemm_tiled call that names none, and whether the call clears the slots of its halved tiles (the tests ask, too)

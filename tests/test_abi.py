@@ -652,3 +652,42 @@ def test_one_row_of_few_bits_in_small_groups_keeps_the_16_column_kernel():
                                          (1, 2496, 2496, 4, 64, False), (2, 2496, 2496, 3, 64, False), (1, 2560, 1024, 3, 128, False),
                                          (1, 2592, 1024, 4, 32, True), (3, 2592, 1024, 3, 32, False)):
         assert (_lib.select_tiled(M, K, N, bits, gs).waves_n == 2) == columns16, (M, K, N, bits, gs)
+
+
+def test_short_calls_take_the_plan_that_the_models_name():
+    """9 to 320 rows of hosts that set the bit for the newer plans: a matmul or PANEL plan gives way to a clearly faster one, for every caller by the
+    same rule; a call without a plan still asks for the workspace of gptq_hip_select_tiled's, and older hosts get the answers they got."""
+    import random
+
+    rng, moved = random.Random(3), 0
+    panel = _lib.COPY_TILED | _lib.COPY_TILED_PANEL
+    shapes = [(138, 4096, 1792, 3, 128, False), (68, 5248, 4576, 4, 128, True), (86, 8064, 4384, 4, 128, True), (104, 1536, 20576, 3, 128, False),
+              (54, 4096, 1184, 3, 128, False), (33, 4480, 1568, 4, 32, True), (320, 1280, 1280, 4, 128, False)]
+    for _ in range(400):
+        gs = rng.choice((128, 64, 32, -1))
+        unit = 32 if gs == -1 else gs
+        shapes.append((rng.choice((9, 13, 16, 17, 32, 33, 64, 65, 128, 129, 256, 320, 321, 700)), unit * rng.randint(1, 20480 // unit),
+                       32 * rng.randint(1, 512), rng.choice((2, 3, 4, 8)), gs, rng.random() < 0.5))
+    for M, K, N, bits, gs, act in shapes:
+        r = _lib.select_route(M, K, N, bits, gs, act, panel).plan
+        old, own = _lib.select_tiled(M, K, N, bits, gs), _lib.select_panel(M, K, N, bits, gs, act)
+        if r.kernel == _lib.KERNEL_TILED_DECODE:
+            continue
+        for have in (0, old.workspace_bytes - 1, old.workspace_bytes, 1 << 40):
+            plan, _ = default_plan(M, K, N, bits, gs, act, have)
+            if have == 1 << 40:
+                assert plan.as_dict() == r.as_dict(), (M, K, N, bits, gs, act)
+            elif own is None:
+                assert (plan.workspace_bytes <= have) == (have >= old.workspace_bytes), (M, K, N, bits, gs, act)
+        before = (own or old).as_dict()
+        if r.as_dict() != before:
+            moved += 1
+            assert (33 if act else 9) <= M <= 320 and not before["flags"]
+            steps = -(-K // 64)
+            if r.kernel == _lib.KERNEL_TILED:
+                assert 32 * r.row_tiles * r.m_blocks >= M and r.split_k * 4 * r.k_chunk >= steps > (r.split_k - 1) * 4 * r.k_chunk
+                assert r.split_k == 1 or 4 * r.split_k * M * N <= 3 * K * N * bits // 8
+            else:
+                assert r.as_dict() == _lib.select_panel(M, K, N, bits, gs, act, False, r.row_tiles, r.split_k).as_dict()
+        assert _lib.select_route(M, K, N, bits, gs, act, _lib.COPY_TILED).plan.as_dict() == old.as_dict()
+    assert moved > 15

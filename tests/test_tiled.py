@@ -192,6 +192,18 @@ def test_tiled_batches_bring_x_through_lds(dev, bits, K, N, gs, M, row_tiles, sp
     assert torch.equal(staged, packed), f"M={M} K={K}: x through LDS and through the pack pass differ"
 
 
+@pytest.mark.parametrize("M,K,N,bits,gs,desc_act", [(138, 4096, 1792, 3, 128, False), (68, 5248, 4576, 4, 128, True), (33, 7552, 1120, 2, 64, True),
+                                                    (104, 1536, 5152, 8, 128, False), (320, 1280, 1280, 4, 32, False), (15, 5632, 2688, 2, 128, False)])
+def test_short_calls_on_the_plan_that_the_models_name(dev, M, K, N, bits, gs, desc_act):
+    L = layer(2700 + M, K, N, bits, gs, desc_act, M=M, bias=True)
+    D = to_dev(L, dev)
+    qtile, sz, xsrc, kinv = prepare(D)
+    maps = (xsrc, kinv) if desc_act else (None, None)
+    y = ops.gemm_tiled(D["x"], qtile, sz, *maps, D["bias"], bits, gs)
+    assert_tight(y, expected_output(L), f"M={M} K={K} N={N}")
+    assert torch.equal(y, torch.ops.gptq_hip.gemm_tiled(D["x"], qtile, sz, *maps, D["bias"], bits, gs))
+
+
 @pytest.mark.parametrize("bits", [2, 3, 4, 8])
 @pytest.mark.parametrize("split", [1, 2, 3, 5])
 @pytest.mark.parametrize("M", [20, 130])
