@@ -88,7 +88,8 @@ struct DecodeTail {
 // E: blocks of 64 positions that share one epilogue (1, or 2 when the groups are multiples of 128 channels and
 // every wave has an even number of blocks: both lane blocks of both blocks then lie in one group).
 // C: the zero point is taken off every code (CENTRE; four rows and more always are built so).
-template <int BITS, int MR, int KW, int E, bool PM, bool RB, bool C>
+// QP: passes over x, eight channels a lane, that are requested ahead of the weights and held in registers (decode_passes).
+template <int BITS, int MR, int KW, int E, bool PM, bool RB, bool C, int QP>
 __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a_x, const uint16_t *a_kinv, const char *a_qtile,
                                                                const uint32_t *a_sz, int a_K, uint32_t a_m_steps, int a_T_total,
                                                                int a_grid_x, uint32_t a_lbg_magic, uint32_t a_flags,
@@ -166,11 +167,6 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     //         for the word of a unit when it asks for the unit's weights and finds it when they are there.) -----
     // (without a map the channels of the range are the range itself)
     const int k8_lo = mapped ? 0 : p0 / 8, k8_hi = mapped ? p.K / 8 : min(p0 + span, p.K) / 8;
-    // passes over x kept in registers (eight rows: 32 registers a pass; a second one only shortens the way of workgroups of
-    // four waves without an activation order, 4096 x 11008 int4 7.55 -> 7.29 us, and costs up to 0.8 us elsewhere: 2048 x 4096 3.9 -> 4.7;
-    // with 8 bits it costs 2 to 9 % where workgroups share a CU or K is short, 2496 x 9792 8.45 us with it, 7.74 without, 1024 x 1024 3.44 and
-    // 3.23, and saves 1 to 4 % of 3008 to 4096 x 8192)
-    constexpr int QP = MR == 16 || (MR == 8 && (PM || KW > 4 || BITS == 8)) ? 1 : 2;
     u4 kq[QP];
     h8 xq[QP][MR];
 #pragma unroll
@@ -561,10 +557,29 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
     }
 }
 
-template <int BITS, int MR, int KW, int E, bool PM, bool RB, bool C>
+// Passes over x held in registers (a lane's eight channels of every row: 4 MR registers a pass); the loop in front of the weight requests
+// stages what they leave.  A second pass that the workgroup's channels do not fill still is a request per row and a wait for it, and the
+// registers of one that they do fill cost workgroups on a CU.  Measured in a graph, us with one / two:
+//   one and two rows: two (a second pass is one or two requests; 5120 x 5120 5.2 / 4.9);
+//   four rows, workgroups of eight waves: one (2048 x 4096 3.34 / 3.56, with an activation order 3.46 / 3.72, 4096 x 4096 3.94 / 4.18 and 4.33 /
+//   4.67, 8192 x 10240 with an order 10.5 / 11.2, 11008 x 11008 16.8 / 17.2), but two without an order where there are more than two workgroups a CU (8192 x
+//   28672 22.4 / 22.3, int3 19.7 / 19.3, 6272 x 21152 int2 13.7 / 13.4);
+//   four and eight rows (eight without an activation order, below 8 bits), workgroups of four: one where it holds them all (1024 x 11008 3.62 / 3.87 and, eight rows,
+//   4.24 / 4.73, 2048 x 11008 4.23 / 4.36 and 5.00 / 5.39), else two (four rows of 4096 x 11008 6.21 / 5.92, 2560 x 14336 5.74 / 5.47, eight of
+//   2560 x 14336 6.70 / 6.63), but one again for four rows with an activation order that nearly fill both, whose walk over all of x the
+//   workgroups of a CU hide from each other (4096 x 11008 6.48 / 6.98, 4096 x 14336 7.70 / 8.01; 3328 x 12960 8.29 / 8.15, 2560 x 14336 6.55 / 6.32);
+//   eight rows otherwise, and sixteen: one (4096 x 4096 4.7 / 5.1, 8192 x 28672 with an order 35.1 / 44).
+constexpr int decode_passes(int mr, int kw) { return mr >= 8 || (mr == 4 && kw > 4) ? 1 : 2; }
+static bool decode_second_pass(int mr, int kw, bool mapped, int K, int channels, int workgroups)
+{
+    if (channels <= 8 * 64 * kw) return false;
+    return kw == 4 ? !(mr == 4 && mapped && K > 3600) : !mapped && workgroups > 2 * kNumCUs;
+}
+
+template <int BITS, int MR, int KW, int E, bool PM, bool RB, bool C, int QP = decode_passes(MR, KW)>
 static int launch_decode_one(const DecodeParams &p, const gptq_hip_plan &plan, hipStream_t stream)
 {
-    auto kern = tiled_decode_kernel<BITS, MR, KW, E, PM, RB, C>;
+    auto kern = tiled_decode_kernel<BITS, MR, KW, E, PM, RB, C, QP>;
     if (plan.lds_bytes > 65536) {
         if (hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, plan.lds_bytes) != hipSuccess) {
             (void)hipGetLastError();
@@ -583,9 +598,23 @@ static int launch_decode_one(const DecodeParams &p, const gptq_hip_plan &plan, h
 template <int BITS, int MR, int E, bool PM, bool RB = false, bool C = tiled_decode_centred(MR)>
 static int launch_decode_kw(const DecodeParams &p, const gptq_hip_plan &plan, hipStream_t stream)
 {
+    // the channels that a workgroup stages: all of K, but for layers whose tiles are all halved or cut into ranges
+    const bool whole = PM || (plan.split_k == 1 && plan.grid_x < 2 * p.T_total);
+    const bool second = decode_second_pass(MR, plan.waves_k, PM, p.K, whole ? p.K : (p.K + 1) / 2, plan.grid_x);
+    (void)second;
     switch (plan.waves_k) {
-        case 4: return launch_decode_one<BITS, MR, 4, E, PM, RB, C>(p, plan, stream);
-        case 8: return launch_decode_one<BITS, MR, 8, E, PM, RB, C>(p, plan, stream);
+        case 4:
+            if constexpr (!RB && (MR == 4 || (MR == 8 && !PM && BITS != 8))) {
+                if (second) return launch_decode_one<BITS, MR, 4, E, PM, RB, C, 2>(p, plan, stream);
+                return launch_decode_one<BITS, MR, 4, E, PM, RB, C, 1>(p, plan, stream);
+            } else {
+                return launch_decode_one<BITS, MR, 4, E, PM, RB, C>(p, plan, stream);
+            }
+        case 8:
+            if constexpr (!RB && MR == 4 && !PM) {
+                if (second) return launch_decode_one<BITS, MR, 8, E, PM, RB, C, 2>(p, plan, stream);
+            }
+            return launch_decode_one<BITS, MR, 8, E, PM, RB, C>(p, plan, stream);
         case 16:
             // (128 registers per lane do not hold two sets of rows)
             if constexpr (MR >= 8 || (C && MR < 4)) return GPTQ_HIP_ERR_UNSUPPORTED;

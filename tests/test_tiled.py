@@ -905,3 +905,18 @@ def test_tiled_decode_small_layers_sum_without_the_bases(dev, bits, K, N, gs, de
     for M in (1, 2, 4, 8):
         y = run_tiled(D, prep, x=D["x"].expand(M, K).contiguous())
         assert float((y.double().cpu() - rest).norm() / (M ** 0.5 * exact.norm())) < 1e-6, M
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("K,N", [(2048, 8224), (2080, 8224), (3616, 8224), (4096, 16448), (4128, 16448)])
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_tiled_decode_passes_over_x(dev, bits, K, N, desc_act):
+    """Three to eight rows: one or two passes over x ahead of the weights, and the loop in front of them: a pass that is just full and one octet more,
+    workgroups of four and eight waves, more than two workgroups a CU."""
+    L = layer(5600 + K, K, N, bits, 32, desc_act, M=8, bias=True)
+    D = to_dev(L, dev)
+    prep, want = prepare(D), expected_output(L)
+    for M in (3, 4, 8):
+        plan = _lib.select_tiled(M, K, N, bits, 32)
+        assert plan.kernel == _lib.KERNEL_TILED_DECODE and plan.waves_k == (4 if K < 4128 else 8)
+        assert_tight(run_tiled(D, prep, x=L["x"][:M].contiguous().to(dev), plan=plan), want[:M], f"int{bits} {K}x{N} M={M}")
