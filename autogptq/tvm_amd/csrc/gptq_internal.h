@@ -187,6 +187,21 @@ inline int tiled_t_lds_bytes(int row_tiles, int waves_k, int wave_steps)
     const int red = tiled_lds_bytes(row_tiles, waves_k), tbl = 2 * waves_k * wave_steps * 256;
     return red > tbl ? red : tbl;
 }
+// The gradient's rows lie in the order that the transposed product reads them in, with an activation order too: workgroups of one and two row
+// tiles stage them themselves where the LDS (their table, and places for two blocks a wave) holds as many of them as the launch puts on a CU:
+// one, or two of one row tile.  The pass stays for the rest (figures at the kernel), and for row blocks past 31 bits.
+inline int tiled_t_staged_lds_bytes(int row_tiles, int waves_k, int wave_steps)
+{
+    return 2 * waves_k * wave_steps * 256 + waves_k * row_tiles * 8192;
+}
+constexpr int kNumCUs = 256;   // MI355X
+inline bool tiled_t_stages_x(int N, const gptq_hip_plan &plan)
+{
+    const long long wgs = (long long)plan.grid_x * plan.split_k * plan.m_blocks;
+    const int per_cu = wgs <= kNumCUs ? 1 : (plan.row_tiles == 1 && wgs <= 2 * kNumCUs ? 2 : 0);
+    return plan.row_tiles <= 2 && per_cu > 0 && 64LL * plan.row_tiles * N < (1LL << 31) &&
+           per_cu * tiled_t_staged_lds_bytes(plan.row_tiles, plan.waves_k, plan.k_chunk) <= 160 * 1024;
+}
 constexpr int kTiledTMaxBlocks = 304;   // blocks of 64 columns a workgroup of the transposed product may walk (LDS)
 inline bool tiled_qualifies(int K, int N, int bits, int gs)
 {
@@ -219,7 +234,6 @@ inline int tiled_decode_lds_bytes(int mr, int span, int groups, int waves_k)
 }
 // decode kernel with one workgroup per CU (16-column units, all of K staged): LDS of a workgroup that takes
 // `units_per_wg` units
-constexpr int kNumCUs = 256;   // MI355X
 inline long long tiled_decode16_lds_bytes(int mr, int K, int groups, int units_per_wg)
 {
     const long long span = ((K + 63) / 64 + 1) / 2 * 128;

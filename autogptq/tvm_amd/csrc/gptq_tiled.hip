@@ -267,7 +267,7 @@ struct TiledParams {
 // register file).
 // TRANS: gx = gy @ W^T, the gradient of the product with respect to x.  The kernel is handed the tiled format of the
 // TRANSPOSED code matrix (gptq_hip_tile_prepare_transposed): its "positions" are the layer's columns n (the
-// reduction runs over them; x here is gy, packed like any x), its "columns" are the layer's sorted positions p, so
+// reduction runs over them; x here is gy, and K the length of its rows), its "columns" are the layer's sorted positions p, so
 // a lane holds 32 columns of one position and a column tile (32 positions) lies in one group.  Scale and zero
 // point then differ per value of an operand instead of per lane: the table p.szt holds them as register pairs
 // per octet of columns; the workgroup copies the part of its tiles' groups and of its K range into LDS, and
@@ -286,6 +286,12 @@ struct TiledParams {
 // 1792 x 5600 9.9 / 8.9; the matmul kernel alone on x that is packed already, which computes nothing useful, 14.1 at the first).  Against
 // X_DIRECT (graph): 16 rows of 18432 x 23552 int8 106.4 / 88.8, 14 of 2048 x 32288 16.4 / 14.1, 16 of 2560 x 1344 8.9 / 8.2; 13 of 4352 x 7392 int2 10.3 /
 // 10.9, 10 of 15360 x 11328 27.4 / 30.6, 5 of 2304 x 15648 6.7 / 7.5: its requests and LDS accesses are for 32 rows always.
+// The transposed product takes X_STAGED with and without an activation order, for a gradient's rows are in the order of the reduction anyway
+// (tiled_t_stages_x; us, graph, pack pass / this: 38 rows of 2176 x 14176 int4 19.3 / 16.1, 342 of 1280 x 1536 16.5 / 14.0, 400 of 1920 x 2496
+// 19.7 / 15.9, 32 of 7040 x 1536 12.2 / 11.0; 155 plans of 70 drawn calls in all 1.14 x as fast on the mean, five of them slower by 2 to 6 %).  Where
+// a CU has more workgroups than fit beside each other with a place for x each, what they hide of one another is worth more than the pass (35 of
+// 15616 x 19872 int3, 488 workgroups of 142 KB, 73.7 / 88.3; launches of more than 512 workgroups 0.92 to 1.2 x as fast); with four row tiles the
+// ring and the fragments do not fit the registers (232 of 5504 x 1824 int3 17.4 / 18.4, 95 of 11264 x 1856 24.0 / 24.6).
 // What the kernel needs before its first requests go out arrives as fourteen dwords that the dispatcher preloads
 // into scalar registers (this source is built with kernel-argument preloading), so that a wave does not begin by
 // waiting ~0.4 us for its argument segment: the source of the A operand (the packed fragments, or x itself for
@@ -373,7 +379,8 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
     const uint32_t x_cut = lane & 4 ? 0x80000000u : 0u;
     // the wave's own two blocks in LDS, [row][octet ^ (row & 7)] of 16 bytes: neither the writes (eight rows of eight octets) nor the reads
     // (32 rows, one octet of each half) meet on a bank
-    unsigned char *x_lds = smem + wave * (AT * 8192);
+    const int wg_blocks = KW * p.wave_steps, S_wg0 = split * wg_blocks;
+    unsigned char *x_lds = smem + (TRANS ? CT * wg_blocks * 256 : 0) + wave * (AT * 8192);   // (TRANS: behind the table)
     const uint32_t x_put = (uint32_t)(lane >> 3) * 128u + (uint32_t)(((lane & 7) ^ (lane >> 3)) * 16);
     auto write_a = [&](int buf, int j, const h8 (&ar)[AT]) {
 #pragma unroll
@@ -447,8 +454,6 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
     __builtin_amdgcn_sched_barrier(0);
     // TRANS: the (scale, base + zero) pairs of the workgroup's K range for the groups of its CT tiles -> LDS,
     // [ct][block of the range][octet][8 words]
-    const int wg_blocks = KW * p.wave_steps;
-    const int S_wg0 = split * wg_blocks;
     if constexpr (TRANS) {
         u4 *tbl = (u4 *)smem;
         for (int i = tid; i < CT * wg_blocks * 16; i += 64 * RW * KW) {
@@ -977,21 +982,23 @@ int launch_tile_prepare_t(const uint32_t *qweight, const uint32_t *qzeros, const
     return hipGetLastError() == hipSuccess ? GPTQ_HIP_OK : GPTQ_HIP_ERR_LAUNCH;
 }
 
-template <int BITS, int AT>
+template <int BITS, int AT, XMode XM>
 static int launch_tiled_t_one(const TiledParams &p, const gptq_hip_plan &plan, hipStream_t stream)
 {
-    auto kern = tiled_gemm_kernel<BITS, AT, 1, 4, tiled_ring(AT), 2, true>;
+    auto kern = tiled_gemm_kernel<BITS, AT, 1, 4, tiled_ring(AT), 2, true, XM>;
     if (plan.lds_bytes < tiled_t_lds_bytes(AT, 4, plan.k_chunk) || plan.waves_k != 4 || plan.block != 256) return GPTQ_HIP_ERR_BAD_ARG;
-    if (plan.lds_bytes > 65536) {
-        if (hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, plan.lds_bytes) != hipSuccess) {
+    const int staged_bytes = tiled_t_staged_lds_bytes(AT, 4, plan.k_chunk);
+    const int lds_bytes = XM == X_STAGED && plan.lds_bytes < staged_bytes ? staged_bytes : plan.lds_bytes;
+    if (lds_bytes > 65536) {
+        if (hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess) {
             (void)hipGetLastError();
             return GPTQ_HIP_ERR_LAUNCH;
         }
     }
-    return launch_gemm_kernel(kern, dim3(plan.grid_x, plan.grid_y, plan.grid_z), dim3(256), plan.lds_bytes, stream, p, false);
+    return launch_gemm_kernel(kern, dim3(plan.grid_x, plan.grid_y, plan.grid_z), dim3(256), lds_bytes, stream, p, XM != X_PACKED);
 }
 
-// gy is packed into the workspace (as x is for the forward product), the matmul runs on the transposed copy, and a
+// The matmul runs on the transposed copy, behind a pass that packs gy into the workspace where it does not stage it itself, and a
 // reduce pass follows when the reduction over N is split over workgroups.
 int launch_tiled_t(const void *gy, const void *qtile_t, const uint32_t *szt, const int32_t *xsrc, void *gx, char *xpack,
                    float *partial, int M, int K, int N, int bits, int group_size, const gptq_hip_plan &plan,
@@ -1018,28 +1025,31 @@ int launch_tiled_t(const void *gy, const void *qtile_t, const uint32_t *szt, con
     p.szt = szt;
     p.out_map = xsrc;
     p.tiles_per_group = group_size / 32;
-    p.x = nullptr;           // (the forward product's direct read of x: not used here)
-    p.K = K;
+    p.x = (const _Float16 *)gy;
+    p.K = N;                 // the length of a row of gy
     const int S_pack = tiled_pack_blocks(plan.split_k, plan.waves_k, plan.k_chunk);
-    hipLaunchKernelGGL(tile_pack_x_kernel, dim3(32 * p.rt_total, pack_parts(32 * p.rt_total, S_pack)), dim3(256), 0, stream, (const _Float16 *)gy,
-                       (const int32_t *)nullptr, xpack, M, N, Np, p.rt_total, S_pack);
-    if (hipGetLastError() != hipSuccess) return GPTQ_HIP_ERR_LAUNCH;
+    const bool staged = tiled_t_stages_x(N, plan);
+    if (!staged) {
+        hipLaunchKernelGGL(tile_pack_x_kernel, dim3(32 * p.rt_total, pack_parts(32 * p.rt_total, S_pack)), dim3(256), 0, stream, (const _Float16 *)gy,
+                           (const int32_t *)nullptr, xpack, M, N, Np, p.rt_total, S_pack);
+        if (hipGetLastError() != hipSuccess) return GPTQ_HIP_ERR_LAUNCH;
+    }
     int rc = GPTQ_HIP_ERR_UNSUPPORTED;
-#define GPTQ_TILED_T_CASE(B, A) \
-    if (bits == B && plan.row_tiles == A) rc = launch_tiled_t_one<B, A>(p, plan, stream)
-    GPTQ_TILED_T_CASE(2, 1);
-    GPTQ_TILED_T_CASE(2, 2);
-    GPTQ_TILED_T_CASE(2, 4);
-    GPTQ_TILED_T_CASE(3, 1);
-    GPTQ_TILED_T_CASE(3, 2);
-    GPTQ_TILED_T_CASE(3, 4);
-    GPTQ_TILED_T_CASE(4, 1);
-    GPTQ_TILED_T_CASE(4, 2);
-    GPTQ_TILED_T_CASE(4, 4);
-    GPTQ_TILED_T_CASE(8, 1);
-    GPTQ_TILED_T_CASE(8, 2);
-    GPTQ_TILED_T_CASE(8, 4);
-#undef GPTQ_TILED_T_CASE
+    auto go = [&](auto bits_c) {
+        constexpr int B = decltype(bits_c)::value;
+        if (plan.row_tiles == 1)
+            return staged ? launch_tiled_t_one<B, 1, X_STAGED>(p, plan, stream) : launch_tiled_t_one<B, 1, X_PACKED>(p, plan, stream);
+        if (plan.row_tiles == 2)
+            return staged ? launch_tiled_t_one<B, 2, X_STAGED>(p, plan, stream) : launch_tiled_t_one<B, 2, X_PACKED>(p, plan, stream);
+        return launch_tiled_t_one<B, 4, X_PACKED>(p, plan, stream);
+    };
+    switch (bits) {
+        case 2: rc = go(std::integral_constant<int, 2>{}); break;
+        case 3: rc = go(std::integral_constant<int, 3>{}); break;
+        case 4: rc = go(std::integral_constant<int, 4>{}); break;
+        case 8: rc = go(std::integral_constant<int, 8>{}); break;
+        default: break;
+    }
     if (rc != GPTQ_HIP_OK) return rc;
     if (plan.split_k > 1) {
         return launch_tiled_reduce(partial, nullptr, gx, M, K, plan.split_k, xsrc, stream);

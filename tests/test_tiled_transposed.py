@@ -246,3 +246,32 @@ def test_a_copied_compact_layer_keeps_its_gradient(dev, M):
     gy = grad_rows(3801, M, N).to(dev)
     assert torch.equal(clone.grad_input(gy), q.grad_input(gy))
     assert_tight(q.grad_input(gy), gy.float().cpu() @ expected_weight(L).float().t(), "compact layer")
+
+
+# a walk shorter than the ring of weights and one of several turns; half a block at the end, alone and behind ranges that go past it;
+# rows one short of and one past a row tile; workgroups that share a CU, and too many for their places in LDS (the packed form)
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("M,K,N,row_tiles,split", [(31, 96, 32, 1, 1), (33, 160, 96, 1, 2), (65, 352, 1056, 2, 1), (63, 96, 2016, 2, 3),
+                                                   (40, 9600, 224, 1, 3), (40, 9600, 544, 2, 1), (33, 17408, 96, 1, 1), (9, 64, 16416, 1, 1)])
+def test_transposed_rows_of_the_gradient_without_the_pack_pass(dev, bits, M, K, N, row_tiles, split):
+    for desc_act in (False, True):
+        L = layer(3700 + N, K, N, bits, 32, desc_act)
+        D = to_dev(L, dev)
+        plan = _lib.select_tiled_transposed(M, K, N, bits, 32)
+        plan.row_tiles, plan.m_blocks = row_tiles, -(-M // (32 * row_tiles))
+        plan.grid_z, plan.split_k, plan.grid_y = plan.m_blocks, split, split
+        plan.k_chunk = -(-(-(-N // 64)) // (plan.waves_k * split))
+        plan.lds_bytes = max(plan.waves_k * row_tiles * 2 * 4096, 2 * plan.waves_k * plan.k_chunk * 256)
+        part = (split * M * K * 4 + 255) // 256 * 256 if split > 1 else 0
+        plan.workspace_bytes = 16384 + part + split * plan.waves_k * plan.k_chunk * 4 * row_tiles * plan.m_blocks * 1024
+        prep = prepare(D)
+        gy = grad_rows(3710 + M, M, N)
+        # what lies before and behind the rows is not read, whatever it holds
+        room = torch.full((M + 2, N), float("nan"), dtype=torch.float16, device=dev)
+        room[1:-1] = gy.to(dev)
+        got = run_t(D, prep, room[1:-1], plan=plan)
+        want = gy.float() @ expected_weight(L).float().t()
+        what = f"transposed bits={bits} K={K} N={N} M={M} row_tiles={row_tiles} split={split} act={desc_act}"
+        assert_close(got, want, what)
+        assert_tight(got, want, what)
+        assert torch.equal(got, run_t(D, prep, room[1:-1], plan=plan)), "two identical calls differ"
