@@ -488,10 +488,8 @@ extern "C" int gptq_hip_gemm_tiled_transposed(const void *gy, const void *qtile_
     if ((long long)K * ((N + 63) / 64 * 64) * bits / 8 >= (1LL << 32)) return GPTQ_HIP_ERR_UNSUPPORTED;
     gptq_hip_plan chosen;
     if (!plan) {
-        int rc = gptq::gptq_panel_plan_within(M, K, N, bits, group_size, GPTQ_HIP_PANEL_TRANSPOSED | (xsrc ? GPTQ_HIP_PANEL_ACT_ORDER : 0),
-                                              workspace && aligned(workspace, 16) ? workspace_bytes : 0, &chosen);
-        if (rc != GPTQ_HIP_OK)
-            rc = gptq_hip_select_tiled_transposed(M, K, N, bits, group_size, &chosen);
+        const int rc = gptq::gptq_transposed_plan_within(M, K, N, bits, group_size, xsrc != nullptr,
+                                                         workspace && aligned(workspace, 16) ? workspace_bytes : 0, &chosen);
         if (rc != GPTQ_HIP_OK) return rc;
         plan = &chosen;
     }

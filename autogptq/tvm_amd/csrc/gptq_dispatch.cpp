@@ -735,7 +735,9 @@ extern "C" int gptq::gptq_tiled_default_plan(int M, int K, int N, int bits, int 
 
 // The transposed product gx[M, K] = gy[M, N] @ W^T on the matmul kernel: the reduction runs over the layer's N
 // columns (blocks of 64), the result has K columns (tiles of 32 positions, two per workgroup).
-extern "C" int gptq_hip_select_tiled_transposed(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
+static void matmul_t_plan(int M, int K, int N, int bits, int at, int split, gptq_hip_plan *plan);
+
+static int plan_tiled_transposed(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
 {
     const int ok = tiled_args_ok(M, K, N, bits, group_size, plan);
     if (ok != GPTQ_HIP_OK) return ok;
@@ -765,25 +767,29 @@ extern "C" int gptq_hip_select_tiled_transposed(int M, int K, int N, int bits, i
     // the table of a workgroup's K range must fit its LDS
     while (ceil_div(S_total, split * kwv) * kwv > gptq::kTiledTMaxBlocks) split++;
     if (split > 1 && (long long)M * K >= (1LL << 32)) return GPTQ_HIP_ERR_UNSUPPORTED;
-    const int wave_steps = ceil_div(S_total, split * kwv);
-    split = ceil_div(S_total, wave_steps * kwv);
+    matmul_t_plan(M, K, N, bits, at, split, plan);
+    return GPTQ_HIP_OK;
+}
+
+// the matmul kernel's plan in blocks of 32 at rows and `split` ranges of the reduction, or fewer where those come out empty
+static void matmul_t_plan(int M, int K, int N, int bits, int at, int split, gptq_hip_plan *plan)
+{
+    const int S_total = ceil_div(N, 64), kwv = 4;
     plan->kernel = GPTQ_HIP_KERNEL_TILED;
     plan->row_tiles = at;
-    plan->m_blocks = m_blocks;
+    plan->m_blocks = plan->grid_z = ceil_div(M, 32 * at);
     plan->waves_n = 1;
     plan->waves_k = kwv;
-    plan->split_k = split;
-    plan->k_chunk = wave_steps;
-    plan->grid_x = col_pairs;
-    plan->grid_y = split;
-    plan->grid_z = m_blocks;
+    plan->k_chunk = ceil_div(S_total, split * kwv);
+    plan->split_k = plan->grid_y = ceil_div(S_total, plan->k_chunk * kwv);
+    plan->grid_x = ceil_div(K / 32, 2);
     plan->block = 64 * kwv;
-    plan->lds_bytes = gptq::tiled_t_lds_bytes(at, kwv, wave_steps);
+    plan->lds_bytes = gptq::tiled_t_lds_bytes(at, kwv, plan->k_chunk);
+    plan->flags = 0;
     size_t ws = gptq::kCounterBytes;
-    if (split > 1) ws += ((size_t)split * M * K * sizeof(float) + 255) / 256 * 256;
-    ws += (size_t)gptq::tiled_pack_blocks(split, kwv, wave_steps) * 4 * (size_t)(at * m_blocks) * 1024;
+    if (plan->split_k > 1) ws += ((size_t)plan->split_k * M * K * sizeof(float) + 255) / 256 * 256;
+    ws += (size_t)gptq::tiled_pack_blocks(plan->split_k, kwv, plan->k_chunk) * 4 * (size_t)(at * plan->m_blocks) * 1024;
     plan->workspace_bytes = ws;
-    return GPTQ_HIP_OK;
 }
 
 namespace {
@@ -903,7 +909,7 @@ static int plan_panel(int M, int K, int N, int bits, int group_size, unsigned fl
             // an activation order: a pass that puts x (or the result) in the layer's order
             if (act) best += transposed ? 2.5 + 0.9e-6 * M * K : 3.5 + 0.7e-6 * M * K;
             gptq_hip_plan other;
-            const int rc = transposed ? gptq_hip_select_tiled_transposed(M, K, N, bits, group_size, &other)
+            const int rc = transposed ? plan_tiled_transposed(M, K, N, bits, group_size, &other)
                                       : gptq_hip_select_tiled(M, K, N, bits, group_size, &other);
             if (rc == GPTQ_HIP_OK && other.kernel != GPTQ_HIP_KERNEL_TILED) return GPTQ_HIP_ERR_UNSUPPORTED;
             if (rc == GPTQ_HIP_OK) {
@@ -939,10 +945,108 @@ static int plan_panel(int M, int K, int N, int bits, int group_size, unsigned fl
     return GPTQ_HIP_OK;
 }
 
+namespace {
+
+// ---- Gradients of 32 to 383 rows of layers within 20480 x 32768: matmul or PANEL plan by two models of both kernels, fitted to 8000 measurements
+// (graph, weights cold) of every row tile and range of 210 calls drawn at random (32 to 600 rows, all widths, with and without an activation order;
+// 6.4 and 5.5 % rms near the best plan).  From 384 rows on a module whose gradient has no PANEL plan takes the library's product: the choice stays. ----
+
+double matmul_t_us(const gptq_hip_plan &p, int M, int K, int N, int bits, bool act)
+{
+    static const double kBlock[3] = {0.817, 1.009, 1.351}, kTurn[3] = {0.87, 2.02, 4.17}, kIdle[3] = {0.79, 0.81, 0.72}, kNext[3] = {0.63, 0.74, 0.84};
+    const int i = p.row_tiles == 1 ? 0 : (p.row_tiles == 2 ? 1 : 2);   // row tiles 1, 2, 4
+    const double block = kBlock[i] * (bits == 8 ? 1.311 : (bits == 3 ? 0.869 : 1.0));
+    auto turn = [&](double n) { return p.k_chunk * block * (kIdle[i] + (1 - kIdle[i]) * n / 256) + kTurn[i]; };
+    const long long wgs = (long long)p.grid_x * p.split_k * p.m_blocks, full = wgs / 256, last = wgs % 256;
+    double us = full * turn(256) + (last ? turn((double)last) : 0.0);
+    if (wgs > 256) us = turn(256) + kNext[i] * (us - turn(256));
+    return 3.5 + us + (p.split_k > 1 ? 1.22 + 2.26e-6 * p.split_k * M * K : 0.0) + (gptq::tiled_t_stages_x(N, p) ? 0.0 : 4.25e-6 * M * N) +
+           (act ? 4.38e-6 * M * K : 0.0);
+}
+
+double panel_t_us(const gptq_hip_plan &p, int M, int K, int N, int bits, bool act)
+{
+    const int rt = p.row_tiles;
+    const double step = (rt <= 4 ? 0.236 + 0.095 * rt : 0.291 + 0.112 * rt) + (bits == 8 || bits == 3 ? 0.087 : 0.0);
+    auto turn = [&](double n) { return p.k_chunk * step * (0.859 + 0.141 * n / 256) + 1.88 + 0.858 * rt; };
+    const long long wgs = (long long)p.grid_x * p.split_k * p.m_blocks, full = wgs / 256, last = wgs % 256;
+    const double ordered = !act ? 0.0 : (p.split_k > 1 || gptq::panel_scatters(M, K) ? 0.56 + 0.423e-3 * K : 4.88 + 5.95e-6 * M * K);
+    return 2.74 + full * turn(256) + (last ? turn((double)last) : 0.0) + (p.split_k > 1 ? 2.91 + 0.748e-6 * p.split_k * M * K : 0.0) + ordered +
+           0.0369e-6 * K * N * bits / 8;
+}
+
+// The plan of such a gradient that has one, replaced by the one that the models name where they give it 5 % at least; panels: PANEL plans are
+// among the choices.  Without that margin six of the 210 calls were slower by more than 3 %, with it three (the worst 1.19 x).  On 154 calls drawn
+// since it moves 16, none to a slower plan, 1.25 x as fast on the mean with the pass for the gradient's rows gone in both where it is gone (us, graph:
+// 68 rows of 1344 x 11008 int4, four row tiles in 11 ranges 23.1, one in four 17.4; 86 of 5248 x 1088 15.0 -> 11.1; to PANEL, all with an
+// activation order: 296 of 5376 x 2144 31.7 -> 21.2, 208 of 6912 x 1728 27.1 -> 19.3, 86 of 11328 x 3136 int4 1.09 x).
+bool short_gradient(int M, int K, int N) { return M >= 32 && M < 384 && K <= 20480 && N <= 32768; }
+void refine_short_gradient(int M, int K, int N, int bits, int group_size, bool act, bool panels, gptq_hip_plan *plan)
+{
+    const bool panel = plan->kernel == GPTQ_HIP_KERNEL_PANEL;
+    if (!short_gradient(M, K, N) || (panel && gptq::panel_main_blocks(*plan) != 0)) return;
+    double best = 0.95 * (panel ? panel_t_us(*plan, M, K, N, bits, act) : matmul_t_us(*plan, M, K, N, bits, act));
+    gptq_hip_plan other = *plan, found = *plan;
+    const int S_total = ceil_div(N, 64);
+    // (the partial tiles of a matmul plan stay within three times the packed weights, as in its own planner)
+    const long long cap = (3LL * N * bits) / (128LL * M);
+    for (int at = 1; at <= 4; at *= 2) {
+        const long long tiles = (long long)ceil_div(K / 32, 2) * ceil_div(M, 32 * at);
+        if (at > 1 && 16 * at >= M) continue;
+        for (int s = 1; s <= 8; s++) {
+            if (s > 1 && (s > cap || tiles * s > 520 || S_total / (4 * s) < 2)) break;
+            matmul_t_plan(M, K, N, bits, at, s, &other);
+            if (other.split_k != s || 4 * other.k_chunk > gptq::kTiledTMaxBlocks) continue;
+            const double us = matmul_t_us(other, M, K, N, bits, act);
+            if (us < best) best = us, found = other;
+        }
+    }
+    const unsigned flags = GPTQ_HIP_PANEL_TRANSPOSED | (act ? GPTQ_HIP_PANEL_ACT_ORDER : 0);
+    for (int rt = 1; panels && rt <= gptq::kPanelMaxTiles && (rt == 1 || 32 * (rt - 1) < M); rt++) {
+        const long long tiles = (long long)ceil_div(K, gptq::kPanelCols) * ceil_div(M, 32 * rt);
+        for (int s = 1; s <= 8; s++) {
+            if (s > 1 && (S_total / s < 6 || tiles * s > 520 || (double)s * M * K > 48e6)) break;
+            if (plan_panel(M, K, N, bits, group_size, flags, rt, s, false, &other) != GPTQ_HIP_OK || other.split_k != s) continue;
+            const double us = panel_t_us(other, M, K, N, bits, act);
+            if (us < best) best = us, found = other;
+        }
+    }
+    *plan = found;
+}
+
+}  // namespace
+
 extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_size, unsigned flags, int row_tiles, int split_k,
                                      gptq_hip_plan *plan)
 {
-    return plan_panel(M, K, N, bits, group_size, flags, row_tiles, split_k, true, plan);
+    int rc = plan_panel(M, K, N, bits, group_size, flags, row_tiles, split_k, true, plan);
+    if ((rc == GPTQ_HIP_OK || rc == GPTQ_HIP_ERR_UNSUPPORTED) && row_tiles == 0 && split_k == 0 && (flags & GPTQ_HIP_PANEL_TRANSPOSED) &&
+        short_gradient(M, K, N) && (rc == GPTQ_HIP_OK || plan_tiled_transposed(M, K, N, bits, group_size, plan) == GPTQ_HIP_OK)) {
+        refine_short_gradient(M, K, N, bits, group_size, flags & GPTQ_HIP_PANEL_ACT_ORDER, true, plan);
+        rc = plan->kernel == GPTQ_HIP_KERNEL_PANEL ? GPTQ_HIP_OK : GPTQ_HIP_ERR_UNSUPPORTED;
+    }
+    return rc;
+}
+
+extern "C" int gptq_hip_select_tiled_transposed(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
+{
+    const int rc = plan_tiled_transposed(M, K, N, bits, group_size, plan);
+    if (rc == GPTQ_HIP_OK) refine_short_gradient(M, K, N, bits, group_size, false, false, plan);
+    return rc;
+}
+
+// The plan of a gradient that names none and brings `have` bytes of workspace: the one that the two entries above name, else what
+// the rules before the models name within that memory, so that a caller with a workspace for those is not refused.
+extern "C" int gptq::gptq_transposed_plan_within(int M, int K, int N, int bits, int group_size, bool act, size_t have, gptq_hip_plan *plan)
+{
+    const unsigned flags = GPTQ_HIP_PANEL_TRANSPOSED | (act ? GPTQ_HIP_PANEL_ACT_ORDER : 0);
+    if (short_gradient(M, K, N)) {
+        int rc = gptq_hip_select_panel(M, K, N, bits, group_size, flags, 0, 0, plan);
+        if (rc == GPTQ_HIP_ERR_UNSUPPORTED) rc = gptq_hip_select_tiled_transposed(M, K, N, bits, group_size, plan);
+        if (rc == GPTQ_HIP_OK && plan->workspace_bytes <= have) return rc;
+    }
+    const int rc = gptq_panel_plan_within(M, K, N, bits, group_size, flags, have, plan);
+    return rc == GPTQ_HIP_OK ? rc : plan_tiled_transposed(M, K, N, bits, group_size, plan);
 }
 
 // The PANEL plan of a call that names none and brings `have` bytes of workspace.  K ranges for the last row blocks take up to

@@ -247,6 +247,7 @@ constexpr int kShortPlanRows = 320;
 void refine_short_plan(int M, int K, int N, int bits, int group_size, bool act_order, gptq_hip_plan *plan);
 // the PANEL plan of a call that names none, if one fits its workspace;
 extern "C" int gptq_panel_plan_within(int M, int K, int N, int bits, int group_size, unsigned flags, size_t have, gptq_hip_plan *plan);
+extern "C" int gptq_transposed_plan_within(int M, int K, int N, int bits, int group_size, bool act, size_t have, gptq_hip_plan *plan);
 // the plan of a gptq_hip_gemm_tiled call that names none, and whether the call clears the slots of its halved tiles (the tests ask, too)
 extern "C" int gptq_tiled_default_plan(int M, int K, int N, int bits, int group_size, int act_order, size_t have, gptq_hip_plan *plan,
                                        int *clear);

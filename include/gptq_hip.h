@@ -277,7 +277,9 @@ int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint32_t *sz, co
  * each sorted position), NULL without an activation order; gy and gx are in the layer's own channel order.  The
  * weights are formed exactly as in the forward product (fp16(scale * (q - zero)), one rounding), sums are fp32.
  * plan: NULL = gptq_hip_select_panel (transposed) where that names a plan and the workspace holds its bytes, with or without ranges
- * for the last row blocks, else gptq_hip_select_tiled_transposed.  workspace: plan.workspace_bytes, zeroed once.
+ * for the last row blocks, else gptq_hip_select_tiled_transposed; for 32 to 383 rows, where both entries know a faster plan than the
+ * general rules, the rules' plan where the workspace holds that one only.  Matmul plans: a pass packs gy first, but for one and two row
+ * tiles in launches that fill the chip once.  workspace: plan.workspace_bytes, zeroed once.
  */
 size_t gptq_hip_tiled_transposed_bytes(int K, int N, int bits);
 size_t gptq_hip_tiled_transposed_table_bytes(int K, int N, int group_size);

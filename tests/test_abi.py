@@ -691,3 +691,44 @@ def test_short_calls_take_the_plan_that_the_models_name():
                 assert r.as_dict() == _lib.select_panel(M, K, N, bits, gs, act, False, r.row_tiles, r.split_k).as_dict()
         assert _lib.select_route(M, K, N, bits, gs, act, _lib.COPY_TILED).plan.as_dict() == old.as_dict()
     assert moved > 15
+
+
+def test_short_gradients_take_the_plan_that_the_models_name():
+    """Gradients of 32 to 383 rows: a matmul or PANEL plan gives way to a clearly faster one; a call without a plan takes it where its workspace
+    does, and no call is refused that has the workspace of the plan that the rules before the models name."""
+    import random
+
+    size, lib = ctypes.c_size_t, _lib.lib()
+
+    def within(M, K, N, bits, gs, act, have):
+        plan = _lib.Plan()
+        rc = lib.gptq_transposed_plan_within(M, K, N, bits, gs, ctypes.c_bool(act), size(have), ctypes.byref(plan))
+        assert rc == _lib.OK
+        return plan
+
+    # measured (us, graph, the rules' plan / this): 23.1 / 17.4, 15.0 / 11.1, 27.1 / 19.3, 31.7 / 21.2, 18.8 / 14.5
+    for M, K, N, bits, gs, act, kind, rt, split in ((68, 1344, 11008, 4, 32, True, _lib.KERNEL_TILED, 1, 4), (86, 5248, 1088, 4, 64, True, _lib.KERNEL_TILED, 1, 1),
+                                                    (208, 6912, 1728, 4, 128, True, _lib.KERNEL_PANEL, 1, 1), (296, 5376, 2144, 4, 128, True, _lib.KERNEL_PANEL, 1, 1)):
+        p = within(M, K, N, bits, gs, act, 1 << 40)
+        assert (p.kernel, p.row_tiles, p.split_k) == (kind, rt, split), (M, K, N, p.as_dict())
+    rng, moved = random.Random(5), 0
+    for _ in range(500):
+        gs = rng.choice((128, 64, 32, -1))
+        unit = 32 if gs == -1 else gs
+        M, bits, act = rng.choice((9, 31, 32, 33, 64, 65, 128, 129, 256, 383, 384, 700)), rng.choice((2, 3, 4, 8)), rng.random() < 0.5
+        K, N = unit * rng.randint(1, 20480 // unit), 32 * rng.randint(1, 600)
+        own = _lib.select_panel(M, K, N, bits, gs, act, transposed=True) or _lib.select_tiled_transposed(M, K, N, bits, gs)
+        assert within(M, K, N, bits, gs, act, 1 << 40).as_dict() == own.as_dict(), (M, K, N, bits, gs, act)
+        blocks = -(-N // 64)
+        if own.kernel == _lib.KERNEL_TILED:
+            assert own.m_blocks * own.row_tiles * 32 >= M and own.split_k * 4 * own.k_chunk >= blocks > (own.split_k - 1) * 4 * own.k_chunk
+            assert 2 * 4 * own.k_chunk * 256 <= own.lds_bytes <= 160 * 1024
+        else:
+            again = _lib.select_panel(M, K, N, bits, gs, act, True, own.row_tiles, own.split_k)
+            assert own.flags or own.as_dict() == again.as_dict()
+        # one byte short of it: what the rules name, which is what every size outside of the models' range has
+        if own.workspace_bytes and 32 <= M < 384:
+            less = within(M, K, N, bits, gs, act, own.workspace_bytes - 1)
+            moved += less.workspace_bytes < own.workspace_bytes
+            assert less.as_dict() != own.as_dict() or less.kernel == _lib.KERNEL_TILED
+    assert moved > 5
