@@ -964,14 +964,13 @@ double matmul_t_us(const gptq_hip_plan &p, int M, int K, int N, int bits, bool a
            (act ? 4.38e-6 * M * K : 0.0);
 }
 
-double panel_t_us(const gptq_hip_plan &p, int M, int K, int N, int bits, bool act)
+double panel_t_us(int rt, int split, int chunk, long long wgs, int M, int K, int N, int bits, bool act)
 {
-    const int rt = p.row_tiles;
     const double step = (rt <= 4 ? 0.236 + 0.095 * rt : 0.291 + 0.112 * rt) + (bits == 8 || bits == 3 ? 0.087 : 0.0);
-    auto turn = [&](double n) { return p.k_chunk * step * (0.859 + 0.141 * n / 256) + 1.88 + 0.858 * rt; };
-    const long long wgs = (long long)p.grid_x * p.split_k * p.m_blocks, full = wgs / 256, last = wgs % 256;
-    const double ordered = !act ? 0.0 : (p.split_k > 1 || gptq::panel_scatters(M, K) ? 0.56 + 0.423e-3 * K : 4.88 + 5.95e-6 * M * K);
-    return 2.74 + full * turn(256) + (last ? turn((double)last) : 0.0) + (p.split_k > 1 ? 2.91 + 0.748e-6 * p.split_k * M * K : 0.0) + ordered +
+    auto turn = [&](double n) { return chunk * step * (0.859 + 0.141 * n / 256) + 1.88 + 0.858 * rt; };
+    const long long full = wgs / 256, last = wgs % 256;
+    const double ordered = !act ? 0.0 : (split > 1 || gptq::panel_scatters(M, K) ? 0.56 + 0.423e-3 * K : 4.88 + 5.95e-6 * M * K);
+    return 2.74 + full * turn(256) + (last ? turn((double)last) : 0.0) + (split > 1 ? 2.91 + 0.748e-6 * split * M * K : 0.0) + ordered +
            0.0369e-6 * K * N * bits / 8;
 }
 
@@ -985,7 +984,8 @@ void refine_short_gradient(int M, int K, int N, int bits, int group_size, bool a
 {
     const bool panel = plan->kernel == GPTQ_HIP_KERNEL_PANEL;
     if (!short_gradient(M, K, N) || (panel && gptq::panel_main_blocks(*plan) != 0)) return;
-    double best = 0.95 * (panel ? panel_t_us(*plan, M, K, N, bits, act) : matmul_t_us(*plan, M, K, N, bits, act));
+    double best = 0.95 * (panel ? panel_t_us(plan->row_tiles, plan->split_k, plan->k_chunk, (long long)plan->grid_x * plan->split_k * plan->m_blocks, M, K, N, bits, act)
+                                : matmul_t_us(*plan, M, K, N, bits, act));
     gptq_hip_plan other = *plan, found = *plan;
     const int S_total = ceil_div(N, 64);
     // (the partial tiles of a matmul plan stay within three times the packed weights, as in its own planner)
@@ -1006,9 +1006,10 @@ void refine_short_gradient(int M, int K, int N, int bits, int group_size, bool a
         const long long tiles = (long long)ceil_div(K, gptq::kPanelCols) * ceil_div(M, 32 * rt);
         for (int s = 1; s <= 8; s++) {
             if (s > 1 && (S_total / s < 6 || tiles * s > 520 || (double)s * M * K > 48e6)) break;
-            if (plan_panel(M, K, N, bits, group_size, flags, rt, s, false, &other) != GPTQ_HIP_OK || other.split_k != s) continue;
-            const double us = panel_t_us(other, M, K, N, bits, act);
-            if (us < best) best = us, found = other;
+            const int chunk = ceil_div(S_total, s);
+            if (ceil_div(S_total, chunk) != s) continue;
+            const double us = panel_t_us(rt, s, chunk, tiles * s, M, K, N, bits, act);
+            if (us < best && plan_panel(M, K, N, bits, group_size, flags, rt, s, false, &other) == GPTQ_HIP_OK) best = us, found = other;
         }
     }
     *plan = found;
