@@ -335,7 +335,6 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
     const int rt0 = (blockIdx.z * RW + rw) * AT;
     const int S_begin = (split * KW + kw) * p.wave_steps;
     const int S_last = p.S_total - 1;
-    const int lb_last = 2 * p.S_total - 1;
 
     // per-lane offsets that never change; the block number lives in scalar registers
     uint32_t tile_off[CT], col[CT];
@@ -343,7 +342,7 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
     for (int ct = 0; ct < CT; ct++) {
         const int T = min(T0 + ct, p.T_total - 1);  // a missing tile repeats the last one; it is never stored
         tile_off[ct] = (uint32_t)T * (uint32_t)p.S_total;
-        col[ct] = (uint32_t)(32 * T + n);
+        col[ct] = (uint32_t)(32 * T + n) * 4u;   // (its (scale, zero) word in bytes)
     }
     const uint32_t b_lane = tile_lane_bytes<BITS>((uint32_t)lane);
     const uint32_t a_lane = (uint32_t)rt0 * 1024u + (uint32_t)lane * 16u;
@@ -352,14 +351,20 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
     uint32_t w[RING][CT][BITS];
     uint32_t szr[RING][CT];
     h8 a[RING][4][AT];
+    // The (scale, zero) words as a buffer (less than 2^31 bytes: an eighth of the codes' number).  A lane block past K reads its word from
+    // behind it, zeros: x is zero there, but times an infinite weight of the last group that would be NaN.  (On 280 drawn calls, graph, the
+    // forms of the forward product cost between 0.5 % less and 0.6 % more than with the last group's words, the gradient's 0.3 to 0.6 % more.)
+    const __amdgpu_buffer_rsrc_t szb = tile_buffer((const char *)p.sz, TRANS ? 0u : (uint32_t)p.G * (uint32_t)p.N * 4u);
+    const uint32_t row_bytes = (uint32_t)p.N * 4u;
+    const uint32_t lb_end = DIRECT ? 0xffffffffu : (uint32_t)p.K >> 5;   // (DIRECT: no wave walks past K)
     auto load_b = [&](int S, uint32_t (&wr)[CT][BITS], uint32_t (&sr)[CT]) {
-        const int Sc = min(S, S_last);  // blocks past K repeat the last one (their x is zero)
-        const uint32_t lb = (uint32_t)min(2 * S + h, lb_last);
-        const uint32_t g = min(lb / (uint32_t)p.lb_per_group, (uint32_t)p.G - 1u);
+        const int Sc = min(S, S_last);  // blocks past K repeat the last one
+        const uint32_t lb = (uint32_t)(2 * S + h);
+        const uint32_t row = lb < lb_end ? min(lb / (uint32_t)p.lb_per_group, (uint32_t)p.G - 1u) * row_bytes : 0x80000000u;
 #pragma unroll
         for (int ct = 0; ct < CT; ct++) {
             tile_load<BITS>(p.qtile + ((size_t)(tile_off[ct] + (uint32_t)Sc) * (256u * BITS) + b_lane), wr[ct]);
-            if constexpr (!TRANS) sr[ct] = p.sz[(size_t)g * p.N + col[ct]];
+            if constexpr (!TRANS) sr[ct] = __builtin_amdgcn_raw_buffer_load_b32(szb, row + col[ct], 0, 0);
         }
     };
     // DIRECT: the lane's rows of x, at its half of a block
@@ -456,11 +461,14 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
     // [ct][block of the range][octet][8 words]
     if constexpr (TRANS) {
         u4 *tbl = (u4 *)smem;
+        const __amdgpu_buffer_rsrc_t sztb = tile_buffer((const char *)p.szt, (uint32_t)p.G * (uint32_t)p.S_total * 256u);
         for (int i = tid; i < CT * wg_blocks * 16; i += 64 * RW * KW) {
             const int ct = i / (wg_blocks * 16), r = i - ct * (wg_blocks * 16);
-            const int Sc = min(S_wg0 + (r >> 4), S_last);   // (blocks past K repeat the last one: their x is zero)
-            const int g = min(T0 + ct, p.T_total - 1) / p.tiles_per_group;
-            tbl[i] = *(const u4 *)(p.szt + ((size_t)g * p.S_total + Sc) * 64 + (r & 15) * 4);
+            const int S = S_wg0 + (r >> 4);
+            const uint32_t g = (uint32_t)(min(T0 + ct, p.T_total - 1) / p.tiles_per_group);
+            // (blocks past the reduction have no scale, as in the forward product; columns past it have none in szt)
+            const uint32_t at = S <= S_last ? (g * (uint32_t)p.S_total + (uint32_t)S) * 256u + (uint32_t)(r & 15) * 16u : 0x80000000u;
+            tbl[i] = __builtin_amdgcn_raw_buffer_load_b128(sztb, at, 0, 0);
         }
         __syncthreads();
     }
