@@ -1036,8 +1036,10 @@ extern "C" int gptq_hip_select_tiled_transposed(int M, int K, int N, int bits, i
     return rc;
 }
 
-// The plan of a gradient that names none and brings `have` bytes of workspace: the one that the two entries above name, else what
-// the rules before the models name within that memory, so that a caller with a workspace for those is not refused.
+// The plan of a gradient that names none and brings `have` bytes of workspace: the one that the two entries above name, else what the rules
+// before the models name within that memory, else gptq_hip_select_tiled_transposed's plan beside a PANEL plan that does not fit: a caller
+// is not refused that has the workspace of any of them (the rules' matmul plan takes more than the models' on a twentieth of drawn layers,
+// 193 rows of 320 x 2880 int2 1.59 and 1.39 MB).
 extern "C" int gptq::gptq_transposed_plan_within(int M, int K, int N, int bits, int group_size, bool act, size_t have, gptq_hip_plan *plan)
 {
     const unsigned flags = GPTQ_HIP_PANEL_TRANSPOSED | (act ? GPTQ_HIP_PANEL_ACT_ORDER : 0);
@@ -1046,8 +1048,13 @@ extern "C" int gptq::gptq_transposed_plan_within(int M, int K, int N, int bits, 
         if (rc == GPTQ_HIP_ERR_UNSUPPORTED) rc = gptq_hip_select_tiled_transposed(M, K, N, bits, group_size, plan);
         if (rc == GPTQ_HIP_OK && plan->workspace_bytes <= have) return rc;
     }
-    const int rc = gptq_panel_plan_within(M, K, N, bits, group_size, flags, have, plan);
-    return rc == GPTQ_HIP_OK ? rc : plan_tiled_transposed(M, K, N, bits, group_size, plan);
+    int rc = gptq_panel_plan_within(M, K, N, bits, group_size, flags, have, plan);
+    if (rc == GPTQ_HIP_OK) return rc;
+    rc = plan_tiled_transposed(M, K, N, bits, group_size, plan);
+    gptq_hip_plan other = *plan;
+    if (rc == GPTQ_HIP_OK && plan->workspace_bytes > have) refine_short_gradient(M, K, N, bits, group_size, false, false, &other);
+    if (other.workspace_bytes <= have) *plan = other;
+    return rc;
 }
 
 // The PANEL plan of a call that names none and brings `have` bytes of workspace.  K ranges for the last row blocks take up to

@@ -732,3 +732,32 @@ def test_short_gradients_take_the_plan_that_the_models_name():
             moved += less.workspace_bytes < own.workspace_bytes
             assert less.as_dict() != own.as_dict() or less.kernel == _lib.KERNEL_TILED
     assert moved > 5
+
+
+def test_gradients_without_a_plan_take_the_workspace_of_any_plan_that_is_offered():
+    """A call that names no plan is sized by what the library answers: gptq_hip_select_panel's plan, gptq_hip_select_tiled_transposed's, or (by callers that
+    kept the answer) what the rules before the models named.  Whichever it brings, it gets a plan that fits."""
+    import random
+
+    size, lib = ctypes.c_size_t, _lib.lib()
+    rng = random.Random(11)
+    shapes = [(193, 320, 2880, 2, 64, False), (147, 16704, 3776, 2, 32, True)]     # (the rules' matmul plan takes more than the models')
+    for _ in range(3000):
+        gs = rng.choice((128, 64, 32, -1))
+        unit = 32 if gs == -1 else gs
+        shapes.append((rng.randint(20, 400), unit * max(1, int(2 ** rng.uniform(5, 14.4)) // unit), 32 * max(1, int(2 ** rng.uniform(5, 15)) // 32),
+                       rng.choice((2, 3, 4, 8)), gs, rng.random() < 0.5))
+    for M, K, N, bits, gs, act in shapes:
+        tiled, panel = _lib.select_tiled_transposed(M, K, N, bits, gs), _lib.select_panel(M, K, N, bits, gs, act, transposed=True)
+        for have in {tiled.workspace_bytes, (panel or tiled).workspace_bytes, 1 << 40}:
+            plan = _lib.Plan()
+            assert lib.gptq_transposed_plan_within(M, K, N, bits, gs, ctypes.c_bool(act), size(have), ctypes.byref(plan)) == _lib.OK
+            what = (M, K, N, bits, gs, act, have, plan.as_dict())
+            assert plan.workspace_bytes <= have, what
+            blocks = -(-N // 64)
+            assert 32 * plan.row_tiles * plan.m_blocks >= M, what
+            if plan.kernel == _lib.KERNEL_TILED:
+                assert plan.split_k * 4 * plan.k_chunk >= blocks > (plan.split_k - 1) * 4 * plan.k_chunk, what
+                assert plan.grid_x == -(-(K // 32) // 2) and (plan.grid_y, plan.grid_z) == (plan.split_k, plan.m_blocks), what
+            else:
+                assert plan.kernel == _lib.KERNEL_PANEL and plan.split_k * plan.k_chunk >= blocks > (plan.split_k - 1) * plan.k_chunk, what
