@@ -701,6 +701,9 @@ static int plan_tiled(int M, int K, int N, int bits, int group_size, bool settle
     return GPTQ_HIP_OK;
 }
 
+static int plan_panel(int M, int K, int N, int bits, int group_size, unsigned flags, int row_tiles, int split_k, bool tails,
+                      gptq_hip_plan *plan);
+
 extern "C" int gptq_hip_select_tiled(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
 {
     return plan_tiled(M, K, N, bits, group_size, false, plan);
@@ -715,12 +718,29 @@ extern "C" int gptq::gptq_tiled_default_plan(int M, int K, int N, int bits, int 
                                              int *clear)
 {
     *clear = 0;
-    int rc = gptq_panel_plan_within(M, K, N, bits, group_size, act_order ? GPTQ_HIP_PANEL_ACT_ORDER : 0, have, plan);
-    if (rc != GPTQ_HIP_OK) rc = gptq_hip_select_tiled(M, K, N, bits, group_size, plan);
-    if (rc != GPTQ_HIP_OK) return rc;
-    gptq_hip_plan other = *plan;
-    refine_short_plan(M, K, N, bits, group_size, act_order, &other);
-    if (plan->workspace_bytes <= have && other.workspace_bytes <= have) *plan = other;
+    gptq_hip_plan other;
+    int rc = GPTQ_HIP_ERR_UNSUPPORTED;
+    // `plan` by the rules, or in its place the models' where both fit; the route's own plan (tails) also where it alone does: it may take fewer
+    // bytes than either kernel's by the rules (66 rows of 15264 x 960 int3 4.2 MB, 7.8)
+    auto fits = [&](bool alone) {
+        other = *plan;
+        refine_short_plan(M, K, N, bits, group_size, act_order, &other);
+        const bool ok = plan->workspace_bytes <= have;
+        if ((ok || alone) && other.workspace_bytes <= have) *plan = other;
+        return plan->workspace_bytes <= have;
+    };
+    bool taken = false;
+    for (const bool tails : {true, false}) {
+        rc = plan_panel(M, K, N, bits, group_size, act_order ? GPTQ_HIP_PANEL_ACT_ORDER : 0, 0, 0, tails, plan);
+        if (rc != GPTQ_HIP_OK && rc != GPTQ_HIP_ERR_UNSUPPORTED) return rc;
+        taken = rc == GPTQ_HIP_OK && fits(tails);
+        if (taken) break;
+    }
+    if (!taken) {
+        rc = gptq_hip_select_tiled(M, K, N, bits, group_size, plan);
+        if (rc != GPTQ_HIP_OK) return rc;
+        fits(false);
+    }
     // row blocks need no workspace, but a call without the one that its size asks for stays refused
     if (plan->workspace_bytes <= have && !matmul_keeps(M, K, N, bits, group_size, act_order) &&
         select_row_blocks(M, K, N, bits, group_size, &other))

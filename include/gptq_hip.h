@@ -249,7 +249,7 @@ int gptq_hip_select_tiled_decode(int M, int K, int N, int bits, int group_size, 
  * NULL means no activation order; pass both or neither).  plan: NULL = what gptq_hip_select_route names for a layer
  * with this copy alone, PANEL included; where the workspace does not hold that plan's bytes, the PANEL plan without ranges for the
  * last row blocks, then gptq_hip_select_tiled.  A call that neither of these PANEL plans takes brings the workspace of
- * gptq_hip_select_tiled's plan, or is refused: also where it would run on row blocks, which need none.  workspace:
+ * gptq_hip_select_tiled's plan, or is refused: also where it would run on row blocks, which need none, or on a plan of fewer bytes.  workspace:
  * plan.workspace_bytes (none for most decode plans).  Decode plans: one launch; matmul plans: one without
  * an activation order, two with one (pack pass, matmul) or with 128 columns per wave; one more when the plan splits K.  A plan whose flags hold
  * GPTQ_HIP_PLAN_PRIVATE_ZERO_WORKSPACE wants ALL bytes of its workspace zero at the first call and leaves them zero

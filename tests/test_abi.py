@@ -761,3 +761,27 @@ def test_gradients_without_a_plan_take_the_workspace_of_any_plan_that_is_offered
                 assert plan.grid_x == -(-(K // 32) // 2) and (plan.grid_y, plan.grid_z) == (plan.split_k, plan.m_blocks), what
             else:
                 assert plan.kernel == _lib.KERNEL_PANEL and plan.split_k * plan.k_chunk >= blocks > (plan.split_k - 1) * plan.k_chunk, what
+
+
+def test_calls_without_a_plan_that_the_panel_kernel_could_take_accept_the_workspace_of_the_route():
+    """gptq_hip_select_route may answer with a plan of fewer bytes than the PANEL plan that the models replaced and than gptq_hip_select_tiled's: a call that
+    names no plan and brings them runs it."""
+    import random
+
+    rng, fewer = random.Random(12), 0
+    panel = _lib.COPY_TILED | _lib.COPY_TILED_PANEL
+    shapes = [(66, 15264, 960, 3, 32, False)]
+    for _ in range(3000):
+        gs = rng.choice((128, 64, 32, -1))
+        unit = 32 if gs == -1 else gs
+        shapes.append((rng.randint(9, 340), unit * max(1, int(2 ** rng.uniform(8, 14.4)) // unit), 32 * max(1, int(2 ** rng.uniform(8, 15)) // 32),
+                       rng.choice((2, 3, 4, 8)), gs, rng.random() < 0.5))
+    for M, K, N, bits, gs, act in shapes:
+        own = _lib.select_panel(M, K, N, bits, gs, act)
+        if own is None:
+            continue
+        r, old = _lib.select_route(M, K, N, bits, gs, act, panel).plan, _lib.select_tiled(M, K, N, bits, gs)
+        fewer += r.workspace_bytes < min(own.workspace_bytes, old.workspace_bytes)
+        plan, _ = default_plan(M, K, N, bits, gs, act, r.workspace_bytes)
+        assert plan.as_dict() == r.as_dict() or r.kernel == _lib.KERNEL_TILED_DECODE, (M, K, N, bits, gs, act, r.as_dict(), plan.as_dict())
+    assert fewer > 20
