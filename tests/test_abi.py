@@ -785,3 +785,20 @@ def test_calls_without_a_plan_that_the_panel_kernel_could_take_accept_the_worksp
         plan, _ = default_plan(M, K, N, bits, gs, act, r.workspace_bytes)
         assert plan.as_dict() == r.as_dict() or r.kernel == _lib.KERNEL_TILED_DECODE, (M, K, N, bits, gs, act, r.as_dict(), plan.as_dict())
     assert fewer > 20
+
+
+def test_short_calls_stay_within_eight_ranges():
+    """The pass that adds K ranges up requests eight at most together.  Measured with nine to twelve (us, graph, those / the plan now): 13 rows of
+    12864 x 1248 int4 11.3 / 9.7, 65 of 11584 x 96 10.0 / 8.3, 147 of 19648 x 320 int8 30.6 / 24.5."""
+    import random
+
+    rng = random.Random(14)
+    panel = _lib.COPY_TILED | _lib.COPY_TILED_PANEL
+    shapes = [(13, 12864, 1248, 4, 64, False), (65, 11584, 96, 4, -1, False), (147, 19648, 320, 8, -1, False), (9, 9216, 64, 4, 128, False)]
+    for _ in range(2000):
+        shapes.append((rng.randint(9, 340), 128 * rng.randint(16, 160), 32 * max(1, int(2 ** rng.uniform(5, 13)) // 32), rng.choice((2, 3, 4, 8)), 128,
+                       rng.random() < 0.3))
+    for M, K, N, bits, gs, act in shapes:
+        r = _lib.select_route(M, K, N, bits, gs, act, panel).plan
+        rules = (_lib.select_tiled(M, K, N, bits, gs).as_dict(), (_lib.select_panel(M, K, N, bits, gs, act) or _lib.Plan()).as_dict())
+        assert r.kernel == _lib.KERNEL_TILED_DECODE or r.split_k <= 8 or r.as_dict() in rules, (M, K, N, bits, act, r.as_dict())
