@@ -1149,12 +1149,17 @@ bool matmul_plan(int M, int K, int N, int bits, int group_size, int at, int spli
 // 5248 x 4576 20.8 -> 16.0, 86 of 8064 x 4384 29.4 -> 22.1, 199 of 1664 x 1216 11.3 -> 10.0).  With an activation order the pack pass is most of what a call
 // of up to 32 rows could lose or gain, and the mean of those was level (0.5 % at 17 to 32 rows, none below): they stay.  So do plans with whole row
 // blocks ahead of their ranges; calls past 320 rows and the gradient were not measured.
+// Outside of the sizes that were fitted, calls drawn and measured where the plan moves (graph): K or N below 1024 120 calls 1.23 x on the mean, one of them
+// slower by more than 2 % (3.2); K past 20480 or N past 32768 140 calls 1.12 x.  There 13 PANEL plans of 3-bit layers for which the models name blocks of 64 or
+// 128 rows were 0.98 x as fast (63 rows of 55616 x 4736 72.6 -> 92.8, 44 of 4288 x 47936 49.6 -> 53.8; two of the other widths 1.23 x): those stay.
+// Four of the others are slower by more than 2 % (38 rows of 1920 x 69056 int2 with an order 32.4 -> 40.6, 11 of 63488 x 3904 42.4 -> 45.3).
 void gptq::refine_short_plan(int M, int K, int N, int bits, int group_size, bool act, gptq_hip_plan *plan)
 {
     if (M <= (act ? 32 : kDecodeMaxRows) || M > kShortPlanRows) return;
     const bool panel = plan->kernel == GPTQ_HIP_KERNEL_PANEL;
     if ((!panel && plan->kernel != GPTQ_HIP_KERNEL_TILED) || (panel && panel_main_blocks(*plan) != 0)) return;
     const int S_total = ceil_div(K, 64), panel_cols = ceil_div(N, kPanelCols);
+    const bool beyond = bits == 3 && (K > 20480 || N > 32768);
     double best = 0.93 * (panel ? panel_call_us(plan->row_tiles, plan->split_k, plan->k_chunk, (long long)plan->grid_x * plan->m_blocks * plan->split_k,
                                                 M, K, N, bits, act)
                                 : matmul_us(*plan, M, K, N, bits, act));
@@ -1164,7 +1169,7 @@ void gptq::refine_short_plan(int M, int K, int N, int bits, int group_size, bool
     const long long cap = (3LL * K * bits) / (128LL * M);
     for (int at = 1; at <= 4; at *= 2) {
         const long long tiles = (long long)ceil_div(N / 32, 2) * ceil_div(M, 32 * at);
-        if ((at > 1 && 16 * at >= M) || tiles > 1100) continue;
+        if ((at > 1 && (16 * at >= M || (panel && beyond))) || tiles > 1100) continue;
         // (at most the eight ranges that their pass requests together, which the model does not know: on 167 drawn calls that nine to twelve were named for, one
         // row block 0.94 x the rules' plans, 1.04 now, several row blocks 1.23 and 1.32; 13 rows of 12864 x 1248 int4 11.3 and 9.7 us, 17 of
         // 11648 x 1216 11.6 and 10.1)

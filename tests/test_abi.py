@@ -802,3 +802,13 @@ def test_short_calls_stay_within_eight_ranges():
         r = _lib.select_route(M, K, N, bits, gs, act, panel).plan
         rules = (_lib.select_tiled(M, K, N, bits, gs).as_dict(), (_lib.select_panel(M, K, N, bits, gs, act) or _lib.Plan()).as_dict())
         assert r.kernel == _lib.KERNEL_TILED_DECODE or r.split_k <= 8 or r.as_dict() in rules, (M, K, N, bits, act, r.as_dict())
+
+
+def test_panel_plans_of_larger_layers_keep_their_row_blocks():
+    """Past 20480 channels or 32768 columns, which the models were not fitted on, a PANEL plan of 3 bits gives way to blocks of 32 rows only.  Measured (us, graph,
+    the matmul kernel in blocks of 64 / PANEL): 92.8 / 72.6, 53.8 / 49.6, 71.8 / 69.1, 53.5 / 51.5."""
+    panel = _lib.COPY_TILED | _lib.COPY_TILED_PANEL
+    for M, K, N, bits, gs in ((63, 55616, 4736, 3, 64), (44, 4288, 47936, 3, 32), (46, 6880, 44544, 3, -1), (50, 4800, 40640, 3, -1)):
+        own = _lib.select_panel(M, K, N, bits, gs, False)
+        r = _lib.select_route(M, K, N, bits, gs, False, panel).plan
+        assert own is not None and (r.kernel, r.row_tiles) in ((_lib.KERNEL_PANEL, own.row_tiles), (_lib.KERNEL_TILED, 1)), (M, K, N, r.as_dict())
