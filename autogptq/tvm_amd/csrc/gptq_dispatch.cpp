@@ -999,6 +999,10 @@ double panel_t_us(int rt, int split, int chunk, long long wgs, int M, int K, int
 // since it moves 16, none to a slower plan, 1.25 x as fast on the mean with the pass for the gradient's rows gone in both where it is gone (us, graph:
 // 68 rows of 1344 x 11008 int4, four row tiles in 11 ranges 23.1, one in four 17.4; 86 of 5248 x 1088 15.0 -> 11.1; to PANEL, all with an
 // activation order: 296 of 5376 x 2144 31.7 -> 21.2, 208 of 6912 x 1728 27.1 -> 19.3, 86 of 11328 x 3136 int4 1.09 x).
+// Below 1024 channels or columns, which the fit had not met, calls drawn and measured where the plan moves: K 60 calls 1.31 x on the mean, one slower by more than
+// 2 %; N 94 calls 1.31 x, of which matmul plans of more than two workgroups a CU were the slowest (71 rows of 13568 x 192 int8 14.8 -> 19.1, 137 of 7360 x
+// 320 19.3 -> 23.9, 70 of 14720 x 512 int4 17.7 -> 19.0): they are not named there (81 of 13440 x 128 int3 16.6, 16.8 then, 10.8 now).  Five of the rest
+// are slower by 3 to 10 % (42 of 13056 x 288 on PANEL 6.4 -> 7.1).
 bool short_gradient(int M, int K, int N) { return M >= 32 && M < 384 && K <= 20480 && N <= 32768; }
 void refine_short_gradient(int M, int K, int N, int bits, int group_size, bool act, bool panels, gptq_hip_plan *plan)
 {
@@ -1012,7 +1016,7 @@ void refine_short_gradient(int M, int K, int N, int bits, int group_size, bool a
     const long long cap = (3LL * N * bits) / (128LL * M);
     for (int at = 1; at <= 4; at *= 2) {
         const long long tiles = (long long)ceil_div(K / 32, 2) * ceil_div(M, 32 * at);
-        if (at > 1 && 16 * at >= M) continue;
+        if ((at > 1 && 16 * at >= M) || (N < 1024 && tiles > 2 * gptq::kNumCUs)) continue;
         for (int s = 1; s <= 8; s++) {
             if (s > 1 && (s > cap || tiles * s > 520 || S_total / (4 * s) < 2)) break;
             matmul_t_plan(M, K, N, bits, at, s, &other);
