@@ -564,10 +564,13 @@ __global__ __launch_bounds__(64 * KW) void tiled_decode_kernel(const _Float16 *a
 //   four rows, workgroups of eight waves: one (2048 x 4096 3.34 / 3.56, with an activation order 3.46 / 3.72, 4096 x 4096 3.94 / 4.18 and 4.33 /
 //   4.67, 8192 x 10240 with an order 10.5 / 11.2, 11008 x 11008 16.8 / 17.2), but two without an order where there are more than two workgroups a CU (8192 x
 //   28672 22.4 / 22.3, int3 19.7 / 19.3, 6272 x 21152 int2 13.7 / 13.4);
+//   four rows, workgroups of sixteen: one (110 drawn calls of 8448 to 28672 channels 1.02 x as fast on the mean, two of them slower by 1 %: with an order
+//   14336 x 5120 11.9 / 12.6, 28672 x 8192 29.0 / 30.7, 10624 x 4928 int2 9.3 / 9.9; without one 13824 x 5120 10.8 / 11.1, 11008 x 8192 level at 11.1);
 //   four and eight rows (eight without an activation order, below 8 bits), workgroups of four: one where it holds them all (1024 x 11008 3.62 / 3.87 and, eight rows,
 //   4.24 / 4.73, 2048 x 11008 4.23 / 4.36 and 5.00 / 5.39), else two (four rows of 4096 x 11008 6.21 / 5.92, 2560 x 14336 5.74 / 5.47, eight of
 //   2560 x 14336 6.70 / 6.63), but one again for four rows with an activation order that nearly fill both, whose walk over all of x the
-//   workgroups of a CU hide from each other (4096 x 11008 6.48 / 6.98, 4096 x 14336 7.70 / 8.01; 3328 x 12960 8.29 / 8.15, 2560 x 14336 6.55 / 6.32);
+//   workgroups of a CU hide from each other (4096 x 11008 6.48 / 6.98, 4096 x 14336 7.70 / 8.01; 2560 x 14336 6.55 / 6.32; the line, in steps of 128
+//   channels: 3456 x 14336 8.28 / 8.08, 3584 x 14336 8.39 / 8.22 and x 11008 6.94 / 6.90, 3712 x 14336 8.50 / 8.95 and x 11008 6.86 / 7.34);
 //   eight rows otherwise, and sixteen: one (4096 x 4096 4.7 / 5.1, 8192 x 28672 with an order 35.1 / 44).
 constexpr int decode_passes(int mr, int kw) { return mr >= 8 || (mr == 4 && kw > 4) ? 1 : 2; }
 static bool decode_second_pass(int mr, int kw, bool mapped, int K, int channels, int workgroups)

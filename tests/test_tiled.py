@@ -920,3 +920,19 @@ def test_tiled_decode_passes_over_x(dev, bits, K, N, desc_act):
         plan = _lib.select_tiled(M, K, N, bits, 32)
         assert plan.kernel == _lib.KERNEL_TILED_DECODE and plan.waves_k == (4 if K < 4128 else 8)
         assert_tight(run_tiled(D, prep, x=L["x"][:M].contiguous().to(dev), plan=plan), want[:M], f"int{bits} {K}x{N} M={M}")
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("K", [8224, 9216, 16416])
+@pytest.mark.parametrize("desc_act", [False, True])
+def test_tiled_decode_passes_over_x_of_sixteen_waves(dev, bits, K, desc_act):
+    """Three and four rows in workgroups of sixteen waves: one pass over x ahead of the weights, four octets, 128 and a whole pass and more left to the loop."""
+    N = 4128
+    L = layer(5700 + K, K, N, bits, 32, desc_act, M=4, bias=True)
+    D = to_dev(L, dev)
+    # (8 bits: weights rounded as the reference's; below, sums of codes are scaled, without that rounding, which is past the tight bound at this length)
+    prep, want = prepare(D), expected_output(L) if bits == 8 else unrounded_output(L, L["x"])
+    for M in (3, 4):
+        plan = _lib.select_tiled(M, K, N, bits, 32)
+        assert plan.kernel == _lib.KERNEL_TILED_DECODE and plan.waves_k == 16
+        assert_tight(run_tiled(D, prep, x=L["x"][:M].contiguous().to(dev), plan=plan), want[:M], f"int{bits} {K}x{N} M={M}")
