@@ -967,6 +967,39 @@ static int plan_panel(int M, int K, int N, int bits, int group_size, unsigned fl
 
 namespace {
 
+// What the models of the short calls chose last, by thread: a choice is a search over 30 to 90 plans (0.3 to 1.4 us), made for every call that names no plan and for
+// every gradient of a module, and depends on nothing but the numbers in its key (forward the plan by the rules among them, which a caller's workspace decides).
+struct Choice {
+    struct Key {
+        int kind, M, K, N, bits, group_size, act;   // kind 1: forward, 2: gradient, 3: gradient on the matmul kernel alone; 0: none yet
+        gptq_hip_plan rules;
+    } key;
+    gptq_hip_plan plan;
+};
+
+template <typename Search>
+void choose_once(int kind, int M, int K, int N, int bits, int group_size, bool act, gptq_hip_plan *plan, Search search)
+{
+    static thread_local Choice kept[64];
+    Choice::Key key;
+    memset(&key, 0, sizeof(key));
+    key.kind = kind, key.M = M, key.K = K, key.N = N, key.bits = bits, key.group_size = group_size, key.act = act;
+    memcpy(&key.rules, plan, sizeof(*plan));
+    const uint32_t mix = ((uint32_t)M * 0x9e3779b1u) ^ ((uint32_t)K * 0x85ebca6bu) ^ ((uint32_t)N * 0xc2b2ae35u) ^ ((uint32_t)(8 * bits + kind) * 0x27d4eb2fu);
+    Choice &c = kept[mix >> 26];
+    if (memcmp(&c.key, &key, sizeof(key)) != 0) {
+        search();
+        c.key = key;
+        c.plan = *plan;
+    } else {
+        *plan = c.plan;
+    }
+}
+
+}  // namespace
+
+namespace {
+
 // ---- Gradients of 32 to 383 rows of layers within 20480 x 32768: matmul or PANEL plan by two models of both kernels, fitted to 8000 measurements
 // (graph, weights cold) of every row tile and range of 210 calls drawn at random (32 to 600 rows, all widths, with and without an activation order;
 // 6.4 and 5.5 % rms near the best plan).  From 384 rows on a module whose gradient has no PANEL plan takes the library's product: the choice stays. ----
@@ -1044,20 +1077,32 @@ void refine_short_gradient(int M, int K, int N, int bits, int group_size, bool a
 extern "C" int gptq_hip_select_panel(int M, int K, int N, int bits, int group_size, unsigned flags, int row_tiles, int split_k,
                                      gptq_hip_plan *plan)
 {
-    int rc = plan_panel(M, K, N, bits, group_size, flags, row_tiles, split_k, true, plan);
-    if ((rc == GPTQ_HIP_OK || rc == GPTQ_HIP_ERR_UNSUPPORTED) && row_tiles == 0 && split_k == 0 && (flags & GPTQ_HIP_PANEL_TRANSPOSED) &&
-        short_gradient(M, K, N) && (rc == GPTQ_HIP_OK || plan_tiled_transposed(M, K, N, bits, group_size, plan) == GPTQ_HIP_OK)) {
-        refine_short_gradient(M, K, N, bits, group_size, flags & GPTQ_HIP_PANEL_ACT_ORDER, true, plan);
-        rc = plan->kernel == GPTQ_HIP_KERNEL_PANEL ? GPTQ_HIP_OK : GPTQ_HIP_ERR_UNSUPPORTED;
-    }
-    return rc;
+    const bool act = flags & GPTQ_HIP_PANEL_ACT_ORDER;
+    if (row_tiles != 0 || split_k != 0 || (flags & ~(unsigned)GPTQ_HIP_PANEL_ACT_ORDER) != GPTQ_HIP_PANEL_TRANSPOSED || !short_gradient(M, K, N))
+        return plan_panel(M, K, N, bits, group_size, flags, row_tiles, split_k, true, plan);
+    const int ok = tiled_args_ok(M, K, N, bits, group_size, plan);
+    if (ok != GPTQ_HIP_OK) return ok;
+    choose_once(2, M, K, N, bits, group_size, act, plan, [&] {
+        if (plan_panel(M, K, N, bits, group_size, flags, 0, 0, true, plan) == GPTQ_HIP_OK || plan_tiled_transposed(M, K, N, bits, group_size, plan) == GPTQ_HIP_OK)
+            refine_short_gradient(M, K, N, bits, group_size, act, true, plan);
+        else
+            plan->kernel = 0;
+    });
+    return plan->kernel == GPTQ_HIP_KERNEL_PANEL ? GPTQ_HIP_OK : GPTQ_HIP_ERR_UNSUPPORTED;
 }
 
 extern "C" int gptq_hip_select_tiled_transposed(int M, int K, int N, int bits, int group_size, gptq_hip_plan *plan)
 {
-    const int rc = plan_tiled_transposed(M, K, N, bits, group_size, plan);
-    if (rc == GPTQ_HIP_OK) refine_short_gradient(M, K, N, bits, group_size, false, false, plan);
-    return rc;
+    if (!short_gradient(M, K, N)) return plan_tiled_transposed(M, K, N, bits, group_size, plan);
+    const int ok = tiled_args_ok(M, K, N, bits, group_size, plan);
+    if (ok != GPTQ_HIP_OK) return ok;
+    choose_once(3, M, K, N, bits, group_size, false, plan, [&] {
+        if (plan_tiled_transposed(M, K, N, bits, group_size, plan) == GPTQ_HIP_OK)
+            refine_short_gradient(M, K, N, bits, group_size, false, false, plan);
+        else
+            plan->kernel = 0;
+    });
+    return plan->kernel == GPTQ_HIP_KERNEL_TILED ? GPTQ_HIP_OK : GPTQ_HIP_ERR_UNSUPPORTED;
 }
 
 // The plan of a gradient that names none and brings `have` bytes of workspace: the one that the two entries above name, else what the rules
@@ -1157,12 +1202,10 @@ bool matmul_plan(int M, int K, int N, int bits, int group_size, int at, int spli
 // slower by more than 2 % (3.2); K past 20480 or N past 32768 140 calls 1.12 x.  There 13 PANEL plans of 3-bit layers for which the models name blocks of 64 or
 // 128 rows were 0.98 x as fast (63 rows of 55616 x 4736 72.6 -> 92.8, 44 of 4288 x 47936 49.6 -> 53.8; two of the other widths 1.23 x): those stay.
 // Four of the others are slower by more than 2 % (38 rows of 1920 x 69056 int2 with an order 32.4 -> 40.6, 11 of 63488 x 3904 42.4 -> 45.3).
-void gptq::refine_short_plan(int M, int K, int N, int bits, int group_size, bool act, gptq_hip_plan *plan)
+static void search_short_plan(int M, int K, int N, int bits, int group_size, bool act, gptq_hip_plan *plan)
 {
-    if (M <= (act ? 32 : kDecodeMaxRows) || M > kShortPlanRows) return;
     const bool panel = plan->kernel == GPTQ_HIP_KERNEL_PANEL;
-    if ((!panel && plan->kernel != GPTQ_HIP_KERNEL_TILED) || (panel && panel_main_blocks(*plan) != 0)) return;
-    const int S_total = ceil_div(K, 64), panel_cols = ceil_div(N, kPanelCols);
+    const int S_total = ceil_div(K, 64), panel_cols = ceil_div(N, gptq::kPanelCols);
     const bool beyond = bits == 3 && (K > 20480 || N > 32768);
     double best = 0.93 * (panel ? panel_call_us(plan->row_tiles, plan->split_k, plan->k_chunk, (long long)plan->grid_x * plan->m_blocks * plan->split_k,
                                                 M, K, N, bits, act)
@@ -1184,7 +1227,7 @@ void gptq::refine_short_plan(int M, int K, int N, int bits, int group_size, bool
             if (us < best) best = us, found = other, better = true;
         }
     }
-    for (int rt = 1; rt <= kPanelMaxTiles && (rt == 1 || 32 * (rt - 1) < M); rt++) {
+    for (int rt = 1; rt <= gptq::kPanelMaxTiles && (rt == 1 || 32 * (rt - 1) < M); rt++) {
         const long long tiles = (long long)panel_cols * ceil_div(M, 32 * rt);
         if (tiles > 1100) continue;
         for (int s = 1; s <= 8; s++) {
@@ -1197,6 +1240,13 @@ void gptq::refine_short_plan(int M, int K, int N, int bits, int group_size, bool
         }
     }
     if (better) *plan = found;
+}
+void gptq::refine_short_plan(int M, int K, int N, int bits, int group_size, bool act, gptq_hip_plan *plan)
+{
+    if (M <= (act ? 32 : kDecodeMaxRows) || M > kShortPlanRows) return;
+    const bool panel = plan->kernel == GPTQ_HIP_KERNEL_PANEL;
+    if ((!panel && plan->kernel != GPTQ_HIP_KERNEL_TILED) || (panel && panel_main_blocks(*plan) != 0)) return;
+    choose_once(1, M, K, N, bits, group_size, act, plan, [&] { search_short_plan(M, K, N, bits, group_size, act, plan); });
 }
 
 namespace {

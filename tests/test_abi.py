@@ -820,3 +820,32 @@ def test_short_gradients_of_narrow_layers_stay_within_two_workgroups_a_cu():
     for M, K, N, bits, gs, act in ((71, 13568, 192, 8, 128, True), (137, 7360, 320, 8, 64, True), (70, 14720, 512, 4, 64, True)):
         p = _lib.select_panel(M, K, N, bits, gs, act, transposed=True) or _lib.select_tiled_transposed(M, K, N, bits, gs)
         assert p.kernel == _lib.KERNEL_PANEL or p.grid_x * p.grid_y * p.grid_z <= 512, (M, K, N, p.as_dict())
+
+
+def test_plans_of_short_calls_are_the_same_whoever_asks_and_however_often():
+    """What the models chose is kept by thread for a few calls: more sizes than are kept, in two orders, from two threads, with and without the workspace for it."""
+    import random
+    import threading
+
+    rng = random.Random(15)
+    shapes = [(rng.choice((9, 33, 64, 100, 200, 320, 383)), 128 * rng.randint(2, 160), 32 * rng.randint(2, 600), rng.choice((2, 3, 4, 8)), 128, rng.random() < 0.5)
+              for _ in range(300)]
+    # (sizes that differ in one number only)
+    shapes += [(M, 4096, 1792, bits, 128, act) for M in range(60, 70) for bits in (3, 4) for act in (False, True)]
+    panel = _lib.COPY_TILED | _lib.COPY_TILED_PANEL
+
+    def ask(M, K, N, bits, gs, act):
+        p = _lib.select_panel(M, K, N, bits, gs, act, transposed=True)
+        r = _lib.select_route(M, K, N, bits, gs, act, panel).plan
+        return [p and p.as_dict(), _lib.select_tiled_transposed(M, K, N, bits, gs).as_dict(), r.as_dict(),
+                default_plan(M, K, N, bits, gs, act, 1 << 40)[0].as_dict(), default_plan(M, K, N, bits, gs, act, 1 << 20)[0].as_dict()]
+
+    want, got = [ask(*s) for s in shapes], {}
+    assert [ask(*s) for s in reversed(shapes)] == want[::-1]
+    assert [a for s in shapes for a in (ask(*s), ask(*s))] == [a for w in want for a in (w, w)]
+    threads = [threading.Thread(target=lambda k=k: got.update({k: [ask(*s) for s in shapes]})) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert got[0] == want and got[1] == want
