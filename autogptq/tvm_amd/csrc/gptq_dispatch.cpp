@@ -604,11 +604,12 @@ bool gptq::select_row_blocks(int M, int K, int N, int bits, int group_size, gptq
 }
 
 // Nine to sixteen rows that the matmul kernel reads itself, in ranges that cover K exactly, are its own again on long layers, whose K it cuts over CUs that
-// row blocks leave idle; with fewer bits or columns sooner (us at 9 / 16 rows, matmul / row blocks: 9216 x 64 int4 6.7 / 9.9 and 7.6 / 10.0,
-// 9216 x 2048 8.3 / 10.4 and 9.2 / 10.5, int3 7.5 / 10.7 and 8.1 / 10.8, 9216 x 4096 int4 10.4 / 10.9 and 11.6 / 10.8, int3 9.4 / 11.1 and
-// 10.7 / 11.2; 7680 x 2048 int4 8.3 / 9.0 and 9.0 / 9.0; 7168 x 2048 int4 8.7 / 8.5 and 9.9 / 8.5, int3 8.0 / 9.0 and 8.6 / 9.0; 8 bits 9216 x 64 7.0 /
-// 9.9, 9216 x 2048 9.9 / 10.5 and 10.8 / 10.6, 7680 x 1024 9.3 / 9.1 and 10.0 / 9.1; with a pack pass row blocks are level or ahead: 8704 x 2048 11.3 /
-// 10.1, 9216 x 512 with an activation order 10.7 / 10.7).
+// row blocks leave idle; with fewer bits or columns sooner (us at 9 / 16 rows, graph, matmul / row blocks: 9216 x 64 int4 7.2 / 10.1 and 7.4 / 10.2,
+// 9216 x 512 8.0 / 10.2 and 8.4 / 10.4, 9216 x 2048 8.8 / 10.8 and 9.3 / 10.7, int3 8.3 / 11.0 and 8.5 / 11.0, 9216 x 4096 int4 10.9 / 11.5 and 11.5 / 10.9, int3 10.1 /
+// 11.3 and 10.9 / 11.3; 7680 x 2048 int4 8.3 / 9.0 and 9.0 / 9.3; 7168 x 2048 int3 7.5 / 9.2 and 7.4 / 9.1; 8 bits 9216 x 64 8.3 / 10.3 and 8.4 / 10.3, 9216 x
+// 2048 10.5 / 11.0 and 10.6 / 10.9, 7680 x 1024 level; with a pack pass row blocks are level or ahead: 9216 x 512 with an activation order 10.7 / 10.7).
+// Drawn with a pass in these calls, the line leaves some to the row blocks that the matmul kernel is ahead on since it stages x: 7168 x 2048 int4
+// 8.3 / 8.9 and 8.4 / 8.8, 8704 x 2048, whose ranges do not cover K exactly, 8.9 / 10.4.
 static bool matmul_keeps(int M, int K, int N, int bits, int group_size, bool mapped)
 {
     gptq_hip_plan plan;
