@@ -245,6 +245,8 @@ class QuantLinear(nn.Module):
             if plan is not None or not past:
                 t = self.prepare_transposed()
                 if t is not None:
+                    if plan is None:   # (named here, so that it is not asked for again below)
+                        plan = _lib.select_tiled_transposed(M, K, N, bits, gs)
                     gx = ops.gemm_tiled_transposed(gy, t[0], t[1], t[2], K, bits, gs, plan=plan)
         if gx is None:
             if self._compact:

@@ -275,3 +275,21 @@ def test_transposed_rows_of_the_gradient_without_the_pack_pass(dev, bits, M, K, 
         assert_close(got, want, what)
         assert_tight(got, want, what)
         assert torch.equal(got, run_t(D, prep, room[1:-1], plan=plan)), "two identical calls differ"
+
+
+@pytest.mark.parametrize("M,K,N", [(38, 2176, 1408), (300, 4096, 1088), (16, 256, 96)])
+def test_a_gradient_asks_for_its_plan_once(dev, monkeypatch, M, K, N):
+    L = layer(3900 + M, K, N, 4, 32, False)
+    D = to_dev(L, dev)
+    q = QuantLinear(4, 32, K, N, False)
+    q.load_state_dict({k: D[k] for k in ("qweight", "qzeros", "scales", "g_idx")})
+    q = q.to(dev)
+    gy = grad_rows(3901, M, N)
+    want = q.grad_input(gy.to(dev))
+    asked = []
+    for name in ("select_panel", "select_tiled_transposed"):
+        entry = getattr(_lib, name)
+        monkeypatch.setattr(_lib, name, lambda *a, entry=entry, name=name, **k: asked.append(name) or entry(*a, **k))
+    assert torch.equal(q.grad_input(gy.to(dev)), want)
+    assert asked.count("select_panel") == 1 and asked.count("select_tiled_transposed") <= 1
+    assert_tight(want, gy.float() @ expected_weight(L).float().t(), f"{M} rows")
