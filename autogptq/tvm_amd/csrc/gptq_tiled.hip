@@ -395,6 +395,13 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
 #pragma unroll
         for (int rt = 0; rt < AT; rt++) fr[rt] = *(const h8 *)(x_lds + (buf * AT + rt) * 4096 + n * 128 + (((4 * h + j) ^ (n & 7)) * 16));
     };
+    // LDS serves the accesses of one wave in order, but a lane writes what others read: the fences keep the compiler from moving the reads
+    // above the writes, or the next block's writes above the reads, where it sees that a lane's own addresses differ
+    auto hand_over = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    };
     auto load_a = [&](int S, int j, h8 (&ar)[AT]) {
         if constexpr (STAGED) {
             const __amdgpu_buffer_rsrc_t xb = tile_buffer((const char *)x_base, S <= S_last ? x_bytes : 0u);
@@ -454,6 +461,7 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
             write_a(0, j, a[0][j]);
             load_a(S, j, a[0][j]);
         }
+        hand_over();
         read_a(0, 0, fr[0]);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -565,6 +573,7 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
 #pragma unroll
                             for (int s = 2; s < RING; s++) load_a(S_of[s], j, a[s][j]);
                         }
+                        if (j == 0) hand_over();   // (the last block's fragments are read)
                         if (j < 2) {
 #pragma unroll
                             for (int i = 2 * j; i < 2 * j + 2; i++) {
@@ -572,6 +581,7 @@ __global__ __launch_bounds__(64 * RW * KW) void tiled_gemm_kernel(const char *a_
                                 if (REFILL) load_a(S_x, i, a[un][i]);
                             }
                         }
+                        if (j == 1) hand_over();
                         if (REFILL && j == 3) {
                             load_b(S_refill, w[u], szr[u]);
                             S_of[u] = S_refill;

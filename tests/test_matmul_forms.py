@@ -102,3 +102,33 @@ def test_infinite_weights_of_the_last_column(dev, bits, N):
             for packed in (False, True) if rt < 4 else (True,):
                 gx = transposed(D, gy[:rows].to(dev), xsrc, transposed_plan(rows, K, N, bits, gs, rt, split, packed))
                 assert_same_specials(gx, want[:rows], f"int{bits} N={N} act={desc_act} rows {rows} tiles {rt} ranges {split} packed {packed}")
+
+
+# Up to 13 rows of a layer whose ranges cover K exactly x is read lane by lane, from 14 on and elsewhere through LDS, with a channels' map packed first:
+# the same fragments and the same order of the sums, so the same bits
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("K,N,gs,split", [(256, 32, 32, 1), (768, 96, 64, 3), (1024, 416, 128, 2), (2048, 160, -1, 1), (4096, 96, 128, 8), (1056, 96, 32, 1)])
+def test_rows_read_in_every_way_give_the_same_bits(dev, bits, K, N, gs, split):
+    D = to_dev(layer(9300 + K, K, N, bits, gs, False, M=16), dev)
+    tiles = prepared(D)
+    want = D["x"].float().cpu() @ expected_weight({k: v.cpu() if torch.is_tensor(v) else v for k, v in D.items()}).float()
+    for M in (1, 9, 12, 13, 14, 16):
+        plan = forward_plan(M, K, N, bits, gs, 1, split)
+        y, packed = forward(D, tiles, plan, x=D["x"][:M]), forward(D, tiles, plan, True, x=D["x"][:M])
+        assert torch.equal(y, packed), f"int{bits} K={K} rows {M}"
+        assert_tight(y, want[:M], f"int{bits} K={K} rows {M}")
+
+
+# the gradient's rows through LDS and packed: the same bits
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("M,K,N,row_tiles,split", [(1, 64, 32, 1, 1), (31, 96, 352, 1, 1), (33, 160, 96, 1, 2), (64, 352, 1056, 2, 1), (65, 96, 2016, 2, 3),
+                                                   (40, 320, 4096, 1, 4)])
+def test_gradient_rows_in_both_ways_give_the_same_bits(dev, bits, M, K, N, row_tiles, split):
+    gy = torch.randn(M, N, generator=torch.Generator().manual_seed(M)).half().to(dev)
+    for desc_act in (False, True):
+        D = to_dev(layer(9400 + N, K, N, bits, 32, desc_act), dev)
+        xsrc = prepared(D)[2] if desc_act else None
+        staged, packed = (transposed(D, gy, xsrc, transposed_plan(M, K, N, bits, 32, row_tiles, split, packed=p)) for p in (False, True))
+        assert torch.equal(staged, packed), f"int{bits} act={desc_act}"
