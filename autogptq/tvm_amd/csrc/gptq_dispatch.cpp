@@ -806,6 +806,10 @@ static void matmul_t_plan(int M, int K, int N, int bits, int at, int split, gptq
     plan->grid_x = ceil_div(K / 32, 2);
     plan->block = 64 * kwv;
     plan->lds_bytes = gptq::tiled_t_lds_bytes(at, kwv, plan->k_chunk);
+    if (gptq::tiled_t_stages_x(N, *plan)) {   // (what the launch takes; smaller plans from elsewhere are taken as they are)
+        const int staged = gptq::tiled_t_staged_lds_bytes(at, kwv, plan->k_chunk);
+        if (staged > plan->lds_bytes) plan->lds_bytes = staged;
+    }
     plan->flags = 0;
     size_t ws = gptq::kCounterBytes;
     if (plan->split_k > 1) ws += ((size_t)plan->split_k * M * K * sizeof(float) + 255) / 256 * 256;
