@@ -13,13 +13,14 @@
 //     no shuffle;
 //   * sz[g][n] = (fp16 scale, fp16 zero point) of group g, column n, one 32-bit word.
 //
-// (The decode kernels for up to four rows of x are in gptq_tiled_decode.hip and gptq_tiled_decode16.hip.)
+// (The decode kernels, for up to eight rows of x and small batches in blocks of 8 or 16, are in gptq_tiled_decode.hip and gptq_tiled_decode16.hip.)
 //
 // tiled_gemm_kernel: a workgroup owns 64 columns (two tiles), 32 * AT rows of x and one K range; its four
 // waves (one per SIMD) split that range and never talk until the end.  A wave holds its whole 32 AT x 64
 // result in registers (AT = 4: 128 rows, 128 accumulator registers), dequantises every weight of its slice
-// exactly once, as the reference does (fp16(scale * (q - zero)), one rounding), and reads x as ready-made A
-// fragments that a small pack pass wrote (rows past M and positions past K as zeros).  One wave per SIMD
+// exactly once, as the reference does (fp16(scale * (q - zero)), one rounding), and multiplies it with A fragments of x (rows past M and
+// positions past K as zeros), which it comes by in one of three ways (XMode): ready-made, from a small pack pass before it (layers with an activation order and
+// plans of 128 columns per wave), or from the rows of x themselves, lane by lane or through LDS (layers without one; the gradient's rows).  One wave per SIMD
 // overlaps its own vector and matrix instructions (measured: up to six packed-fp16 instructions per
 // 32x32x16 matrix instruction are free), so the dequantisation of the next B operand is interleaved with the
 // matrix instructions of the current one.  Weights, (scale, zero) words and fragments ride in register
