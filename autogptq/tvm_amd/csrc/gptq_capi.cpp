@@ -440,7 +440,7 @@ extern "C" int gptq_hip_gemm_tiled(const void *x, const void *qtile, const uint3
     if (!workspace || !aligned(workspace, 16) || workspace_bytes < gptq::kCounterBytes + part + xb) return GPTQ_HIP_ERR_WORKSPACE;
     float *partial = (float *)((char *)workspace + gptq::kCounterBytes);
     char *xpack = (char *)workspace + gptq::kCounterBytes + part;
-    return gptq::launch_tiled(x, qtile, sz, xsrc, bias, y, xpack, partial, M, K, N, K / gs, bits, gs, *plan, stream);
+    return gptq::launch_tiled(x, qtile, sz, xsrc, bias, y, xpack, partial, M, K, N, bits, gs, *plan, stream);
 }
 
 extern "C" size_t gptq_hip_tiled_transposed_bytes(int K, int N, int bits)

@@ -353,7 +353,7 @@ int launch_panel(const void *x, const void *qtile, const uint32_t *sz, const int
                  void *stream);
 
 int launch_tiled(const void *x, const void *qtile, const uint32_t *sz, const int32_t *xsrc, const void *bias, void *y,
-                 char *xpack, float *partial, int M, int K, int N, int G, int bits, int group_size,
+                 char *xpack, float *partial, int M, int K, int N, int bits, int group_size,
                  const gptq_hip_plan &plan, void *stream);
 
 }  // namespace gptq

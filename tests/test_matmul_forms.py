@@ -132,3 +132,16 @@ def test_gradient_rows_in_both_ways_give_the_same_bits(dev, bits, M, K, N, row_t
         xsrc = prepared(D)[2] if desc_act else None
         staged, packed = (transposed(D, gy, xsrc, transposed_plan(M, K, N, bits, 32, row_tiles, split, packed=p)) for p in (False, True))
         assert torch.equal(staged, packed), f"int{bits} act={desc_act}"
+
+
+# the group of a lane block: groups of one block, of odd numbers of them, of half and of all of K
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [3, 4])
+@pytest.mark.parametrize("K,gs", [(1920, 32), (1920, 64), (1920, 96), (2080, 160), (4032, 224), (3936, 1312), (2112, 1056), (2016, -1)])
+def test_groups_of_every_number_of_blocks(dev, bits, K, gs):
+    N = 64
+    D = to_dev(layer(9500 + K, K, N, bits, gs, True, M=40), dev)
+    tiles, W = prepared(D), expected_weight({k: v.cpu() if torch.is_tensor(v) else v for k, v in D.items()}).float()
+    for rt, split in ((1, 1), (2, 3)):
+        y = forward(D, tiles, forward_plan(40, K, N, bits, gs, rt, split))
+        assert_tight(y, D["x"].float().cpu() @ W, f"int{bits} K={K} groups of {gs} tiles {rt}")
