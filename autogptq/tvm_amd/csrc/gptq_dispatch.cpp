@@ -1291,6 +1291,11 @@ namespace {
 //     31.4 / 32.0, 64 / 128 / 256 rows 30.2 / 45.9 / 64.3 against 36.2 / 48.4 / 72.6; 12288 x 12288 level at 28); with an activation order also
 //     beyond 20480 channels (28672 x 8192 at 17 / 32 rows, int4 48.4 / 48.4 against 47.9 / 49.0, int3 48.4 / 49.0 against
 //     49.6 / 50.7; 64 rows 61.6 / 65.5 against 64.9 / 67.9);
+//   * (the figures of 9 to 64 rows without an activation order above, and those in the function, hold a pack pass, which these calls of the matmul kernel no
+//     longer have; both sides now, the tiled copy as gptq_hip_select_route runs it / STREAM, at 9 / 16 rows: 11008 x 4096 int4 12.2 / 13.2 and 12.2 /
+//     14.1, int3 11.5 / 14.3 and 11.9 / 16.1; 8192 x 8192 int4 15.5 / 15.4 and 15.9 / 16.7, int3 13.8 / 15.2 and 14.4 / 16.2; 8192 x 6144 15.0 / 14.5 and 15.7 /
+//     15.1; 8192 x 10240 int4 18.4 / 18.3 and 17.6 / 19.8, at 17 / 32 rows 17.7 / 24.3 and 18.8 / 24.4: the lines leave a layer that holds other copies up to
+//     4 us there, and 6 at the last, for a copy less);
 //   * above 128 rows: K up to 8192 (4096 x 11008, 512 rows: 75 against 95; 11008 x 4096: 127 against 81), and up to
 //     256 rows the longer layers named in the function.
 bool tiled_wins(int M, int K, int N, bool act_order, int bits, bool one_group)
