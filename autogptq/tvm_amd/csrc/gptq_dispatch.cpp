@@ -1223,7 +1223,7 @@ static void search_short_plan(int M, int K, int N, int bits, int group_size, boo
         const long long tiles = (long long)ceil_div(N / 32, 2) * ceil_div(M, 32 * at);
         if ((at > 1 && (16 * at >= M || (panel && beyond))) || tiles > 1100) continue;
         // (at most the eight ranges that their pass requests together, which the model does not know: on 167 drawn calls that nine to twelve were named for, one
-        // row block 0.94 x the rules' plans, 1.04 now, several row blocks 1.23 and 1.32; 13 rows of 12864 x 1248 int4 11.3 and 9.7 us, 17 of
+        // row block 0.96 x as fast as the rules' plans, 1.04 now, several row blocks 1.22 and 1.31; 13 rows of 12864 x 1248 int4 11.3 and 9.7 us, 17 of
         // 11648 x 1216 11.6 and 10.1)
         for (int s = 1; s <= 8; s++) {
             if (s > 1 && (s > cap || tiles * s > 520 || S_total / (4 * s) < (at == 1 ? 3 : 2))) break;
